@@ -2267,6 +2267,15 @@ inline int num_cus() {
     return n;
 }
 
+// Workgroups of a persistent launch over `total` tiles, at most `most`: a multiple of 8, which the tile walk needs to keep
+// "position % 8 = XCD", rounded UP while there is room.  (Rounded down, 44 tiles ran on 40 workgroups, four of which then
+// had two tiles: 44 us instead of 22 for 256 x 2 x 5632 x 2048.)  A workgroup without a tile returns at once.
+inline int persistent_grid(int total, int most) {
+    if (total < kXcds) return total;
+    const int up = (total + kXcds - 1) / kXcds * kXcds;
+    return up <= most ? up : most / kXcds * kXcds;
+}
+
 template <int FMT, int EPI, int SCALE>
 int launch_tiled(const GemmArgs& p, hipStream_t st) {
     static std::once_flag once;
@@ -2304,11 +2313,9 @@ int launch_tiled(const GemmArgs& p, hipStream_t st) {
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kRingLds);
         });
         if (ring_err != hipSuccess) return static_cast<int>(ring_err);
-        // persistent: one workgroup per CU (the kernel uses a CU's whole LDS and register file);
-        // a grid that is a multiple of 8 keeps "position % 8 = XCD" true for every tile a workgroup walks
+        // persistent: one workgroup per CU (the kernel uses a CU's whole LDS and register file)
         const int total = p.tiles_m * p.tiles_n;     // grouped: tiles_m is the host-side upper bound of row tiles
-        int grid = total < num_cus() ? total : num_cus();
-        if (grid >= kXcds) grid -= grid % kXcds;
+        const int grid = persistent_grid(total, num_cus());
         if constexpr (EPI == EPI_NONE || EPI == EPI_BIAS || EPI == EPI_SILU_GATE) {
             // the bf16 epilogues on an even number of K-tiles: the kernel on the 16 x 16 x 128 MFMA
             if (!p.mfma32 && (p.K / BK) % 2 == 0) {
@@ -2345,8 +2352,7 @@ int launch_duo(GemmArgs p, hipStream_t st) {
     p.tiles_m = (p.M + DM - 1) / DM;
     p.tiles_n = p.N / out_bn;
     const int total = p.tiles_m * p.tiles_n;
-    int grid = total < 2 * num_cus() ? total : 2 * num_cus();
-    if (grid >= kXcds) grid -= grid % kXcds;
+    const int grid = persistent_grid(total, 2 * num_cus());
     if (p.duo == 2) k_gemm_nt_duo<EPI, false><<<grid, kThreads, kDuoLds, st>>>(p);
     else            k_gemm_nt_duo<EPI, true><<<grid, kThreads, kDuoLds, st>>>(p);
     return launch_status();
@@ -2497,8 +2503,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
             });
             if (ring_err != hipSuccess) return static_cast<int>(ring_err);
             const int total = p.tiles_m * p.tiles_n;
-            int grid = total < num_cus() ? total : num_cus();
-            if (grid >= kXcds) grid -= grid % kXcds;
+            const int grid = persistent_grid(total, num_cus());
             k_gemm_nt_block_ring<<<grid, kBsThreads, kBsLds, st>>>(p);
             return launch_status();
         }
@@ -2740,8 +2745,7 @@ int launch_ring_only(const GemmArgs& p, hipStream_t st) {
     });
     if (err != hipSuccess) return static_cast<int>(err);
     const int total = p.tiles_m * p.tiles_n;
-    int grid = total < num_cus() ? total : num_cus();
-    if (grid >= kXcds) grid -= grid % kXcds;
+    const int grid = persistent_grid(total, num_cus());
     k_gemm_nt_ring<FMT, EPI, SCALE, MX><<<grid, kThreads, kRingLds, st>>>(p);
     return launch_status();
 }
