@@ -1,6 +1,7 @@
 // Scaled FP8 GEMM for gfx950:  C[M,N] = epilogue( (A[M,K] * sa) . (B[N,K] * sb)^T ).
 //
-// Kernels in this file, in the order a call tries them:
+// Calls with few rows or few tiles go to gemm_direct.hip (gemm_nt compares the estimates).  Kernels in this file, in the
+// order the others try them:
 //   k_gemm_nt_ring        the fast path: persistent, operand tiles copied global -> LDS without staging registers
 //                         into a ring of five 32 KiB slots, epilogue through an LDS-staged drain (plain, bias,
 //                         SiLU-gate, fp32 / bf16 accumulate; per-tensor or per-row x per-channel scales; dense or
@@ -39,7 +40,6 @@ constexpr int kStageBytes = 2 * kTileBytes;       // X tile + W tile
 constexpr int kLdsBytes = 2 * kStageBytes;        // double buffered: 128 KiB
 constexpr int kXcds = 8;
 
-enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_SILU_GATE = 2, EPI_ACCUM_F32 = 3, EPI_ACCUM_BF16 = 4, EPI_STORE_F32 = 5 };
 enum { SCALE_TENSOR = 0, SCALE_ROWCOL = 1, SCALE_BLOCK = 2, SCALE_ROW = 3 };   // SCALE_ROW: sa per row, sb one scalar (ring kernel)
 
 struct GemmArgs {
@@ -55,7 +55,8 @@ struct GemmArgs {
     float* Cf;                   // fp32 [M,N] for EPI_ACCUM_F32 (C += product)
     int tiles_m, tiles_n;
     int force_staged;            // take the register-staged kernel even when the ring kernel applies
-    int duo;                     // 1: the two-workgroups-per-CU kernel where it applies, 2: the same without the stagger
+    int duo;                     // 1: the two-workgroups-per-CU kernel where it applies, 2: the same without the stagger, 0: where its estimate is lowest
+    int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
     // grouped (per-expert) form, ring kernel only; all null / 0 for a dense GEMM
     const int* tile_map;         // [0] = number of row tiles, then (expert, first row, end row) per row tile
@@ -2353,7 +2354,7 @@ int launch_duo(GemmArgs p, hipStream_t st) {
     p.tiles_n = p.N / out_bn;
     const int total = p.tiles_m * p.tiles_n;
     const int grid = persistent_grid(total, 2 * num_cus());
-    if (p.duo == 2) k_gemm_nt_duo<EPI, false><<<grid, kThreads, kDuoLds, st>>>(p);
+    if (p.duo != 1) k_gemm_nt_duo<EPI, false><<<grid, kThreads, kDuoLds, st>>>(p);
     else            k_gemm_nt_duo<EPI, true><<<grid, kThreads, kDuoLds, st>>>(p);
     return launch_status();
 }
@@ -2363,6 +2364,16 @@ inline bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
            p.K >= 2 * BK && p.N % out_bn == 0 && p.ldc % 8 == 0 && aligned16(p.C) && aligned16(p.sb) &&
            (epi != EPI_SILU_GATE || aligned16(p.sb2)) && static_cast<size_t>(p.M) * p.lda < (1ull << 32) &&
            static_cast<size_t>(p.N) * p.ldb < (1ull << 32);
+}
+
+// Its time on a dense problem, microseconds: 0.48 a K-tile where a CU holds one of its workgroups, 0.875 for both where it
+// holds two (measured, 4096 columns, K 4096 to 14336).
+float duo_estimate_us(const GemmArgs& p, int epi) {
+    const int out_bn = epi == EPI_SILU_GATE ? DM / 2 : DM;
+    const long long wgs = static_cast<long long>((p.M + DM - 1) / DM) * (p.N / out_bn);
+    const long long full = wgs / 512, rest = wgs % 512;
+    const float kt = static_cast<float>(p.K / BK);
+    return static_cast<float>(full) * (kt * 0.875f + 2.5f) + (rest == 0 ? 0.0f : (rest > 256 ? kt * 0.875f : kt * 0.48f) + (full ? 0.0f : 2.5f));
 }
 
 template <int FMT, int EPI>
@@ -2461,6 +2472,41 @@ __global__ __launch_bounds__(256) void k_bank_setup(const int* __restrict__ coun
     }
 }
 
+// What the kernels of this file take for a dense problem, in microseconds: tiles in rounds over the CUs, so much per K-tile and
+// so much per tile.  Measured with a tile on every CU: 256 x 256 tiles 0.95 a K-tile, 128 x 256 block-scaled tiles 0.72,
+// the register-staged kernels about twice that.  (At the power limit all of them slow down together.)
+float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile, float per_tile) {
+    const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
+    return static_cast<float>((tiles + 255) / 256) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
+}
+float tiled_estimate_us(const GemmArgs& p, int fmt, int epi, int scale_mode) {
+    if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, p.K % BK == 0 && p.N % BN == 0 ? 0.72f : 2.0f, 5.0f);
+    const bool ring = p.K % BK == 0 && (epi == EPI_SILU_GATE ? p.N % (BN / 2) == 0 : p.N % 8 == 0) && p.ldc % 8 == 0;
+    float best = ring_estimate_us(p.M, p.N, p.K, BM, epi == EPI_SILU_GATE ? BN / 2 : BN, ring ? 0.95f : 2.0f, epi == EPI_SILU_GATE ? 10.0f : 6.0f);
+    if (duo_ok(p, fmt, epi, scale_mode)) {
+        const float duo = duo_estimate_us(p, epi);
+        if (duo < best) best = duo;
+    }
+    return best;
+}
+DirectArgs direct_args(const GemmArgs& p, int epi, int scale_mode) {
+    DirectArgs d{};
+    d.M = p.M; d.N = p.N; d.K = p.K;
+    d.A = p.A; d.lda = p.lda;
+    d.B = p.B; d.ldb = p.ldb;
+    d.B2 = p.B2;
+    d.sa = p.sa; d.sb = p.sb; d.sb2 = p.sb2;
+    d.bias = p.bias;
+    d.C = p.C; d.ldc = p.ldc;
+    d.epi = epi;
+    d.scale_rowcol = scale_mode == SCALE_ROWCOL;
+    d.c_vec = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0;
+    d.tile_map = p.tile_map; d.tiles_m = p.tiles_m;
+    d.a_row_index = p.a_row_index;
+    d.b_expert_stride = p.b_expert_stride; d.sb_expert_stride = p.sb_expert_stride;
+    return d;
+}
+
 int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_stream_t stream) {
     if (p.M < 0 || p.N < 0 || p.K < 0) return CF_ERR_INVALID_ARG;
     if (p.M == 0 || p.N == 0) return CF_OK;
@@ -2479,6 +2525,16 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         const long long total = static_cast<long long>(p.M) * p.N;
         k_gemm_nt_naive<<<static_cast<unsigned>((total + 255) / 256), 256, 0, st>>>(p, fmt, epi, scale_mode);
         return launch_status();
+    }
+    // Few rows or few tiles: the kernel with small tiles and K split inside the workgroup, where its estimate is the lowest
+    if (epi <= EPI_SILU_GATE && !(fmt & 2) && !p.force_staged && !p.ring && !p.duo && p.K >= BK &&
+        static_cast<size_t>(p.M) * p.lda < (1ull << 32) && static_cast<size_t>(p.N) * p.ldb < (1ull << 32) && !(epi == EPI_SILU_GATE && fmt)) {
+        int shape = 0;
+        const float direct = direct_estimate_us(p.M, p.N, p.K, epi == EPI_SILU_GATE, scale_mode == SCALE_BLOCK, &shape);
+        if (direct < tiled_estimate_us(p, fmt, epi, scale_mode)) {
+            const int rc = gemm_nt_direct(direct_args(p, epi, scale_mode), fmt, epi == EPI_SILU_GATE, scale_mode == SCALE_BLOCK, shape, st);
+            if (rc != CF_ERR_UNSUPPORTED) return rc;
+        }
     }
     if (scale_mode == SCALE_BLOCK) {
         static std::once_flag once;
@@ -2525,7 +2581,8 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         }
     }
     if (fmt & 2) return CF_ERR_UNSUPPORTED;     // forward weights are always E4M3
-    if (p.duo && duo_ok(p, fmt, epi, scale_mode))
+    if (duo_ok(p, fmt, epi, scale_mode) &&
+        (p.duo || (!p.force_staged && !p.ring && duo_estimate_us(p, epi) < ring_estimate_us(p.M, p.N, p.K, BM, out_bn, 0.95f, epi == EPI_SILU_GATE ? 10.0f : 6.0f))))
         return epi == EPI_SILU_GATE ? launch_duo<EPI_SILU_GATE>(p, st) : launch_duo<EPI_NONE>(p, st);
     return (fmt & 1) ? dispatch_epi<1>(p, epi, scale_mode, st) : dispatch_epi<0>(p, epi, scale_mode, st);
 }
@@ -2564,6 +2621,7 @@ int cf_fp8_gemm_nt_bf16_ex(int M, int N, int K, const void* A, int lda, int a_is
     p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;
     p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) ? 2 : 1) : 0;
     p.mfma32 = (flags & CF_GEMM_FLAG_MFMA32) != 0;
+    p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
     return gemm_nt(p, a_is_e5m2 ? 1 : 0, epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE, stream);
 }
 
@@ -2727,6 +2785,18 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
     const int out_bn = epilogue == EPI_SILU_GATE ? BN / 2 : BN;
     p.tiles_m = max_row_tiles;
     p.tiles_n = (N + out_bn - 1) / out_bn;
+    // Few rows per expert: the small-tile kernel, which walks an expert's rows 16 mb at a time, where its estimate is lower.
+    // It is sized for half as many rows again as the bound's average, so that most experts take one pass over their weights.
+    if (static_cast<size_t>(total_rows) <= static_cast<size_t>(40) * num_experts) {
+        const bool gate = epilogue == EPI_SILU_GATE;
+        int shape = 0;
+        const float direct = grouped_direct_estimate_us(total_rows, N, K, num_experts, gate, &shape);
+        const int row_tiles = total_rows < num_experts ? total_rows : num_experts;
+        if (direct < ring_estimate_us(row_tiles * BM, N, K, BM, out_bn, 0.95f, 6.0f)) {
+            const int rc = grouped_gemm_nt_direct(direct_args(p, epilogue, scale_mode), a_is_e5m2, gate, shape, st);
+            if (rc != CF_ERR_UNSUPPORTED) return rc;
+        }
+    }
     if (a_is_e5m2) return launch_tiled<1, EPI_NONE, SCALE_ROWCOL>(p, st);
     return epilogue == EPI_SILU_GATE ? launch_tiled<0, EPI_SILU_GATE, SCALE_ROWCOL>(p, st)
                                      : launch_tiled<0, EPI_NONE, SCALE_ROWCOL>(p, st);

@@ -1,0 +1,433 @@
+// FP8 GEMM tiles whose operands go from memory straight to the matrix cores' registers:
+//     C[M,N] = epilogue( (A[M,K] * sa) . (B[N,K] * sb)^T )  for few rows, few tiles or few rows per expert.
+//
+// The persistent kernels of gemm.hip stage 256 x 256 tiles through LDS, one workgroup per tile: a decode batch of 16 rows
+// against a [4096, 14336] weight is 16 tiles, so 240 of the 256 CUs idle and each of the others streams 3.7 MB of weights
+// alone (108 us).  Here a workgroup owns a small output tile and its four wavefronts split K: wavefront w takes K-tiles w,
+// w + 4, w + 8, ... of 128 bytes and copies their operand rows to LDS for itself alone, so that nothing synchronises inside
+// the K loop; the fp32 partial sums are added through LDS at the end, in wavefront order.
+//
+// What bounds it.  Few rows: HBM (16 rows: 10.9 us, the 58.7 MB weight at 5.4 TB/s; 64 rows 13.4 us).  More rows: what the
+// eight L2s deliver, about 24 TB/s here, 93 KB per microsecond and CU, whatever the tile: 256 rows 24 us, 512 rows 36 us,
+// 1000 rows 53 us (256 x 256 tiles: 108-110 us throughout).  So the rule is the largest tile that still gives every CU one.
+// Reading the operands from memory straight into registers was built first: a lane's MFMA row is lane % 16, so 16 consecutive
+// lanes read 16 different lines, and the same L2s delivered 8.6 TB/s (16 rows 15.0 us, 256 rows 52 us).  Copies to LDS take
+// whole 128-byte lines, eight lanes each.
+#include "common.hpp"
+#include "internal.hpp"
+
+#include <mutex>
+#include <type_traits>
+
+namespace cf {
+namespace {
+
+constexpr int kXcds = 8;
+constexpr int kMapWords = 5;          // words per entry of the row-tile table (build_tile_map)
+constexpr int kMapRows = 256;         // rows of a table entry
+constexpr int BK = 128;
+
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+__device__ __forceinline__ float fast_silu(float x) {
+    const float e = __builtin_amdgcn_exp2f(-1.44269504f * x);
+    return x * __builtin_amdgcn_rcpf(1.0f + e);
+}
+
+// vmcnt(n), the other counters left alone
+constexpr int wait_vm(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
+constexpr int kWaitLgkm0 = 0xc07f;
+
+template <int FMT, bool GATE, bool BLOCK, bool GROUPED, int MB, int NB, int WK, int S>
+// BLOCK: two wavefronts per SIMD at most 256 registers each, so that the products land where the vector ALU can fold them
+__global__ __launch_bounds__(64 * WK) __attribute__((amdgpu_waves_per_eu(BLOCK ? 2 : 1)))
+void k_gemm_nt_direct(const DirectArgs p) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    constexpr int NT = GATE ? 2 * NB : NB;          // weight blocks: NB gate blocks, then NB up blocks
+    constexpr int TM = 16 * MB, TN = 16 * NB;
+    constexpr int kBlk = 16 * BK;                   // a 16-row block of a K-tile
+    constexpr int kStage = (MB + NT) * kBlk;
+    constexpr int kCopies = 2 * (MB + NT);          // copy instructions per K-tile
+    // block rows whose partial sums fit LDS together
+    constexpr int MR = WK * MB * NT * 1024 > 128 * 1024 ? MB / 2 : MB;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+
+    const int total = p.tiles_m * p.tiles_n;
+    const int pos = blockIdx.x;
+    const int t = total % kXcds == 0 ? (pos % kXcds) * (total / kXcds) + pos / kXcds : pos;
+    const int tm = t % p.tiles_m, tn = t / p.tiles_m;
+    const int n0 = tn * TN;
+    int m_first = tm * TM, m_end = min(m_first + TM, p.M), expert = 0;
+    if constexpr (GROUPED) {
+        if (tm >= p.tile_map[0]) return;
+        const int* e = p.tile_map + 1 + kMapWords * tm;
+        expert = __builtin_amdgcn_readfirstlane(e[0]);
+        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (tm - __builtin_amdgcn_readfirstlane(e[3])) * kMapRows;
+        m_end = min(m_first + kMapRows, __builtin_amdgcn_readfirstlane(e[2]));
+    }
+    const uint8_t* B = p.B + static_cast<size_t>(expert) * p.b_expert_stride;
+    const uint8_t* B2 = GATE ? p.B2 + static_cast<size_t>(expert) * p.b_expert_stride : B;
+
+    // ---- memory -> LDS: one instruction copies 8 whole 128-byte row pieces, so that every line is asked for once ----
+    const int crow = lane >> 3;
+    uint32_t cchunk[2];                             // this lane's 16-byte chunk of rows 0-7 and 8-15 of a block
+    cchunk[0] = ((lane & 7) ^ crow) * 16u;
+    cchunk[1] = ((lane & 7) ^ crow ^ 1) * 16u;
+    uint32_t woff[NB][2];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            woff[b][h] = static_cast<uint32_t>(min(n0 + b * 16 + h * 8 + crow, p.N - 1)) * static_cast<uint32_t>(p.ldb) + cchunk[h];
+    uint8_t* const mine = smem + wave * (S * kStage);
+    const uint32_t lds_mine = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * (S * kStage);
+    // ---- LDS -> operands: row r16, chunks 2 g and 2 g + 1 ----
+    const int fs = (r16 ^ (r16 >> 3)) & 7;
+    const int rd0 = r16 * BK + (((2 * g) ^ fs) << 4), rd1 = r16 * BK + (((2 * g + 1) ^ fs) << 4);
+
+    const int kfull = p.K / BK;
+    const int nk = kfull > wave ? (kfull - wave + WK - 1) / WK : 0;
+    const int kgroups = (p.K + BK - 1) / BK;        // scale groups along K (BLOCK)
+    const int kpad = kgroups | 1;
+    float* const lds_sa = reinterpret_cast<float*>(smem + WK * S * kStage);
+    float* const lds_sb = lds_sa + TM * kpad;
+
+    for (int m0 = m_first; m0 < m_end; m0 += TM) {
+        uint32_t xoff[MB][2];
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                int row = min(m0 + b * 16 + h * 8 + crow, m_end - 1);
+                if (GROUPED && p.a_row_index) row = p.a_row_index[row];
+                xoff[b][h] = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.lda) + cchunk[h];
+            }
+        if constexpr (BLOCK) {
+            // the tile's scales: [TM][groups] of the activations, [groups] of the weights
+            for (int i = threadIdx.x; i < TM * kgroups; i += 64 * WK) {
+                const int r = i / kgroups, k = i - r * kgroups;
+                lds_sa[r * kpad + k] = p.sa[static_cast<size_t>(min(m0 + r, m_end - 1)) * kgroups + k];
+            }
+            for (int i = threadIdx.x; i < kgroups; i += 64 * WK) lds_sb[i] = p.sb[static_cast<size_t>(n0 / 128) * kgroups + i];
+            __syncthreads();
+        }
+
+        // the epilogue's factors, on their way while K is walked: one row and one column per lane
+        float f_row = 0.0f, f_col = 0.0f, f_col2 = 0.0f;
+        const int tid = threadIdx.x;
+        if constexpr (!BLOCK) {
+            const float* sb = p.sb + static_cast<size_t>(expert) * p.sb_expert_stride;
+            const float* sb2 = GATE ? p.sb2 + static_cast<size_t>(expert) * p.sb_expert_stride : sb;
+            int row = min(m0 + (tid < TM ? tid : 0), m_end - 1), col = min(n0 + (tid < TN ? tid : 0), p.N - 1);
+            if (GROUPED && p.a_row_index) row = p.a_row_index[row];
+            f_row = p.sa[p.scale_rowcol ? row : 0];
+            f_col = sb[p.scale_rowcol ? col : 0];
+            if constexpr (GATE) f_col2 = sb2[p.scale_rowcol ? col : 0];
+        }
+
+        v4f acc[MB][NT];
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+        auto copy = [&](uint32_t dst, uint32_t voff, const uint8_t* base) {
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(dst), "v"(voff), "s"(base) : "memory");
+        };
+        auto fetch = [&](int stage, int kt) {
+            const size_t k0 = static_cast<size_t>(kt) * BK;
+            const uint32_t dst = lds_mine + stage * kStage;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    copy(dst + b * kBlk + h * (kBlk / 2), woff[b][h], B + k0);
+                    if constexpr (GATE) copy(dst + (NB + b) * kBlk + h * (kBlk / 2), woff[b][h], B2 + k0);
+                }
+#pragma unroll
+            for (int b = 0; b < MB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) copy(dst + (NT + b) * kBlk + h * (kBlk / 2), xoff[b][h], p.A + k0);
+        };
+        v8i x[MB], w[NT];
+        auto read = [&](int stage) {
+            const uint8_t* s = mine + stage * kStage;
+            auto one = [&](v8i& d, const uint8_t* blk) {
+                const uint4 lo = *reinterpret_cast<const uint4*>(blk + rd0), hi = *reinterpret_cast<const uint4*>(blk + rd1);
+                d = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+            };
+#pragma unroll
+            for (int j = 0; j < NT; ++j) one(w[j], s + j * kBlk);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) one(x[i], s + (NT + i) * kBlk);
+        };
+        auto multiply = [&](int kt) {
+            float fx[MB], fw = 0.0f;
+            if constexpr (BLOCK) {
+                fw = lds_sb[kt];
+#pragma unroll
+                for (int i = 0; i < MB; ++i) fx[i] = lds_sa[(i * 16 + r16) * kpad + kt] * fw;
+            }
+            if constexpr (BLOCK) {
+                // a column's products are folded while the next column's are on the matrix cores
+                v4f part[2][MB];
+#pragma unroll
+                for (int j = 0; j <= NT; ++j) {
+                    if (j < NT) {
+#pragma unroll
+                        for (int i = 0; i < MB; ++i) {
+                            const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+                            part[j & 1][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[j < NT ? j : 0], x[i], zero, (FMT >> 1) & 1, FMT & 1, 0, 0, 0, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (j > 0) {
+#pragma unroll
+                        for (int i = 0; i < MB; ++i)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q)
+                                acc[i][j > 0 ? j - 1 : 0][q] = __builtin_fmaf(part[(j + 1) & 1][i][q], fx[i], acc[i][j > 0 ? j - 1 : 0][q]);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int i = 0; i < MB; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[j], x[i], acc[i][j], (FMT >> 1) & 1, FMT & 1, 0, 0, 0, 0);
+            }
+        };
+
+        // (loads issued before the copies are older than them: a wait that leaves n copies in flight covers them)
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (s < nk) fetch(s, wave + s * WK);
+        int i = 0, stage = 0;
+        for (; i + S < nk; ++i) {
+            __builtin_amdgcn_s_waitcnt(wait_vm((S - 1) * kCopies));
+            __builtin_amdgcn_sched_barrier(0);
+            read(stage);
+            __builtin_amdgcn_s_waitcnt(kWaitLgkm0);    // the stage is free for the copies of the K-tile S ahead
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(stage, wave + (i + S) * WK);
+            multiply(wave + i * WK);
+            stage = stage + 1 == S ? 0 : stage + 1;
+        }
+        for (; i < nk; ++i) {
+            // the last K-tiles: nothing is issued behind them
+            if (nk - i >= S) __builtin_amdgcn_s_waitcnt(wait_vm((S - 1) * kCopies));
+            else             __builtin_amdgcn_s_waitcnt(wait_vm(0));
+            __builtin_amdgcn_sched_barrier(0);
+            read(stage);
+            multiply(wave + i * WK);
+            stage = stage + 1 == S ? 0 : stage + 1;
+        }
+        // the last, partial K-tile (K % 16 == 0): bytes beyond K count as zeros
+        if (kfull * BK < p.K && wave == kfull % WK) {
+            const uint32_t left = p.K - kfull * BK;
+            const size_t k0 = static_cast<size_t>(kfull) * BK;
+            auto part = [&](int blk, int h, uint32_t voff, const uint8_t* base) {
+                uint4 v = make_uint4(0, 0, 0, 0);
+                if (cchunk[h] < left) v = *reinterpret_cast<const uint4*>(base + k0 + voff);
+                *reinterpret_cast<uint4*>(mine + blk * kBlk + h * (kBlk / 2) + lane * 16) = v;
+            };
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    part(b, h, woff[b][h], B);
+                    if constexpr (GATE) part(NB + b, h, woff[b][h], B2);
+                }
+#pragma unroll
+                for (int b = 0; b < MB; ++b) part(NT + b, h, xoff[b][h], p.A);
+            }
+            read(0);
+            multiply(kfull);
+        }
+        __syncthreads();          // every wavefront is done with its stages: their LDS takes the partial sums
+
+        // ---- the wavefronts' partial sums, added in wavefront order; MR block rows at a time ----
+        float4* red = reinterpret_cast<float4*>(smem);
+        float* const lds_f = reinterpret_cast<float*>(smem + WK * MR * NT * 1024);      // [TM] rows, [TN] columns, [TN] up columns
+        if constexpr (!BLOCK) {
+            if (tid < TM) lds_f[tid] = f_row;
+            if (tid < TN) lds_f[TM + tid] = f_col;
+            if (GATE && tid < TN) lds_f[TM + TN + tid] = f_col2;
+        }
+        static_for<0, MB / MR>([&](auto pass) {
+        constexpr int base = decltype(pass)::value * MR;
+        if constexpr (base > 0) __syncthreads();
+#pragma unroll
+        for (int b = 0; b < MR; ++b)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                red[(wave * (MR * NT) + b * NT + j) * 64 + lane] =
+                    make_float4(acc[base + b][j][0], acc[base + b][j][1], acc[base + b][j][2], acc[base + b][j][3]);
+        __syncthreads();
+        auto summed = [&](int blk, float (&v)[4]) {
+            v[0] = v[1] = v[2] = v[3] = 0.0f;
+#pragma unroll
+            for (int k = 0; k < WK; ++k) {
+                const float4 s = red[(k * (MR * NT) + blk) * 64 + lane];
+                v[0] += s.x; v[1] += s.y; v[2] += s.z; v[3] += s.w;
+            }
+        };
+        // ---- epilogue: one 16 x 16 block of outputs per wavefront and step; a lane holds four columns of one row ----
+#pragma unroll
+        for (int u = 0; u < (MR * NB + WK - 1) / WK; ++u) {
+            const int unit = wave + u * WK;
+            if (MR * NB % WK != 0 && unit >= MR * NB) break;
+            const int mb = unit / NB, nb = unit % NB;
+            const int ml = (base + mb) * 16 + r16, nl = nb * 16 + g * 4;
+            const int m = m0 + ml, n = n0 + nl;
+            float v[4], up[4];
+            summed(mb * NT + nb, v);
+            if constexpr (GATE) summed(mb * NT + NB + nb, up);
+            if constexpr (!BLOCK) {
+                const float sa = lds_f[ml];
+                const float4 c = *reinterpret_cast<const float4*>(lds_f + TM + nl);
+                const float c4[4] = {c.x, c.y, c.z, c.w};
+                float4 d = c;
+                if constexpr (GATE) d = *reinterpret_cast<const float4*>(lds_f + TM + TN + nl);
+                const float d4[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    v[q] *= sa * c4[q];
+                    if constexpr (GATE) {
+                        // the reference rounds gate and up to bf16 before the SiLU product
+                        const uint32_t gu = pack_bf16x2_hw(v[q], up[q] * (sa * d4[q]));
+                        v[q] = fast_silu(bf16_lo(gu)) * bf16_hi(gu);
+                    }
+                }
+            }
+            if (m >= m_end || n >= p.N) continue;
+            const bool whole = n + 3 < p.N;
+            if (p.epi == EPI_BIAS)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = round_bf16_hw(v[q]) + bf16_to_f32(p.bias[min(n + q, p.N - 1)]);
+            uint16_t* c = p.C + static_cast<size_t>(m) * p.ldc + n;
+            const uint32_t o01 = pack_bf16x2_hw(v[0], v[1]), o23 = pack_bf16x2_hw(v[2], v[3]);
+            if (whole && p.c_vec) {
+                *reinterpret_cast<uint2*>(c) = make_uint2(o01, o23);
+            } else {
+                c[0] = static_cast<uint16_t>(o01);
+                if (n + 1 < p.N) c[1] = static_cast<uint16_t>(o01 >> 16);
+                if (n + 2 < p.N) c[2] = static_cast<uint16_t>(o23);
+                if (n + 3 < p.N) c[3] = static_cast<uint16_t>(o23 >> 16);
+            }
+        }
+        });
+        if (GROUPED) __syncthreads();
+    }
+}
+
+constexpr int kLds = 160 * 1024;
+
+template <int FMT, bool GATE, bool BLOCK, bool GROUPED, int MB, int NB, int WK, int S>
+int launch(DirectArgs p, hipStream_t st) {
+    constexpr int NT = GATE ? 2 * NB : NB;
+    constexpr int stages = WK * S * (MB + NT) * 2048;
+    constexpr int one = WK * MB * NT * 1024, sums = (one > 128 * 1024 ? one / 2 : one) + (16 * MB + 32 * NB) * 4;
+    constexpr int base = stages > sums ? stages : sums;
+    static_assert(base <= kLds);
+    const int kg = (p.K + 127) / 128;
+    const int lds = base + (BLOCK ? (16 * MB * (kg | 1) + kg) * 4 : 0);
+    if (lds > kLds) return CF_ERR_UNSUPPORTED;
+    static std::once_flag once;
+    static hipError_t err = hipSuccess;
+    std::call_once(once, [] {
+        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_nt_direct<FMT, GATE, BLOCK, GROUPED, MB, NB, WK, S>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    });
+    if (err != hipSuccess) return static_cast<int>(err);
+    if (!GROUPED) p.tiles_m = (p.M + 16 * MB - 1) / (16 * MB);
+    p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
+    k_gemm_nt_direct<FMT, GATE, BLOCK, GROUPED, MB, NB, WK, S><<<p.tiles_m * p.tiles_n, 64 * WK, lds, st>>>(p);
+    return launch_status();
+}
+
+// The tile shapes, smallest first: 16 mb rows x 16 nt weight rows (nt counts gate and up blocks), whether two workgroups fit a
+// CU's LDS, and what a workgroup costs beside its operand bytes (pipeline fill, reduction, epilogue; microseconds).
+struct Shape { int mb, nt; bool shared; float fixed; };
+constexpr Shape kPlain[6] = {{1, 1, true, 1.5f}, {2, 2, true, 2.0f}, {4, 2, false, 2.5f}, {4, 4, false, 4.0f}, {8, 4, false, 6.0f}, {8, 8, false, 12.0f}};
+constexpr Shape kGate[4] = {{1, 2, true, 1.5f}, {2, 4, true, 2.5f}, {4, 8, false, 6.0f}, {8, 8, false, 12.0f}};
+
+template <int FMT, bool BLOCK, bool GROUPED>
+int launch_plain(const DirectArgs& p, int shape, hipStream_t st) {
+    switch (shape) {
+        case 0: return launch<FMT, false, BLOCK, GROUPED, 1, 1, 4, 3>(p, st);
+        case 1: return launch<FMT, false, BLOCK, GROUPED, 2, 2, 4, 2>(p, st);
+        case 2: return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, st);
+        case 3: return launch<FMT, false, BLOCK, GROUPED, 4, 4, 4, 2>(p, st);
+        default:
+            if constexpr (BLOCK || GROUPED) return CF_ERR_UNSUPPORTED;
+            else return shape == 4 ? launch<FMT, false, BLOCK, GROUPED, 8, 4, 4, 1>(p, st) : launch<FMT, false, BLOCK, GROUPED, 8, 8, 4, 1>(p, st);
+    }
+}
+template <bool GROUPED>
+int launch_gate(const DirectArgs& p, int shape, hipStream_t st) {
+    switch (shape) {
+        case 0: return launch<0, true, false, GROUPED, 1, 1, 4, 3>(p, st);
+        case 1: return launch<0, true, false, GROUPED, 2, 2, 4, 1>(p, st);
+        case 2: return launch<0, true, false, GROUPED, 4, 4, 4, 1>(p, st);
+        default:
+            if constexpr (GROUPED) return CF_ERR_UNSUPPORTED;
+            else return launch<0, true, false, GROUPED, 8, 4, 4, 1>(p, st);
+    }
+}
+
+}  // namespace
+
+// Picks the tile shape and says what it would take, in microseconds: every workgroup moves K bytes of each of its rows and weight rows, and a CU takes them in at 93 KB
+// per microsecond whatever the shape (measured, K 1024 to 14336; 62 KB where the folds of the block scales are as many as in
+// a 64 x 64 tile); a CU whose LDS holds one workgroup works in whole rounds.
+// A shape with more rows than the next one smaller would do is not looked at: its extra rows are copies.
+float direct_estimate_us(int M, int N, int K, bool gate, bool block, int* shape) {
+    const Shape* s = gate ? kGate : kPlain;
+    const int count = gate ? 4 : block ? 4 : 6;
+    float best = 1e30f;
+    for (int i = 0; i < count; ++i) {
+        if (i > 0 && s[i].mb > s[i - 1].mb && M <= 16 * s[i - 1].mb) break;
+        const int tn = 16 * s[i].nt / (gate ? 2 : 1);
+        const double wgs = static_cast<double>((M + 16 * s[i].mb - 1) / (16 * s[i].mb)) * ((N + tn - 1) / tn);
+        double rounds = wgs / 256.0;
+        if (!s[i].shared) rounds = static_cast<double>(static_cast<long long>(rounds + 0.999));
+        if (rounds < 1.0) rounds = 1.0;
+        const double rate = block && s[i].mb * s[i].nt >= 16 ? 62e3 : 93e3;
+        const float t = static_cast<float>(rounds * (s[i].fixed + static_cast<double>(K) * 16.0 * (s[i].mb + s[i].nt) / rate));
+        if (t < best) { best = t; *shape = i; }
+    }
+    return best;
+}
+
+float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape) {
+    const Shape* s = gate ? kGate : kPlain;
+    const int count = gate ? 3 : 4;
+    const float rows = static_cast<float>(total_rows) / static_cast<float>(num_experts);
+    int i = 0;
+    while (i + 1 < count && (16 * s[i].mb < 1.5f * rows + 2.0f || s[i + 1].mb == s[i].mb)) ++i;
+    *shape = i;
+    const int tn = 16 * s[i].nt / (gate ? 2 : 1);
+    const float rounds = static_cast<float>(num_experts) * static_cast<float>((N + tn - 1) / tn) / 256.0f;
+    return (rounds < 1.0f ? 1.0f : rounds) * (s[i].fixed + static_cast<float>(K) * 16.0f * static_cast<float>(s[i].mb + s[i].nt) / 93e3f);
+}
+
+int gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, bool block, int shape, hipStream_t st) {
+    if (gate) return fmt == 0 ? launch_gate<false>(p, shape, st) : CF_ERR_UNSUPPORTED;
+    if (block) return launch_plain<0, true, false>(p, shape, st);
+    return fmt == 1 ? launch_plain<1, false, false>(p, shape, st) : fmt == 0 ? launch_plain<0, false, false>(p, shape, st) : CF_ERR_UNSUPPORTED;
+}
+int grouped_gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, int shape, hipStream_t st) {
+    if (gate) return fmt == 0 ? launch_gate<true>(p, shape, st) : CF_ERR_UNSUPPORTED;
+    return fmt == 1 ? launch_plain<1, false, true>(p, shape, st) : launch_plain<0, false, true>(p, shape, st);
+}
+
+}  // namespace cf
