@@ -1,7 +1,7 @@
 // Scaled FP8 GEMM for gfx950:  C[M,N] = epilogue( (A[M,K] * sa) . (B[N,K] * sb)^T ).
 //
-// Calls with few rows or few tiles go to gemm_direct.hip (gemm_nt compares the estimates).  Kernels in this file, in the
-// order the others try them:
+// Calls with few rows or few tiles go to gemm_direct.hip or gemm_duo.hip (gemm_nt compares the estimates), accumulating ones
+// over a short K to gemm_duo.hip.  Kernels in this file, in the order the others try them:
 //   k_gemm_nt_ring        the fast path: persistent, operand tiles copied global -> LDS without staging registers
 //                         into a ring of five 32 KiB slots, epilogue through an LDS-staged drain (plain, bias,
 //                         SiLU-gate, fp32 / bf16 accumulate; per-tensor or per-row x per-channel scales; dense or
@@ -24,68 +24,23 @@
 //
 // Workgroup -> tile mapping is XCD aware: consecutive workgroup ids go round-robin to the 8 XCDs, so each XCD is
 // given a contiguous range of tiles, walked in 8 (M) x 4 (N) patches whose operands share its own L2.
-#include "common.hpp"
-#include "internal.hpp"
+#include "gemm_common.hpp"
 
 #include <mutex>
-#include <type_traits>
 
 namespace cf {
 namespace {
 
-constexpr int BM = 256, BN = 256, BK = 128;
 constexpr int kThreads = 256;
 constexpr int kTileBytes = BM * BK;               // 32 KiB per operand tile
 constexpr int kStageBytes = 2 * kTileBytes;       // X tile + W tile
 constexpr int kLdsBytes = 2 * kStageBytes;        // double buffered: 128 KiB
-constexpr int kXcds = 8;
 
-enum { SCALE_TENSOR = 0, SCALE_ROWCOL = 1, SCALE_BLOCK = 2, SCALE_ROW = 3 };   // SCALE_ROW: sa per row, sb one scalar (ring kernel)
-
-struct GemmArgs {
-    int M, N, K;                 // N = output columns
-    const uint8_t* A; int lda;   // activations [M,K]
-    const uint8_t* B; int ldb;   // weights [N,K] (gate weights for EPI_SILU_GATE)
-    const uint8_t* B2;           // up weights [N,K] for EPI_SILU_GATE
-    const float* sa;             // descale of A: [1] or [M]
-    const float* sb;             // descale of B: [1] or [N]
-    const float* sb2;            // descale of B2
-    const uint16_t* bias;        // bf16 [N] for EPI_BIAS
-    uint16_t* C; int ldc;        // bf16 [M,N]
-    float* Cf;                   // fp32 [M,N] for EPI_ACCUM_F32 (C += product)
-    int tiles_m, tiles_n;
-    int force_staged;            // take the register-staged kernel even when the ring kernel applies
-    int duo;                     // 1: the two-workgroups-per-CU kernel where it applies, 2: the same without the stagger, 0: where its estimate is lowest
-    int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
-    int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
-    // grouped (per-expert) form, ring kernel only; all null / 0 for a dense GEMM
-    const int* tile_map;         // [0] = number of row tiles, then (expert, first row, end row) per row tile
-    const int* a_row_index;      // compact row r reads A row (and its descale) a_row_index[r]; null = r
-    int a_rows;                  // rows of the A buffer (= M without a row index)
-    long long b_expert_stride;   // bytes between the weight matrices of consecutive experts
-    int sb_expert_stride;        // elements between the channel descales of consecutive experts
-    // term-split form (ring kernel, MX instantiation only): A's K axis is `K / b_k_period` terms laid side by side,
-    // term t = the residual of the terms before it scaled by 16^t; every term multiplies the same b_k_period
-    // columns of B, and the matrix cores scale its products by 2^(-4 t)
-    int b_k_period;
-};
 
 // where a workgroup's tile lives: rows [m0, m_end) of the output, columns from n0, weights of `expert`
 struct TilePos { int m0, m_end, n0, expert; };
 
-__device__ __forceinline__ int swz(int row) { return (row ^ ((row >> 3) & 3)) & 7; }
 
-// Tile t of the walk order -> (tile_m, tile_n): patches of 8 (M) x tiles_n, row tiles varying fastest, so that
-// 32 consecutive tiles form an 8 x 4 patch whose operands an XCD's L2 can hold.
-__device__ __forceinline__ void tile_coords(int t, int tiles_m, int tiles_n, int& tm, int& tn) {
-    constexpr int GM = 8;
-    const int group = t / (GM * tiles_n);
-    const int first_m = group * GM;
-    const int gm = min(GM, tiles_m - first_m);
-    const int in_group = t - group * GM * tiles_n;
-    tm = first_m + in_group % gm;
-    tn = in_group / gm;
-}
 // Workgroups are handed to the 8 XCDs round-robin, so launch positions with the same pos % 8 share an XCD
 // (and its L2).  One tile per workgroup: position pos works on tile (pos % 8) * (total / 8) + pos / 8 of the walk
 // order, so each XCD is given a contiguous range of tiles (ragged counts keep the plain order).
@@ -97,14 +52,6 @@ __device__ __forceinline__ int xcd_chunked(int pos, int total) {
 // acc[a][b][r]: output row m = m0 + wm*128 + b*32 + (lane & 31); weight row within the
 // wave's 128 = a*32 + 8*(r/4) + 4*(lane>>5) + r%4, i.e. four consecutive output columns per quad.
 // Column scales are fetched once per quad as a float4 and reused for the four row tiles.
-
-// SiLU gate for the fused epilogue: x * 1/(1 + 2^(-x*log2 e)) on the hardware exp2 and reciprocal
-// (1 ulp each).  The stand-alone swiglu kernel keeps the correctly-rounded divide and the
-// reproducible expf; the two differ by at most one bf16 ulp of the product.
-__device__ __forceinline__ float fast_silu(float x) {
-    const float e = __builtin_amdgcn_exp2f(-1.44269504f * x);
-    return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
 
 __device__ __forceinline__ float4 load_scale4(const float* s, int n, int N, bool fast) {
     if (fast) return *reinterpret_cast<const float4*>(s + n);
@@ -492,19 +439,10 @@ constexpr int kRingLds = kSlots * kSlotBytes;     // 160 KiB: all of a CU's LDS
 // s_waitcnt immediates: vmcnt in bits [3:0] and [15:14], expcnt [6:4] and lgkmcnt [11:8] left at no-wait
 constexpr int kWaitVm0 = 0x0f70, kWaitVm8 = 0x0f78, kWaitVm16 = 0x4f70;
 
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
 // Tile `lin` of a workgroup's walk order -> where it lives.  Dense: the patch order of tile_coords.  Grouped:
 // the table holds, per row tile, its expert's number, row range, first row tile and row-tile count, experts back
 // to back; an expert's tiles are walked in groups of 4 column tiles with its row tiles varying fastest, so that
 // 32 consecutive tiles are (up to) 8 row tiles x 4 column tiles of one expert.
-constexpr int kMapWords = 5;
 template <int OUT_BN>
 __device__ __forceinline__ TilePos locate_tile(const GemmArgs& p, int lin) {
     TilePos t;
@@ -1579,307 +1517,6 @@ void k_gemm_nt_ring16(const GemmArgs p) {
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
 }
 
-// ---- duo kernel: the ring kernel at half the tile edge, two workgroups per CU ------------------------------
-// Workgroup tile 128 x 128 x 128, four wavefronts 2 x 2, each 64 x 64 = 2 x 2 MFMA tiles (64 accumulator
-// registers), the same ring of five slots at 16 KiB each: 80 KiB, so a CU holds TWO workgroups and every SIMD two
-// wavefronts.  A tile's drain is vector-ALU work (scales, SiLU, bf16 rounding) during which the matrix cores of a
-// one-wavefront-per-SIMD kernel idle; here the other workgroup's MFMAs run under it, provided the two are out of
-// step.  The workgroup that got the upper half of the CU's LDS (readable from the hardware's LDS allocation
-// register) therefore starts half a tile late.  The price is twice the LDS and L2 bytes per FLOP of the 256 x 256
-// tile.  Dense and grouped per expert (128-row tiles over the 256-row tile table: an entry's second half may be
-// empty), E4M3 activations and weights, per-row x per-channel scales, plain or SiLU-gate epilogue; N a multiple of
-// the tile's output width.
-constexpr int DM = 128;
-constexpr int kDuoSlot = DM * BK;                  // 16 KiB
-constexpr int kDuoLds = kSlots * kDuoSlot;         // 80 KiB
-constexpr int kWaitVm4 = 0x0f74;
-
-template <int EPI, bool STAGGER>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_gemm_nt_duo(const GemmArgs p) {
-    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr bool GATE = EPI == EPI_SILU_GATE;
-    constexpr int OUT_BN = GATE ? DM / 2 : DM;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
-    const int total_tiles = p.tiles_m * p.tiles_n;
-    int my_tiles, lin0, lstep;
-    if (gridDim.x % kXcds == 0) {
-        const int per = (total_tiles + kXcds - 1) / kXcds;
-        const int x = blockIdx.x % kXcds, i = blockIdx.x / kXcds;
-        lstep = gridDim.x / kXcds;
-        const int cnt = max(0, min(per, total_tiles - x * per));
-        my_tiles = (cnt - i + lstep - 1) / lstep;
-        lin0 = x * per + i;
-    } else {
-        lstep = gridDim.x;
-        my_tiles = (total_tiles - static_cast<int>(blockIdx.x) + lstep - 1) / lstep;
-        lin0 = blockIdx.x;
-    }
-    if (my_tiles <= 0) return;
-    const int ktiles = p.K / BK;      // >= 2, checked by the launcher
-
-    if constexpr (STAGGER) {
-        // the second workgroup of a CU (its LDS starts above the first one's) waits about half a tile's MFMA time
-        unsigned alloc;
-        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_LDS_ALLOC, 0, 12)" : "=s"(alloc));
-        if (alloc != 0) {
-            for (int i = 0; i < (ktiles + 15) / 16; ++i) __builtin_amdgcn_s_sleep(127);
-        }
-    }
-
-    auto tile_at = [&](int seq, int& m0, int& n0) {
-        int tm, tn;
-        tile_coords(lin0 + seq * lstep, p.tiles_m, p.tiles_n, tm, tn);
-        m0 = tm * DM;
-        n0 = tn * OUT_BN;
-    };
-
-    // ---- global -> LDS: wave w copies rows [32w, 32w+32) of an operand tile, 8 rows per instruction ----
-    const int lrow = lane >> 3, lslot = lane & 7;
-    uint32_t xoff[4], woff[4];
-    // SiLU-gate: the W tile's rows are [gate 32 | up 32] for the columns of wavefront column 0, then the same for
-    // column 1, so wave w copies from one matrix only: gate for even w, up for odd w
-    const uint8_t* wsrc = (GATE && (wave & 1)) ? p.B2 : p.B;
-    auto aim = [&](int seq) {
-        int m0, n0;
-        tile_at(seq, m0, n0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = wave * 32 + j * 8 + lrow;
-            const uint32_t gchunk = (lslot ^ swz(row)) * 16;
-            xoff[j] = static_cast<uint32_t>(min(m0 + row, p.M - 1)) * static_cast<uint32_t>(p.lda) + gchunk;
-            const int n = GATE ? n0 + (row >> 6) * 32 + (row & 31) : n0 + row;
-            woff[j] = static_cast<uint32_t>(min(n, p.N - 1)) * static_cast<uint32_t>(p.ldb) + gchunk;
-        }
-    };
-    uint32_t lds_wave = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(smem)) + wave * (32 * BK);
-    auto dma = [&](int slot, uint32_t voff, const uint8_t* base, auto jc) {
-        constexpr int J = decltype(jc)::value;
-        const uint32_t dst = lds_wave + slot;
-        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3"
-                     :: "s"(dst), "n"(J * 8 * BK), "v"(voff), "s"(base) : "memory", "scc");
-    };
-    auto dma_x = [&](int slot, int k0, auto jc) { dma(slot, xoff[decltype(jc)::value], p.A + k0, jc); };
-    auto dma_w = [&](int slot, int k0, auto jc) { dma(slot, woff[decltype(jc)::value], wsrc + k0, jc); };
-
-    // ---- LDS -> MFMA operands ----
-    const int frow = lane & 31, khalf = lane >> 5, fs = swz(frow);
-    int rd[2][2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) rd[h][j] = frow * BK + (((h * 4 + khalf * 2 + j) ^ fs) << 4);
-    const uint8_t* xrd = smem + wm * 64 * BK;
-    const uint8_t* wrd = smem + wn * 64 * BK;
-
-    v16f acc[2][2];       // [weight tile][activation tile]
-    v8i wq[2][2], xq[2][2];
-    auto put = [](v8i& dst, int half, const uint4 v) {
-        dst[4 * half + 0] = (int)v.x; dst[4 * half + 1] = (int)v.y; dst[4 * half + 2] = (int)v.z; dst[4 * half + 3] = (int)v.w;
-    };
-    // read I (0..7) of k-half H: w0 x0 x1 w1, two reads each
-    auto read_one = [&](int sx, int sw, auto hc, auto ic) {
-        constexpr int H = decltype(hc)::value, I = decltype(ic)::value;
-        constexpr int t = I >> 1, half = I & 1;
-        const int r = rd[H][half];
-        if constexpr (t == 0)      put(wq[H][0], half, *reinterpret_cast<const uint4*>(wrd + sw + r));
-        else if constexpr (t <= 2) put(xq[H][t - 1], half, *reinterpret_cast<const uint4*>(xrd + sx + (t - 1) * 32 * BK + r));
-        else                       put(wq[H][1], half, *reinterpret_cast<const uint4*>(wrd + sw + 32 * BK + r));
-    };
-    auto mfma_one = [&](auto hc, auto ic, auto first_c) {
-        constexpr int H = decltype(hc)::value, I = decltype(ic)::value;
-        constexpr int a = I >> 1, b = I & 1;
-        v16f c = acc[a][b];
-        if constexpr (decltype(first_c)::value != 0) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) c[r] = 0.0f;
-        }
-        acc[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wq[H][a], xq[H][b], c, 0, 0, 0, 0, 0, 0);
-    };
-    using C0 = std::integral_constant<int, 0>;
-    using C1 = std::integral_constant<int, 1>;
-
-    int a0 = 0, a1 = kDuoSlot, a2 = 2 * kDuoSlot, a3 = 3 * kDuoSlot, a4 = 4 * kDuoSlot;
-
-    // what the drain needs in registers: row descales of this lane's two output rows and the channel descales of its
-    // columns (plain: cs[a][g] = four columns of quad g of weight tile a; SiLU-gate: cs[0][g] gate, cs[1][g] up)
-    float sa[2];
-    float4 cs[2][4];
-    auto load_scales = [&](int m0, int n0) {
-#pragma unroll
-        for (int b = 0; b < 2; ++b) sa[b] = p.sa[min(m0 + wm * 64 + b * 32 + (lane & 31), p.M - 1)];
-        if constexpr (GATE) {
-            const int col = n0 + wn * 32 + khalf * 4;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                cs[0][g] = *reinterpret_cast<const float4*>(p.sb + col + g * 8);
-                cs[1][g] = *reinterpret_cast<const float4*>(p.sb2 + col + g * 8);
-            }
-        } else {
-            const int col = n0 + wn * 64 + khalf * 4;
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) cs[a][g] = *reinterpret_cast<const float4*>(p.sb + col + a * 32 + g * 8);
-        }
-    };
-
-    auto ktile = [&](auto first_c, auto end_c, int dk0, int m0, int n0, bool wait) {
-        constexpr bool END = decltype(end_c)::value != 0;
-        // step (g,0): 4 MFMAs, the operand reads of (g,1), the copies of X(g+2)
-        static_for<0, 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            mfma_one(C0{}, ic, first_c);
-            read_one(a0, a1, C1{}, std::integral_constant<int, 2 * i>{});
-            read_one(a0, a1, C1{}, std::integral_constant<int, 2 * i + 1>{});
-            dma_x(a4, dk0, ic);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        // step (g,1)
-        mfma_one(C1{}, C0{}, C0{});
-        __builtin_amdgcn_sched_barrier(0);
-        if (wait) __builtin_amdgcn_s_waitcnt(kWaitVm4);
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        static_for<1, 4>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            mfma_one(C1{}, ic, C0{});
-            if constexpr (!END) {
-                static_for<0, 3>([&](auto jc) {
-                    constexpr int j = (i - 1) * 3 + decltype(jc)::value;
-                    if constexpr (j < 8) read_one(a2, a3, C0{}, std::integral_constant<int, j < 8 ? j : 0>{});
-                });
-            }
-            if constexpr (i == 1) { dma_w(a0, dk0, C0{}); dma_w(a0, dk0, C1{}); }
-            if constexpr (i == 2) dma_w(a0, dk0, std::integral_constant<int, 2>{});
-            if constexpr (i == 3) dma_w(a0, dk0, std::integral_constant<int, 3>{});
-            if constexpr (END && i == 1) load_scales(m0, n0);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    };
-    auto rotate = [&]() {
-        const int b0 = a0, b1 = a1;
-        a0 = a2; a1 = a3; a2 = a4; a3 = b0; a4 = b1;
-    };
-
-    // copy position: two K-tiles ahead of the compute position; past the last tile the stream re-reads that tile
-    int dkt = 2 % ktiles, dseq = 2 / ktiles;
-    aim(0);
-    static_for<0, 4>([&](auto jc) { dma_x(a0, 0, jc); });
-    static_for<0, 4>([&](auto jc) { dma_w(a1, 0, jc); });
-    static_for<0, 4>([&](auto jc) { dma_x(a2, BK, jc); });
-    static_for<0, 4>([&](auto jc) { dma_w(a3, BK, jc); });
-    if (dseq == 1 && my_tiles > 1) aim(1);
-    __builtin_amdgcn_s_waitcnt(kWaitVm8);
-    __syncthreads();
-    static_for<0, 8>([&](auto ic) { read_one(a0, a1, C0{}, ic); });
-
-    auto advance_copy = [&]() {
-        if (++dkt == ktiles) {
-            dkt = 0;
-            if (++dseq < my_tiles) aim(dseq);
-        }
-    };
-
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    for (int seq = 0; seq < my_tiles; ++seq) {
-        int m0, n0;
-        tile_at(seq, m0, n0);
-        ktile(C1{}, C0{}, dkt * BK, m0, n0, seq == 0);
-        rotate(); advance_copy();
-        for (int kt = 1; kt + 1 < ktiles; ++kt) {
-            ktile(C0{}, C0{}, dkt * BK, m0, n0, true);
-            rotate(); advance_copy();
-        }
-        ktile(C0{}, C1{}, dkt * BK, m0, n0, true);
-        rotate(); advance_copy();
-
-        // ---- drain: a4 is free until this workgroup's own copies of the stream's next K-tile but one ----
-        const int row = lane & 31;
-        const int wswz = (row >> 1) & 7;
-        const int rr = lane >> 3, rc = lane & 7;
-        if constexpr (GATE) {
-            // the two wavefronts of a row half share 64 rows x 128 bytes: each writes the 64 bytes per row of its 32
-            // output columns, then (barrier) each streams out 32 whole rows
-            uint8_t* stage = smem + a4 + wm * (64 * 128);
-            uint8_t* wr = stage + row * 128 + khalf * 8;
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float c4[4] = {cs[0][g].x, cs[0][g].y, cs[0][g].z, cs[0][g].w};
-                    const float u4[4] = {cs[1][g].x, cs[1][g].y, cs[1][g].z, cs[1][g].w};
-                    float v[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        // the reference rounds gate and up to bf16 before the SiLU product
-                        const uint32_t gu = pack_bf16x2_hw(acc[0][b][g * 4 + q] * (sa[b] * c4[q]), acc[1][b][g * 4 + q] * (sa[b] * u4[q]));
-                        v[q] = fast_silu(bf16_lo(gu)) * bf16_hi(gu);
-                    }
-                    *reinterpret_cast<uint2*>(wr + b * 32 * 128 + (((wn * 4 + g) ^ wswz) << 4)) =
-                        make_uint2(pack_bf16x2_hw(v[0], v[1]), pack_bf16x2_hw(v[2], v[3]));
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // every copy in flight is waited for before the first store (stores and copies share one counter); the tile
-            // that follows skips the wait of its first K-tile
-            __builtin_amdgcn_s_waitcnt(kWaitVm0);
-            __syncthreads();
-            const uint8_t* rdp0 = stage + (wn * 32 + rr) * 128 + ((rc ^ (rr >> 1)) << 4);
-            const uint8_t* rdp1 = stage + (wn * 32 + rr) * 128 + ((rc ^ (rr >> 1) ^ 4) << 4);
-            uint8_t* cu = reinterpret_cast<uint8_t*>(p.C + static_cast<size_t>(m0 + wm * 64 + wn * 32) * p.ldc + n0);
-            const uint32_t coff = (static_cast<uint32_t>(rr) * static_cast<uint32_t>(p.ldc) + rc * 8u) * 2u;
-            const size_t cstep = static_cast<size_t>(p.ldc) * 16;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint4 v = *reinterpret_cast<const uint4*>(((i & 1) ? rdp1 : rdp0) + i * 8 * 128);
-                if (m0 + wm * 64 + wn * 32 + rr + i * 8 < p.M) {
-                    const u32x4 vv = {v.x, v.y, v.z, v.w};
-                    __builtin_nontemporal_store(vv, reinterpret_cast<u32x4*>(cu + i * cstep + coff));
-                }
-            }
-        } else {
-            // per 32 output rows: 32 rows x 128 bytes in this wavefront's own 4 KiB, then out as whole lines
-            uint8_t* stage = smem + a4 + wave * (32 * BK);
-            uint8_t* wr = stage + row * 128 + khalf * 8;
-            const uint8_t* rdp0 = stage + rr * 128 + ((rc ^ (rr >> 1)) << 4);
-            const uint8_t* rdp1 = stage + rr * 128 + ((rc ^ (rr >> 1) ^ 4) << 4);
-            uint8_t* cu = reinterpret_cast<uint8_t*>(p.C + static_cast<size_t>(m0 + wm * 64) * p.ldc + n0 + wn * 64);
-            const uint32_t coff = (static_cast<uint32_t>(rr) * static_cast<uint32_t>(p.ldc) + rc * 8u) * 2u;
-            const size_t cstep = static_cast<size_t>(p.ldc) * 16;
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g) {
-                        const float c4[4] = {cs[a][g].x, cs[a][g].y, cs[a][g].z, cs[a][g].w};
-                        float v[4];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) v[q] = acc[a][b][g * 4 + q] * (sa[b] * c4[q]);
-                        *reinterpret_cast<uint2*>(wr + (((a * 4 + g) ^ wswz) << 4)) =
-                            make_uint2(pack_bf16x2_hw(v[0], v[1]), pack_bf16x2_hw(v[2], v[3]));
-                    }
-                __builtin_amdgcn_sched_barrier(0);
-                if (b == 0) __builtin_amdgcn_s_waitcnt(kWaitVm0);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint4 v = *reinterpret_cast<const uint4*>(((i & 1) ? rdp1 : rdp0) + i * 8 * 128);
-                    if (m0 + wm * 64 + b * 32 + rr + i * 8 < p.M) {
-                        const u32x4 vv = {v.x, v.y, v.z, v.w};
-                        __builtin_nontemporal_store(vv, reinterpret_cast<u32x4*>(cu + (b * 4 + i) * cstep + coff));
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        static_for<0, 8>([&](auto ic) { read_one(a0, a1, C0{}, ic); });
-    }
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-}
-
 // ---- block-scaled ring kernel ---------------------------------------------------------------
 // The block-scaled GEMM on the persistent direct-to-LDS structure.  Needs K % 128 == 0, K >= 384,
 // N % 256 == 0, operands smaller than 4 GiB, K / 128 <= 256.
@@ -2258,25 +1895,6 @@ __global__ __launch_bounds__(256) void k_gemm_nt_naive(const GemmArgs p, int fmt
     p.C[static_cast<size_t>(m) * p.ldc + n] = f32_to_bf16(v);
 }
 
-inline int num_cus() {
-    static int n = [] {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return 256;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) return 256;
-        return v;
-    }();
-    return n;
-}
-
-// Workgroups of a persistent launch over `total` tiles, at most `most`: a multiple of 8, which the tile walk needs to keep
-// "position % 8 = XCD", rounded UP while there is room.  (Rounded down, 44 tiles ran on 40 workgroups, four of which then
-// had two tiles: 44 us instead of 22 for 256 x 2 x 5632 x 2048.)  A workgroup without a tile returns at once.
-inline int persistent_grid(int total, int most) {
-    if (total < kXcds) return total;
-    const int up = (total + kXcds - 1) / kXcds * kXcds;
-    return up <= most ? up : most / kXcds * kXcds;
-}
-
 template <int FMT, int EPI, int SCALE>
 int launch_tiled(const GemmArgs& p, hipStream_t st) {
     static std::once_flag once;
@@ -2336,44 +1954,6 @@ int launch_tiled(const GemmArgs& p, hipStream_t st) {
     }
     k_gemm_nt<FMT, EPI, SCALE><<<p.tiles_m * p.tiles_n, kThreads, kLdsBytes, st>>>(p);
     return launch_status();
-}
-
-// the duo kernel: E4M3 operands, per-row x per-channel scales, plain or SiLU-gate epilogue, whole column tiles
-template <int EPI>
-int launch_duo(GemmArgs p, hipStream_t st) {
-    static std::once_flag once;
-    static hipError_t err = hipSuccess;
-    std::call_once(once, [] {
-        err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_nt_duo<EPI, true>), hipFuncAttributeMaxDynamicSharedMemorySize, kDuoLds);
-        if (err == hipSuccess)
-            err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_nt_duo<EPI, false>), hipFuncAttributeMaxDynamicSharedMemorySize, kDuoLds);
-    });
-    if (err != hipSuccess) return static_cast<int>(err);
-    constexpr int out_bn = EPI == EPI_SILU_GATE ? DM / 2 : DM;
-    p.tiles_m = (p.M + DM - 1) / DM;
-    p.tiles_n = p.N / out_bn;
-    const int total = p.tiles_m * p.tiles_n;
-    const int grid = persistent_grid(total, 2 * num_cus());
-    if (p.duo != 1) k_gemm_nt_duo<EPI, false><<<grid, kThreads, kDuoLds, st>>>(p);
-    else            k_gemm_nt_duo<EPI, true><<<grid, kThreads, kDuoLds, st>>>(p);
-    return launch_status();
-}
-inline bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
-    const int out_bn = epi == EPI_SILU_GATE ? DM / 2 : DM;
-    return fmt == 0 && scale_mode == SCALE_ROWCOL && (epi == EPI_NONE || epi == EPI_SILU_GATE) && !p.tile_map && p.K % BK == 0 &&
-           p.K >= 2 * BK && p.N % out_bn == 0 && p.ldc % 8 == 0 && aligned16(p.C) && aligned16(p.sb) &&
-           (epi != EPI_SILU_GATE || aligned16(p.sb2)) && static_cast<size_t>(p.M) * p.lda < (1ull << 32) &&
-           static_cast<size_t>(p.N) * p.ldb < (1ull << 32);
-}
-
-// Its time on a dense problem, microseconds: 0.48 a K-tile where a CU holds one of its workgroups, 0.875 for both where it
-// holds two (measured, 4096 columns, K 4096 to 14336).
-float duo_estimate_us(const GemmArgs& p, int epi) {
-    const int out_bn = epi == EPI_SILU_GATE ? DM / 2 : DM;
-    const long long wgs = static_cast<long long>((p.M + DM - 1) / DM) * (p.N / out_bn);
-    const long long full = wgs / 512, rest = wgs % 512;
-    const float kt = static_cast<float>(p.K / BK);
-    return static_cast<float>(full) * (kt * 0.875f + 2.5f) + (rest == 0 ? 0.0f : (rest > 256 ? kt * 0.875f : kt * 0.48f) + (full ? 0.0f : 2.5f));
 }
 
 template <int FMT, int EPI>
@@ -2479,32 +2059,20 @@ float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile,
     const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
     return static_cast<float>((tiles + 255) / 256) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
 }
+float persistent_estimate_us(const GemmArgs& p, int epi) {
+    const bool gate = epi == EPI_SILU_GATE, f32 = epi == EPI_ACCUM_F32, accum = f32 || epi == EPI_ACCUM_BF16;
+    const bool ring = p.K % BK == 0 && p.ldc % 8 == 0 && (gate ? p.N % (BN / 2) == 0 : accum ? p.N % BN == 0 : p.N % 8 == 0);
+    // a tile's epilogue; the accumulating ones read and write a round's C (134 MB fp32) with the matrix cores idle
+    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.0f : f32 ? 25.0f : accum ? 14.0f : 6.0f);
+}
 float tiled_estimate_us(const GemmArgs& p, int fmt, int epi, int scale_mode) {
     if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, p.K % BK == 0 && p.N % BN == 0 ? 0.72f : 2.0f, 5.0f);
-    const bool ring = p.K % BK == 0 && (epi == EPI_SILU_GATE ? p.N % (BN / 2) == 0 : p.N % 8 == 0) && p.ldc % 8 == 0;
-    float best = ring_estimate_us(p.M, p.N, p.K, BM, epi == EPI_SILU_GATE ? BN / 2 : BN, ring ? 0.95f : 2.0f, epi == EPI_SILU_GATE ? 10.0f : 6.0f);
+    float best = persistent_estimate_us(p, epi);
     if (duo_ok(p, fmt, epi, scale_mode)) {
         const float duo = duo_estimate_us(p, epi);
         if (duo < best) best = duo;
     }
     return best;
-}
-DirectArgs direct_args(const GemmArgs& p, int epi, int scale_mode) {
-    DirectArgs d{};
-    d.M = p.M; d.N = p.N; d.K = p.K;
-    d.A = p.A; d.lda = p.lda;
-    d.B = p.B; d.ldb = p.ldb;
-    d.B2 = p.B2;
-    d.sa = p.sa; d.sb = p.sb; d.sb2 = p.sb2;
-    d.bias = p.bias;
-    d.C = p.C; d.ldc = p.ldc;
-    d.epi = epi;
-    d.scale_rowcol = scale_mode == SCALE_ROWCOL;
-    d.c_vec = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0;
-    d.tile_map = p.tile_map; d.tiles_m = p.tiles_m;
-    d.a_row_index = p.a_row_index;
-    d.b_expert_stride = p.b_expert_stride; d.sb_expert_stride = p.sb_expert_stride;
-    return d;
 }
 
 int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_stream_t stream) {
@@ -2532,7 +2100,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         int shape = 0;
         const float direct = direct_estimate_us(p.M, p.N, p.K, epi == EPI_SILU_GATE, scale_mode == SCALE_BLOCK, &shape);
         if (direct < tiled_estimate_us(p, fmt, epi, scale_mode)) {
-            const int rc = gemm_nt_direct(direct_args(p, epi, scale_mode), fmt, epi == EPI_SILU_GATE, scale_mode == SCALE_BLOCK, shape, st);
+            const int rc = gemm_nt_direct(p, fmt, epi, scale_mode, shape, st);
             if (rc != CF_ERR_UNSUPPORTED) return rc;
         }
     }
@@ -2566,6 +2134,9 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         k_gemm_nt_block<<<p.tiles_m * p.tiles_n, kThreads, kBlkLds, st>>>(p);
         return launch_status();
     }
+    if (duo_ok(p, fmt, epi, scale_mode) &&
+        (p.duo || (!p.force_staged && !p.ring && duo_estimate_us(p, epi) < persistent_estimate_us(p, epi))))
+        return gemm_nt_duo(p, fmt, epi, scale_mode, st);
     const int out_bn = epi == EPI_SILU_GATE ? BN / 2 : BN;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + out_bn - 1) / out_bn;
@@ -2581,9 +2152,6 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         }
     }
     if (fmt & 2) return CF_ERR_UNSUPPORTED;     // forward weights are always E4M3
-    if (duo_ok(p, fmt, epi, scale_mode) &&
-        (p.duo || (!p.force_staged && !p.ring && duo_estimate_us(p, epi) < ring_estimate_us(p.M, p.N, p.K, BM, out_bn, 0.95f, epi == EPI_SILU_GATE ? 10.0f : 6.0f))))
-        return epi == EPI_SILU_GATE ? launch_duo<EPI_SILU_GATE>(p, st) : launch_duo<EPI_NONE>(p, st);
     return (fmt & 1) ? dispatch_epi<1>(p, epi, scale_mode, st) : dispatch_epi<0>(p, epi, scale_mode, st);
 }
 
@@ -2793,7 +2361,7 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
         const float direct = grouped_direct_estimate_us(total_rows, N, K, num_experts, gate, &shape);
         const int row_tiles = total_rows < num_experts ? total_rows : num_experts;
         if (direct < ring_estimate_us(row_tiles * BM, N, K, BM, out_bn, 0.95f, 6.0f)) {
-            const int rc = grouped_gemm_nt_direct(direct_args(p, epilogue, scale_mode), a_is_e5m2, gate, shape, st);
+            const int rc = grouped_gemm_nt_direct(p, a_is_e5m2, epilogue, shape, st);
             if (rc != CF_ERR_UNSUPPORTED) return rc;
         }
     }
@@ -2894,6 +2462,8 @@ int cf_fp8_gemm_nt_accum_f32_ex(int M, int N, int K, const void* A, int lda, int
     p.sa = a_descale; p.sb = b_descale;
     p.Cf = C; p.ldc = ldc;
     p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;
+    p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) == CF_GEMM_FLAG_DUO_IN_STEP ? 2 : 1) : 0;
+    p.ring = (flags & CF_GEMM_FLAG_RING) != 0;
     return gemm_nt(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), EPI_ACCUM_F32, SCALE_TENSOR,
                    flags & CF_GEMM_FLAG_NAIVE, stream);
 }

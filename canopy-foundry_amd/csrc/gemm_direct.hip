@@ -13,32 +13,12 @@
 // Reading the operands from memory straight into registers was built first: a lane's MFMA row is lane % 16, so 16 consecutive
 // lanes read 16 different lines, and the same L2s delivered 8.6 TB/s (16 rows 15.0 us, 256 rows 52 us).  Copies to LDS take
 // whole 128-byte lines, eight lanes each.
-#include "common.hpp"
-#include "internal.hpp"
+#include "gemm_common.hpp"
 
 #include <mutex>
-#include <type_traits>
 
 namespace cf {
 namespace {
-
-constexpr int kXcds = 8;
-constexpr int kMapWords = 5;          // words per entry of the row-tile table (build_tile_map)
-constexpr int kMapRows = 256;         // rows of a table entry
-constexpr int BK = 128;
-
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
-
-__device__ __forceinline__ float fast_silu(float x) {
-    const float e = __builtin_amdgcn_exp2f(-1.44269504f * x);
-    return x * __builtin_amdgcn_rcpf(1.0f + e);
-}
 
 // vmcnt(n), the other counters left alone
 constexpr int wait_vm(int n) { return 0x0f70 | (n & 15) | ((n >> 4) << 14); }
@@ -47,7 +27,7 @@ constexpr int kWaitLgkm0 = 0xc07f;
 template <int FMT, bool GATE, bool BLOCK, bool GROUPED, int MB, int NB, int WK, int S>
 // BLOCK: two wavefronts per SIMD at most 256 registers each, so that the products land where the vector ALU can fold them
 __global__ __launch_bounds__(64 * WK) __attribute__((amdgpu_waves_per_eu(BLOCK ? 2 : 1)))
-void k_gemm_nt_direct(const DirectArgs p) {
+void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const int c_vec) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int NT = GATE ? 2 * NB : NB;          // weight blocks: NB gate blocks, then NB up blocks
     constexpr int TM = 16 * MB, TN = 16 * NB;
@@ -70,8 +50,8 @@ void k_gemm_nt_direct(const DirectArgs p) {
         if (tm >= p.tile_map[0]) return;
         const int* e = p.tile_map + 1 + kMapWords * tm;
         expert = __builtin_amdgcn_readfirstlane(e[0]);
-        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (tm - __builtin_amdgcn_readfirstlane(e[3])) * kMapRows;
-        m_end = min(m_first + kMapRows, __builtin_amdgcn_readfirstlane(e[2]));
+        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (tm - __builtin_amdgcn_readfirstlane(e[3])) * BM;
+        m_end = min(m_first + BM, __builtin_amdgcn_readfirstlane(e[2]));
     }
     const uint8_t* B = p.B + static_cast<size_t>(expert) * p.b_expert_stride;
     const uint8_t* B2 = GATE ? p.B2 + static_cast<size_t>(expert) * p.b_expert_stride : B;
@@ -128,9 +108,9 @@ void k_gemm_nt_direct(const DirectArgs p) {
             const float* sb2 = GATE ? p.sb2 + static_cast<size_t>(expert) * p.sb_expert_stride : sb;
             int row = min(m0 + (tid < TM ? tid : 0), m_end - 1), col = min(n0 + (tid < TN ? tid : 0), p.N - 1);
             if (GROUPED && p.a_row_index) row = p.a_row_index[row];
-            f_row = p.sa[p.scale_rowcol ? row : 0];
-            f_col = sb[p.scale_rowcol ? col : 0];
-            if constexpr (GATE) f_col2 = sb2[p.scale_rowcol ? col : 0];
+            f_row = p.sa[rowcol ? row : 0];
+            f_col = sb[rowcol ? col : 0];
+            if constexpr (GATE) f_col2 = sb2[rowcol ? col : 0];
         }
 
         v4f acc[MB][NT];
@@ -310,12 +290,12 @@ void k_gemm_nt_direct(const DirectArgs p) {
             }
             if (m >= m_end || n >= p.N) continue;
             const bool whole = n + 3 < p.N;
-            if (p.epi == EPI_BIAS)
+            if (bias)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) v[q] = round_bf16_hw(v[q]) + bf16_to_f32(p.bias[min(n + q, p.N - 1)]);
             uint16_t* c = p.C + static_cast<size_t>(m) * p.ldc + n;
             const uint32_t o01 = pack_bf16x2_hw(v[0], v[1]), o23 = pack_bf16x2_hw(v[2], v[3]);
-            if (whole && p.c_vec) {
+            if (whole && c_vec) {
                 *reinterpret_cast<uint2*>(c) = make_uint2(o01, o23);
             } else {
                 c[0] = static_cast<uint16_t>(o01);
@@ -332,7 +312,7 @@ void k_gemm_nt_direct(const DirectArgs p) {
 constexpr int kLds = 160 * 1024;
 
 template <int FMT, bool GATE, bool BLOCK, bool GROUPED, int MB, int NB, int WK, int S>
-int launch(DirectArgs p, hipStream_t st) {
+int launch(GemmArgs p, int epi, int scale_mode, hipStream_t st) {
     constexpr int NT = GATE ? 2 * NB : NB;
     constexpr int stages = WK * S * (MB + NT) * 2048;
     constexpr int one = WK * MB * NT * 1024, sums = (one > 128 * 1024 ? one / 2 : one) + (16 * MB + 32 * NB) * 4;
@@ -350,7 +330,8 @@ int launch(DirectArgs p, hipStream_t st) {
     if (err != hipSuccess) return static_cast<int>(err);
     if (!GROUPED) p.tiles_m = (p.M + 16 * MB - 1) / (16 * MB);
     p.tiles_n = (p.N + 16 * NB - 1) / (16 * NB);
-    k_gemm_nt_direct<FMT, GATE, BLOCK, GROUPED, MB, NB, WK, S><<<p.tiles_m * p.tiles_n, 64 * WK, lds, st>>>(p);
+    k_gemm_nt_direct<FMT, GATE, BLOCK, GROUPED, MB, NB, WK, S><<<p.tiles_m * p.tiles_n, 64 * WK, lds, st>>>(
+        p, scale_mode == SCALE_ROWCOL, epi == EPI_BIAS, p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0);
     return launch_status();
 }
 
@@ -361,26 +342,26 @@ constexpr Shape kPlain[6] = {{1, 1, true, 1.5f}, {2, 2, true, 2.0f}, {4, 2, fals
 constexpr Shape kGate[4] = {{1, 2, true, 1.5f}, {2, 4, true, 2.5f}, {4, 8, false, 6.0f}, {8, 8, false, 12.0f}};
 
 template <int FMT, bool BLOCK, bool GROUPED>
-int launch_plain(const DirectArgs& p, int shape, hipStream_t st) {
+int launch_plain(const GemmArgs& p, int epi, int scale_mode, int shape, hipStream_t st) {
     switch (shape) {
-        case 0: return launch<FMT, false, BLOCK, GROUPED, 1, 1, 4, 3>(p, st);
-        case 1: return launch<FMT, false, BLOCK, GROUPED, 2, 2, 4, 2>(p, st);
-        case 2: return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, st);
-        case 3: return launch<FMT, false, BLOCK, GROUPED, 4, 4, 4, 2>(p, st);
+        case 0: return launch<FMT, false, BLOCK, GROUPED, 1, 1, 4, 3>(p, epi, scale_mode, st);
+        case 1: return launch<FMT, false, BLOCK, GROUPED, 2, 2, 4, 2>(p, epi, scale_mode, st);
+        case 2: return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, epi, scale_mode, st);
+        case 3: return launch<FMT, false, BLOCK, GROUPED, 4, 4, 4, 2>(p, epi, scale_mode, st);
         default:
             if constexpr (BLOCK || GROUPED) return CF_ERR_UNSUPPORTED;
-            else return shape == 4 ? launch<FMT, false, BLOCK, GROUPED, 8, 4, 4, 1>(p, st) : launch<FMT, false, BLOCK, GROUPED, 8, 8, 4, 1>(p, st);
+            else return shape == 4 ? launch<FMT, false, BLOCK, GROUPED, 8, 4, 4, 1>(p, epi, scale_mode, st) : launch<FMT, false, BLOCK, GROUPED, 8, 8, 4, 1>(p, epi, scale_mode, st);
     }
 }
 template <bool GROUPED>
-int launch_gate(const DirectArgs& p, int shape, hipStream_t st) {
+int launch_gate(const GemmArgs& p, int scale_mode, int shape, hipStream_t st) {
     switch (shape) {
-        case 0: return launch<0, true, false, GROUPED, 1, 1, 4, 3>(p, st);
-        case 1: return launch<0, true, false, GROUPED, 2, 2, 4, 1>(p, st);
-        case 2: return launch<0, true, false, GROUPED, 4, 4, 4, 1>(p, st);
+        case 0: return launch<0, true, false, GROUPED, 1, 1, 4, 3>(p, EPI_SILU_GATE, scale_mode, st);
+        case 1: return launch<0, true, false, GROUPED, 2, 2, 4, 1>(p, EPI_SILU_GATE, scale_mode, st);
+        case 2: return launch<0, true, false, GROUPED, 4, 4, 4, 1>(p, EPI_SILU_GATE, scale_mode, st);
         default:
             if constexpr (GROUPED) return CF_ERR_UNSUPPORTED;
-            else return launch<0, true, false, GROUPED, 8, 4, 4, 1>(p, st);
+            else return launch<0, true, false, GROUPED, 8, 4, 4, 1>(p, EPI_SILU_GATE, scale_mode, st);
     }
 }
 
@@ -420,14 +401,16 @@ float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, 
     return (rounds < 1.0f ? 1.0f : rounds) * (s[i].fixed + static_cast<float>(K) * 16.0f * static_cast<float>(s[i].mb + s[i].nt) / 93e3f);
 }
 
-int gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, bool block, int shape, hipStream_t st) {
-    if (gate) return fmt == 0 ? launch_gate<false>(p, shape, st) : CF_ERR_UNSUPPORTED;
-    if (block) return launch_plain<0, true, false>(p, shape, st);
-    return fmt == 1 ? launch_plain<1, false, false>(p, shape, st) : fmt == 0 ? launch_plain<0, false, false>(p, shape, st) : CF_ERR_UNSUPPORTED;
+int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st) {
+    if (epi == EPI_SILU_GATE) return fmt == 0 ? launch_gate<false>(p, scale_mode, shape, st) : CF_ERR_UNSUPPORTED;
+    if (scale_mode == SCALE_BLOCK) return launch_plain<0, true, false>(p, epi, scale_mode, shape, st);
+    return fmt == 1 ? launch_plain<1, false, false>(p, epi, scale_mode, shape, st)
+         : fmt == 0 ? launch_plain<0, false, false>(p, epi, scale_mode, shape, st) : CF_ERR_UNSUPPORTED;
 }
-int grouped_gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, int shape, hipStream_t st) {
-    if (gate) return fmt == 0 ? launch_gate<true>(p, shape, st) : CF_ERR_UNSUPPORTED;
-    return fmt == 1 ? launch_plain<1, false, true>(p, shape, st) : launch_plain<0, false, true>(p, shape, st);
+int grouped_gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int shape, hipStream_t st) {
+    if (epi == EPI_SILU_GATE) return fmt == 0 ? launch_gate<true>(p, SCALE_ROWCOL, shape, st) : CF_ERR_UNSUPPORTED;
+    return fmt == 1 ? launch_plain<1, false, true>(p, epi, SCALE_ROWCOL, shape, st)
+                    : launch_plain<0, false, true>(p, epi, SCALE_ROWCOL, shape, st);
 }
 
 }  // namespace cf

@@ -11,35 +11,6 @@ enum { AMAX = 0, SCALE, DESCALE, SCALE_SNAP, DESCALE_SNAP, CALIB_MIN, CALIB_MAX,
        HISTORY = 16 };
 }
 
-// Epilogues of the FP8 GEMMs (CF_EPI_* and the accumulate / fp32 forms behind other entry points)
-enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_SILU_GATE = 2, EPI_ACCUM_F32 = 3, EPI_ACCUM_BF16 = 4, EPI_STORE_F32 = 5 };
-
-// Small-tile FP8 GEMM with operands loaded straight into registers (gemm_direct.hip)
-struct DirectArgs {
-    int M, N, K;
-    const uint8_t* A; int lda;
-    const uint8_t* B; int ldb;
-    const uint8_t* B2;
-    const float* sa;
-    const float* sb;
-    const float* sb2;
-    const uint16_t* bias;
-    uint16_t* C; int ldc;
-    int epi;
-    int scale_rowcol;            // 1: sa per row, sb per column; 0: one scalar each
-    int c_vec;                   // C takes 8-byte stores at multiples of four columns
-    int tiles_m, tiles_n;
-    const int* tile_map;         // grouped form: the table of build_tile_map
-    const int* a_row_index;
-    long long b_expert_stride;
-    int sb_expert_stride;
-};
-// Time of its best tile shape on this problem and which one that is, and the launches (dense; grouped over a row-tile table).
-float direct_estimate_us(int M, int N, int K, bool gate, bool block, int* shape);
-float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape);
-int gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, bool block, int shape, hipStream_t st);
-int grouped_gemm_nt_direct(const DirectArgs& p, int fmt, bool gate, int shape, hipStream_t st);
-
 // The grouped GEMM behind cf_fp8_grouped_gemm_nt_bf16_ex, for callers inside the library that run several
 // projections over one routing: build_map = false reuses the tile table an earlier call left in d_workspace;
 // a_is_e5m2 takes E5M2 activations (plain epilogue only).
