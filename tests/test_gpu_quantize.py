@@ -154,7 +154,8 @@ def test_update_delayed_scale(cf, dev, hlen, cursor, count):
             assert np.array_equal(host(hist), st.history)
 
 
-@pytest.mark.parametrize("K,N", [(128, 128), (256, 384), (1024, 2048), (1, 1), (3, 5), (65, 130), (200, 77), (128, 130)])
+@pytest.mark.parametrize("K,N", [(128, 128), (256, 384), (1024, 2048), (1, 1), (3, 5), (65, 130), (200, 77), (128, 130),
+                                 (16, 8), (112, 120), (144, 264), (2000, 136), (128, 1400), (1408, 128), (136, 128), (144, 130)])
 def test_transposing_kernels(cf, dev, K, N):
     case(f"transposes K={K} N={N}")
     rng = np.random.default_rng(K * 7 + N)
