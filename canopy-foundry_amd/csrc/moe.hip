@@ -881,16 +881,33 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma(const ui
 }
 
 // ---- 32-row form ------------------------------------------------------------------------------------
-// The 16-row kernel above re-reads its expert's weights once per 16 rows, and that traffic through the L2s is what
-// it waits for.  This form takes 32 rows per workgroup (two groups of 16 token rows against every weight fetch) and
-// still keeps the GELU output at 4 bytes per element in LDS by walking Ie in chunks: fc_in + GELU for a chunk of
-// columns, then that chunk's share of fc_out added into accumulators that stay in registers across chunks: a
-// wavefront owns the output blocks wave, wave + 8, ... (H / 128 of them, at most kWideBlocks: H <= 2048), two
-// accumulators each.  Blocks are walked in pairs so an activation read from LDS feeds two blocks.  One rounding
-// per (row, expert) as before: the compare-and-swap comes after the last chunk.
+// The 16-row kernel above re-reads its expert's weights once per 16 rows.  This form takes 32 rows per workgroup (two groups
+// of 16 token rows against every weight fetch) and still keeps the GELU output at 4 bytes per element in LDS by walking Ie in
+// chunks: fc_in + GELU for a chunk of columns, then that chunk's share of fc_out added into accumulators that stay in
+// registers across chunks: a wavefront owns the output blocks wave, wave + 8, ... (H / 128 of them, at most kWideBlocks:
+// H <= 2048), two accumulators each.  One rounding per (row, expert) as before: the compare-and-swap comes after the last chunk.
+// What bounds it is how fast a CU gets the weights into the MFMAs' layout: there, 16 neighbouring lanes hold 16 rows, and a
+// load so addressed touches a line per lane (25 bytes a nanosecond and CU).  So weights are fetched as runs of 64 or 128
+// bytes of a row by neighbouring lanes and turned in 4 KiB of LDS per wavefront; the sums go to `mixed` as whole rows.
+// 2048 tokens, 6 of 64 experts, 2048 x 1408: 620 -> 375 us (the swaps alone 160 us of the former); 64 tokens 280 -> 187.
 constexpr int kWideRows = 32;
 constexpr int kWideBlocks = 16;
-constexpr int kWideDepth = 2;
+constexpr int kWideInDepth = 4;     // weight fetches in flight per wavefront in fc_in
+constexpr int kWideGroup = 4;          // output blocks that share an activation read
+constexpr int kWideTurn = 4096;        // bytes per wavefront in which weights change from lines of memory to MFMA operands
+
+// LDS rows: 16 lanes of neighbouring token rows read the same k, and the LDS serves lanes 0-7 of one k-group together with
+// lanes 8-15 of the next (0 with 1, 2 with 3).  The row stride is 16 bytes beyond a multiple of 256, so 8 rows cover half of
+// the banks and 16 all of them, if the two k-groups are a multiple of 256 bytes apart: the pieces of neighbouring 128-element
+// runs are interleaved to make it so.  Positions of hidden byte k (32 per k-group and step) and activation element k (16):
+__device__ __host__ __forceinline__ int wide_hidden_at(int k) {
+    return (k & ~511) | ((k >> 5 & 1) << 8) | ((k >> 7 & 3) << 6) | ((k >> 6 & 1) << 5) | (k & 31);
+}
+__device__ __host__ __forceinline__ int wide_act_at(int k) {
+    return (k & ~255) | ((k >> 4 & 1) << 7) | ((k >> 5 & 7) << 4) | (k & 15);
+}
+__device__ __host__ __forceinline__ int wide_hidden_stride(int H) { return (H + 511) / 512 * 512 + 16; }        // bytes
+__device__ __host__ __forceinline__ int wide_act_stride(int chunk) { return (chunk + 255) / 256 * 256 + 8; }     // elements
 
 template <bool E5M2>
 __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const uint8_t* __restrict__ hidden, const float* __restrict__ fcin_descale,
@@ -901,11 +918,11 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
                                                                           int rows, int H, int Ie, int E, int tiles_per_expert, int chunk) {
     extern __shared__ __align__(16) uint8_t smem[];
     constexpr int kWaves = kMfmaThreads / 64;
-    const int hs = H + 16;                          // hidden row stride in bytes
-    const int as = chunk + 8;                       // activation row stride in elements
+    const int hs = wide_hidden_stride(H), as = wide_act_stride(chunk);
     uint8_t* sh_hidden = smem;                                                        // [32][hs] fp8
     uint16_t* sh_hi = reinterpret_cast<uint16_t*>(smem + kWideRows * hs);             // [32][as] bf16 head of gelu
     uint16_t* sh_lo = sh_hi + kWideRows * as;                                         // [32][as] bf16 remainder
+    uint8_t* sh_turn = reinterpret_cast<uint8_t*>(sh_lo + kWideRows * as);            // [8 wavefronts][4 KiB], private to each
     const int xcd = blockIdx.x % kXcdCount, slot = blockIdx.x / kXcdCount;
     const int e = (slot / tiles_per_expert) * kXcdCount + xcd, tile = slot % tiles_per_expert;
     if (e >= E) return;
@@ -915,17 +932,23 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
     const int* my_rows = row_indices + static_cast<size_t>(e) * rows + first;
     const uint8_t* w_in = fc_in_w + static_cast<size_t>(e) * H * Ie;
     const uint8_t* w_out = fc_out_w + static_cast<size_t>(e) * Ie * H;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = lane & 15, g = lane >> 4;
 
     const int vec_per_row = H / 16;
     for (int i = threadIdx.x; i < kWideRows * vec_per_row; i += kMfmaThreads) {
         const int r = i / vec_per_row, c = i % vec_per_row;
         const int src = my_rows[min(r, n_rows - 1)];
-        *reinterpret_cast<uint4*>(sh_hidden + r * hs + c * 16) =
+        *reinterpret_cast<uint4*>(sh_hidden + r * hs + wide_hidden_at(c * 16)) =
             *reinterpret_cast<const uint4*>(hidden + static_cast<size_t>(src) * H + c * 16);
     }
     __syncthreads();
 
+    uint8_t* turn = sh_turn + wave * kWideTurn;
+    // orders a wavefront's own LDS writes and reads (the LDS serves them in order: nothing to wait for)
+    auto turned = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     const float s_in = *fcin_descale * *fc_in_descale;
     const int in_steps = H / 128;
     const int nblk = H / 128;                       // output blocks of this wavefront
@@ -939,34 +962,56 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
     for (int c0 = 0; c0 < Ie; c0 += chunk) {
         const int cw = min(chunk, Ie - c0);         // a multiple of 64
         // ---- fc_in + GELU for columns c0 .. c0 + cw - 1 ----
+        // A step is 16 weight rows x 128 bytes, fetched 8 lanes to a row and turned in LDS.  One stream of fetches over the
+        // wavefront's column blocks, kWideInDepth steps ahead: the first ones of the next block are requested under the last
+        // ones of this.  in_pad: steps of a block, rounded up to the ring's length.
+        const int in_pad = (in_steps + kWideInDepth - 1) / kWideInDepth * kWideInDepth;
+        // addresses are a scalar base plus one 32-bit lane offset, here and in fc_out: the registers go to the fetches
+        const uint32_t in_lane = static_cast<uint32_t>(lane >> 3) * static_cast<uint32_t>(H) + (lane & 7) * 16;
+        v4u w0[kWideInDepth], w1[kWideInDepth];
+        auto fetch_in = [&](int j, int n0, int st) {          // clamped, not skipped: loads under a condition cannot be counted
+            const uint8_t* wr = w_in + static_cast<size_t>(c0 + min(n0, cw - 16)) * H + min(st, in_steps - 1) * 128;
+            w0[j] = *reinterpret_cast<const v4u*>(wr + in_lane);
+            w1[j] = *reinterpret_cast<const v4u*>(wr + static_cast<size_t>(8) * H + in_lane);
+        };
+        // row r's 16-byte piece c sits at slot c ^ (r / 2): rows 0-7 of one k-group and 8-15 of the next fill 256 bytes each
+        uint8_t* in_put = turn + (lane >> 3) * 128;
+        const int in_put0 = ((lane & 7) ^ (lane >> 4)) << 4, in_put1 = ((lane & 7) ^ (4 + (lane >> 4))) << 4;
+        const uint8_t* in_get = turn + t * 128;
+        const int in_get0 = ((2 * g) ^ (t >> 1)) << 4, in_get1 = ((2 * g + 1) ^ (t >> 1)) << 4;
+#pragma unroll
+        for (int j = 0; j < kWideInDepth; ++j) fetch_in(j, wave * 16, j);
         for (int n0 = wave * 16; n0 < cw; n0 += kWaves * 16) {
             v4f a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = {0.0f, 0.0f, 0.0f, 0.0f};
-            const uint8_t* wr = w_in + static_cast<size_t>(c0 + n0 + t) * H + 32 * g;
-            const uint8_t* hr0 = sh_hidden + t * hs + 32 * g;
+            const uint8_t* hr0 = sh_hidden + t * hs + wide_hidden_at(32 * g);
             const uint8_t* hr1 = hr0 + 16 * hs;
-            uint4 w0[kWideDepth], w1[kWideDepth];
+            for (int s0 = 0; s0 < in_pad; s0 += kWideInDepth) {
+                const bool last = s0 + kWideInDepth == in_pad;
 #pragma unroll
-            for (int j = 0; j < kWideDepth; ++j)
-                if (j < in_steps) {
-                    w0[j] = *reinterpret_cast<const uint4*>(wr + j * 128);
-                    w1[j] = *reinterpret_cast<const uint4*>(wr + j * 128 + 16);
-                }
-            for (int s0 = 0; s0 < in_steps; s0 += kWideDepth) {
+                for (int j = 0; j < kWideInDepth; j += 2) {             // two steps to a turn
+                    turned();
 #pragma unroll
-                for (int j = 0; j < kWideDepth; ++j) {
-                    const int st = s0 + j;
-                    if (st < in_steps) {
-                        const v8i a = {(int)w0[j].x, (int)w0[j].y, (int)w0[j].z, (int)w0[j].w, (int)w1[j].x, (int)w1[j].y, (int)w1[j].z, (int)w1[j].w};
-                        if (st + kWideDepth < in_steps) {
-                            w0[j] = *reinterpret_cast<const uint4*>(wr + (st + kWideDepth) * 128);
-                            w1[j] = *reinterpret_cast<const uint4*>(wr + (st + kWideDepth) * 128 + 16);
+                    for (int q = 0; q < 2; ++q) {
+                        *reinterpret_cast<v4u*>(in_put + q * 2048 + in_put0) = w0[j + q];
+                        *reinterpret_cast<v4u*>(in_put + q * 2048 + 1024 + in_put1) = w1[j + q];
+                        fetch_in(j + q, last ? n0 + kWaves * 16 : n0, last ? j + q : s0 + j + q + kWideInDepth);
+                    }
+                    turned();
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const int st = s0 + j + q;
+                        if (st < in_steps) {
+                            const uint4 u0 = *reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get0);
+                            const uint4 u1 = *reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get1);
+                            const v8i a = {(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
+                            const int at = wide_hidden_at(st * 128);
+                            const uint4 x0 = *reinterpret_cast<const uint4*>(hr0 + at), x1 = *reinterpret_cast<const uint4*>(hr0 + at + 16);
+                            const uint4 y0 = *reinterpret_cast<const uint4*>(hr1 + at), y1 = *reinterpret_cast<const uint4*>(hr1 + at + 16);
+                            const v8i b0 = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
+                            const v8i b1 = {(int)y0.x, (int)y0.y, (int)y0.z, (int)y0.w, (int)y1.x, (int)y1.y, (int)y1.z, (int)y1.w};
+                            a0 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b0, a0, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
+                            a1 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b1, a1, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
                         }
-                        const uint4 x0 = *reinterpret_cast<const uint4*>(hr0 + st * 128), x1 = *reinterpret_cast<const uint4*>(hr0 + st * 128 + 16);
-                        const uint4 y0 = *reinterpret_cast<const uint4*>(hr1 + st * 128), y1 = *reinterpret_cast<const uint4*>(hr1 + st * 128 + 16);
-                        const v8i b0 = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
-                        const v8i b1 = {(int)y0.x, (int)y0.y, (int)y0.z, (int)y0.w, (int)y1.x, (int)y1.y, (int)y1.z, (int)y1.w};
-                        a0 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b0, a0, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
-                        a1 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b1, a1, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
                     }
                 }
             }
@@ -980,117 +1025,110 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
                     hb[r] = __float_as_uint(act) & 0xffff0000u;
                     lb[r] = f32_to_bf16(act - __uint_as_float(hb[r]));
                 }
-                const int at = (tg * 16 + t) * as + n0 + 4 * g;
+                const int at = (tg * 16 + t) * as + wide_act_at(n0 + 4 * g);
                 *reinterpret_cast<uint2*>(sh_hi + at) = make_uint2((hb[0] >> 16) | hb[1], (hb[2] >> 16) | hb[3]);
                 *reinterpret_cast<uint2*>(sh_lo + at) = make_uint2(lb[0] | (lb[1] << 16), lb[2] | (lb[3] << 16));
             }
         }
-        __syncthreads();
-
         // ---- this chunk's share of fc_out ----
-        const int steps = cw / 128, tail = steps * 128;     // whole 128-byte runs of the chunk; cw % 128 == 64 leaves half a run
-        const uint32_t lane_row = static_cast<uint32_t>(wave * 16 + t) * static_cast<uint32_t>(Ie);
-        const uint16_t* ah0 = sh_hi + t * as;
-        const uint16_t* al0 = sh_lo + t * as;
-        const uint16_t* ah1 = ah0 + 16 * as;
-        const uint16_t* al1 = al0 + 16 * as;
+        // Four blocks at a time (an activation read feeds eight MFMAs).  A step is 64 k: 64 bytes of each of a block's 16 weight
+        // rows, fetched 4 lanes to a row and turned in LDS; one stream of fetches over the groups of blocks, two steps ahead.
+        const int steps = cw / 64, out_pad = (steps + 1) & ~1;
+        const uint32_t out_lane = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(Ie) + (lane & 3) * 16;
+        // the weights of this wavefront's block blk (past the last one: that one again; those sums are not used)
+        auto block = [&](int blk) { return w_out + c0 + static_cast<size_t>((min(blk, nblk - 1) * kWaves + wave) * 16) * Ie; };
+        v4u w[2][kWideGroup];
+        auto fetch_out = [&](int j, int blk, int st) {
 #pragma unroll
-        for (int bp = 0; bp < kWideBlocks; bp += 2) {
-            if (bp < nblk) {
-                // rows of the two blocks' weights (the second repeats the first where nblk is odd; its sums are not used)
-                // uniform base + 32-bit lane offsets: no 64-bit per-lane addresses to keep alive across the pairs
-                const int bq = bp + 1 < nblk ? bp + 1 : bp;
-                const uint8_t* wbase = w_out + c0;
-                const uint32_t oA = lane_row + static_cast<uint32_t>(kWaves * 16 * bp) * static_cast<uint32_t>(Ie);
-                const uint32_t oB = lane_row + static_cast<uint32_t>(kWaves * 16 * bq) * static_cast<uint32_t>(Ie);
-                auto ldw = [&](uint32_t off) { return *reinterpret_cast<const uint4*>(wbase + off); };
-                v4f pA0 = acc[bp][0], pA1 = acc[bp][1], pB0 = acc[bp + 1][0], pB1 = acc[bp + 1][1];
-                auto mm = [&](uint32_t xa, uint32_t ya, uint32_t xb, uint32_t yb, int k) {
-                    const v8bf wa = e4m3x8_to_bf16(xa, ya), wb = e4m3x8_to_bf16(xb, yb);
-                    const v8bf h0 = *reinterpret_cast<const v8bf*>(ah0 + k), h1 = *reinterpret_cast<const v8bf*>(ah1 + k);
-                    const v8bf l0 = *reinterpret_cast<const v8bf*>(al0 + k), l1 = *reinterpret_cast<const v8bf*>(al1 + k);
-                    pA0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, h0, pA0, 0, 0, 0);
-                    pA1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, h1, pA1, 0, 0, 0);
-                    pB0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, h0, pB0, 0, 0, 0);
-                    pB1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, h1, pB1, 0, 0, 0);
-                    pA0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, l0, pA0, 0, 0, 0);
-                    pA1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, l1, pA1, 0, 0, 0);
-                    pB0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, l0, pB0, 0, 0, 0);
-                    pB1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, l1, pB1, 0, 0, 0);
-                };
-                uint4 a0[kWideDepth], a1[kWideDepth], b0[kWideDepth], b1[kWideDepth];
+            for (int i = 0; i < kWideGroup; ++i) w[j][i] = *reinterpret_cast<const v4u*>(block(blk + i) + min(st, steps - 1) * 64 + out_lane);
+        };
+        fetch_out(0, 0, 0);
+        fetch_out(1, 0, 1);
+        __syncthreads();                            // the activations are complete
+        // row r's piece c sits at slot c ^ (r / 4), for the same reason as above
+        uint8_t* out_put = turn + (lane >> 2) * 64 + (((lane & 3) ^ (lane >> 4)) << 4);
+        const uint8_t* out_get = turn + t * 64 + ((g ^ (t >> 2)) << 4);
+        const int act_lane = t * as + wide_act_at(16 * g);
 #pragma unroll
-                for (int j = 0; j < kWideDepth; ++j)
-                    if (j < steps) {                                                // step s: k = 128 s + 32 g .. + 31 of the chunk
-                        a0[j] = ldw(oA + 32 * g + j * 128);
-                        a1[j] = ldw(oA + 32 * g + j * 128 + 16);
-                        b0[j] = ldw(oB + 32 * g + j * 128);
-                        b1[j] = ldw(oB + 32 * g + j * 128 + 16);
-                    }
-                for (int s0 = 0; s0 < steps; s0 += kWideDepth) {
+        for (int bg = 0; bg < kWideBlocks; bg += kWideGroup) {
+            if (bg < nblk) {
+                v4f p0[kWideGroup], p1[kWideGroup];
 #pragma unroll
-                    for (int j = 0; j < kWideDepth; ++j) {
-                        const int st = s0 + j;
-                        if (st < steps) {
-                            const uint4 ca0 = a0[j], ca1 = a1[j], cb0 = b0[j], cb1 = b1[j];
-                            if (st + kWideDepth < steps) {
-                                a0[j] = ldw(oA + 32 * g + (st + kWideDepth) * 128);
-                                a1[j] = ldw(oA + 32 * g + (st + kWideDepth) * 128 + 16);
-                                b0[j] = ldw(oB + 32 * g + (st + kWideDepth) * 128);
-                                b1[j] = ldw(oB + 32 * g + (st + kWideDepth) * 128 + 16);
+                for (int i = 0; i < kWideGroup; ++i) { p0[i] = acc[bg + i][0]; p1[i] = acc[bg + i][1]; }
+                for (int s0 = 0; s0 < out_pad; s0 += 2) {
+                    const bool last = s0 + 2 == out_pad;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        turned();
+#pragma unroll
+                        for (int i = 0; i < kWideGroup; ++i) *reinterpret_cast<v4u*>(out_put + i * 1024) = w[j][i];
+                        fetch_out(j, last ? bg + kWideGroup : bg, last ? j : s0 + j + 2);
+                        turned();
+                        if (s0 + j < steps) {
+                            uint4 x[kWideGroup];
+#pragma unroll
+                            for (int i = 0; i < kWideGroup; ++i) x[i] = *reinterpret_cast<const uint4*>(out_get + i * 1024);
+                            const int at0 = act_lane + wide_act_at((s0 + j) * 64);
+#pragma unroll
+                            for (int half = 0; half < 2; ++half) {              // eight k of this lane's two token rows
+                                const int at = at0 + 8 * half;
+                                const v8bf h0 = *reinterpret_cast<const v8bf*>(sh_hi + at), h1 = *reinterpret_cast<const v8bf*>(sh_hi + at + 16 * as);
+                                const v8bf l0 = *reinterpret_cast<const v8bf*>(sh_lo + at), l1 = *reinterpret_cast<const v8bf*>(sh_lo + at + 16 * as);
+#pragma unroll
+                                for (int i = 0; i < kWideGroup; ++i) {
+                                    const v8bf q = half ? e4m3x8_to_bf16(x[i].z, x[i].w) : e4m3x8_to_bf16(x[i].x, x[i].y);
+                                    p0[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, h0, p0[i], 0, 0, 0);
+                                    p1[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, h1, p1[i], 0, 0, 0);
+                                    p0[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, l0, p0[i], 0, 0, 0);
+                                    p1[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(q, l1, p1[i], 0, 0, 0);
+                                }
                             }
-                            const int k = st * 128 + 32 * g;
-                            mm(ca0.x, ca0.y, cb0.x, cb0.y, k);
-                            mm(ca0.z, ca0.w, cb0.z, cb0.w, k + 8);
-                            mm(ca1.x, ca1.y, cb1.x, cb1.y, k + 16);
-                            mm(ca1.z, ca1.w, cb1.z, cb1.w, k + 24);
                         }
                     }
                 }
-                if (cw & 64) {                                                      // half run: k = tail + 16 g .. + 15
-                    const uint4 ta = ldw(oA + tail + 16 * g);
-                    const uint4 tb = ldw(oB + tail + 16 * g);
-                    mm(ta.x, ta.y, tb.x, tb.y, tail + 16 * g);
-                    mm(ta.z, ta.w, tb.z, tb.w, tail + 16 * g + 8);
-                }
-                acc[bp][0] = pA0; acc[bp][1] = pA1; acc[bp + 1][0] = pB0; acc[bp + 1][1] = pB1;
+#pragma unroll
+                for (int i = 0; i < kWideGroup; ++i) { acc[bg + i][0] = p0[i]; acc[bg + i][1] = p1[i]; }
             }
         }
         __syncthreads();                            // the next chunk overwrites the activations
     }
 
-    // ---- one compare-and-swap per (token row, 4 output columns), four in flight at a time ----
+    // ---- one compare-and-swap per (token row, 4 output columns) ----
+    // Sixteen token rows at a time pass through LDS, so that a wavefront's accesses to `mixed` are 512 bytes of one row:
+    // straight from the accumulators an access covers 32 bytes of each of 16 rows.
     const float d_wout = *fc_out_descale;
+    const int ys = 4 * H + 16;                      // row stride in bytes
 #pragma unroll
     for (int tg = 0; tg < 2; ++tg) {
-        const int r = tg * 16 + t;
-        const bool live = r < n_rows;
-        const int row = live ? my_rows[r] : 0;
-        const float rw = live ? route_weights[static_cast<size_t>(row) * E + e] : 0.0f;
-        uint16_t* mrow = mixed + static_cast<size_t>(row) * H + 4 * g + wave * 16;
+        if (tg) __syncthreads();
 #pragma unroll
-        for (int b0 = 0; b0 < kWideBlocks; b0 += 4) {
-            if (b0 < nblk && live) {
+        for (int b = 0; b < kWideBlocks; ++b)
+            if (b < nblk) *reinterpret_cast<v4f*>(smem + t * ys + ((b * kWaves + wave) * 16 + 4 * g) * 4) = acc[b][tg];
+        __syncthreads();
+        for (int r = wave; r < 16 && tg * 16 + r < n_rows; r += kWaves) {
+            const int row = my_rows[tg * 16 + r];
+            const float rw = route_weights[static_cast<size_t>(row) * E + e];
+            unsigned long long* mrow = reinterpret_cast<unsigned long long*>(mixed + static_cast<size_t>(row) * H) + lane;
+            const uint8_t* y = smem + r * ys + lane * 16;
+            for (int i0 = 0; i0 < H / 4; i0 += 4 * 64) {                // four in flight at a time
                 unsigned long long before[4], got[4];
                 float v[4][4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (b0 + i < nblk)
-                        before[i] = __builtin_nontemporal_load(reinterpret_cast<unsigned long long*>(mrow + (b0 + i) * kWaves * 16));
+                    if (i0 + i * 64 + lane < H / 4) before[i] = __builtin_nontemporal_load(mrow + i0 + i * 64);
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (b0 + i < nblk) {
+                    if (i0 + i * 64 + lane < H / 4) {
+                        const v4f sum = *reinterpret_cast<const v4f*>(y + (i0 + i * 64) * 16);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) v[i][q] = rw * (acc[b0 + i][tg][q] * d_wout);
-                        got[i] = atomicCAS(reinterpret_cast<unsigned long long*>(mrow + (b0 + i) * kWaves * 16), before[i],
-                                           add_bf16x4(before[i], v[i]));
+                        for (int q = 0; q < 4; ++q) v[i][q] = rw * (sum[q] * d_wout);
+                        got[i] = atomicCAS(mrow + i0 + i * 64, before[i], add_bf16x4(before[i], v[i]));
                     }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (b0 + i < nblk && got[i] != before[i])                     // lost a race: redo from the value found
-                        atomic_add_bf16x4(reinterpret_cast<unsigned long long*>(mrow + (b0 + i) * kWaves * 16), got[i], v[i]);
+                    if (i0 + i * 64 + lane < H / 4 && got[i] != before[i])      // lost a race: redo from the value found
+                        atomic_add_bf16x4(mrow + i0 + i * 64, got[i], v[i]);
             }
-            __builtin_amdgcn_sched_barrier(0);      // keeps the groups apart: their loads hoisted together would not fit the registers
         }
     }
 }
@@ -1640,36 +1678,35 @@ int cf::expert_forward_fp8_one_kernel(const void* d_hidden, const float* d_fcin_
                                       cf_stream_t stream) {
     const bool mfma_ok = H % 128 == 0 && Ie % 64 == 0 && aligned16(d_hidden) && aligned16(d_fc_in_w) && aligned16(d_fc_out_w) &&
                          (reinterpret_cast<uintptr_t>(d_mixed) & 7u) == 0;
-    // 32 rows per workgroup where the output blocks fit a wavefront's registers and LDS holds the hidden rows plus
-    // a chunk of at least 64 activation columns: Ie is walked in the fewest equal chunks that fit
+    // 32 rows per workgroup where the output blocks fit a wavefront's registers; Ie is walked in the fewest equal chunks whose
+    // activations fit the LDS beside the hidden rows
     if (mfma_ok && H <= 128 * kWideBlocks) {
-        const long long room = 160 * 1024 - static_cast<long long>(kWideRows) * (H + 16);
-        const int max_chunk = room > 0 ? static_cast<int>(((room / (4 * kWideRows)) - 8) / 64 * 64) : 0;
-        if (max_chunk >= 64) {
-            const int passes = (Ie + max_chunk - 1) / max_chunk;
-            const int chunk = ((Ie + passes - 1) / passes + 63) / 64 * 64;
-            const size_t smem32 = static_cast<size_t>(kWideRows) * (H + 16) + 4u * kWideRows * (static_cast<size_t>(chunk) + 8);
-            static std::once_flag once32;
-            static hipError_t err32 = hipSuccess;
-            std::call_once(once32, [] {
-                err32 = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_grouped_gelu_fp8_mfma32<false>),
+        const int room = 160 * 1024 - kWideRows * wide_hidden_stride(H) - (kMfmaThreads / 64) * kWideTurn;
+        const int most = (room / (4 * kWideRows) - 8) / 256 * 256, passes = (Ie + most - 1) / most;     // >= 256 at H = 2048
+        const int chunk = ((Ie + passes - 1) / passes + 63) / 64 * 64;
+        // never less than the 16 output rows of fp32 that pass through it at the end
+        const size_t smem32 = max(static_cast<size_t>(kWideRows) * (wide_hidden_stride(H) + 4 * wide_act_stride(chunk)) + (kMfmaThreads / 64) * kWideTurn,
+                                  static_cast<size_t>(16) * (4 * static_cast<size_t>(H) + 16));
+        static std::once_flag once32;
+        static hipError_t err32 = hipSuccess;
+        std::call_once(once32, [] {
+            err32 = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_grouped_gelu_fp8_mfma32<false>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+            if (err32 == hipSuccess)
+                err32 = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_grouped_gelu_fp8_mfma32<true>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-                if (err32 == hipSuccess)
-                    err32 = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_grouped_gelu_fp8_mfma32<true>),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-            });
-            if (err32 != hipSuccess) return static_cast<int>(err32);
-            const int tiles = (rows + kWideRows - 1) / kWideRows;
-            auto launch = [&](auto kernel) {
-                kernel<<<kXcdCount * ((num_experts + kXcdCount - 1) / kXcdCount) * tiles, kMfmaThreads, smem32, as_stream(stream)>>>(
-                    static_cast<const uint8_t*>(d_hidden), d_fcin_descale, d_route_weights, d_counts, d_row_indices,
-                    static_cast<const uint8_t*>(d_fc_in_w), d_fc_in_descale, static_cast<const uint8_t*>(d_fc_out_w), d_fc_out_descale,
-                    d_mixed, rows, H, Ie, num_experts, tiles, chunk);
-            };
-            if (fcin_is_e5m2) launch(k_grouped_gelu_fp8_mfma32<true>);
-            else launch(k_grouped_gelu_fp8_mfma32<false>);
-            return launch_status();
-        }
+        });
+        if (err32 != hipSuccess) return static_cast<int>(err32);
+        const int tiles = (rows + kWideRows - 1) / kWideRows;
+        auto launch = [&](auto kernel) {
+            kernel<<<kXcdCount * ((num_experts + kXcdCount - 1) / kXcdCount) * tiles, kMfmaThreads, smem32, as_stream(stream)>>>(
+                static_cast<const uint8_t*>(d_hidden), d_fcin_descale, d_route_weights, d_counts, d_row_indices,
+                static_cast<const uint8_t*>(d_fc_in_w), d_fc_in_descale, static_cast<const uint8_t*>(d_fc_out_w), d_fc_out_descale,
+                d_mixed, rows, H, Ie, num_experts, tiles, chunk);
+        };
+        if (fcin_is_e5m2) launch(k_grouped_gelu_fp8_mfma32<true>);
+        else launch(k_grouped_gelu_fp8_mfma32<false>);
+        return launch_status();
     }
     // the matrix-core form where the shapes are whole MFMA steps and its tile fits the LDS
     const size_t smem_mfma = static_cast<size_t>(kMfmaRows) * (H + 16) + 4u * kMfmaRows * (static_cast<size_t>(Ie) + 8);

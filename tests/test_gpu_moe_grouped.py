@@ -150,7 +150,7 @@ def test_config5_full_size(cf, dev):
                                                  (300, 6, 3, 256, 320, True), (200, 4, 2, 128, 64, False), (1000, 5, 2, 384, 448, False),
                                                  (70, 3, 3, 2048, 1408, False),
                                                  # three unequal chunks of Ie in the 32-row form; H > 2048: the 16-row form
-                                                 (50, 2, 2, 2048, 1472, True), (40, 3, 2, 2304, 128, False), (90, 2, 1, 2176, 192, True)])
+                                                 (50, 2, 2, 2048, 1472, True), (60, 2, 1, 1664, 832, False), (35, 2, 2, 1152, 64, True), (40, 3, 2, 2304, 128, False), (90, 2, 1, 2176, 192, True)])
 def test_grouped_gelu_expert_bank_reference_form(cf, dev, rows, E, k, H, Ie, e5m2):
     """moe_grouped_expert_forward_fp8: per-tensor descales, float GELU intermediate, bf16 CAS accumulate."""
     case(f"grouped gelu bank rows={rows} E={E} k={k} H={H} Ie={Ie} e5m2={e5m2}")
