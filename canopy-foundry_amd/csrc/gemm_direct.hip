@@ -339,6 +339,11 @@ int launch(GemmArgs p, int epi, int scale_mode, hipStream_t st) {
 // CU's LDS, and what a workgroup costs beside its operand bytes (pipeline fill, reduction, epilogue; microseconds).
 struct Shape { int mb, nt; bool shared; float fixed; };
 constexpr Shape kPlain[6] = {{1, 1, true, 1.5f}, {2, 2, true, 2.0f}, {4, 2, false, 2.5f}, {4, 4, false, 4.0f}, {8, 4, false, 6.0f}, {8, 8, false, 12.0f}};
+// Grouped only: the first two with 64 weight rows per workgroup.  With experts enough to fill the chip many times over, the cost
+// per workgroup counts for more than their number: 64 experts of 2048 x 1408 and 6 rows each,
+// the routed layer around them 157 -> 145 us; 18 rows each 157 -> 148; 16 tokens, 1.5 rows each 129 -> 114.
+constexpr Shape kWide[2] = {{1, 4, true, 2.0f}, {2, 4, true, 2.5f}};
+constexpr int kWideShape = 6;           // shape numbers 6 and 7
 constexpr Shape kGate[4] = {{1, 2, true, 1.5f}, {2, 4, true, 2.5f}, {4, 8, false, 6.0f}, {8, 8, false, 12.0f}};
 
 template <int FMT, bool BLOCK, bool GROUPED>
@@ -349,7 +354,10 @@ int launch_plain(const GemmArgs& p, int epi, int scale_mode, int shape, hipStrea
         case 2: return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, epi, scale_mode, st);
         case 3: return launch<FMT, false, BLOCK, GROUPED, 4, 4, 4, 2>(p, epi, scale_mode, st);
         default:
-            if constexpr (BLOCK || GROUPED) return CF_ERR_UNSUPPORTED;
+            if constexpr (GROUPED) {
+                return shape == kWideShape ? launch<FMT, false, BLOCK, GROUPED, 1, 4, 4, 2>(p, epi, scale_mode, st)
+                                           : launch<FMT, false, BLOCK, GROUPED, 2, 4, 4, 1>(p, epi, scale_mode, st);
+            } else if constexpr (BLOCK) return CF_ERR_UNSUPPORTED;
             else return shape == 4 ? launch<FMT, false, BLOCK, GROUPED, 8, 4, 4, 1>(p, epi, scale_mode, st) : launch<FMT, false, BLOCK, GROUPED, 8, 8, 4, 1>(p, epi, scale_mode, st);
     }
 }
@@ -396,9 +404,17 @@ float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, 
     int i = 0;
     while (i + 1 < count && (16 * s[i].mb < 1.5f * rows + 2.0f || s[i + 1].mb == s[i].mb)) ++i;
     *shape = i;
-    const int tn = 16 * s[i].nt / (gate ? 2 : 1);
-    const float rounds = static_cast<float>(num_experts) * static_cast<float>((N + tn - 1) / tn) / 256.0f;
-    return (rounds < 1.0f ? 1.0f : rounds) * (s[i].fixed + static_cast<float>(K) * 16.0f * static_cast<float>(s[i].mb + s[i].nt) / 93e3f);
+    auto estimate = [&](const Shape& sh) {
+        const int tn = 16 * sh.nt / (gate ? 2 : 1);
+        const float rounds = static_cast<float>(num_experts) * static_cast<float>((N + tn - 1) / tn) / 256.0f;
+        return (rounds < 1.0f ? 1.0f : rounds) * (sh.fixed + static_cast<float>(K) * 16.0f * static_cast<float>(sh.mb + sh.nt) / 93e3f);
+    };
+    float best = estimate(s[i]);
+    if (!gate && i < 2 && estimate(kWide[i]) < best) {
+        best = estimate(kWide[i]);
+        *shape = kWideShape + i;
+    }
+    return best;
 }
 
 int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st) {

@@ -90,15 +90,17 @@ def test_small_tiles_block_scales(cf, dev, M, N, K):
     orc.assert_gemm_close(got[:, :N], ref, absdot, what=f"block {M}x{N}x{K}")
 
 
-@pytest.mark.parametrize("gate", [False, True])
-@pytest.mark.parametrize("scale", [1, 3])       # counts times this: 16-row tiles, then 64-row ones
-def test_small_tiles_grouped(cf, dev, gate, scale):
+# counts times `scale`: 16-row tiles, then 32- and 64-row ones; the plain form takes 64 columns instead of 16 or 32 per workgroup
+# where there are many
+@pytest.mark.parametrize("gate,scale,N", [(False, 1, 128), (False, 1, 256), (False, 1, 520), (False, 2, 256), (False, 2, 1000), (False, 3, 256),
+                                          (True, 1, 256), (True, 3, 256)])
+def test_small_tiles_grouped(cf, dev, gate, scale, N):
     """Experts without rows, with one row, with a tile and a row more, and with rows in two entries of the row-tile table."""
     counts = np.array([0, 1, 16, 17, 33, 130, 0, 3] + [0] * 16, np.int32) * scale
-    E, N, K = len(counts), 256, 384
+    E, K = len(counts), 384
     offsets = np.concatenate([[0], np.cumsum(counts)[:-1]]).astype(np.int32)
     total = int(counts.sum())
-    case(f"small-tile grouped gemm total={total} gate={gate}")
+    case(f"small-tile grouped gemm total={total} N={N} gate={gate}")
     assert total <= 40 * E
     rng = np.random.default_rng(total)
     rows = 50
