@@ -1,6 +1,6 @@
 // Scaled FP8 GEMM for gfx950:  C[M,N] = epilogue( (A[M,K] * sa) . (B[N,K] * sb)^T ).
 //
-// Calls with few rows or few tiles go to gemm_direct.hip or gemm_duo.hip (gemm_nt compares the estimates), accumulating ones
+// Calls with few rows or few tiles go to gemm_direct.hip or gemm_duo.hip (gemm_route compares the estimates), accumulating ones
 // over a short K to gemm_duo.hip.  Kernels in this file, in the order the others try them:
 //   k_gemm_nt_ring        the fast path: persistent, operand tiles copied global -> LDS without staging registers
 //                         into a ring of five 32 KiB slots, epilogue through an LDS-staged drain (plain, bias,
@@ -1895,6 +1895,32 @@ __global__ __launch_bounds__(256) void k_gemm_nt_naive(const GemmArgs p, int fmt
     p.C[static_cast<size_t>(m) * p.ldc + n] = f32_to_bf16(v);
 }
 
+// What the persistent kernels take.  The launches and the estimates of gemm_route both ask here.
+bool ring_ok(const GemmArgs& p, int epi, int scale_mode) {
+    // operand rows are addressed by 32-bit byte offsets
+    if (p.K % BK != 0 || p.K < 2 * BK || static_cast<size_t>(p.a_rows) * p.lda >= (1ull << 32) ||
+        static_cast<size_t>(p.N) * p.ldb >= (1ull << 32))
+        return false;
+    // the accumulating drains add into full-width tiles with 16-byte (bf16 C: 8-byte) accesses
+    if (epi == EPI_ACCUM_F32) return p.N % BN == 0 && p.ldc % 4 == 0 && aligned16(p.Cf);
+    if (epi == EPI_ACCUM_BF16) return p.N % BN == 0 && p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0;
+    // the bf16 drains write full-width tiles with 16-byte stores and read the channel descales as float4
+    // (N may cut the last column tile short at a multiple of 8; the fused gate/up form interleaves two weight
+    // matrices per tile and keeps whole tiles)
+    if (epi == EPI_SILU_GATE ? p.N % (BN / 2) != 0 : p.N % 8 != 0 || p.N < 8) return false;
+    if (p.ldc % 8 != 0 || !aligned16(p.C)) return false;
+    if (scale_mode == SCALE_ROWCOL && (!aligned16(p.sb) || p.sb_expert_stride % 4 != 0 || (epi == EPI_SILU_GATE && !aligned16(p.sb2))))
+        return false;
+    return epi != EPI_BIAS || aligned16(p.bias);
+}
+// of those, what the kernel on the 16 x 16 x 128 MFMA takes: the bf16 epilogues on an even number of K-tiles
+bool ring16_ok(const GemmArgs& p) { return !p.mfma32 && (p.K / BK) % 2 == 0; }
+bool block_ring_ok(const GemmArgs& p) {
+    const int kb = p.K / BK;
+    return p.K % BK == 0 && kb >= 3 && kb <= kBsMaxKb && p.N % BN == 0 && static_cast<size_t>(p.M) * p.lda < (1ull << 32) &&
+           static_cast<size_t>(p.N) * p.ldb < (1ull << 32) && static_cast<size_t>(p.M) * kb * 4 < (1ull << 32);
+}
+
 template <int FMT, int EPI, int SCALE>
 int launch_tiled(const GemmArgs& p, hipStream_t st) {
     static std::once_flag once;
@@ -1904,27 +1930,7 @@ int launch_tiled(const GemmArgs& p, hipStream_t st) {
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     });
     if (attr_err != hipSuccess) return static_cast<int>(attr_err);
-    // the ring kernel addresses operand rows by 32-bit byte offsets
-    bool ring_ok = p.K % BK == 0 && p.K >= 2 * BK && static_cast<size_t>(p.a_rows) * p.lda < (1ull << 32) &&
-                   static_cast<size_t>(p.N) * p.ldb < (1ull << 32);
-    if constexpr (EPI == EPI_ACCUM_F32) {
-        // its drain adds into full-width fp32 tiles with 16-byte accesses
-        ring_ok = ring_ok && p.N % BN == 0 && p.ldc % 4 == 0 && aligned16(p.Cf);
-    }
-    if constexpr (EPI == EPI_ACCUM_BF16) {
-        // the same with 8-byte accesses to bf16 tiles
-        ring_ok = ring_ok && p.N % BN == 0 && p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 7u) == 0;
-    }
-    if constexpr (EPI == EPI_NONE || EPI == EPI_BIAS || EPI == EPI_SILU_GATE) {
-        // its drain writes full-width tiles with 16-byte stores and reads the channel descales as float4
-        // (N may cut the last column tile short at a multiple of 8; the fused gate/up form interleaves two weight
-        // matrices per tile and keeps whole tiles)
-        ring_ok = ring_ok && (EPI == EPI_SILU_GATE ? p.N % (BN / 2) == 0 : p.N % 8 == 0 && p.N >= 8) && p.ldc % 8 == 0 && aligned16(p.C);
-        if (SCALE == SCALE_ROWCOL)
-            ring_ok = ring_ok && aligned16(p.sb) && p.sb_expert_stride % 4 == 0 && (EPI != EPI_SILU_GATE || aligned16(p.sb2));
-        if (EPI == EPI_BIAS) ring_ok = ring_ok && aligned16(p.bias);
-    }
-    if (ring_ok && !p.force_staged) {
+    if (ring_ok(p, EPI, SCALE) && !p.force_staged) {
         static std::once_flag once_ring;
         static hipError_t ring_err = hipSuccess;
         std::call_once(once_ring, [] {
@@ -1936,8 +1942,7 @@ int launch_tiled(const GemmArgs& p, hipStream_t st) {
         const int total = p.tiles_m * p.tiles_n;     // grouped: tiles_m is the host-side upper bound of row tiles
         const int grid = persistent_grid(total, num_cus());
         if constexpr (EPI == EPI_NONE || EPI == EPI_BIAS || EPI == EPI_SILU_GATE) {
-            // the bf16 epilogues on an even number of K-tiles: the kernel on the 16 x 16 x 128 MFMA
-            if (!p.mfma32 && (p.K / BK) % 2 == 0) {
+            if (ring16_ok(p)) {
                 static std::once_flag once16;
                 static hipError_t err16 = hipSuccess;
                 std::call_once(once16, [] {
@@ -2059,18 +2064,35 @@ float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile,
     const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
     return static_cast<float>((tiles + 255) / 256) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
 }
-float persistent_estimate_us(const GemmArgs& p, int epi) {
+float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
     const bool gate = epi == EPI_SILU_GATE, f32 = epi == EPI_ACCUM_F32, accum = f32 || epi == EPI_ACCUM_BF16;
-    const bool ring = p.K % BK == 0 && p.ldc % 8 == 0 && (gate ? p.N % (BN / 2) == 0 : accum ? p.N % BN == 0 : p.N % 8 == 0);
+    if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, block_ring_ok(p) ? 0.72f : 2.0f, 5.0f);
     // a tile's epilogue; the accumulating ones read and write a round's C (134 MB fp32) with the matrix cores idle
-    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.0f : f32 ? 25.0f : accum ? 14.0f : 6.0f);
+    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring_ok(p, epi, scale_mode) ? 0.95f : 2.3f,
+                            gate ? 10.0f : f32 ? 25.0f : accum ? 14.0f : 6.0f);
 }
-float tiled_estimate_us(const GemmArgs& p, int fmt, int epi, int scale_mode) {
-    if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, p.K % BK == 0 && p.N % BN == 0 ? 0.72f : 2.0f, 5.0f);
-    float best = persistent_estimate_us(p, epi);
-    if (duo_ok(p, fmt, epi, scale_mode)) {
-        const float duo = duo_estimate_us(p, epi);
-        if (duo < best) best = duo;
+
+// Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.
+struct Route { int kernel, shape; };
+Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_naive) {
+    if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
+        (epi == EPI_SILU_GATE && !aligned16(p.B2)))
+        return {CF_GEMM_KERNEL_NAIVE, 0};
+    const bool duo = duo_ok(p, fmt, epi, scale_mode), small = direct_ok(p, fmt, epi, scale_mode);
+    const bool ring = scale_mode == SCALE_BLOCK ? block_ring_ok(p) : ring_ok(p, epi, scale_mode);
+    Route best{!ring || p.force_staged                       ? CF_GEMM_KERNEL_STAGED
+               : epi <= EPI_SILU_GATE && scale_mode != SCALE_BLOCK && ring16_ok(p) ? CF_GEMM_KERNEL_RING16 : CF_GEMM_KERNEL_RING, 0};
+    if (p.small && small && direct_takes(p, epi, scale_mode, p.small - 1)) return {CF_GEMM_KERNEL_SMALL, p.small - 1};
+    if (p.duo && duo) return {CF_GEMM_KERNEL_DUO, 0};
+    if (p.small || p.duo || p.ring || p.force_staged) return best;
+    float t = persistent_estimate_us(p, epi, scale_mode);
+    if (duo) {
+        const float d = duo_estimate_us(p, epi);
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
+    }
+    if (small) {
+        int shape = 0;
+        if (direct_estimate_us(p, epi, scale_mode, &shape) < t) best = {CF_GEMM_KERNEL_SMALL, shape};
     }
     return best;
 }
@@ -2087,23 +2109,14 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
     if (p.lda < p.K || p.ldb < p.K || p.ldc < p.N) return CF_ERR_INVALID_ARG;
     hipStream_t st = as_stream(stream);
     p.a_rows = p.M;
-    const bool tiled_ok = p.K > 0 && p.K % 16 == 0 && p.lda % 16 == 0 && p.ldb % 16 == 0 && aligned16(p.A) &&
-                          aligned16(p.B) && (epi != EPI_SILU_GATE || aligned16(p.B2));
-    if (force_naive || !tiled_ok) {
+    const Route route = gemm_route(p, fmt, epi, scale_mode, force_naive);
+    if (route.kernel == CF_GEMM_KERNEL_NAIVE) {
         const long long total = static_cast<long long>(p.M) * p.N;
         k_gemm_nt_naive<<<static_cast<unsigned>((total + 255) / 256), 256, 0, st>>>(p, fmt, epi, scale_mode);
         return launch_status();
     }
-    // Few rows or few tiles: the kernel with small tiles and K split inside the workgroup, where its estimate is the lowest
-    if (epi <= EPI_SILU_GATE && !(fmt & 2) && !p.force_staged && !p.ring && !p.duo && p.K >= BK &&
-        static_cast<size_t>(p.M) * p.lda < (1ull << 32) && static_cast<size_t>(p.N) * p.ldb < (1ull << 32) && !(epi == EPI_SILU_GATE && fmt)) {
-        int shape = 0;
-        const float direct = direct_estimate_us(p.M, p.N, p.K, epi == EPI_SILU_GATE, scale_mode == SCALE_BLOCK, &shape);
-        if (direct < tiled_estimate_us(p, fmt, epi, scale_mode)) {
-            const int rc = gemm_nt_direct(p, fmt, epi, scale_mode, shape, st);
-            if (rc != CF_ERR_UNSUPPORTED) return rc;
-        }
-    }
+    if (route.kernel == CF_GEMM_KERNEL_SMALL) return gemm_nt_direct(p, fmt, epi, scale_mode, route.shape, st);
+    if (route.kernel == CF_GEMM_KERNEL_DUO) return gemm_nt_duo(p, fmt, epi, scale_mode, st);
     if (scale_mode == SCALE_BLOCK) {
         static std::once_flag once;
         static hipError_t attr_err = hipSuccess;
@@ -2114,11 +2127,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         if (attr_err != hipSuccess) return static_cast<int>(attr_err);
         p.tiles_m = (p.M + BSM - 1) / BSM;
         p.tiles_n = (p.N + BN - 1) / BN;
-        const int kb = p.K / BK;
-        const bool ring_ok = p.K % BK == 0 && kb >= 3 && kb <= kBsMaxKb && p.N % BN == 0 && !p.force_staged &&
-                             static_cast<size_t>(p.M) * p.lda < (1ull << 32) && static_cast<size_t>(p.N) * p.ldb < (1ull << 32) &&
-                             static_cast<size_t>(p.M) * kb * 4 < (1ull << 32);
-        if (ring_ok) {
+        if (route.kernel == CF_GEMM_KERNEL_RING) {
             static std::once_flag once_ring;
             static hipError_t ring_err = hipSuccess;
             std::call_once(once_ring, [] {
@@ -2134,9 +2143,6 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         k_gemm_nt_block<<<p.tiles_m * p.tiles_n, kThreads, kBlkLds, st>>>(p);
         return launch_status();
     }
-    if (duo_ok(p, fmt, epi, scale_mode) &&
-        (p.duo || (!p.force_staged && !p.ring && duo_estimate_us(p, epi) < persistent_estimate_us(p, epi))))
-        return gemm_nt_duo(p, fmt, epi, scale_mode, st);
     const int out_bn = epi == EPI_SILU_GATE ? BN / 2 : BN;
     p.tiles_m = (p.M + BM - 1) / BM;
     p.tiles_n = (p.N + out_bn - 1) / out_bn;
@@ -2190,7 +2196,25 @@ int cf_fp8_gemm_nt_bf16_ex(int M, int N, int K, const void* A, int lda, int a_is
     p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) ? 2 : 1) : 0;
     p.mfma32 = (flags & CF_GEMM_FLAG_MFMA32) != 0;
     p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
+    p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
     return gemm_nt(p, a_is_e5m2 ? 1 : 0, epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE, stream);
+}
+
+int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int scale_mode, int epilogue, int ldc, int flags,
+                      int* kernel) {
+    if (M <= 0 || N <= 0 || K <= 0 || ldc < N || !kernel || epilogue < EPI_NONE || epilogue > EPI_ACCUM_BF16 ||
+        scale_mode < SCALE_TENSOR || scale_mode > SCALE_BLOCK)
+        return CF_ERR_INVALID_ARG;
+    GemmArgs p{};                     // null pointers are aligned ones
+    p.M = M; p.N = N; p.K = K; p.lda = K; p.ldb = K; p.ldc = ldc; p.a_rows = M;
+    p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;
+    p.duo = (flags & CF_GEMM_FLAG_DUO) != 0;
+    p.mfma32 = (flags & CF_GEMM_FLAG_MFMA32) != 0;
+    p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
+    p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
+    const Route r = gemm_route(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE);
+    *kernel = r.kernel + r.shape;
+    return CF_OK;
 }
 
 // dW[M,N] += X^T . dY with both operands pre-transposed to K-contiguous rows:
@@ -2447,25 +2471,39 @@ int grouped_gemm_nt_terms(int total_rows, int N, int Kb, int terms, int num_expe
     return c_is_f32 ? launch_ring_only<0, EPI_STORE_F32, SCALE_ROW, 1>(p, as_stream(stream))
                     : launch_ring_only<0, EPI_NONE, SCALE_ROW, 1>(p, as_stream(stream));
 }
-}  // namespace cf
 
-extern "C" {
-
-// Cross-check form of the accumulate GEMMs: any format pair, optional naive kernel.
-int cf_fp8_gemm_nt_accum_f32_ex(int M, int N, int K, const void* A, int lda, int a_is_e5m2, const float* a_descale,
-                                const void* B, int ldb, int b_is_e5m2, const float* b_descale, float* C, int ldc,
-                                int flags, cf_stream_t stream) {
+namespace {
+int accum_ex(int M, int N, int K, const void* A, int lda, int a_is_e5m2, const float* a_descale, const void* B, int ldb,
+             int b_is_e5m2, const float* b_descale, float* Cf, uint16_t* C, int ldc, int flags, cf_stream_t stream) {
     GemmArgs p{};
     p.M = M; p.N = N; p.K = K;
     p.A = static_cast<const uint8_t*>(A); p.lda = lda;
     p.B = static_cast<const uint8_t*>(B); p.ldb = ldb;
     p.sa = a_descale; p.sb = b_descale;
-    p.Cf = C; p.ldc = ldc;
+    p.Cf = Cf; p.C = C; p.ldc = ldc;
     p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;
-    p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) == CF_GEMM_FLAG_DUO_IN_STEP ? 2 : 1) : 0;
+    p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) ? 2 : 1) : 0;
     p.ring = (flags & CF_GEMM_FLAG_RING) != 0;
-    return gemm_nt(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), EPI_ACCUM_F32, SCALE_TENSOR,
+    return gemm_nt(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), Cf ? EPI_ACCUM_F32 : EPI_ACCUM_BF16, SCALE_TENSOR,
                    flags & CF_GEMM_FLAG_NAIVE, stream);
+}
+}  // namespace
+}  // namespace cf
+
+extern "C" {
+
+// Cross-check forms of the accumulate GEMMs: any format pair, a kernel of the caller's choice.
+int cf_fp8_gemm_nt_accum_f32_ex(int M, int N, int K, const void* A, int lda, int a_is_e5m2, const float* a_descale,
+                                const void* B, int ldb, int b_is_e5m2, const float* b_descale, float* C, int ldc,
+                                int flags, cf_stream_t stream) {
+    if (!C && M > 0 && N > 0) return CF_ERR_INVALID_ARG;
+    return accum_ex(M, N, K, A, lda, a_is_e5m2, a_descale, B, ldb, b_is_e5m2, b_descale, C, nullptr, ldc, flags, stream);
+}
+
+int cf_fp8_gemm_nt_accum_bf16_ex(int M, int N, int K, const void* A, int lda, int a_is_e5m2, const float* a_descale,
+                                 const void* B, int ldb, int b_is_e5m2, const float* b_descale, uint16_t* C, int ldc,
+                                 int flags, cf_stream_t stream) {
+    return accum_ex(M, N, K, A, lda, a_is_e5m2, a_descale, B, ldb, b_is_e5m2, b_descale, nullptr, C, ldc, flags, stream);
 }
 
 }  // extern "C"

@@ -28,6 +28,7 @@ struct GemmArgs {
     int tiles_m, tiles_n;
     int force_staged;            // take the register-staged kernel even when the ring kernel applies
     int duo;                     // 1: the two-workgroups-per-CU kernel where it applies, 2: the same without the stagger, 0: where its estimate is lowest
+    int small;                   // 1 + the tile shape of the small-tile kernel a caller asks for, 0: where its estimate is lowest
     int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
     // grouped (per-expert) form, ring kernel only; all null / 0 for a dense GEMM
@@ -89,9 +90,11 @@ inline int persistent_grid(int total, int most) {
     return up <= most ? up : most / kXcds * kXcds;
 }
 
-// gemm_direct.hip: time of its best tile shape on a problem and which one that is; the launches (dense; grouped over a row-tile
-// table)
-float direct_estimate_us(int M, int N, int K, bool gate, bool block, int* shape);
+// gemm_direct.hip: whether it takes a problem (at all; with a tile shape), the time of its best tile shape and which one that is,
+// the launches (dense; grouped over a row-tile table)
+bool direct_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
+bool direct_takes(const GemmArgs& p, int epi, int scale_mode, int shape);
+float direct_estimate_us(const GemmArgs& p, int epi, int scale_mode, int* shape);
 float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape);
 int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st);
 int grouped_gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int shape, hipStream_t st);

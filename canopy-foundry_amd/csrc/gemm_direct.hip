@@ -311,6 +311,12 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
 
 constexpr int kLds = 160 * 1024;
 
+// bytes of LDS the scales of a block-scaled tile take beside the operands: [16 mb] rows and one row of weights
+constexpr size_t block_scale_bytes(int mb, int K) {
+    const size_t kg = (static_cast<size_t>(K) + BK - 1) / BK;
+    return (16 * mb * (kg | 1) + kg) * 4;
+}
+
 template <int FMT, bool GATE, bool BLOCK, bool GROUPED, int MB, int NB, int WK, int S>
 int launch(GemmArgs p, int epi, int scale_mode, hipStream_t st) {
     constexpr int NT = GATE ? 2 * NB : NB;
@@ -318,9 +324,8 @@ int launch(GemmArgs p, int epi, int scale_mode, hipStream_t st) {
     constexpr int one = WK * MB * NT * 1024, sums = (one > 128 * 1024 ? one / 2 : one) + (16 * MB + 32 * NB) * 4;
     constexpr int base = stages > sums ? stages : sums;
     static_assert(base <= kLds);
-    const int kg = (p.K + 127) / 128;
-    const int lds = base + (BLOCK ? (16 * MB * (kg | 1) + kg) * 4 : 0);
-    if (lds > kLds) return CF_ERR_UNSUPPORTED;
+    const size_t lds = base + (BLOCK ? block_scale_bytes(MB, p.K) : 0);
+    if (lds > kLds) return CF_ERR_UNSUPPORTED;          // direct_takes() is stricter
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {
@@ -375,19 +380,35 @@ int launch_gate(const GemmArgs& p, int scale_mode, int shape, hipStream_t st) {
 
 }  // namespace
 
+bool direct_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
+    return epi <= EPI_SILU_GATE && !(fmt & 2) && !(epi == EPI_SILU_GATE && fmt) && !(scale_mode == SCALE_BLOCK && (fmt || epi != EPI_NONE)) &&
+           p.K >= BK && static_cast<size_t>(p.M) * p.lda < (1ull << 32) && static_cast<size_t>(p.N) * p.ldb < (1ull << 32);
+}
+// Whether the shape exists for the epilogue and scales and its LDS suffices (block scales: the stages of the four shapes take 48,
+// 64, 96 and 128 KiB, their sums less, the scales the rest)
+bool direct_takes(const GemmArgs& p, int epi, int scale_mode, int shape) {
+    if (shape < 0 || shape >= (epi == EPI_SILU_GATE ? 4 : scale_mode == SCALE_BLOCK ? 4 : 6)) return false;
+    if (scale_mode != SCALE_BLOCK) return true;
+    constexpr size_t stages[4] = {48 * 1024, 64 * 1024, 96 * 1024, 128 * 1024};
+    return stages[shape] + block_scale_bytes(kPlain[shape].mb, p.K) <= kLds;
+}
+
 // Picks the tile shape and says what it would take, in microseconds: every workgroup moves K bytes of each of its rows and weight rows, and a CU takes them in at 93 KB
 // per microsecond whatever the shape (measured, K 1024 to 14336; 62 KB where the folds of the block scales are as many as in
 // a 64 x 64 tile); a CU whose LDS holds one workgroup works in whole rounds.
 // A shape with more rows than the next one smaller would do is not looked at: its extra rows are copies.
-float direct_estimate_us(int M, int N, int K, bool gate, bool block, int* shape) {
+float direct_estimate_us(const GemmArgs& p, int epi, int scale_mode, int* shape) {
+    const bool gate = epi == EPI_SILU_GATE, block = scale_mode == SCALE_BLOCK;
+    const int M = p.M, N = p.N, K = p.K;
     const Shape* s = gate ? kGate : kPlain;
     const int count = gate ? 4 : block ? 4 : 6;
     float best = 1e30f;
     for (int i = 0; i < count; ++i) {
         if (i > 0 && s[i].mb > s[i - 1].mb && M <= 16 * s[i - 1].mb) break;
+        if (!direct_takes(p, epi, scale_mode, i)) break;
         const int tn = 16 * s[i].nt / (gate ? 2 : 1);
         const double wgs = static_cast<double>((M + 16 * s[i].mb - 1) / (16 * s[i].mb)) * ((N + tn - 1) / tn);
-        double rounds = wgs / 256.0;
+        double rounds = wgs / num_cus();
         if (!s[i].shared) rounds = static_cast<double>(static_cast<long long>(rounds + 0.999));
         if (rounds < 1.0) rounds = 1.0;
         const double rate = block && s[i].mb * s[i].nt >= 16 ? 62e3 : 93e3;

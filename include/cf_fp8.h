@@ -260,6 +260,9 @@ int cf_cross_entropy_fwd_bwd_chunk_quant_e5m2(const uint16_t* d_logits, const in
                                   8 - 9 % more MFMA throughput at the same socket power) */
 #define CF_GEMM_FLAG_RING 32   /* keep the persistent 256 x 256-tile kernels (128 x 256 with block scales) where few rows or few
                                   tiles would take a kernel with smaller tiles */
+#define CF_GEMM_FLAG_SMALL 64  /* take the small-tile kernel where it applies, with the tile shape in bits 8 to 11: plain and
+                                  bias 0 to 5, block scales 0 to 3: 16x16, 32x32, 64x32, 64x64, 128x64, 128x128 outputs; SiLU gate
+                                  0 to 3: 16x16, 32x32, 64x64, 128x64 */
 
 /* lt_gemm_fp8_nt, static at src/trainer.cu:4498-4534 (plan lookup :4402-4496).
  * C[M,N] bf16 (row stride ldc) = (A[M,K] fp8, row stride lda, E4M3 or E5M2) .
@@ -291,13 +294,30 @@ int cf_fp8_gemm_tn_accum_f32(int M, int N, int K, const void* d_Xt_e4m3, const f
 int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const float* d_ds_x,
                               const void* d_dYt_e5m2, const float* d_ds_dy, uint16_t* d_dW,
                               int ldc_dw, cf_stream_t stream);
-/* The accumulate GEMM of src/trainer.cu:4596-4627 with free operand formats and row strides, and
- * CF_GEMM_FLAG_NAIVE for the cross-check kernel; used by the tests and for fp32 inspection of
- * the accumulators. */
+#define CF_GEMM_KERNEL_NAIVE  0    /* one lane per output: K no multiple of 16, or asked for */
+#define CF_GEMM_KERNEL_STAGED 1    /* 256 x 256 (block scales: 128 x 256) tiles through registers and LDS */
+#define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: its own) */
+#define CF_GEMM_KERNEL_RING16 3    /* the same on 16 x 16 x 128 MFMAs */
+#define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU */
+#define CF_GEMM_KERNEL_SMALL  16   /* + tile shape (see CF_GEMM_FLAG_SMALL): K split over a workgroup's wavefronts */
+
+/* Which kernel (CF_GEMM_KERNEL_*) the dense GEMM entry points run a problem on (16-byte aligned operands, descales and
+ * C, operand rows back to back); launches nothing and needs no GPU.  epilogue: a CF_EPI_* value, or 3 / 4 for C +=
+ * product into an fp32 / bf16 C.  flags: CF_GEMM_FLAG_*.  The order in which K is summed is a kernel's own: calls whose kernels differ may differ in
+ * the last bits of a result.  It has no counterpart in the reference, whose plan cache asks cuBLASLt. */
+int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int scale_mode, int epilogue, int ldc,
+                      int flags, int* kernel);
+/* The accumulate GEMMs of src/trainer.cu:4596-4627 and :4670-4691 with free operand formats and row strides, and a
+ * kernel of the caller's choice: CF_GEMM_FLAG_NAIVE, _STAGED, _DUO (E4M3 x E5M2, N and ldc multiples of 4), _RING; used
+ * by the tests and for fp32 inspection of the accumulators. */
 int cf_fp8_gemm_nt_accum_f32_ex(int M, int N, int K, const void* d_A, int lda, int a_is_e5m2,
                                 const float* d_a_descale, const void* d_B, int ldb, int b_is_e5m2,
                                 const float* d_b_descale, float* d_C, int ldc, int flags,
                                 cf_stream_t stream);
+int cf_fp8_gemm_nt_accum_bf16_ex(int M, int N, int K, const void* d_A, int lda, int a_is_e5m2,
+                                 const float* d_a_descale, const void* d_B, int ldb, int b_is_e5m2,
+                                 const float* d_b_descale, uint16_t* d_C, int ldc, int flags,
+                                 cf_stream_t stream);
 
 /* ---- MoE routing and dispatch: kernels/moe.cu, kernels/cross_entropy.cu --------
  * Routing results are reproducible bit for bit: fixed reduction order, a

@@ -1,0 +1,41 @@
+"""Which kernel a dense FP8 GEMM runs on (cf_fp8_gemm_route; decided on the host).  Times are microseconds on one MI355X from
+captured graphs, weights from HBM; each case names the two kernels between which the choice lies."""
+import ctypes
+
+import pytest
+
+NAIVE, STAGED, RING, RING16, DUO, SMALL = 0, 1, 2, 3, 4, 16
+TENSOR, ROW_COL, BLOCK = 0, 1, 2
+PLAIN, BIAS, GATE, ACCUM_F32, ACCUM_BF16 = range(5)
+F_NAIVE, F_STAGED, F_DUO, F_MFMA32, F_RING, F_SMALL = 1, 2, 4, 16, 32, 64
+
+
+def route(cf, M, N, K, mode=TENSOR, epi=PLAIN, flags=0, pad=0, a_e5m2=0):
+    k = ctypes.c_int(-1)
+    cf.cf_fp8_gemm_route(M, N, K, a_e5m2, int(epi >= ACCUM_F32), mode, epi, N + pad, flags, ctypes.byref(k))
+    return k.value
+
+
+def test_flags_name_kernels(cf):
+    assert route(cf, 512, 512, 512, flags=F_NAIVE) == NAIVE == route(cf, 512, 512, 40)
+    assert route(cf, 512, 512, 512, flags=F_STAGED) == STAGED
+    assert route(cf, 512, 512, 512, flags=F_RING) == RING16 and route(cf, 512, 512, 640, flags=F_RING) == RING
+    assert route(cf, 512, 512, 512, flags=F_MFMA32) == RING
+    assert route(cf, 512, 512, 512, flags=F_RING, mode=BLOCK) == RING
+    assert route(cf, 512, 512, 512, flags=F_DUO) == DUO == route(cf, 512, 512, 512, flags=F_DUO, epi=ACCUM_BF16)
+    for shape in range(6):
+        assert route(cf, 512, 512, 512, flags=F_SMALL | shape << 8) == SMALL + shape
+    # what a kernel does not take falls to the persistent or the staged one
+    assert route(cf, 512, 516, 512, flags=F_DUO) == STAGED
+    assert route(cf, 512, 512, 512, flags=F_SMALL | 4 << 8, epi=GATE) == RING16
+    assert route(cf, 512, 512, 512, flags=F_SMALL, epi=ACCUM_F32) == RING
+    assert route(cf, 512, 512, 112, flags=F_SMALL) == STAGED
+
+
+def test_estimates_ask_what_the_launch_asks(cf):
+    """The persistent kernels' rate is assumed where they are launched, and only there."""
+    # rows of C a multiple of 4 and not of 8: the accumulating ring takes them (306 us; two workgroups per CU 369)
+    assert route(cf, 4096, 14336, 4096, epi=ACCUM_F32, pad=4) == RING
+    assert route(cf, 4096, 14336, 4096, epi=ACCUM_BF16, pad=4) == RING
+    # block scales with K of two K-tiles: the register-staged kernel (9.6 us against 4.4), priced as such
+    assert route(cf, 1000, 512, 256, mode=BLOCK) >= SMALL
