@@ -2065,11 +2065,14 @@ float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile,
     return static_cast<float>((tiles + 255) / 256) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
 }
 float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
-    const bool gate = epi == EPI_SILU_GATE, f32 = epi == EPI_ACCUM_F32, accum = f32 || epi == EPI_ACCUM_BF16;
     if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, block_ring_ok(p) ? 0.72f : 2.0f, 5.0f);
-    // a tile's epilogue; the accumulating ones read and write a round's C (134 MB fp32) with the matrix cores idle
-    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring_ok(p, epi, scale_mode) ? 0.95f : 2.3f,
-                            gate ? 10.0f : f32 ? 25.0f : accum ? 14.0f : 6.0f);
+    const bool ring = ring_ok(p, epi, scale_mode);
+    // The accumulating ones read and write a round's C with the matrix cores idle (134 MB fp32); the register-staged ones hide
+    // nothing of it under their K-tiles.  14336 x 4096 +=, 896 tiles in four rounds: K 256 fp32 107 us, bf16 62; K 4096 243, 205.
+    if (epi == EPI_ACCUM_F32) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, 25.0f);
+    if (epi == EPI_ACCUM_BF16) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, c_lines_shared(p, 2) ? 13.7f : 11.1f);
+    const bool gate = epi == EPI_SILU_GATE;
+    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.0f : 6.0f);
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.

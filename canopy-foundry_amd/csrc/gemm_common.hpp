@@ -90,6 +90,9 @@ inline int persistent_grid(int total, int most) {
     return up <= most ? up : most / kXcds * kXcds;
 }
 
+// Whether a row of C begins inside a 128-byte line, so that neighbouring tiles write parts of the same lines.
+inline bool c_lines_shared(const GemmArgs& p, int elem_bytes) { return static_cast<long long>(p.ldc) * elem_bytes % 128 != 0; }
+
 // gemm_direct.hip: whether it takes a problem (at all; with a tile shape), the time of its best tile shape and which one that is,
 // the launches (dense; grouped over a row-tile table)
 bool direct_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);

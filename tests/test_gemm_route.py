@@ -39,3 +39,17 @@ def test_estimates_ask_what_the_launch_asks(cf):
     assert route(cf, 4096, 14336, 4096, epi=ACCUM_BF16, pad=4) == RING
     # block scales with K of two K-tiles: the register-staged kernel (9.6 us against 4.4), priced as such
     assert route(cf, 1000, 512, 256, mode=BLOCK) >= SMALL
+
+
+# ring (or register-staged, where N is no multiple of 256) against two workgroups per CU
+@pytest.mark.parametrize("M,N,K,pad,epi,kernel", [
+    (4096, 4096, 256, 0, ACCUM_BF16, RING),          # 21.8, 29.2
+    (4096, 14336, 512, 0, ACCUM_BF16, RING),         # 74.2, 85.6
+    (4096, 14336, 512, 4, ACCUM_F32, RING),          # 191, 222: rows of C that do not begin at a line
+    (4100, 5636, 256, 0, ACCUM_F32, DUO),            # 116 (register-staged), 94
+    (1024, 4096, 1024, 0, ACCUM_F32, DUO),           # 24.1, 13.5: 64 tiles
+    (14336, 4096, 2000, 0, ACCUM_F32, DUO),          # 262, 188: K no multiple of 128
+    (14336, 4096, 8192, 0, ACCUM_F32, RING),         # 389, 431
+])
+def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
+    assert route(cf, M, N, K, epi=epi, pad=pad) == kernel
