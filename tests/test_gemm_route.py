@@ -53,3 +53,16 @@ def test_estimates_ask_what_the_launch_asks(cf):
 ])
 def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
     assert route(cf, M, N, K, epi=epi, pad=pad) == kernel
+
+
+# times of the tile shapes 32x32, 64x32, 64x64 and of the persistent kernel (128 x 256 tiles)
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (3000, 512, 4096, (RING, SMALL + 3)),            # 33.9, 42.4, 28.7, 29.9
+    (3000, 512, 2048, (RING, SMALL + 3)),            # 19.1, 23.6, 18.0, 16.9
+    (6000, 1000, 7168, (STAGED,)),                   # 197, 227, 137, 103 (register-staged)
+    (4096, 1000, 2000, (STAGED,)),                   # 56.6, 70.0, 44.1, 35.6 (register-staged)
+    (1000, 512, 4096, (SMALL + 1, SMALL + 2)),       # 11.7, 12.1, 13.7, 28.6
+    (4096, 7168, 7168, (RING,)),
+])
+def test_block_scaled_kernel(cf, M, N, K, kernel):
+    assert route(cf, M, N, K, mode=BLOCK) in kernel
