@@ -2072,7 +2072,7 @@ float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
     if (epi == EPI_ACCUM_F32) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, 25.0f);
     if (epi == EPI_ACCUM_BF16) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, c_lines_shared(p, 2) ? 13.7f : 11.1f);
     const bool gate = epi == EPI_SILU_GATE;
-    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.0f : 6.0f);
+    return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.4f : 6.0f);
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.

@@ -459,11 +459,14 @@ bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
     return p.N % 8 == 0 && (epi != EPI_BIAS || aligned16(p.bias));
 }
 
-// Microseconds: 0.48 a K-tile where a CU holds one workgroup, 0.875 for both where it holds two (measured, 4096 columns, K 4096 to
-// 14336); a third more where K is no multiple of 128 and a row's 128-byte pieces therefore lie across lines.  Per round of
-// tiles 2.5 for the fill and the bf16 store, 8 for what is left of adding to an fp32 C under the other workgroup's MFMAs, 5.5 to
-// a bf16 C, whose 64-byte pieces are half lines; more where the rows of C do not begin at lines.  So a short K and a bf16 C stay
-// with the ring kernel (+= bf16 4096 x 4096: K 256 21.8 us there, 29.2 here; 4096 x 14336: K 512 74.2, 85.6), as do rows off the
+// Microseconds: 0.48 a K-tile where a CU holds one workgroup (0.62 with the SiLU gate), 0.875 for both where it holds two
+// (measured, 4096 columns, K 4096 to 14336); a third more where K is no multiple of 128 and a row's 128-byte pieces therefore
+// lie across lines.  Per round of tiles 2.5 for the fill and the bf16 store (hidden in a last round that follows others), 3 for
+// those and the SiLU gate's arithmetic (1.2 there).  512 x 2 x 14336 over K 1024, a round and three quarters: 26.0 us, 20.8 in
+// the ring kernel; 1500 x 2 x 4096: 16.5, 19.1.
+// Accumulating forms, per round: 8 for what is left of adding to an fp32 C under the other workgroup's MFMAs, 5.5 to a bf16 C,
+// whose 64-byte pieces are half lines; more where the rows of C do not begin at lines.  So a short K and a bf16 C stay with
+// the ring kernel (+= bf16 4096 x 4096: K 256 21.8 us there, 29.2 here; 4096 x 14336: K 512 74.2, 85.6), as do rows off the
 // lines (fp32 4096 x 14336, ldc + 4, K 512: 191, 222); few tiles come here (fp32 1024 x 4096, K 1024: 24.1, 13.5).  One
 // shape is still misjudged: fp32 4096 x 8192, K up to 512, whose two whole rounds take the ring 70 us, this kernel 75.
 float duo_estimate_us(const GemmArgs& p, int epi) {
@@ -471,9 +474,11 @@ float duo_estimate_us(const GemmArgs& p, int epi) {
     const long long wgs = static_cast<long long>((p.M + DM - 1) / DM) * ((p.N + out_bn - 1) / out_bn);
     const long long full = wgs / (2 * most), rest = wgs % (2 * most);
     const float kt = static_cast<float>((p.K + BK - 1) / BK) * (p.K % BK ? 1.33f : 1.0f);
-    const float tile = epi == EPI_ACCUM_F32 ? (c_lines_shared(p, 4) ? 14.0f : 8.0f) : epi == EPI_ACCUM_BF16 ? (c_lines_shared(p, 2) ? 6.2f : 5.5f) : 2.5f;
-    return static_cast<float>(full) * (kt * 0.875f + tile) +
-           (rest == 0 ? 0.0f : (rest > most ? kt * 0.875f : kt * 0.48f) + (full && tile == 2.5f ? 0.0f : tile));
+    const bool gate = epi == EPI_SILU_GATE, accum = epi == EPI_ACCUM_F32 || epi == EPI_ACCUM_BF16;
+    const float tile = epi == EPI_ACCUM_F32 ? (c_lines_shared(p, 4) ? 14.0f : 8.0f) : epi == EPI_ACCUM_BF16 ? (c_lines_shared(p, 2) ? 6.2f : 5.5f)
+                     : gate ? 3.0f : 2.5f;
+    const float last = full == 0 || accum ? tile : gate ? 1.2f : 0.0f;
+    return static_cast<float>(full) * (kt * 0.875f + tile) + (rest == 0 ? 0.0f : kt * (rest > most ? 0.875f : gate ? 0.62f : 0.48f) + last);
 }
 
 int gemm_nt_duo(GemmArgs p, int fmt, int epi, int scale_mode, hipStream_t st) {

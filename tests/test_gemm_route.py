@@ -66,3 +66,16 @@ def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
 ])
 def test_block_scaled_kernel(cf, M, N, K, kernel):
     assert route(cf, M, N, K, mode=BLOCK) in kernel
+
+
+# 256 x 128-output persistent tiles against 128 x 64-output ones, two workgroups per CU
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (512, 14336, 1024, RING16),                      # 20.8, 26.0: a round and three quarters of the smaller tiles
+    (1024, 7168, 1024, RING16),                      # 20.1, 24.5
+    (700, 7168, 2048, RING16),                       # 28.0, 32.7
+    (1000, 896, 1024, DUO),                          # 56 tiles instead of 28
+    (1500, 4096, 1024, DUO),                         # 19.1, 16.5
+    (8192, 14336, 4096, RING16),
+])
+def test_silu_gate_kernel(cf, M, N, K, kernel):
+    assert route(cf, M, N, K, mode=ROW_COL, epi=GATE) == kernel
