@@ -45,13 +45,25 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
     const int t = total % kXcds == 0 ? (pos % kXcds) * (total / kXcds) + pos / kXcds : pos;
     const int tm = t % p.tiles_m, tn = t / p.tiles_m;
     const int n0 = tn * TN;
-    int m_first = tm * TM, m_end = min(m_first + TM, p.M), expert = 0;
+    int m_first = tm * TM, m_end = min(m_first + TM, p.M), m_step = TM, expert = 0;
     if constexpr (GROUPED) {
-        if (tm >= p.tile_map[0]) return;
-        const int* e = p.tile_map + 1 + kMapWords * tm;
+        // A table entry is up to 256 rows of an expert, walked TM at a time.  Where the rows lie on few experts there are fewer entries
+        // than workgroups to a column of tiles: those beyond the last entry take every second, third, ... pass of the entries
+        // before.  (64 experts of 2 x 1408 x 2048, 1280 rows all on one: 53 us with its entries walked by a workgroup each.)
+        const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], p.tiles_m));
+        if (entries <= 0) return;
+        int entry = tm, part = 0, parts = tm + entries < p.tiles_m ? 2 : 1;
+        if (tm >= entries || 2 * entries < p.tiles_m) {
+            part = tm / entries;
+            entry = tm - part * entries;
+            parts = (p.tiles_m - 1 - entry) / entries + 1;
+        }
+        const int* e = p.tile_map + 1 + kMapWords * entry;
         expert = __builtin_amdgcn_readfirstlane(e[0]);
-        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (tm - __builtin_amdgcn_readfirstlane(e[3])) * BM;
+        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (entry - __builtin_amdgcn_readfirstlane(e[3])) * BM;
         m_end = min(m_first + BM, __builtin_amdgcn_readfirstlane(e[2]));
+        m_first += part * TM;
+        m_step = parts * TM;
     }
     const uint8_t* B = p.B + static_cast<size_t>(expert) * p.b_expert_stride;
     const uint8_t* B2 = GATE ? p.B2 + static_cast<size_t>(expert) * p.b_expert_stride : B;
@@ -80,7 +92,7 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
     float* const lds_sa = reinterpret_cast<float*>(smem + WK * S * kStage);
     float* const lds_sb = lds_sa + TM * kpad;
 
-    for (int m0 = m_first; m0 < m_end; m0 += TM) {
+    for (int m0 = m_first; m0 < m_end; m0 += m_step) {
         uint32_t xoff[MB][2];
 #pragma unroll
         for (int b = 0; b < MB; ++b)
@@ -305,7 +317,7 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
             }
         }
         });
-        if (GROUPED) __syncthreads();
+        if (GROUPED) __syncthreads();          // the sums' LDS takes the next pass's stages
     }
 }
 

@@ -90,14 +90,8 @@ def test_small_tiles_block_scales(cf, dev, M, N, K):
     orc.assert_gemm_close(got[:, :N], ref, absdot, what=f"block {M}x{N}x{K}")
 
 
-# counts times `scale`: 16-row tiles, then 32- and 64-row ones; the plain form takes 64 columns instead of 16 or 32 per workgroup
-# where there are many
-@pytest.mark.parametrize("gate,scale,N", [(False, 1, 128), (False, 1, 256), (False, 1, 520), (False, 2, 256), (False, 2, 1000), (False, 3, 256),
-                                          (True, 1, 256), (True, 3, 256)])
-def test_small_tiles_grouped(cf, dev, gate, scale, N):
-    """Experts without rows, with one row, with a tile and a row more, and with rows in two entries of the row-tile table."""
-    counts = np.array([0, 1, 16, 17, 33, 130, 0, 3] + [0] * 16, np.int32) * scale
-    E, K = len(counts), 384
+def check_grouped(cf, dev, counts, N, K, gate):
+    E = len(counts)
     offsets = np.concatenate([[0], np.cumsum(counts)[:-1]]).astype(np.int32)
     total = int(counts.sum())
     case(f"small-tile grouped gemm total={total} N={N} gate={gate}")
@@ -134,6 +128,27 @@ def test_small_tiles_grouped(cf, dev, gate, scale, N):
             assert np.sqrt(((mine - exact) ** 2).sum() / (exact ** 2).sum()) <= 4e-3, e
         else:
             orc.assert_gemm_close(mine, ref, absdot, what=f"expert {e}")
+
+
+# counts times `scale`: 16-row tiles, then 32- and 64-row ones; the plain form takes 64 columns instead of 16 or 32 per workgroup
+# where there are many
+@pytest.mark.parametrize("gate,scale,N", [(False, 1, 128), (False, 1, 256), (False, 1, 520), (False, 2, 256), (False, 2, 1000), (False, 3, 256),
+                                          (True, 1, 256), (True, 3, 256)])
+def test_small_tiles_grouped(cf, dev, gate, scale, N):
+    """Experts without rows, with one row, with a tile and a row more, and with rows in two entries of the row-tile table."""
+    check_grouped(cf, dev, np.array([0, 1, 16, 17, 33, 130, 0, 3] + [0] * 16, np.int32) * scale, N, 384, gate)
+
+
+# the same number of workgroups whatever the counts: all rows on one expert (one entry and several), on the first and the last,
+# on just under and just over half of the experts, and no entry to spare
+@pytest.mark.parametrize("rows", [{7: 90}, {0: 300}, {23: 600}, {0: 1, 23: 257}, {i: 17 for i in range(11)}, {i: 35 for i in range(13)},
+                                  {i: 20 for i in range(23)}, {i: 33 for i in range(24)}])
+@pytest.mark.parametrize("gate", [False, True])
+def test_small_tiles_grouped_skewed(cf, dev, rows, gate):
+    counts = np.zeros(24, np.int32)
+    for e, n in rows.items():
+        counts[e] = n
+    check_grouped(cf, dev, counts, 256, 256, gate)
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 512, 512), (770, 256, 384), (1024, 1024, 256), (300, 264, 512), (512, 1000, 384), (256, 8, 256),
