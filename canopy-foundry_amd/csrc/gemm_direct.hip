@@ -369,7 +369,9 @@ int launch_plain(const GemmArgs& p, int epi, int scale_mode, int shape, hipStrea
     switch (shape) {
         case 0: return launch<FMT, false, BLOCK, GROUPED, 1, 1, 4, 3>(p, epi, scale_mode, st);
         case 1: return launch<FMT, false, BLOCK, GROUPED, 2, 2, 4, 2>(p, epi, scale_mode, st);
-        case 2: return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, epi, scale_mode, st);
+        case 2:
+            if constexpr (GROUPED) return CF_ERR_UNSUPPORTED;          // of two shapes of as many rows the wider is taken
+            else return launch<FMT, false, BLOCK, GROUPED, 4, 2, 4, 2>(p, epi, scale_mode, st);
         case 3: return launch<FMT, false, BLOCK, GROUPED, 4, 4, 4, 2>(p, epi, scale_mode, st);
         default:
             if constexpr (GROUPED) {
