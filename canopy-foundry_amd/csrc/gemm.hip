@@ -36,10 +36,8 @@ constexpr int kTileBytes = BM * BK;               // 32 KiB per operand tile
 constexpr int kStageBytes = 2 * kTileBytes;       // X tile + W tile
 constexpr int kLdsBytes = 2 * kStageBytes;        // double buffered: 128 KiB
 
-
 // where a workgroup's tile lives: rows [m0, m_end) of the output, columns from n0, weights of `expert`
 struct TilePos { int m0, m_end, n0, expert; };
-
 
 // Workgroups are handed to the 8 XCDs round-robin, so launch positions with the same pos % 8 share an XCD
 // (and its L2).  One tile per workgroup: position pos works on tile (pos % 8) * (total / 8) + pos / 8 of the walk
@@ -2062,7 +2060,8 @@ __global__ __launch_bounds__(256) void k_bank_setup(const int* __restrict__ coun
 // register-staged kernel 2.3), 128 x 256 block-scaled tiles 0.65 (1.45).  (At the power limit all of them slow down together.)
 float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile, float per_tile) {
     const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
-    return static_cast<float>((tiles + 255) / 256) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
+    const int cus = num_cus();
+    return static_cast<float>((tiles + cus - 1) / cus) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
 }
 float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
     if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, block_ring_ok(p) ? 0.65f : 1.45f, 6.0f);
@@ -2354,7 +2353,7 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
     size_t need = 0;
     cf_fp8_grouped_gemm_workspace_bytes(total_rows, num_experts, &need);
     if (workspace_bytes < need || (reinterpret_cast<uintptr_t>(d_workspace) & 3u)) return CF_ERR_INVALID_ARG;
-    // the grouped form runs on the ring kernel only
+    // what the ring kernel takes (the small-tile kernel would take more: a refusal must not depend on the number of rows)
     if (K % BK != 0 || K < 2 * BK || lda % 16 != 0 || !aligned16(A) || !aligned16(B) ||
         (epilogue == EPI_SILU_GATE && !aligned16(B_up)) || lda < K || ldc < N ||
         static_cast<size_t>(a_rows) * lda >= (1ull << 32) || static_cast<size_t>(N) * K >= (1ull << 32) ||

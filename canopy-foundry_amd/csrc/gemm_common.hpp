@@ -31,8 +31,8 @@ struct GemmArgs {
     int small;                   // 1 + the tile shape of the small-tile kernel a caller asks for, 0: where its estimate is lowest
     int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
-    // grouped (per-expert) form, ring kernel only; all null / 0 for a dense GEMM
-    const int* tile_map;         // [0] = number of row tiles, then (expert, first row, end row) per row tile
+    // grouped (per-expert) form, ring and small-tile kernels; all null / 0 for a dense GEMM
+    const int* tile_map;         // [0] = number of row tiles, then kMapWords words per row tile: expert, its first row, end row, first tile, tiles
     const int* a_row_index;      // compact row r reads A row (and its descale) a_row_index[r]; null = r
     int a_rows;                  // rows of the A buffer (= M without a row index)
     long long b_expert_stride;   // bytes between the weight matrices of consecutive experts

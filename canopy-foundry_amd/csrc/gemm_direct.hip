@@ -1,4 +1,4 @@
-// FP8 GEMM tiles whose operands go from memory straight to the matrix cores' registers:
+// FP8 GEMM on small tiles, K split over a workgroup's wavefronts:
 //     C[M,N] = epilogue( (A[M,K] * sa) . (B[N,K] * sb)^T )  for few rows, few tiles or few rows per expert.
 //
 // The persistent kernels of gemm.hip stage 256 x 256 tiles through LDS, one workgroup per tile: a decode batch of 16 rows
@@ -444,7 +444,7 @@ float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, 
     *shape = i;
     auto estimate = [&](const Shape& sh) {
         const int tn = 16 * sh.nt / (gate ? 2 : 1);
-        const float rounds = static_cast<float>(num_experts) * static_cast<float>((N + tn - 1) / tn) / 256.0f;
+        const float rounds = static_cast<float>(num_experts) * static_cast<float>((N + tn - 1) / tn) / static_cast<float>(num_cus());
         return (rounds < 1.0f ? 1.0f : rounds) * (sh.fixed + static_cast<float>(K) * 16.0f * static_cast<float>(sh.mb + sh.nt) / 93e3f);
     };
     float best = estimate(s[i]);

@@ -237,7 +237,11 @@ int cf_cross_entropy_fwd_bwd_chunk_quant_e5m2(const uint16_t* d_logits, const in
 /* ---- scaled FP8 GEMM -------------------------------------------------------
  * Replaces the reference's cuBLASLt wrappers, which are static functions of
  * src/trainer.cu bound to its Fp8Ctx (handle, workspace, plan cache); the
- * entry points take the same operands without the context.  fp32 accumulate. */
+ * entry points take the same operands without the context.  fp32 accumulate.
+ * Without flags the kernel follows from M, N, K, the epilogue, the scales and the alignment, and with it the order in
+ * which K is summed: the same row in a batch of another size may differ in the last bits of a result, as it may where
+ * cuBLASLt picks another algorithm.  CF_GEMM_FLAG_RING keeps one order for every M (K % 128 == 0); the grouped entry
+ * points choose by total_rows and num_experts and take no flag. */
 
 #define CF_SCALE_PER_TENSOR 0  /* a_descale[1], b_descale[1] (device scalars)   */
 #define CF_SCALE_ROW_COL    1  /* a_descale[M] per token, b_descale[N] per channel */
@@ -252,12 +256,13 @@ int cf_cross_entropy_fwd_bwd_chunk_quant_e5m2(const uint16_t* d_logits, const in
 #define CF_GEMM_FLAG_NAIVE 1   /* run the one-lane-per-output cross-check kernel  */
 #define CF_GEMM_FLAG_STAGED 2  /* take the register-staged tile kernel (the K % 64 != 0 path) */
 #define CF_GEMM_FLAG_DUO 4     /* take the 128 x 128-tile kernel that runs two workgroups per CU (a tile's epilogue under
-                                  the other workgroup's MFMAs) where it applies: E4M3, CF_SCALE_ROW_COL, plain or SiLU-gate
-                                  epilogue, N a multiple of 128 (64 with the SiLU gate) */
+                                  the other workgroup's MFMAs) where it applies: K above 128 and a multiple of 16, per-tensor or
+                                  CF_SCALE_ROW_COL scales, ldc and N multiples of 8 (N of 64 with the SiLU gate, which takes E4M3
+                                  only); accumulating E4M3 x E5M2 forms: ldc and N multiples of 4 */
 #define CF_GEMM_FLAG_DUO_IN_STEP 8 /* with CF_GEMM_FLAG_DUO: do not start the CU's second workgroup half a tile late */
 #define CF_GEMM_FLAG_MFMA32 16 /* plain, bias and SiLU-gate epilogues: keep the ring kernel on v_mfma_f32_32x32x64_f8f6f4
                                   instead of the one on v_mfma_f32_16x16x128_f8f6f4 (the default; same tiles and drain,
-                                  8 - 9 % more MFMA throughput at the same socket power) */
+                                  8 - 9 % more MFMA throughput at the same socket power); implies CF_GEMM_FLAG_RING */
 #define CF_GEMM_FLAG_RING 32   /* keep the persistent 256 x 256-tile kernels (128 x 256 with block scales) where few rows or few
                                   tiles would take a kernel with smaller tiles */
 #define CF_GEMM_FLAG_SMALL 64  /* take the small-tile kernel where it applies, with the tile shape in bits 8 to 11: plain and
