@@ -79,3 +79,10 @@ def test_block_scaled_kernel(cf, M, N, K, kernel):
 ])
 def test_silu_gate_kernel(cf, M, N, K, kernel):
     assert route(cf, M, N, K, mode=ROW_COL, epi=GATE) == kernel
+
+
+def test_block_scales_shape_without_the_lds_for_its_scales(cf):
+    """Groups of scales along K lie in LDS beside the operands: a 64 x 64 tile has room for 125 of them."""
+    assert route(cf, 64, 4096, 16000, mode=BLOCK, flags=F_SMALL | 3 << 8) == SMALL + 3
+    assert route(cf, 64, 4096, 16384, mode=BLOCK, flags=F_SMALL | 3 << 8) == RING
+    assert SMALL <= route(cf, 64, 4096, 16384, mode=BLOCK) < SMALL + 3

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 PER_TENSOR, ROW_COL = 0, 1
 EPI_NONE, EPI_BIAS, EPI_SILU = 0, 1, 2
-NAIVE = 1
+NAIVE, STAGED, DUO, DUO_IN_STEP, MFMA32, RING = 1, 2, 4, 12, 16, 32
 
 
 def rand_fp8(rng, shape, e5m2=False, sigma=1.0):
@@ -56,7 +56,7 @@ SHAPES = [(256, 256, 128), (512, 768, 1024), (300, 200, 144), (1, 1, 16), (33, 5
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
-@pytest.mark.parametrize("flags", [0, NAIVE])
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING])
 def test_gemm_per_tensor(cf, dev, M, N, K, flags):
     case(f"gemm per-tensor {M}x{N}x{K} flags={flags}")
     rng = np.random.default_rng(M + N + K)
@@ -64,17 +64,18 @@ def test_gemm_per_tensor(cf, dev, M, N, K, flags):
     B, sb = rand_fp8(rng, (N, K), sigma=0.02)
     got = run_gemm(cf, dev, A, B, sa, sb, flags=flags)
     ref, absdot = orc.gemm_nt_ref(A, B, [sa], [sb])
-    orc.assert_gemm_close(got, ref, absdot, what=f"{M}x{N}x{K}", acc=orc.ACC_FP32 if flags else orc.ACC_MFMA)
+    orc.assert_gemm_close(got, ref, absdot, what=f"{M}x{N}x{K}", acc=orc.ACC_FP32 if flags == NAIVE else orc.ACC_MFMA)
     # without any allowance: only cancellation points (|ref| << sum|a b|) may exceed 2 bf16 ulps
     off = np.abs(got - ref) > 2 * orc.bf16_ulp(ref)
     assert off.mean() <= 0.03 and np.all(np.abs(ref[off]) <= 2.0 ** -9 * absdot[off])
 
 
 @pytest.mark.parametrize("epi", [EPI_NONE, EPI_BIAS])
-def test_gemm_short_last_column_tile_leaves_row_padding_alone(cf, dev, epi):
+@pytest.mark.parametrize("flags", [0, RING])
+def test_gemm_short_last_column_tile_leaves_row_padding_alone(cf, dev, epi, flags):
     """N = 3 x 256 + 136 with rows of C padded to ldc > N: the persistent kernel stores whole 8-column chunks up to
     N and nothing after it; the element-per-thread kernel is the cross-check."""
-    case(f"gemm N=904 ldc=960 epi={epi}")
+    case(f"gemm N=904 ldc=960 epi={epi} flags={flags}")
     rng = np.random.default_rng(904)
     M, N, K, ldc = 300, 904, 512, 960
     A, _ = rand_fp8(rng, (M, K))
@@ -82,13 +83,13 @@ def test_gemm_short_last_column_tile_leaves_row_padding_alone(cf, dev, epi):
     sa = rng.uniform(0.001, 0.02, M).astype(np.float32)
     sb = rng.uniform(1e-5, 1e-4, N).astype(np.float32)
     bias = orc.bf16_from_f32((rng.standard_normal(N) * 1e-3).astype(np.float32)) if epi == EPI_BIAS else None
-    got = run_gemm(cf, dev, A, B, sa, sb, mode=ROW_COL, epi=epi, bias=bias, ldc=ldc)
+    got = run_gemm(cf, dev, A, B, sa, sb, mode=ROW_COL, epi=epi, bias=bias, ldc=ldc, flags=flags)
     naive = run_gemm(cf, dev, A, B, sa, sb, mode=ROW_COL, epi=epi, bias=bias, ldc=ldc, flags=NAIVE)
     assert np.all(np.isnan(got[:, N:])) and not np.any(np.isnan(got[:, :N]))
     ref, absdot = orc.gemm_nt_ref(A, B, sa, sb, scale_mode=1)
     if epi == EPI_BIAS:
         # bias is added to the bf16-rounded product: exact given the plain result
-        plain = run_gemm(cf, dev, A, B, sa, sb, mode=ROW_COL, ldc=ldc)[:, :N]
+        plain = run_gemm(cf, dev, A, B, sa, sb, mode=ROW_COL, ldc=ldc, flags=flags)[:, :N]
         want = orc.bf16_to_f32(orc.bf16_from_f32((plain + orc.bf16_to_f32(bias)[None, :].astype(np.float64)).astype(np.float32)))
         assert np.array_equal(got[:, :N], want)
     else:
@@ -113,7 +114,7 @@ def test_gemm_exact_small_integers_equals_numpy_matmul(cf, dev):
     assert not np.array_equal(got[:256, :256], got[:256, :256].T)
 
 
-@pytest.mark.parametrize("flags", [0, NAIVE])
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING])
 def test_gemm_e5m2_activations_and_row_stride(cf, dev, flags):
     case(f"gemm e5m2 A + lda flags={flags}")
     rng = np.random.default_rng(5)
@@ -126,7 +127,7 @@ def test_gemm_e5m2_activations_and_row_stride(cf, dev, flags):
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 260, 384), (300, 512, 384), (1100, 256, 640), (300, 264, 384), (520, 904, 640)])
-@pytest.mark.parametrize("flags", [0, NAIVE])
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING])
 def test_gemm_row_col_scales_and_bias(cf, dev, M, N, K, flags):
     case(f"gemm row/col scales + bias {M}x{N}x{K} flags={flags}")
     rng = np.random.default_rng(6)
@@ -146,8 +147,12 @@ def test_gemm_row_col_scales_and_bias(cf, dev, M, N, K, flags):
 
 @pytest.mark.parametrize("M,N,K", [(256, 128, 256), (300, 200, 512), (512, 1408, 2048), (300, 256, 512), (1024, 384, 256)])
 @pytest.mark.parametrize("mode", [PER_TENSOR, ROW_COL])
-def test_gemm_fused_silu_gate(cf, dev, M, N, K, mode):
-    case(f"gemm silu-gate {M}x{N}x{K} mode={mode}")
+@pytest.mark.parametrize("flags", [0, STAGED, RING])
+def test_gemm_fused_silu_gate(cf, dev, M, N, K, mode, flags):
+    """flags: the kernel of the fused call, and of the two plain ones (the persistent one keeps whole column tiles with two
+    weight matrices; the register-staged one sums K as its 32 x 32 x 64 form does, so where N cuts a tile the plain calls follow)."""
+    plain = STAGED if flags == RING and N % 128 else flags
+    case(f"gemm silu-gate {M}x{N}x{K} mode={mode} flags={flags}")
     rng = np.random.default_rng(M + N + mode)
     A, sa = rand_fp8(rng, (M, K))
     Bg, sg = rand_fp8(rng, (N, K), sigma=0.02)
@@ -156,10 +161,10 @@ def test_gemm_fused_silu_gate(cf, dev, M, N, K, mode):
         sa = (sa * rng.uniform(0.5, 2, M)).astype(np.float32)
         sg = (sg * rng.uniform(0.5, 2, N)).astype(np.float32)
         su = (su * rng.uniform(0.5, 2, N)).astype(np.float32)
-    fused = run_gemm(cf, dev, A, Bg, sa, sg, mode=mode, epi=EPI_SILU, B2=Bu, sb2=su)
+    fused = run_gemm(cf, dev, A, Bg, sa, sg, mode=mode, epi=EPI_SILU, B2=Bu, sb2=su, flags=flags)
     # (1) identical to running the two plain GEMMs and the stand-alone swiglu kernel
-    gate = run_gemm(cf, dev, A, Bg, sa, sg, mode=mode)
-    up = run_gemm(cf, dev, A, Bu, sa, su, mode=mode)
+    gate = run_gemm(cf, dev, A, Bg, sa, sg, mode=mode, flags=plain)
+    up = run_gemm(cf, dev, A, Bu, sa, su, mode=mode, flags=plain)
     want = orc.bf16_to_f32(orc.swiglu_forward(orc.bf16_from_f32(gate.astype(np.float32)), orc.bf16_from_f32(up.astype(np.float32)))).astype(np.float64)
     # the fused epilogue evaluates the sigmoid on the hardware exp2 / reciprocal (1 ulp fp32 each): the bf16
     # result may land on the neighbouring value when the product sits at a rounding boundary
@@ -179,16 +184,14 @@ def test_gemm_fused_silu_gate(cf, dev, M, N, K, mode):
         assert rel <= 4e-3, rel      # three bf16 roundings (gate, up, product): ~2^-9 * sqrt(3) relative
 
 
-DUO, DUO_IN_STEP = 4, 12
-
-
 # (300, 256, 384): ragged last row tile, three K-tiles; (1100, 384, 256): two K-tiles (the copy stream a whole tile ahead);
 # (3000, 768, 512): more tiles than workgroups; (128, 128, 1024): a single tile
 @pytest.mark.parametrize("M,N,K", [(300, 256, 384), (1100, 384, 256), (3000, 768, 512), (128, 128, 1024), (520, 512, 640)])
 @pytest.mark.parametrize("epi", [EPI_NONE, EPI_SILU])
 def test_gemm_two_workgroups_per_cu_kernel_matches_the_ring_kernel(cf, dev, M, N, K, epi):
     """CF_GEMM_FLAG_DUO: the 128 x 128-tile kernel accumulates every output over the same sequence of MFMA steps as the
-    256 x 256-tile kernel and runs the same epilogue arithmetic, so the bits are the same; started in step or half a tile apart."""
+    256 x 256-tile kernel on the 32 x 32 x 64 MFMA and runs the same epilogue arithmetic, so the bits are the same; started in
+    step or half a tile apart."""
     case(f"gemm duo {M}x{N}x{K} epi={epi}")
     rng = np.random.default_rng(M + N + K + epi)
     A, sa = rand_fp8(rng, (M, K))
@@ -198,7 +201,7 @@ def test_gemm_two_workgroups_per_cu_kernel_matches_the_ring_kernel(cf, dev, M, N
     sg = (sg * rng.uniform(0.5, 2, N)).astype(np.float32)
     su = (su * rng.uniform(0.5, 2, N)).astype(np.float32)
     kw = dict(mode=ROW_COL, epi=epi, B2=Bu if epi == EPI_SILU else None, sb2=su if epi == EPI_SILU else None)
-    ring = run_gemm(cf, dev, A, Bg, sa, sg, **kw)
+    ring = run_gemm(cf, dev, A, Bg, sa, sg, flags=MFMA32, **kw)
     assert np.array_equal(run_gemm(cf, dev, A, Bg, sa, sg, flags=DUO, **kw), ring)
     assert np.array_equal(run_gemm(cf, dev, A, Bg, sa, sg, flags=DUO_IN_STEP, **kw), ring)
     if epi == EPI_NONE:
@@ -207,9 +210,6 @@ def test_gemm_two_workgroups_per_cu_kernel_matches_the_ring_kernel(cf, dev, M, N
     # a row stride wider than N: the padding stays untouched
     wide = run_gemm(cf, dev, A, Bg, sa, sg, flags=DUO, ldc=N + 40, **kw)
     assert np.array_equal(wide[:, :N], ring) and np.isnan(wide[:, N:]).all()
-
-
-MFMA32 = 16
 
 
 # (300, 256, 384): ragged last row tile, three K-tiles (odd); (1100, 384, 256): two K-tiles; (3000, 768, 512): more tiles than
@@ -234,7 +234,7 @@ def test_gemm_both_mfma_shapes_of_the_ring_kernel(cf, dev, M, N, K, epi, mode):
         su = (su * rng.uniform(0.5, 2, N)).astype(np.float32)
     bias = orc.bf16_from_f32((rng.standard_normal(N) * 0.05).astype(np.float32)) if epi == EPI_BIAS else None
     kw = dict(mode=mode, epi=epi, bias=bias, B2=Bu if epi == EPI_SILU else None, sb2=su if epi == EPI_SILU else None)
-    new = run_gemm(cf, dev, A, Bg, sa, sg, ldc=N + 24, **kw)
+    new = run_gemm(cf, dev, A, Bg, sa, sg, flags=RING, ldc=N + 24, **kw)      # odd K-tile counts: 32 x 32 x 64 as well
     old = run_gemm(cf, dev, A, Bg, sa, sg, flags=MFMA32, ldc=N + 24, **kw)
     assert np.isnan(new[:, N:]).all() and np.isnan(old[:, N:]).all()
     new, old = new[:, :N], old[:, :N]
@@ -249,27 +249,29 @@ def test_gemm_both_mfma_shapes_of_the_ring_kernel(cf, dev, M, N, K, epi, mode):
     assert (new != old).mean() < 0.02
 
 
-def test_gemm_exact_integers_on_both_mfma_shapes(cf, dev):
-    case("gemm exact small integers, 16x16x128 and 32x32x64")
+@pytest.mark.parametrize("K", [640, 512])          # an odd number of K-tiles stays on 32 x 32 x 64
+def test_gemm_exact_integers_on_both_mfma_shapes(cf, dev, K):
+    case(f"gemm exact small integers, 16x16x128 and 32x32x64, K={K}")
     rng = np.random.default_rng(21)
-    M, N, K = 520, 384, 640
+    M, N = 520, 384
     ai = rng.integers(-3, 4, (M, K)).astype(np.float32)
     bi = rng.integers(-2, 3, (N, K)).astype(np.float32)
     A, B = orc.e4m3_satfinite(ai), orc.e4m3_satfinite(bi)
     want = orc.bf16_to_f32(orc.bf16_from_f32((ai @ bi.T).astype(np.float32))).astype(np.float64)
     one = np.float32(1.0)
-    for flags in (0, MFMA32):
+    for flags in (0, RING, MFMA32):
         assert np.array_equal(run_gemm(cf, dev, A, B, one, one, flags=flags), want), flags
 
 
 def test_gemm_duo_flag_on_other_shapes_takes_the_usual_kernels(cf, dev):
     case("gemm duo flag on shapes the kernel does not take")
     rng = np.random.default_rng(9)
-    A, sa = rand_fp8(rng, (300, 384))
-    B, sb = rand_fp8(rng, (200, 384), sigma=0.02)                # N not a multiple of 128
-    assert np.array_equal(run_gemm(cf, dev, A, B, sa, sb, flags=DUO), run_gemm(cf, dev, A, B, sa, sb))
-    B, sb = rand_fp8(rng, (256, 384), sigma=0.02)                # per-tensor scales
-    assert np.array_equal(run_gemm(cf, dev, A, B, sa, sb, flags=DUO), run_gemm(cf, dev, A, B, sa, sb))
+    for N, K in ((204, 384), (256, 128)):                        # N not a multiple of 8; a single K-tile
+        A, sa = rand_fp8(rng, (300, K))
+        B, sb = rand_fp8(rng, (N, K), sigma=0.02)
+        duo = run_gemm(cf, dev, A, B, sa, sb, flags=DUO)
+        assert np.array_equal(duo, run_gemm(cf, dev, A, B, sa, sb, flags=RING))
+        orc.assert_gemm_close(duo, *orc.gemm_nt_ref(A, B, [sa], [sb]), what=f"{N} x {K}")
 
 
 def test_gemm_config2_shape_sampled_rows_and_naive_crosscheck(cf, dev):
@@ -483,7 +485,11 @@ def run_accum(cf, dev, A, B, sa, sb, C0, *, a_e5m2, b_e5m2, flags=0, bf16_out=Fa
     if bf16_out:
         C = dev_bf16(orc.bf16_from_f32(C0.astype(np.float32)), dev)
         assert a_e5m2 is False and b_e5m2 is True
-        cf.cf_fp8_gemm_tn_accum_bf16(M, N, K, dev_arr(A, dev), s(sa), dev_arr(B, dev), s(sb), C, ldc, stream())
+        if flags == 0:
+            cf.cf_fp8_gemm_tn_accum_bf16(M, N, K, dev_arr(A, dev), s(sa), dev_arr(B, dev), s(sb), C, ldc, stream())
+        else:
+            cf.cf_fp8_gemm_nt_accum_bf16_ex(M, N, K, dev_arr(A, dev), K, 0, s(sa), dev_arr(B, dev), K, 1, s(sb), C, ldc, flags,
+                                            stream())
         torch.cuda.synchronize()
         return orc.bf16_to_f32(bf16_bits(C)).astype(np.float64)
     C = torch.from_numpy(C0.astype(np.float32)).to(dev)
@@ -494,7 +500,7 @@ def run_accum(cf, dev, A, B, sa, sb, C0, *, a_e5m2, b_e5m2, flags=0, bf16_out=Fa
 
 
 @pytest.mark.parametrize("M,N,K", [(256, 256, 256), (300, 200, 384), (512, 1024, 2048), (130, 260, 80), (300, 512, 512), (1024, 768, 256)])
-@pytest.mark.parametrize("flags", [0, NAIVE])
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING, DUO_IN_STEP])
 def test_wgrad_tn_accumulate_f32(cf, dev, M, N, K, flags):
     """dW[M,N] fp32 += X^T[M,K](E4M3) . dY^T[N,K](E5M2)^T, beta = 1 (lt_gemm_fp8_tn_accum_f32)."""
     case(f"wgrad accumulate f32 {M}x{N}x{K} flags={flags}")
@@ -508,7 +514,7 @@ def test_wgrad_tn_accumulate_f32(cf, dev, M, N, K, flags):
     # fp32 output: relative L2 against the unrounded reference, elementwise within the accumulation allowance
     rel = np.sqrt(((got - want) ** 2).sum() / (want ** 2).sum())
     assert rel <= 1e-3, rel
-    acc = orc.ACC_FP32 if flags else orc.ACC_MFMA
+    acc = orc.ACC_FP32 if flags == NAIVE else orc.ACC_MFMA
     assert np.all(np.abs(got - want) <= acc * absdot + 2.0 ** -22 * (np.abs(want) + np.abs(C0)))
     if flags == 0 and K % 128 == 0:
         # the named entry point is the same kernel
@@ -520,15 +526,16 @@ def test_wgrad_tn_accumulate_f32(cf, dev, M, N, K, flags):
 
 
 @pytest.mark.parametrize("M,N,K", [(300, 260, 512), (300, 512, 512), (1024, 768, 256), (700, 256, 1152)])
-def test_wgrad_tn_accumulate_bf16(cf, dev, M, N, K):
-    """N a multiple of 256 takes the persistent kernel (ragged last row tile included), 260 the staged one."""
-    case(f"wgrad accumulate bf16 {M}x{N}x{K}")
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING])
+def test_wgrad_tn_accumulate_bf16(cf, dev, M, N, K, flags):
+    """RING: N a multiple of 256 takes the persistent kernel (ragged last row tile included), 260 the staged one."""
+    case(f"wgrad accumulate bf16 {M}x{N}x{K} flags={flags}")
     rng = np.random.default_rng(77 + M + N + K)
     Xt, sx = rand_fp8(rng, (M, K))
     dYt, sy = rand_fp8(rng, (N, K), e5m2=True, sigma=1e-3)
     ref, absdot = orc.gemm_nt_ref(Xt, dYt, [sx], [sy], b_e5m2=True)
     C0 = rng.standard_normal((M, N)) * np.abs(ref).mean()
-    got = run_accum(cf, dev, Xt, dYt, sx, sy, C0, a_e5m2=False, b_e5m2=True, bf16_out=True)
+    got = run_accum(cf, dev, Xt, dYt, sx, sy, C0, a_e5m2=False, b_e5m2=True, bf16_out=True, flags=flags)
     want = orc.bf16_to_f32(orc.bf16_from_f32(C0.astype(np.float32))).astype(np.float64) + ref
     assert np.all(np.abs(got - want) <= 1.01 * orc.bf16_ulp(want) / 2 + orc.ACC_MFMA * absdot)
 
@@ -597,10 +604,10 @@ def block_quant_gpu(cf, dev, x_bf16, kind):
     return q, s, d
 
 
-# (300, 512, 640), (1000, 256, 384), (3000, 768, 512): the persistent kernel (ragged rows; three K-tiles per tile; many tiles per workgroup)
+# RING: (300, 512, 640), (1000, 256, 384), (3000, 768, 512) the persistent kernel (ragged rows; three K-tiles per tile; many tiles)
 @pytest.mark.parametrize("M,N,K", [(128, 256, 128), (256, 256, 256), (300, 200, 384), (130, 260, 208), (64, 512, 1024),
                                    (300, 512, 640), (1000, 256, 384), (3000, 768, 512)])
-@pytest.mark.parametrize("flags", [0, NAIVE])
+@pytest.mark.parametrize("flags", [0, NAIVE, STAGED, RING])
 def test_gemm_block_scaled(cf, dev, M, N, K, flags):
     case(f"gemm block-scaled {M}x{N}x{K} flags={flags}")
     rng = np.random.default_rng(M * 3 + N + K)
@@ -616,14 +623,15 @@ def test_gemm_block_scaled(cf, dev, M, N, K, flags):
     assert np.array_equal(host(xq), oq) and np.array_equal(host(xd), odx)
     ref, absdot = orc.gemm_nt_ref(host(xq), host(wq), host(xd), host(wd), scale_mode=2)
     got = orc.bf16_to_f32(bf16_bits(C)).astype(np.float64)
-    orc.assert_gemm_close(got, ref, absdot, what=f"block {M}x{N}x{K}", acc=orc.ACC_FP32 * 4 if flags else orc.ACC_MFMA)
+    orc.assert_gemm_close(got, ref, absdot, what=f"block {M}x{N}x{K}", acc=orc.ACC_FP32 * 4 if flags == NAIVE else orc.ACC_MFMA)
 
 
 @pytest.mark.parametrize("pad", [4, 2, 8])
-def test_gemm_block_scaled_row_strides_of_c(cf, dev, pad):
+@pytest.mark.parametrize("flags", [0, STAGED, RING])
+def test_gemm_block_scaled_row_strides_of_c(cf, dev, pad, flags):
     """The persistent block-scaled kernel stores whole 128-byte lines when C's rows allow 16-byte accesses and falls
     back to 8-byte or 2-byte stores otherwise: the same bits in all three, and the padding of C's rows untouched."""
-    case(f"gemm block-scaled, ldc = N + {pad}")
+    case(f"gemm block-scaled, ldc = N + {pad}, flags={flags}")
     M, N, K = 300, 512, 640
     rng = np.random.default_rng(pad)
     xb = orc.bf16_from_f32(rng.standard_normal((M, K)).astype(np.float32))
@@ -631,9 +639,9 @@ def test_gemm_block_scaled_row_strides_of_c(cf, dev, pad):
     xq, xs, xd = block_quant_gpu(cf, dev, dev_bf16(xb, dev), "1x128")
     wq, ws, wd = block_quant_gpu(cf, dev, dev_bf16(wb, dev), "128x128")
     C0 = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
-    cf.cf_fp8_gemm_nt_bf16_ex(M, N, K, xq, K, 0, xd, wq, K, wd, BLOCK, EPI_NONE, None, None, None, C0, N, 0, stream())
+    cf.cf_fp8_gemm_nt_bf16_ex(M, N, K, xq, K, 0, xd, wq, K, wd, BLOCK, EPI_NONE, None, None, None, C0, N, flags, stream())
     C1 = torch.full((M, N + pad), float("nan"), dtype=torch.bfloat16, device=dev)
-    cf.cf_fp8_gemm_nt_bf16_ex(M, N, K, xq, K, 0, xd, wq, K, wd, BLOCK, EPI_NONE, None, None, None, C1, N + pad, 0, stream())
+    cf.cf_fp8_gemm_nt_bf16_ex(M, N, K, xq, K, 0, xd, wq, K, wd, BLOCK, EPI_NONE, None, None, None, C1, N + pad, flags, stream())
     torch.cuda.synchronize()
     got = bf16_bits(C1)
     assert np.array_equal(got[:, :N], bf16_bits(C0))

@@ -12,7 +12,16 @@ from test_gpu_gemm import EPI_BIAS, EPI_NONE, EPI_SILU, PER_TENSOR, ROW_COL, ran
 
 pytestmark = pytest.mark.gpu
 
-BLOCK, RING = 2, 32
+BLOCK, RING, SMALL = 2, 32, 64
+KERNEL_SMALL = 16
+
+
+def runs_shape(cf, M, N, K, mode, epi, shape, a_e5m2=0):
+    """Flags that ask for a tile shape, checked to get it."""
+    k, flags = ctypes.c_int(-1), SMALL | shape << 8
+    cf.cf_fp8_gemm_route(M, N, K, a_e5m2, 0, mode, epi, N + 8, flags, ctypes.byref(k))
+    assert k.value == KERNEL_SMALL + shape
+    return flags
 
 
 def pick_rows(M, at_most=40):
@@ -21,9 +30,70 @@ def pick_rows(M, at_most=40):
     return np.unique(np.concatenate([some, [r for r in edges if r < M]]))
 
 
-# one row; one 16-row tile and its neighbours; a K of one tile, of fewer K-tiles than wavefronts, with a last K-tile of 16 and
-# of 112 bytes; columns that end inside a 16-column block, at an odd count; (300, 2000), (700, 2304): 64 x 64 and 128 x 64
-# tiles with ragged edges; (1000, 4080, 4112): 128 x 128 tiles
+# every tile shape by its number: rows and columns that end inside a tile of each (150 = 9 x 16 + 6 = 2 x 64 + 22 = 128 + 22), five
+# whole K-tiles (one wavefront has two) and 16 bytes; a single row and K-tile
+@pytest.mark.parametrize("M,N,K", [(150, 200, 656), (1, 8, 128), (257, 392, 1152)])
+@pytest.mark.parametrize("shape", range(6))
+@pytest.mark.parametrize("kind", ["tensor", "rows_bias", "e5m2"])
+def test_every_tile_shape(cf, dev, M, N, K, shape, kind):
+    case(f"small-tile gemm shape {shape} {M}x{N}x{K} {kind}")
+    e5m2, mode = kind == "e5m2", ROW_COL if kind == "rows_bias" else PER_TENSOR
+    rng = np.random.default_rng(M + N + K + shape)
+    A, sa = rand_fp8(rng, (M, K), e5m2=e5m2)
+    B, sb = rand_fp8(rng, (N, K), sigma=0.02)
+    if mode:
+        sa, sb = (sa * rng.uniform(0.5, 2, M)).astype(np.float32), (sb * rng.uniform(0.5, 2, N)).astype(np.float32)
+    flags = runs_shape(cf, M, N, K, mode, EPI_NONE, shape, int(e5m2))
+    got = run_gemm(cf, dev, A, B, sa, sb, mode=mode, a_e5m2=e5m2, ldc=N + 8, flags=flags)
+    assert np.isnan(got[:, N:]).all()
+    ref, absdot = orc.gemm_nt_ref(A, B, np.atleast_1d(sa), np.atleast_1d(sb), scale_mode=mode, a_e5m2=e5m2)
+    orc.assert_gemm_close(got[:, :N], ref, absdot, what=f"shape {shape} {M}x{N}x{K}")
+    if kind == "rows_bias":                      # added to the bf16 result
+        bias = orc.bf16_from_f32(rng.standard_normal(N).astype(np.float32))
+        biased = run_gemm(cf, dev, A, B, sa, sb, mode=mode, epi=EPI_BIAS, bias=bias, ldc=N + 8, flags=flags)
+        want = orc.bf16_to_f32(orc.bf16_from_f32((got[:, :N] + orc.bf16_to_f32(bias)).astype(np.float32)))
+        assert np.array_equal(biased[:, :N], want)
+
+
+@pytest.mark.parametrize("M,N,K", [(150, 200, 656), (257, 392, 1152)])
+@pytest.mark.parametrize("shape", range(4))
+@pytest.mark.parametrize("mode", [PER_TENSOR, ROW_COL])
+def test_every_tile_shape_silu_gate(cf, dev, M, N, K, shape, mode):
+    case(f"small-tile gemm silu-gate shape {shape} {M}x{N}x{K} mode={mode}")
+    rng = np.random.default_rng(M + N + shape)
+    A, sa = rand_fp8(rng, (M, K))
+    G, sg = rand_fp8(rng, (N, K), sigma=0.02)
+    U, su = rand_fp8(rng, (N, K), sigma=0.02)
+    if mode:
+        sa = (sa * rng.uniform(0.5, 2, M)).astype(np.float32)
+        sg, su = (sg * rng.uniform(0.5, 2, N)).astype(np.float32), (su * rng.uniform(0.5, 2, N)).astype(np.float32)
+    got = run_gemm(cf, dev, A, G, sa, sg, mode=mode, epi=EPI_SILU, B2=U, sb2=su, ldc=N + 8,
+                   flags=runs_shape(cf, M, N, K, mode, EPI_SILU, shape))
+    assert np.isnan(got[:, N:]).all()
+    gref, _ = orc.gemm_nt_ref(A, G, np.atleast_1d(sa), np.atleast_1d(sg), scale_mode=mode, want_abs=False)
+    uref, _ = orc.gemm_nt_ref(A, U, np.atleast_1d(sa), np.atleast_1d(su), scale_mode=mode, want_abs=False)
+    exact = silu_ref(gref, uref)
+    assert np.sqrt(((got[:, :N] - exact) ** 2).sum() / (exact ** 2).sum()) <= 4e-3      # three bf16 roundings
+
+
+# the last: 112 groups of scales along K, the most LDS
+@pytest.mark.parametrize("M,N,K", [(150, 200, 656), (1, 136, 128), (70, 136, 14336)])
+@pytest.mark.parametrize("shape", range(4))
+def test_every_tile_shape_block_scales(cf, dev, M, N, K, shape):
+    case(f"small-tile gemm block scales shape {shape} {M}x{N}x{K}")
+    rng = np.random.default_rng(M + K + shape)
+    A, _ = rand_fp8(rng, (M, K))
+    B, _ = rand_fp8(rng, (N, K), sigma=0.02)
+    sa = rng.uniform(0.5, 2, (M, -(-K // 128))).astype(np.float32)
+    sb = rng.uniform(0.5, 2, (-(-N // 128), -(-K // 128))).astype(np.float32)
+    got = run_gemm(cf, dev, A, B, sa, sb, mode=BLOCK, ldc=N + 8, flags=runs_shape(cf, M, N, K, BLOCK, EPI_NONE, shape))
+    assert np.isnan(got[:, N:]).all()
+    ref, absdot = orc.gemm_nt_ref(A, B, sa, sb, scale_mode=BLOCK)
+    orc.assert_gemm_close(got[:, :N], ref, absdot, what=f"block shape {shape} {M}x{N}x{K}")
+
+
+# What the sizes choose.  One row; one 16-row tile and its neighbours; a K of one tile, of fewer K-tiles than wavefronts, with a
+# last K-tile of 16 and of 112 bytes; columns that end inside a 16-column block, at an odd count
 SHAPES = [(1, 40, 128), (16, 64, 256), (17, 33, 144), (15, 16, 624), (33, 520, 1264), (64, 1032, 512), (130, 1000, 400), (300, 2000, 528),
           (700, 2304, 1040), (1000, 4080, 4112)]
 
