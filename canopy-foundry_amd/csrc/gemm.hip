@@ -2057,19 +2057,19 @@ __global__ __launch_bounds__(256) void k_bank_setup(const int* __restrict__ coun
 
 // What the kernels of this file take for a dense problem, in microseconds: tiles in rounds over the CUs, so much per K-tile and
 // so much per tile.  Measured with a tile on every CU: 256 x 256 tiles 0.95 a K-tile (the
-// register-staged kernel 2.3), 128 x 256 block-scaled tiles 0.65 (1.45).  (At the power limit all of them slow down together.)
+// register-staged kernel 2.3), 128 x 256 block-scaled tiles 0.65 (1.5).  (At the power limit all of them slow down together.)
 float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile, float per_tile) {
     const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
     const int cus = num_cus();
     return static_cast<float>((tiles + cus - 1) / cus) * (static_cast<float>((K + BK - 1) / BK) * per_ktile + per_tile);
 }
 float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
-    if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, block_ring_ok(p) ? 0.65f : 1.45f, 6.0f);
+    if (scale_mode == SCALE_BLOCK) return ring_estimate_us(p.M, p.N, p.K, BSM, BN, block_ring_ok(p) ? 0.65f : 1.5f, 6.0f);
     const bool ring = ring_ok(p, epi, scale_mode);
     // The accumulating ones read and write a round's C with the matrix cores idle (134 MB fp32); the register-staged ones hide
     // nothing of it under their K-tiles.  14336 x 4096 +=, 896 tiles in four rounds: K 256 fp32 107 us, bf16 62; K 4096 243, 205.
     if (epi == EPI_ACCUM_F32) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, 25.0f);
-    if (epi == EPI_ACCUM_BF16) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, c_lines_shared(p, 2) ? 13.7f : 11.1f);
+    if (epi == EPI_ACCUM_BF16) return ring_estimate_us(p.M, p.N, p.K, BM, BN, ring ? 0.95f : 4.0f, c_lines_shared(p, 2) ? 13.3f : 10.7f);
     const bool gate = epi == EPI_SILU_GATE;
     return ring_estimate_us(p.M, p.N, p.K, BM, gate ? BN / 2 : BN, ring ? 0.95f : 2.3f, gate ? 10.4f : 6.0f);
 }

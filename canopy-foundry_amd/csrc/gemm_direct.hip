@@ -361,7 +361,7 @@ constexpr Shape kPlain[6] = {{1, 1, true, 1.5f}, {2, 2, true, 2.0f}, {4, 2, fals
 // the routed layer around them 157 -> 145 us; 18 rows each 157 -> 148; 16 tokens, 1.5 rows each 129 -> 114.
 constexpr Shape kWide[2] = {{1, 4, true, 2.0f}, {2, 4, true, 2.5f}};
 constexpr int kWideShape = 6;           // shape numbers 6 and 7
-constexpr double kBlockRate[4] = {93e3, 75e3, 62e3, 75e3};     // bytes per microsecond and CU with block scales
+constexpr double kBlockRate[4] = {70e3, 75e3, 62e3, 72e3};     // bytes per microsecond and CU with block scales
 constexpr Shape kGate[4] = {{1, 2, true, 1.5f}, {2, 4, true, 2.5f}, {4, 8, false, 6.0f}, {8, 8, false, 12.0f}};
 
 template <int FMT, bool BLOCK, bool GROUPED>
@@ -410,9 +410,9 @@ bool direct_takes(const GemmArgs& p, int epi, int scale_mode, int shape) {
 
 // Picks the tile shape and says what it would take, in microseconds: every workgroup moves K bytes of each of its rows and weight
 // rows, and a CU takes them in at 93 KB per microsecond whatever the shape (measured, K 1024 to 14336); a CU whose LDS holds one
-// workgroup works in whole rounds.  With block scales the folds lower the rate from the second shape on (fitted to 990 sizes):
+// workgroup works in whole rounds.  With block scales the folds lower the rate (fitted to 1400 sizes):
 // 3000 x 512 over K 4096 takes 33.9, 42.4 and 28.7 us in the last three shapes and 29.9 in the persistent kernel, 1000 x 512:
-// 11.7, 12.1, 13.7 and 28.6.
+// 11.7, 12.1, 13.7 and 28.6; 100 x 1000 over K 4096 8.3, 6.7, 8.9 and 11.5 in the four shapes.
 // A shape with more rows than the next one smaller would do is not looked at: its extra rows are copies.
 float direct_estimate_us(const GemmArgs& p, int epi, int scale_mode, int* shape) {
     const bool gate = epi == EPI_SILU_GATE, block = scale_mode == SCALE_BLOCK;

@@ -45,6 +45,7 @@ def test_estimates_ask_what_the_launch_asks(cf):
 @pytest.mark.parametrize("M,N,K,pad,epi,kernel", [
     (4096, 4096, 256, 0, ACCUM_BF16, RING),          # 21.8, 29.2
     (4096, 14336, 512, 0, ACCUM_BF16, RING),         # 74.2, 85.6
+    (4096, 14336, 256, 0, ACCUM_BF16, RING),         # 64.1, 79.9
     (4096, 14336, 512, 4, ACCUM_F32, RING),          # 191, 222: rows of C that do not begin at a line
     (4100, 5636, 256, 0, ACCUM_F32, DUO),            # 116 (register-staged), 94
     (1024, 4096, 1024, 0, ACCUM_F32, DUO),           # 24.1, 13.5: 64 tiles
@@ -61,6 +62,8 @@ def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
     (3000, 512, 2048, (RING, SMALL + 3)),            # 19.1, 23.6, 18.0, 16.9
     (6000, 1000, 7168, (STAGED,)),                   # 197, 227, 137, 103 (register-staged)
     (4096, 1000, 2000, (STAGED,)),                   # 56.6, 70.0, 44.1, 35.6 (register-staged)
+    (100, 1000, 4096, (SMALL + 1,)),                 # 16x16 8.3; 6.7, 8.9, 11.5, 55.5 (register-staged)
+    (1024, 128, 7168, (SMALL + 1,)),                 # 16x16 12.5; 10.7, 15.5, 16.6, 97.4
     (1000, 512, 4096, (SMALL + 1, SMALL + 2)),       # 11.7, 12.1, 13.7, 28.6
     (4096, 7168, 7168, (RING,)),
 ])
