@@ -50,6 +50,8 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
         // A table entry is up to 256 rows of an expert, walked TM at a time.  Where the rows lie on few experts there are fewer entries
         // than workgroups to a column of tiles: those beyond the last entry take every second, third, ... pass of the entries
         // before.  (64 experts of 2 x 1408 x 2048, 1280 rows all on one: 53 us with its entries walked by a workgroup each.)
+        const int* e = p.tile_map + 1 + kMapWords * tm;            // the usual one, read beside the number of entries
+        int number = e[0], first = e[1], last = e[2], first_tile = e[3];
         const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], p.tiles_m));
         if (entries <= 0) return;
         int entry = tm, part = 0, parts = tm + entries < p.tiles_m ? 2 : 1;
@@ -57,11 +59,12 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
             part = tm / entries;
             entry = tm - part * entries;
             parts = (p.tiles_m - 1 - entry) / entries + 1;
+            e = p.tile_map + 1 + kMapWords * entry;
+            number = e[0]; first = e[1]; last = e[2]; first_tile = e[3];
         }
-        const int* e = p.tile_map + 1 + kMapWords * entry;
-        expert = __builtin_amdgcn_readfirstlane(e[0]);
-        m_first = __builtin_amdgcn_readfirstlane(e[1]) + (entry - __builtin_amdgcn_readfirstlane(e[3])) * BM;
-        m_end = min(m_first + BM, __builtin_amdgcn_readfirstlane(e[2]));
+        expert = __builtin_amdgcn_readfirstlane(number);
+        m_first = __builtin_amdgcn_readfirstlane(first) + (entry - __builtin_amdgcn_readfirstlane(first_tile)) * BM;
+        m_end = min(m_first + BM, __builtin_amdgcn_readfirstlane(last));
         m_first += part * TM;
         m_step = parts * TM;
     }
