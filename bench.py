@@ -37,7 +37,7 @@ sys.path.insert(0, str(ROOT))
 FP8_PEAK_TFLOPS = 5000.0      # MI355X dense FP8 MFMA peak (published)
 HBM_PEAK_GBPS = 8000.0        # MI355X HBM3E peak (published)
 TRAFFIC_PROFILE = ROOT / "profiles" / "mlp_config2_hbm_traffic_pmc.txt"
-GEMM_SOURCES = [ROOT / "canopy-foundry_amd" / "csrc" / "gemm.hip", ROOT / "canopy-foundry_amd" / "csrc" / "common.hpp"]
+GEMM_SOURCES = [ROOT / "canopy-foundry_amd" / "csrc" / f for f in ("gemm.hip", "gemm_common.hpp", "common.hpp")]
 
 
 def gemm_source_hash():
