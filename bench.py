@@ -145,7 +145,7 @@ def cpu_baseline(config2_rows=1024):
     workload (first rows of config 2's gate projection), one pass."""
     import numpy as np
     sys.path.insert(0, str(ROOT / "tests"))
-    import oracle_lib as orc      # checker code, used here only as the reported CPU baseline
+    import oracle_lib as orc      # the oracle, used here only as the reported CPU baseline
 
     threads, reported = host_threads()
     rng = np.random.default_rng(1)
