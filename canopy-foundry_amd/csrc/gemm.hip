@@ -2207,6 +2207,9 @@ int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int sca
     if (M <= 0 || N <= 0 || K <= 0 || ldc < N || !kernel || epilogue < EPI_NONE || epilogue > EPI_ACCUM_BF16 ||
         scale_mode < SCALE_TENSOR || scale_mode > SCALE_BLOCK)
         return CF_ERR_INVALID_ARG;
+    const bool accum = epilogue >= EPI_ACCUM_F32;            // what the entry points refuse, or have no argument for
+    if ((scale_mode == SCALE_BLOCK && (epilogue != EPI_NONE || a_is_e5m2)) || (accum ? scale_mode != SCALE_TENSOR : b_is_e5m2 != 0))
+        return CF_ERR_UNSUPPORTED;
     GemmArgs p{};                     // null pointers are aligned ones
     p.M = M; p.N = N; p.K = K; p.lda = K; p.ldb = K; p.ldc = ldc; p.a_rows = M;
     p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;

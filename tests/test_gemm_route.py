@@ -89,3 +89,13 @@ def test_block_scales_shape_without_the_lds_for_its_scales(cf):
     assert route(cf, 64, 4096, 16000, mode=BLOCK, flags=F_SMALL | 3 << 8) == SMALL + 3
     assert route(cf, 64, 4096, 16384, mode=BLOCK, flags=F_SMALL | 3 << 8) == RING
     assert SMALL <= route(cf, 64, 4096, 16384, mode=BLOCK) < SMALL + 3
+
+
+def test_route_refuses_what_the_entry_points_refuse(cf):
+    k = ctypes.c_int(-1)
+    ask = lambda M, N, K, a, b, mode, epi, ldc: cf.raw_cf_fp8_gemm_route(M, N, K, a, b, mode, epi, ldc, 0, ctypes.byref(k))
+    assert ask(64, 256, 256, 0, 0, BLOCK, BIAS, 256) == -2 and ask(64, 256, 256, 1, 0, BLOCK, PLAIN, 256) == -2
+    assert ask(64, 256, 256, 0, 1, TENSOR, PLAIN, 256) == -2 and ask(64, 256, 256, 0, 1, ROW_COL, ACCUM_F32, 256) == -2
+    assert ask(64, 256, 256, 0, 0, TENSOR, 5, 256) == -1 and ask(64, 256, 256, 0, 0, 3, PLAIN, 256) == -1
+    assert ask(64, 256, 256, 0, 0, TENSOR, PLAIN, 255) == -1 and ask(0, 256, 256, 0, 0, TENSOR, PLAIN, 256) == -1
+    assert k.value == -1
