@@ -34,6 +34,11 @@ int grouped_gemm_nt_terms(int total_rows, int N, int Kb, int terms, int num_expe
 int grouped_gemm_bf16_nt(int total_rows, int N, int Kb, int terms, int num_experts, const uint16_t* A, int a_rows, int lda,
                          const int* d_a_row_index, const uint16_t* B, void* C, int ldc, bool c_is_f32, const int* d_tile_map,
                          cf_stream_t stream);
+// What both bf16 GEMM sources ask of their operands (their epilogues address a wavefront's 128 rows of C by 32-bit byte offsets from the block's first element)
+inline bool bf16_operands_ok(const void* A, int lda, const void* B, int ldb, const void* C, int ldc, int c_elem_bytes) {
+    return aligned16(A) && aligned16(B) && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && ldc < (1 << 21) &&
+           (reinterpret_cast<uintptr_t>(C) & (4u * c_elem_bytes - 1u)) == 0;
+}
 // The tile table of a grouped GEMM (k_build_tile_map in gemm.hip): tile_map[0] = number of row tiles of 256 rows,
 // then per row tile (expert, its first row, its end row, its first row tile, its row-tile count), experts back to back.
 // An expert's row range is cut at total_rows, the number of rows the compact buffers hold.

@@ -1,0 +1,62 @@
+"""GPU parity: the weight-gradient kernel of gemm_bf16_duo.hip where its tiles, steps and rules have their edges, on small
+integers: every product and partial sum is exact in fp32, so the result must match a float64 matmul to the bit (bf16: its one
+rounding)."""
+import pytest
+import torch
+
+from gpu_util import case, stream
+
+pytestmark = pytest.mark.gpu
+
+
+def ints(g, *shape):
+    return torch.randint(-4, 5, shape, generator=g).to(torch.bfloat16)
+
+
+def padded(x, ld):
+    out = torch.full((*x.shape[:-1], ld), float("nan"), dtype=x.dtype)
+    out[..., :x.shape[-1]] = x
+    return out
+
+
+# tiles of 256 x 128 and of 128 x 256 (whichever are fewer), one column short of and beyond them; K around the steps of 32, the
+# pairs of steps and the shortest pipeline of four; the last size is beyond the limit from which C is streamed
+@pytest.mark.parametrize("M,N,K", [(256, 128, 1), (128, 256, 31), (264, 120, 33), (120, 264, 64), (248, 136, 65), (8, 8, 127), (512, 384, 129),
+                                   (384, 512, 200), (2048, 2056, 96), (5128, 5192, 40)])
+@pytest.mark.parametrize("f32", [True, False])
+def test_wgrad_edges(cf, dev, M, N, K, f32):
+    case(f"bf16 wgrad {M}x{N}x{K} f32 {f32}")
+    g = torch.Generator().manual_seed(M + N + K)
+    A, B = ints(g, K, M), ints(g, K, N)
+    C0 = ints(g, M, N).to(torch.float32 if f32 else torch.bfloat16)
+    lda, ldb, ldc = M + 8, N + 16, N + 4
+    C = padded(C0, ldc).to(dev)
+    call = cf.cf_gemm_bf16_tn_accum_f32 if f32 else cf.cf_gemm_bf16_tn_accum_bf16
+    call(M, N, K, padded(A, lda).to(dev), lda, padded(B, ldb).to(dev), ldb, C, ldc, stream())
+    want = (C0.double() + A.double().T @ B.double()).to(C0.dtype)
+    got = C.cpu()
+    assert torch.equal(got[:, :N], want)
+    assert torch.isnan(got[:, N:]).all()           # the row padding of C is left alone
+
+
+# rows per expert from none to several tiles' worth of steps; enough tiles for every workgroup to walk several
+@pytest.mark.parametrize("M,N,counts", [(264, 136, [0, 1, 63, 64, 65, 0, 129, 300, 5]), (136, 264, [40, 0, 0, 7]),
+                                        (1408, 1024, [70, 0, 33, 1, 0, 64, 97, 128, 3, 200, 0, 32])])
+@pytest.mark.parametrize("f32", [True, False])
+def test_grouped_wgrad_edges(cf, dev, M, N, counts, f32):
+    case(f"grouped bf16 wgrad {M}x{N} {counts} f32 {f32}")
+    g = torch.Generator().manual_seed(sum(counts) + M)
+    R, E = sum(counts), len(counts)
+    A, B = ints(g, R, M), ints(g, R, N)
+    C0 = ints(g, E, M, N).to(torch.float32 if f32 else torch.bfloat16)
+    C0[counts.index(0)] = -0.0                      # an expert without rows keeps its bits
+    offsets = [sum(counts[:e]) for e in range(E)]
+    C = C0.to(dev)
+    call = cf.cf_moe_grouped_gemm_bf16_tn_accum_f32 if f32 else cf.cf_moe_grouped_gemm_bf16_tn_accum_bf16
+    call(M, N, R, E, torch.tensor(counts, dtype=torch.int32, device=dev), torch.tensor(offsets, dtype=torch.int32, device=dev),
+         A.to(dev), M, B.to(dev), N, C, stream())
+    got = C.cpu()
+    for e, (o, n) in enumerate(zip(offsets, counts)):
+        want = (C0[e].double() + A[o:o + n].double().T @ B[o:o + n].double()).to(C0.dtype) if n else C0[e]
+        assert torch.equal(got[e], want), f"expert {e}"
+        assert n or torch.equal(torch.signbit(got[e]), torch.signbit(want))
