@@ -2080,17 +2080,22 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
     if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
         (epi == EPI_SILU_GATE && !aligned16(p.B2)))
         return {CF_GEMM_KERNEL_NAIVE, 0};
-    const bool duo = duo_ok(p, fmt, epi, scale_mode), small = direct_ok(p, fmt, epi, scale_mode);
+    const bool duo = duo_ok(p, fmt, epi, scale_mode), half = half_ok(p, fmt, epi, scale_mode), small = direct_ok(p, fmt, epi, scale_mode);
     const bool ring = scale_mode == SCALE_BLOCK ? block_ring_ok(p) : ring_ok(p, epi, scale_mode);
     Route best{!ring || p.force_staged                       ? CF_GEMM_KERNEL_STAGED
                : epi <= EPI_SILU_GATE && scale_mode != SCALE_BLOCK && ring16_ok(p) ? CF_GEMM_KERNEL_RING16 : CF_GEMM_KERNEL_RING, 0};
     if (p.small && small && direct_takes(p, epi, scale_mode, p.small - 1)) return {CF_GEMM_KERNEL_SMALL, p.small - 1};
     if (p.duo && duo) return {CF_GEMM_KERNEL_DUO, 0};
-    if (p.small || p.duo || p.ring || p.force_staged) return best;
+    if (p.half && half) return {CF_GEMM_KERNEL_HALF, 0};
+    if (p.small || p.duo || p.half || p.ring || p.force_staged) return best;
     float t = persistent_estimate_us(p, epi, scale_mode);
     if (duo) {
         const float d = duo_estimate_us(p, epi);
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
+    }
+    if (half && p.M > 128) {          // (with fewer rows half of the tile or more is padding)
+        const float d = half_estimate_us(p, epi);
+        if (d * (best.kernel == CF_GEMM_KERNEL_DUO ? 1.03f : 1.0f) < t) { t = d; best = {CF_GEMM_KERNEL_HALF, 0}; }
     }
     if (small) {
         int shape = 0;
@@ -2119,6 +2124,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
     }
     if (route.kernel == CF_GEMM_KERNEL_SMALL) return gemm_nt_direct(p, fmt, epi, scale_mode, route.shape, st);
     if (route.kernel == CF_GEMM_KERNEL_DUO) return gemm_nt_duo(p, fmt, epi, scale_mode, st);
+    if (route.kernel == CF_GEMM_KERNEL_HALF) return gemm_nt_half(p, fmt, epi, scale_mode, st);
     if (scale_mode == SCALE_BLOCK) {
         static std::once_flag once;
         static hipError_t attr_err = hipSuccess;
@@ -2199,6 +2205,7 @@ int cf_fp8_gemm_nt_bf16_ex(int M, int N, int K, const void* A, int lda, int a_is
     p.mfma32 = (flags & CF_GEMM_FLAG_MFMA32) != 0;
     p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
     p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
+    p.half = (flags & CF_GEMM_FLAG_HALF) != 0;
     return gemm_nt(p, a_is_e5m2 ? 1 : 0, epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE, stream);
 }
 
@@ -2217,6 +2224,7 @@ int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int sca
     p.mfma32 = (flags & CF_GEMM_FLAG_MFMA32) != 0;
     p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
     p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
+    p.half = (flags & CF_GEMM_FLAG_HALF) != 0;
     const Route r = gemm_route(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE);
     *kernel = r.kernel + r.shape;
     return CF_OK;

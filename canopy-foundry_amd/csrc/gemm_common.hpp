@@ -29,6 +29,7 @@ struct GemmArgs {
     int force_staged;            // take the register-staged kernel even when the ring kernel applies
     int duo;                     // 1: the two-workgroups-per-CU kernel where it applies, 2: the same without the stagger, 0: where its estimate is lowest
     int small;                   // 1 + the tile shape of the small-tile kernel a caller asks for, 0: where its estimate is lowest
+    int half;                    // take the half-tile kernel where it applies
     int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
     // grouped (per-expert) form, ring and small-tile kernels; all null / 0 for a dense GEMM
@@ -101,6 +102,10 @@ float direct_estimate_us(const GemmArgs& p, int epi, int scale_mode, int* shape)
 float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape);
 int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st);
 int grouped_gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int shape, hipStream_t st);
+// gemm_half.hip: whether it takes a problem, its time, the launch
+bool half_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
+float half_estimate_us(const GemmArgs& p, int epi);
+int gemm_nt_half(const GemmArgs& p, int fmt, int epi, int scale_mode, hipStream_t st);
 // gemm_duo.hip: whether it takes a problem, its time, the launch
 bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
 float duo_estimate_us(const GemmArgs& p, int epi);

@@ -459,8 +459,8 @@ bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
     return p.N % 8 == 0 && (epi != EPI_BIAS || aligned16(p.bias));
 }
 
-// Microseconds: 0.48 a K-tile where a CU holds one workgroup (0.62 with the SiLU gate), 0.875 for both where it holds two
-// (measured, 4096 columns, K 4096 to 14336); a third more where K is no multiple of 128 and a row's 128-byte pieces therefore
+// Microseconds: 0.48 a K-tile where a CU holds one workgroup (0.62 with the SiLU gate), 0.875 for both where it holds two, less where
+// only some CUs hold two and there is one round (measured, 4096 columns, K 4096 to 14336: 288 workgroups 0.70 to 0.74, 384 0.77 to 0.80, 448 0.82); a third more where K is no multiple of 128 and a row's 128-byte pieces therefore
 // lie across lines.  Per round of tiles 2.5 for the fill and the bf16 store (hidden in a last round that follows others), 3 for
 // those and the SiLU gate's arithmetic (1.2 there).  512 x 2 x 14336 over K 1024, a round and three quarters: 26.0 us, 20.8 in
 // the ring kernel; 1500 x 2 x 4096: 16.5, 19.1.
@@ -477,8 +477,9 @@ float duo_estimate_us(const GemmArgs& p, int epi) {
     const bool gate = epi == EPI_SILU_GATE, accum = epi == EPI_ACCUM_F32 || epi == EPI_ACCUM_BF16;
     const float tile = epi == EPI_ACCUM_F32 ? (c_lines_shared(p, 4) ? 14.0f : 8.0f) : epi == EPI_ACCUM_BF16 ? (c_lines_shared(p, 2) ? 6.2f : 5.5f)
                      : gate ? 3.0f : 2.5f;
+    const float two = accum || full > 0 || p.M <= DM ? 0.875f : 0.70f + 0.175f * static_cast<float>(rest - most) / static_cast<float>(most);
     const float last = full == 0 || accum ? tile : gate ? 1.2f : 0.0f;
-    return static_cast<float>(full) * (kt * 0.875f + tile) + (rest == 0 ? 0.0f : kt * (rest > most ? 0.875f : gate ? 0.62f : 0.48f) + last);
+    return static_cast<float>(full) * (kt * 0.875f + tile) + (rest == 0 ? 0.0f : kt * (rest > most ? two : gate ? 0.62f : 0.48f) + last);
 }
 
 int gemm_nt_duo(GemmArgs p, int fmt, int epi, int scale_mode, hipStream_t st) {

@@ -269,6 +269,9 @@ int cf_cross_entropy_fwd_bwd_chunk_quant_e5m2(const uint16_t* d_logits, const in
                                   bias 0 to 5, block scales 0 to 3: 16x16, 32x32, 64x32, 64x64, 128x64, 128x128 outputs; SiLU gate
                                   0 to 3: 16x16, 32x32, 64x64, 128x64 */
 
+#define CF_GEMM_FLAG_HALF 128  /* take the kernel of 256 x 128 or 128 x 256 tiles (SiLU gate: 128 x 128 outputs) where it applies:
+                                  plain, bias and SiLU-gate epilogues, otherwise as CF_GEMM_FLAG_DUO (gate: N a multiple of 8) */
+
 /* lt_gemm_fp8_nt, static at src/trainer.cu:4498-4534 (plan lookup :4402-4496).
  * C[M,N] bf16 (row stride ldc) = (A[M,K] fp8, row stride lda, E4M3 or E5M2) .
  * (B[N,K] E4M3, contiguous)^T, per-tensor device descales, alpha 1, beta 0. */
@@ -304,6 +307,7 @@ int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const 
 #define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: its own) */
 #define CF_GEMM_KERNEL_RING16 3    /* the same on 16 x 16 x 128 MFMAs */
 #define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU */
+#define CF_GEMM_KERNEL_HALF   5    /* persistent, 256 x 128 or 128 x 256 tiles, one workgroup per CU */
 #define CF_GEMM_KERNEL_SMALL  16   /* + tile shape (see CF_GEMM_FLAG_SMALL): K split over a workgroup's wavefronts */
 
 /* Which kernel (CF_GEMM_KERNEL_*) the dense GEMM entry points run a problem on (16-byte aligned operands, descales and

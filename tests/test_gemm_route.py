@@ -4,10 +4,10 @@ import ctypes
 
 import pytest
 
-NAIVE, STAGED, RING, RING16, DUO, SMALL = 0, 1, 2, 3, 4, 16
+NAIVE, STAGED, RING, RING16, DUO, HALF, SMALL = 0, 1, 2, 3, 4, 5, 16
 TENSOR, ROW_COL, BLOCK = 0, 1, 2
 PLAIN, BIAS, GATE, ACCUM_F32, ACCUM_BF16 = range(5)
-F_NAIVE, F_STAGED, F_DUO, F_MFMA32, F_RING, F_SMALL = 1, 2, 4, 16, 32, 64
+F_NAIVE, F_STAGED, F_DUO, F_MFMA32, F_RING, F_SMALL, F_HALF = 1, 2, 4, 16, 32, 64, 128
 
 
 def route(cf, M, N, K, mode=TENSOR, epi=PLAIN, flags=0, pad=0, a_e5m2=0):
@@ -82,6 +82,22 @@ def test_block_scaled_kernel(cf, M, N, K, kernel):
 ])
 def test_silu_gate_kernel(cf, M, N, K, kernel):
     assert route(cf, M, N, K, mode=ROW_COL, epi=GATE) == kernel
+
+
+# half tiles against the kernel that was the fastest of the others (two workgroups per CU, 128 x 128 small tiles, 256 x 256 tiles)
+@pytest.mark.parametrize("M,N,K,epi,kernel", [
+    (2048, 4096, 50304, PLAIN, HALF),                # 317 us, small tiles 361: 256 half tiles
+    (2048, 4096, 14336, PLAIN, HALF),                # 90.8, two per CU 102.6
+    (1000, 4096, 14336, PLAIN, SMALL + 5),           # 71.8, small tiles 52.8: 128 half tiles
+    (4000, 2048, 32000, PLAIN, HALF),                # 189, small tiles 302
+    (257, 14336, 4096, PLAIN, DUO),                  # 27.0, two per CU 24.9
+    (8192, 4096, 14336, PLAIN, RING16),              # 346, 256 x 256 tiles 294
+    (700, 14336, 4096, GATE, HALF),                  # 79.3, 256 x 256 tiles 88.7: 336 of those are one and a third rounds
+    (8192, 14336, 4096, GATE, RING16),               # 733, 653
+])
+def test_half_tiles(cf, M, N, K, epi, kernel):
+    assert route(cf, M, N, K, mode=ROW_COL, epi=epi) == kernel
+    assert route(cf, M, N, K, mode=ROW_COL, epi=epi, flags=F_HALF) == HALF
 
 
 def test_block_scales_shape_without_the_lds_for_its_scales(cf):
