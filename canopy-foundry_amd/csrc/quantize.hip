@@ -6,6 +6,7 @@
 // two 128-bit loads and one 128-bit store, a wavefront reduces with xor
 // shuffles, and a workgroup issues one atomic.
 #include "common.hpp"
+#include "gelu_table.hpp"
 #include "internal.hpp"
 #include <mutex>
 
@@ -485,18 +486,16 @@ __global__ __launch_bounds__(kThreads) void k_quant_rows(const uint16_t* __restr
     }
 }
 
-// GELU + per-row quantize for many rows: the exact-erf GELU of a bf16 value is a function of its 16 bits, so a
-// workgroup that stays on its CU builds the table of all 65536 results once (128 KiB of LDS, 64 erff per lane) and then
-// looks every element up instead of evaluating erff, which is what the plain form above waits for (about 40 vector
-// instructions per element).  Same bits: the table holds bf16(gelu_fwd(x)) for every x.
+// GELU + per-row quantize for many rows: workgroups that stay on their CU look every element up (gelu_table.hpp) instead of
+// evaluating erff, which is what the plain form above waits for.  Same bits.  24576 x 1408: direct 47.4 us, 25.6; x from memory 55.0
+// and 41.8.
 constexpr int kLutThreads = 1024;
 __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint16_t* __restrict__ x, int rows, int K,
                                                                      uint8_t* __restrict__ out, float* __restrict__ scale,
                                                                      float* __restrict__ descale) {
-    extern __shared__ uint16_t lut[];
-    for (int i = threadIdx.x; i < 65536; i += kLutThreads) lut[i] = f32_to_bf16(gelu_fwd(bf16_to_f32(static_cast<uint16_t>(i))));
+    __shared__ uint16_t table[kGeluEntries];
+    gelu_table_build(table);
     __syncthreads();
-    auto look2 = [&](uint32_t pair) { return static_cast<uint32_t>(lut[pair & 0xffffu]) | (static_cast<uint32_t>(lut[pair >> 16]) << 16); };
     constexpr int MAXS = 4;
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (kLutThreads / 64);
@@ -514,8 +513,8 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
         for (int s = 0; s < MAXS; ++s) {
             const int k = (s * 64 + lane) * kVec;
             if (k < K) {
-                v[s].lo = make_uint4(look2(v[s].lo.x), look2(v[s].lo.y), look2(v[s].lo.z), look2(v[s].lo.w));
-                v[s].hi = make_uint4(look2(v[s].hi.x), look2(v[s].hi.y), look2(v[s].hi.z), look2(v[s].hi.w));
+                v[s].lo = gelu_look8(table, v[s].lo);
+                v[s].hi = gelu_look8(table, v[s].hi);
                 acc = absmax16(acc, v[s]);
             }
         }
@@ -540,14 +539,15 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
     }
 }
 
-// k_grouped_quant_delayed with GELU for large banks, on the same table: one workgroup per CU stays resident, builds
-// the 65536-entry table once and then takes the (expert, part) items w = blockIdx.x, blockIdx.x + gridDim.x, ...
+// k_grouped_quant_delayed with GELU for all but small banks, on the same table: two workgroups per CU stay resident, build
+// the table once and then take the (expert, part) items w = blockIdx.x, blockIdx.x + gridDim.x, ...
 // (part p of `per` covers the expert's 16-element vectors p * 1024 + lane, stepping per * 1024).  An item ends as a
 // workgroup of the plain form does: maximum into the slot's running amax, one arrival; the item that arrives last of an
 // expert's `per` updates the slot.  The slot's state changes only in that last step, and only after every item of the
 // expert has arrived, so what a workgroup reads of it at the start of the kernel (row range and scale pair of every
-// expert, into LDS, under the table build) is the state the call started with; the history is read by the last
-// arrival alone.  Same bits as the plain form: the table holds bf16(gelu_fwd(x)) for every x.
+// expert, into LDS, under the table build, and of an expert's history at the start of an item) is the state the call started
+// with.  Same bits as the plain form.
+// 24576 x 1408, 64 experts: direct 43.8 us, 28.6 (5.2 of 3 bytes an element); x from memory 51.9 and 46.3.
 constexpr int kLutMaxExperts = 1024;
 template <bool E5M2, bool RECOMPUTE>
 __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(const uint16_t* __restrict__ x, uint8_t* __restrict__ out,
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
                                                                                int num_experts, int per, float* __restrict__ states,
                                                                                int stride, int history_len, float fp8_max,
                                                                                float* __restrict__ row_descale) {
-    extern __shared__ uint16_t lut[];
+    __shared__ uint16_t table[kGeluEntries];
     __shared__ float sh[2][kLutThreads / 64];
     __shared__ int sh_first[kLutMaxExperts], sh_rows[kLutMaxExperts];
     __shared__ float sh_scale[kLutMaxExperts], sh_descale[kLutMaxExperts];
@@ -568,9 +568,8 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
         sh_scale[e] = st[RECOMPUTE ? slotw::SCALE_SNAP : slotw::SCALE];
         sh_descale[e] = st[RECOMPUTE ? slotw::DESCALE_SNAP : slotw::DESCALE];
     }
-    for (int i = threadIdx.x; i < 65536; i += kLutThreads) lut[i] = f32_to_bf16(gelu_fwd(bf16_to_f32(static_cast<uint16_t>(i))));
+    gelu_table_build(table);
     __syncthreads();
-    auto look2 = [&](uint32_t pair) { return static_cast<uint32_t>(lut[pair & 0xffffu]) | (static_cast<uint32_t>(lut[pair >> 16]) << 16); };
     const int items = num_experts * per;
     int parity = 0;
     for (int w = blockIdx.x; w < items; w += gridDim.x) {
@@ -579,6 +578,18 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
         if (rows <= 0) continue;                                     // uniform over the workgroup
         const int first = sh_first[e];
         const float s = sh_scale[e], ds = sh_descale[e];
+        // what the last arrival needs of the history, read under the streaming work
+        float pre_max = 0.0f;
+        int cursor = 0, count = 0;
+        if (!RECOMPUTE && threadIdx.x == 0 && history_len > 0) {
+            const float* st = states + static_cast<size_t>(e) * stride;
+            cursor = reinterpret_cast<const int*>(st)[slotw::CURSOR];
+            count = reinterpret_cast<const int*>(st)[slotw::COUNT];
+            if (cursor < 0 || cursor >= history_len) cursor = 0;
+            if (count < history_len) ++count;
+            for (int i = 0; i < count; ++i)
+                if (i != cursor) pre_max = fmaxf(pre_max, st[slotw::HISTORY + i]);
+        }
         const bool s_finite = fabsf(s) < __uint_as_float(0x7f800000u);
         const size_t tid = static_cast<size_t>(part) * kLutThreads + threadIdx.x;
         const size_t stride_t = static_cast<size_t>(per) * kLutThreads;
@@ -598,8 +609,8 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
             for (int b = 0; b < kBatch; ++b) {
                 const size_t i = i0 + b * stride_t;
                 if (i < nvec) {
-                    v[b].lo = make_uint4(look2(v[b].lo.x), look2(v[b].lo.y), look2(v[b].lo.z), look2(v[b].lo.w));
-                    v[b].hi = make_uint4(look2(v[b].hi.x), look2(v[b].hi.y), look2(v[b].hi.z), look2(v[b].hi.w));
+                    v[b].lo = gelu_look8(table, v[b].lo);
+                    v[b].hi = gelu_look8(table, v[b].hi);
                     store_stream16(oe + i * kVec, quant16_track<E5M2, !RECOMPUTE>(v[b], s, s_finite, local_bits, local));
                 }
             }
@@ -621,13 +632,6 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
                     const float a = fmaxf(amax, 1e-12f);
                     float hist_max = a;
                     if (history_len > 0) {
-                        int cursor = reinterpret_cast<const int*>(st)[slotw::CURSOR];
-                        int count = reinterpret_cast<const int*>(st)[slotw::COUNT];
-                        if (cursor < 0 || cursor >= history_len) cursor = 0;
-                        if (count < history_len) ++count;
-                        float pre_max = 0.0f;
-                        for (int i = 0; i < count; ++i)
-                            if (i != cursor) pre_max = fmaxf(pre_max, st[slotw::HISTORY + i]);
                         st[slotw::HISTORY + cursor] = a;
                         hist_max = fmaxf(cursor < count ? fmaxf(pre_max, a) : pre_max, 1e-12f);
                         reinterpret_cast<int*>(st)[slotw::CURSOR] = (cursor + 1) % history_len;
@@ -912,6 +916,16 @@ int launch_quant(const uint16_t* x, void* out, const float* scale, float* amax, 
     return launch_status();
 }
 
+// From here on the table form of the row quantize is the faster one (2048 x 1408: 8.7 us direct, 7.0; 512 x 1408 7.5, 7.5), the
+// grouped one with its arrivals from twice that (64 experts, 1536 x 1408 in all: 12.8, 13.9; 6144 x 1408: 19.7, 15.5).
+constexpr size_t kGeluTableFrom = 2u << 20;
+int resident_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        return (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : 256;
+    }();
+    return cus;
+}
 // per-row quantize: the register-resident forms where the row fits, the two-pass form otherwise
 template <bool E5M2, bool GELU>
 int launch_quant_rows(const uint16_t* d_x, int rows, int K, void* d_out, float* d_scale, float* d_descale, cf_stream_t stream) {
@@ -923,21 +937,8 @@ int launch_quant_rows(const uint16_t* d_x, int rows, int K, void* d_out, float* 
     const bool vec = aligned16(d_x) && aligned16(d_out) && K % kVec == 0 && K > 0;
     const unsigned grid = ceil_div(rows, kThreads / 64);
     if constexpr (GELU && !E5M2) {
-        // enough rows to pay for 256 tables of 65536 entries (each costs what 64 rows of 1024 elements cost directly)
-        if (vec && K <= 4 * 1024 && static_cast<size_t>(rows) * K >= (64u << 20)) {
-            static std::once_flag once;
-            static hipError_t err = hipSuccess;
-            static int cus = 256;
-            std::call_once(once, [] {
-                err = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gelu_quant_rows_lut),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-                int dev = 0, n = 0;
-                if (hipGetDevice(&dev) == hipSuccess &&
-                    hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-                    cus = n;
-            });
-            if (err != hipSuccess) return static_cast<int>(err);
-            k_gelu_quant_rows_lut<<<cus, kLutThreads, 128 * 1024, st>>>(d_x, rows, K, o, d_scale, d_descale);
+        if (vec && K <= 4 * 1024 && static_cast<size_t>(rows) * K >= kGeluTableFrom) {
+            k_gelu_quant_rows_lut<<<2 * resident_cus(), kLutThreads, 0, st>>>(d_x, rows, K, o, d_scale, d_descale);
             return launch_status();
         }
     }
@@ -1043,32 +1044,16 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
                                           fp8_max, d_row_descale);
     };
     const int which = (is_e5m2 ? 4 : 0) | (apply_gelu ? 2 : 0) | (is_recompute ? 1 : 0);
-    // GELU over a large bank: the table form (the direct form waits for erff, about 40 vector instructions per element)
-    if (apply_gelu && num_experts <= kLutMaxExperts && static_cast<size_t>(total_rows) * K >= (64u << 20)) {
-        static std::once_flag once;
-        static hipError_t err = hipSuccess;
-        static int cus = 256;
-        std::call_once(once, [] {
-            const void* ks[4] = {reinterpret_cast<const void*>(&k_grouped_gelu_quant_delayed_lut<false, false>),
-                                 reinterpret_cast<const void*>(&k_grouped_gelu_quant_delayed_lut<false, true>),
-                                 reinterpret_cast<const void*>(&k_grouped_gelu_quant_delayed_lut<true, false>),
-                                 reinterpret_cast<const void*>(&k_grouped_gelu_quant_delayed_lut<true, true>)};
-            for (const void* k : ks) {
-                const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-                if (e != hipSuccess) err = e;
-            }
-            int dev = 0, n = 0;
-            if (hipGetDevice(&dev) == hipSuccess &&
-                hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-                cus = n;
-        });
-        if (err != hipSuccess) return static_cast<int>(err);
-        // parts per expert: about four items per resident workgroup, so ragged experts even out
-        int parts = (4 * cus + num_experts - 1) / num_experts;
+    // GELU: the table form (the direct form waits for erff)
+    if (apply_gelu && num_experts <= kLutMaxExperts && static_cast<size_t>(total_rows) * K >= 2 * kGeluTableFrom) {
+        const int cus = resident_cus();
+        // Parts per expert: an item per resident workgroup.  An item ends in an arrival of a few dependent atomics: with two items each
+        // 31.8 us at 24576 x 1408 and 64 experts instead of 28.6 (four: 45.2).
+        int parts = (2 * cus + num_experts - 1) / num_experts;
         parts = parts < 1 ? 1 : (parts > 64 ? 64 : parts);
         auto launch_lut = [&](auto kernel) {
-            kernel<<<cus, kLutThreads, 128 * 1024, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
-                                                         state_stride_words, history_len, fp8_max, d_row_descale);
+            kernel<<<2 * cus, kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
+                                                    state_stride_words, history_len, fp8_max, d_row_descale);
         };
         switch (which & 5) {
             case 0: launch_lut(k_grouped_gelu_quant_delayed_lut<false, false>); break;
