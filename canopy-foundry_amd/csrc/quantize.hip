@@ -8,7 +8,6 @@
 #include "common.hpp"
 #include "gelu_table.hpp"
 #include "internal.hpp"
-#include <mutex>
 
 namespace cf {
 namespace {
@@ -487,16 +486,17 @@ __global__ __launch_bounds__(kThreads) void k_quant_rows(const uint16_t* __restr
 }
 
 // GELU + per-row quantize for many rows: workgroups that stay on their CU look every element up (gelu_table.hpp) instead of
-// evaluating erff, which is what the plain form above waits for.  Same bits.  24576 x 1408: direct 47.4 us, 25.6; x from memory 55.0
-// and 41.8.
+// evaluating erff, which is what the plain form above waits for.  Same bits.  MAXS 16-element vectors per lane: with four of them for
+// rows that need two, 24576 x 1408 takes 25.6 us and 98304 x 1408 104, with two 21.3 and 81 (direct 47.3; looked up in a table of all
+// bf16 values 103); x from memory 45, 139 against 38, 131.
 constexpr int kLutThreads = 1024;
+template <int MAXS>
 __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint16_t* __restrict__ x, int rows, int K,
                                                                      uint8_t* __restrict__ out, float* __restrict__ scale,
                                                                      float* __restrict__ descale) {
     __shared__ uint16_t table[kGeluEntries];
     gelu_table_build(table);
     __syncthreads();
-    constexpr int MAXS = 4;
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (kLutThreads / 64);
     for (int row = blockIdx.x * (kLutThreads / 64) + (threadIdx.x >> 6); row < rows; row += waves) {
@@ -539,7 +539,7 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
     }
 }
 
-// k_grouped_quant_delayed with GELU for all but small banks, on the same table: two workgroups per CU stay resident, build
+// k_grouped_quant_delayed with GELU for all but small banks, on the same table: up to two workgroups per CU stay, build
 // the table once and then take the (expert, part) items w = blockIdx.x, blockIdx.x + gridDim.x, ...
 // (part p of `per` covers the expert's 16-element vectors p * 1024 + lane, stepping per * 1024).  An item ends as a
 // workgroup of the plain form does: maximum into the slot's running amax, one arrival; the item that arrives last of an
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
 // expert has arrived, so what a workgroup reads of it at the start of the kernel (row range and scale pair of every
 // expert, into LDS, under the table build, and of an expert's history at the start of an item) is the state the call started
 // with.  Same bits as the plain form.
-// 24576 x 1408, 64 experts: direct 43.8 us, 28.6 (5.2 of 3 bytes an element); x from memory 51.9 and 46.3.
+// 24576 x 1408, 64 experts: direct 43.7 us, 22.9 (104 MB: 4.5 TB/s); x from memory 51.6 and 43.7.
 constexpr int kLutMaxExperts = 1024;
 template <bool E5M2, bool RECOMPUTE>
 __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(const uint16_t* __restrict__ x, uint8_t* __restrict__ out,
@@ -916,9 +916,11 @@ int launch_quant(const uint16_t* x, void* out, const float* scale, float* amax, 
     return launch_status();
 }
 
-// From here on the table form of the row quantize is the faster one (2048 x 1408: 8.7 us direct, 7.0; 512 x 1408 7.5, 7.5), the
-// grouped one with its arrivals from twice that (64 experts, 1536 x 1408 in all: 12.8, 13.9; 6144 x 1408: 19.7, 15.5).
-constexpr size_t kGeluTableFrom = 2u << 20;
+// From here on the table form of the row quantize is the faster one.  Rows of up to 2048 elements: 512 x 1408 7.5 us both ways, 1024 x
+// 2048 7.5 directly and 6.6.  Wider rows have few wavefronts at work in small tensors: 512 x 4096 5.5 and 9.5, 2048 x 4096 10.9 and
+// 10.0, 4096 x 4096 18.5 and 10.4.  The grouped form with its arrivals from twice the first line: 8 experts, 1500 x 1408 9.6 and 8.0,
+// 64 experts, 3072 x 1408 12.7 and 10.3.
+constexpr size_t kGeluTableFrom = 2u << 20, kGeluTableFromWide = 8u << 20, kGeluOneItem = 48u << 20, kGeluTableFromUneven = 32u << 20;
 int resident_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -937,8 +939,13 @@ int launch_quant_rows(const uint16_t* d_x, int rows, int K, void* d_out, float* 
     const bool vec = aligned16(d_x) && aligned16(d_out) && K % kVec == 0 && K > 0;
     const unsigned grid = ceil_div(rows, kThreads / 64);
     if constexpr (GELU && !E5M2) {
-        if (vec && K <= 4 * 1024 && static_cast<size_t>(rows) * K >= kGeluTableFrom) {
-            k_gelu_quant_rows_lut<<<2 * resident_cus(), kLutThreads, 0, st>>>(d_x, rows, K, o, d_scale, d_descale);
+        const size_t n = static_cast<size_t>(rows) * K;
+        if (vec && K <= 2 * 1024 && n >= kGeluTableFrom) {
+            k_gelu_quant_rows_lut<2><<<2 * resident_cus(), kLutThreads, 0, st>>>(d_x, rows, K, o, d_scale, d_descale);
+            return launch_status();
+        }
+        if (vec && K > 2 * 1024 && K <= 4 * 1024 && n >= kGeluTableFromWide) {
+            k_gelu_quant_rows_lut<4><<<2 * resident_cus(), kLutThreads, 0, st>>>(d_x, rows, K, o, d_scale, d_descale);
             return launch_status();
         }
     }
@@ -1044,15 +1051,22 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
                                           fp8_max, d_row_descale);
     };
     const int which = (is_e5m2 ? 4 : 0) | (apply_gelu ? 2 : 0) | (is_recompute ? 1 : 0);
-    // GELU: the table form (the direct form waits for erff)
-    if (apply_gelu && num_experts <= kLutMaxExperts && static_cast<size_t>(total_rows) * K >= 2 * kGeluTableFrom) {
-        const int cus = resident_cus();
-        // Parts per expert: an item per resident workgroup.  An item ends in an arrival of a few dependent atomics: with two items each
-        // 31.8 us at 24576 x 1408 and 64 experts instead of 28.6 (four: 45.2).
-        int parts = (2 * cus + num_experts - 1) / num_experts;
-        parts = parts < 1 ? 1 : (parts > 64 ? 64 : parts);
+    // GELU: the table form (the direct form waits for erff).  Parts per expert: an item ends in an arrival of a few dependent atomics on
+    // the expert's slot, so at most one item per CU (64 experts, 6144 x 1408: 10.4 us, with two 15.7; 24576 x 1408 22.9 and 29.2) until
+    // the streaming outweighs that and wants both workgroups of a CU (180000 x 1408 from memory: 212 and 206).  Rounded down: a few CUs
+    // with a second item hold up all others (100 experts, 4200 x 1408: 10.0 us, rounded up 14.2, direct 12.5).  Where that leaves more
+    // than a quarter of the CUs idle the direct form stays until two per CU pay (300 experts from memory, 12000 x 1408: 30.9 directly,
+    // 34.8 in table form; 24576 x 1408: 51.3, 49.7).
+    const size_t n = static_cast<size_t>(total_rows) * K;
+    const int cus = resident_cus();
+    int parts = cus / num_experts;
+    parts = parts > 64 ? 64 : parts;
+    const bool fills = parts * num_experts * 4 >= min(cus, 64 * num_experts) * 3;      // of the CUs that a part each can give work to
+    const bool two_per_cu = n >= (fills ? kGeluOneItem : kGeluTableFromUneven);
+    if (two_per_cu) parts = min((2 * cus + num_experts - 1) / num_experts, 64);
+    if (apply_gelu && num_experts <= kLutMaxExperts && (two_per_cu || (fills && n >= 2 * kGeluTableFrom))) {
         auto launch_lut = [&](auto kernel) {
-            kernel<<<2 * cus, kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
+            kernel<<<min(2 * cus, parts * num_experts), kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
                                                     state_stride_words, history_len, fp8_max, d_row_descale);
         };
         switch (which & 5) {
