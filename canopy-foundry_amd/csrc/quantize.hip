@@ -114,6 +114,11 @@ __device__ __forceinline__ uint4 quant16_track(const Vec16& v, float s, bool sca
 // atomic on the same address, and those serialise, so there should be few of them.
 constexpr int kAmaxThreads = 1024;
 constexpr unsigned kAmaxBlocks = 256;
+// fp32 tensors of this range: up to 256 workgroups of 1024 with four loads in flight per lane.  With one of 256 lanes per 1024 elements, up
+// to 4096, their atomics on one address are what it waits for: with the two small launches around it 512 Ki elements 8.6 us, 7.3 with
+// few; 1 Mi 15.3 and 7.2; 8 Mi 25.1 and 7.9; from memory 1 Mi 17.8 and 12.1, 32 Mi 57.8 and 52.0.  Below there are few workgroups
+// either way (64 Ki from memory 9.6 and 10.2); above, more loads in flight win (64 Mi from memory 87 and 92).
+constexpr size_t kAmaxFewFrom = 256u << 10, kAmaxFewTo = 32u << 20;
 template <bool VEC>
 __global__ __launch_bounds__(kAmaxThreads) void k_amax_bf16(const uint16_t* __restrict__ x, size_t n,
                                                             float* __restrict__ amax) {
@@ -139,18 +144,22 @@ __global__ __launch_bounds__(kAmaxThreads) void k_amax_bf16(const uint16_t* __re
     if (threadIdx.x == 0) atomic_max_nonneg(amax, m);
 }
 
-__global__ __launch_bounds__(kThreads) void k_amax_f32(const float* __restrict__ x, size_t n,
-                                                       float* __restrict__ amax, int vec) {
-    __shared__ float sh[kThreads / 64];
+template <int THREADS, int LOADS>
+__global__ __launch_bounds__(THREADS) void k_amax_f32(const float* __restrict__ x, size_t n, float* __restrict__ amax, int vec) {
+    __shared__ float sh[THREADS / 64];
     float local = 0.0f;
-    const size_t tid = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+    const size_t tid = static_cast<size_t>(blockIdx.x) * THREADS + threadIdx.x;
+    const size_t stride = static_cast<size_t>(gridDim.x) * THREADS;
     size_t done = 0;
     if (vec) {
         const size_t nvec = n / 4;
-        for (size_t i = tid; i < nvec; i += stride) {
-            const float4 v = reinterpret_cast<const float4*>(x)[i];
-            local = fmaxf(fmaxf(local, fabsf(v.x)), fmaxf(fmaxf(fabsf(v.y), fabsf(v.z)), fabsf(v.w)));
+        for (size_t i = tid; i < nvec; i += LOADS * stride) {
+            float4 v[LOADS];
+#pragma unroll
+            for (int b = 0; b < LOADS; ++b) v[b] = reinterpret_cast<const float4*>(x)[min(i + b * stride, nvec - 1)];
+#pragma unroll
+            for (int b = 0; b < LOADS; ++b)
+                local = fmaxf(fmaxf(local, fabsf(v[b].x)), fmaxf(fmaxf(fabsf(v[b].y), fabsf(v[b].z)), fabsf(v[b].w)));
         }
         done = nvec * 4;
     }
@@ -987,7 +996,10 @@ int cf_fp8_amax_f32(const float* d_x, size_t n, float* d_amax, cf_stream_t strea
     k_zero_f32<<<1, 1, 0, as_stream(stream)>>>(d_amax);
     if (n == 0) return launch_status();
     const int vec = aligned16(d_x);
-    k_amax_f32<<<blocks_for(vec ? (n + 3) / 4 : n), kThreads, 0, as_stream(stream)>>>(d_x, n, d_amax, vec);
+    if (vec && n >= kAmaxFewFrom && n <= kAmaxFewTo)
+        k_amax_f32<kAmaxThreads, 4><<<min(ceil_div(n, 8 * kAmaxThreads), kAmaxBlocks), kAmaxThreads, 0, as_stream(stream)>>>(d_x, n, d_amax, vec);
+    else
+        k_amax_f32<kThreads, 1><<<blocks_for(vec ? (n + 3) / 4 : n), kThreads, 0, as_stream(stream)>>>(d_x, n, d_amax, vec);
     return launch_status();
 }
 
