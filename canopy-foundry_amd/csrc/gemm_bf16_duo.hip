@@ -146,17 +146,19 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
     Tile F = decode(xi_fetch);
     if (!F.valid) return;
     int fk = 0;
+    // (A k row beyond the operand's last starts at its end: 32 bits hold that offset for every stride, which row * stride they
+    // would not, fewer than 32 rows of more than 128 Mi elements being within the launcher's limits.)
     auto aim = [&]() {
         const int w0 = WIDE_M ? F.m0 : F.n0, s0 = WIDE_M ? F.n0 : F.m0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int row = 8 * wave + 2 * j + (lane >> 5), chunk = (lane & 31) ^ (unit_swz(row) << 1);
-            voff_w[j] = w0 + chunk * 8 < ext_w ? static_cast<uint32_t>(row) * ldw + chunk * 16u : kOutside;
+            voff_w[j] = w0 + chunk * 8 < ext_w ? static_cast<uint32_t>(min(row, p.K)) * ldw + chunk * 16u : kOutside;
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int row = 8 * wave + 4 * j + (lane >> 4), chunk = (lane & 15) ^ (unit_swz(row) << 1);
-            voff_s[j] = s0 + chunk * 8 < ext_s ? static_cast<uint32_t>(row) * lds_ + chunk * 16u : kOutside;
+            voff_s[j] = s0 + chunk * 8 < ext_s ? static_cast<uint32_t>(min(row, p.K)) * lds_ + chunk * 16u : kOutside;
         }
         base_w = reinterpret_cast<uint64_t>(Wp) + static_cast<uint64_t>(F.k_begin) * ldw + 2ull * w0;
         base_s = reinterpret_cast<uint64_t>(Sp) + static_cast<uint64_t>(F.k_begin) * lds_ + 2ull * s0;

@@ -60,3 +60,28 @@ def test_grouped_wgrad_edges(cf, dev, M, N, counts, f32):
         want = (C0[e].double() + A[o:o + n].double().T @ B[o:o + n].double()).to(C0.dtype) if n else C0[e]
         assert torch.equal(got[e], want), f"expert {e}"
         assert n or torch.equal(torch.signbit(got[e]), torch.signbit(want))
+
+
+# rows so far apart that 32 bits do not hold the offset of a k row beyond the last: row 16 of one with 2^27 elements a row, row 8 of
+# 2^28, row 9 of nearly that (which would land in row 1).  A wrapped row would be added a second time.
+@pytest.mark.parametrize("K,ld", [(1, 1 << 27), (2, 1 << 28), (3, (1 << 28) - 8)])
+@pytest.mark.parametrize("M,N", [(136, 264), (264, 120)])
+def test_wgrad_row_stride(cf, dev, K, ld, M, N):
+    case(f"bf16 wgrad {M}x{N}x{K}, {ld} elements a row")
+    g = torch.Generator().manual_seed(M + K)
+    A, B = ints(g, K, M), ints(g, K, N)
+
+    def far(x):
+        buf = torch.zeros((K - 1) * ld + x.shape[1], dtype=torch.bfloat16, device=dev)
+        for k in range(K): buf[k * ld:k * ld + x.shape[1]] = x[k].to(dev)
+        return buf
+    a, b = far(A), far(B)
+    want = (A.double().T @ B.double()).float()
+    C = torch.zeros(M, N, device=dev)
+    cf.cf_gemm_bf16_tn_accum_f32(M, N, K, a, ld, b, ld, C, N, stream())
+    assert torch.equal(C.cpu(), want)
+    if K > 1:                           # an expert per row
+        C = torch.zeros(K, M, N, device=dev)
+        counts, offsets = torch.ones(K, dtype=torch.int32, device=dev), torch.arange(K, dtype=torch.int32, device=dev)
+        cf.cf_moe_grouped_gemm_bf16_tn_accum_f32(M, N, K, K, counts, offsets, a, ld, b, ld, C, stream())
+        assert torch.equal(C.cpu(), (A.double()[:, :, None] * B.double()[:, None, :]).float())
