@@ -121,7 +121,7 @@ void k_gemm_bf16(const BfArgs p) {
     const int x = blockIdx.x % 8, xi_step = gridDim.x / 8;
     constexpr int TK = 64;
     constexpr int NA = 8, NB = TK / 8;       // 16-byte chunks per lane and K-tile
-    constexpr uint32_t kOutside = 0x80000000u;
+    constexpr uint32_t kOutside = 0x80000000u, kFar = 0x7ffffff0u;      // kOutside + kFar does not wrap; no operand is larger than kFar
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     int row_tiles = p.tiles_m;
     if constexpr (GROUPED) row_tiles = __builtin_amdgcn_readfirstlane(p.tile_map[0]);
@@ -191,7 +191,8 @@ void k_gemm_bf16(const BfArgs p) {
     // (nothing, past the end of the k range).  A lane's offset is its row within the first eight-row (32-row) group and
     // its 16-byte column, plus the group's distance from the tile's first row; a lane whose columns lie outside the
     // operand (or, for the K-contiguous form, whose k chunk lies beyond K) starts from an offset beyond every size.
-    // The launcher keeps operands below 2 GiB, so the sum does not wrap.  (A descriptor per load costs about ten
+    // The launcher keeps operands below 2 GiB, so the sum does not wrap for rows that are there; a row beyond them that
+    // does belongs to outputs that are not stored, except for a group of k rows beyond K, which is sent to kFar (see load_one).  (A descriptor per load costs about ten
     // scalar instructions in front of one MFMA in every eight, more than the MFMA's 16 cycles cover.)
     // rows [row0, row_end) of a row-major operand with `ld` elements per row, seen from element `col0` of row row0
     auto rows_rsrc = [](const uint16_t* base, int ld, int row0, int row_end, int col0) {
@@ -315,7 +316,9 @@ void k_gemm_bf16(const BfArgs p) {
                 ra[c] = load_at(rs_a, off_a + c * a_step);
             }
         } else {
-            rb[c - NA] = load_at(rs_b, off_b + (c - NA) * b_step);
+            // [k][columns] rows of more than 32 Mi elements, fewer than 64 of them: c groups of eight rows down may be 2^32 bytes.  (K is a
+            // multiple of 8.)
+            rb[c - NA] = load_at(rs_b, off_b + (B_KC || 8 * (c - NA) < p.K ? (c - NA) * b_step : kFar));
         }
     };
     // the same chunk from its staging register into LDS stage `stage`

@@ -56,6 +56,21 @@ def test_gemm_bf16_nn(cf, dev, M, N, K, pad):
     check_bf16_out(got[:, :N], orc.gemm_bf16_nn_ref(A, B), absdot(A, B), f"nn {M}x{N}x{K}")
 
 
+def test_gemm_bf16_nn_row_stride(cf, dev):
+    """Eight k rows 2^26 elements apart: 32 bits do not hold the offset of row 32 (of a K step's 64), and one that wraps to row 0
+    would be multiplied by zeros: NaN where B is infinite."""
+    case("gemm_bf16_nn, 2^26 elements a row of B")
+    M, N, K, ldb = 40, 264, 8, 1 << 26
+    rng = np.random.default_rng(9)
+    a, b = rng.integers(1, 5, (M, K)).astype(np.float32), rng.integers(-4, 5, (K, N)).astype(np.float32)
+    b[0, 5], b[0, 200] = np.inf, -np.inf
+    B = torch.zeros((K - 1) * ldb + N, dtype=torch.bfloat16, device=dev)
+    for k in range(K): B[k * ldb:k * ldb + N] = torch.from_numpy(b[k])
+    C = torch.zeros((M, N), dtype=torch.bfloat16, device=dev)
+    cf.cf_gemm_bf16_nn(M, N, K, torch.from_numpy(a).to(torch.bfloat16).to(dev), K, B, ldb, C, N, stream())
+    assert np.array_equal(C.float().cpu().numpy(), a @ b)      # whole numbers below 257
+
+
 def test_gemm_bf16_exact_integers_equal_numpy(cf, dev):
     """Small integers: every product and partial sum is exact in fp32, so all three forms must match numpy to the
     bit; the operands are far from symmetric, so a transposed or misindexed operand cannot pass."""
