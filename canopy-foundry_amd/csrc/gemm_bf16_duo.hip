@@ -429,11 +429,15 @@ int launch(TnArgs p, hipStream_t st) {
 }
 template <bool WIDE_M, bool F32, bool GROUPED>
 int launch(const TnArgs& p, hipStream_t st) {
-    // A small C may still lie in the 256 MiB memory-side cache from the call that added to it before, and is left there for the next:
-    // 64 MiB fp32 (8 experts of 2048 x 1024, 1024 rows each) over and over 49 us, streamed 59; with C from memory 73 and 68.
-    // 196 MiB and more (12288 columns of 4096) do not fit beside the operands: 50304 x 4096 over 2048 rows 817 us streamed, 852 not.
+    // A C that the 256 MiB memory-side cache still holds from the call that added to it before is best left there, one that comes from
+    // memory is best streamed: 64 MiB fp32 (4096^2 over 256 rows) over and over 28 us, streamed 36, from memory 44 and 42; 96 MiB 39
+    // and 45, 59 and 50; 144 MiB 60 and 69, 85 and 73; 192 MiB 73 and 102, 110 and 105; 256 MiB 124 and 125, 133 and 132.  The larger, the less
+    // of it is likely to be left, so the line lies inside that range.
+    // Streamed rows have to begin at lines: a line shared by two rows' accesses would be read and written twice (32000 x 2968 bf16 over
+    // 848 rows 225 us streamed, 171 not; 30000 x 2056 fp32 over 256 213 and 107; rows at half lines 14336 x 4080 fp32 313 and 317).
     const long long bytes = static_cast<long long>(p.M) * p.ldc * (F32 ? 4 : 2) * (GROUPED ? p.num_experts : 1);
-    return bytes > kStreamBytes ? launch<WIDE_M, F32, GROUPED, true>(p, st) : launch<WIDE_M, F32, GROUPED, false>(p, st);
+    const bool lines = (static_cast<long long>(p.ldc) * (F32 ? 4 : 2)) % 128 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 127u) == 0;
+    return bytes > kStreamBytes && lines ? launch<WIDE_M, F32, GROUPED, true>(p, st) : launch<WIDE_M, F32, GROUPED, false>(p, st);
 }
 template <bool F32, bool GROUPED>
 int launch(const TnArgs& p, hipStream_t st) {

@@ -20,7 +20,7 @@ def padded(x, ld):
 
 
 # tiles of 256 x 128 and of 128 x 256 (whichever are fewer), one column short of and beyond them; K around the steps of 32, the
-# pairs of steps and the shortest pipeline of four; the last size is beyond the limit from which C is streamed
+# pairs of steps and the shortest pipeline of four; the last size is as large as what is streamed, but its rows begin off the lines
 @pytest.mark.parametrize("M,N,K", [(256, 128, 1), (128, 256, 31), (264, 120, 33), (120, 264, 64), (248, 136, 65), (8, 8, 127), (512, 384, 129),
                                    (384, 512, 200), (2048, 2056, 96), (5128, 5192, 40)])
 @pytest.mark.parametrize("f32", [True, False])
@@ -37,6 +37,26 @@ def test_wgrad_edges(cf, dev, M, N, K, f32):
     got = C.cpu()
     assert torch.equal(got[:, :N], want)
     assert torch.isnan(got[:, N:]).all()           # the row padding of C is left alone
+
+
+# C larger than what is left to the caches: streamed where its rows begin at 128-byte lines, not where C itself begins off one
+@pytest.mark.parametrize("M,N,ldc,f32", [(5000, 5168, 5184, True), (10008, 5168, 5184, False)])
+@pytest.mark.parametrize("off", [0, 4])
+def test_wgrad_large_c(cf, dev, M, N, ldc, f32, off):
+    case(f"bf16 wgrad {M}x{N}, C of more than 96 MiB, f32 {f32} off {off}")
+    dt = torch.float32 if f32 else torch.bfloat16
+    assert ldc * dt.itemsize % 128 == 0 and M * ldc * dt.itemsize > 96 << 20
+    g = torch.Generator().manual_seed(M + off)
+    A, B = ints(g, 40, M).to(dev), ints(g, 40, N).to(dev)
+    buf = torch.full((M * ldc + 64,), float("nan"), dtype=dt, device=dev)
+    C = buf[off:off + M * ldc].view(M, ldc)
+    C0 = torch.randint(-4, 5, (M, N), device=dev, generator=torch.Generator(device=dev).manual_seed(M)).to(dt)
+    C[:, :N] = C0
+    call = cf.cf_gemm_bf16_tn_accum_f32 if f32 else cf.cf_gemm_bf16_tn_accum_bf16
+    call(M, N, 40, A, M, B, N, C, ldc, stream())
+    want = (C0.double() + A.double().T.contiguous() @ B.double()).to(dt)
+    assert torch.equal(C[:, :N], want)
+    assert torch.isnan(C[:, N:]).all() and torch.isnan(buf[:off]).all() and torch.isnan(buf[off + M * ldc:]).all()
 
 
 # rows per expert from none to several tiles' worth of steps; enough tiles for every workgroup to walk several
