@@ -105,14 +105,24 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
         size_t c_base;
         bool valid;
     };
+    // tile `i` of an order that walks the tiles in patches of `rows` row tiles, column after column
+    auto place = [&](Tile& t, int i, int rows) {
+        const int group = i / (rows * p.tiles_n), first = group * rows;
+        const int gm = min(rows, p.tiles_m - first), in_group = i - group * rows * p.tiles_n;
+        t.m0 = __builtin_amdgcn_readfirstlane((first + in_group % gm) * TM);
+        t.n0 = __builtin_amdgcn_readfirstlane((in_group / gm) * TN);
+    };
     auto decode = [&](int xi) {
         Tile t{};
         if constexpr (GROUPED) {
             const int round = xi / tiles_mn, e = x + 8 * round, ti = xi - round * tiles_mn;
             t.valid = e < p.num_experts;
             if (t.valid) {
-                t.m0 = __builtin_amdgcn_readfirstlane((ti % p.tiles_m) * TM);
-                t.n0 = __builtin_amdgcn_readfirstlane((ti / p.tiles_m) * TN);
+                // An expert's tiles in patches too, of 1024 columns of A where it has 2048 or more: 64 tiles are worked on at a time, and of an
+                // expert with many rows of tiles (14336 x 1024: 56) that would be all of A.  16 experts of 14336 x 1024 over 4473 rows
+                // each 3298 us without, 1812 so (2048 columns: 2051); of 8192 x 1024 over 3305 1214 and 806; 8 of 8192 x 8192 over 2310
+                // 3591 and 2522; of 2048 x 8192 over 11371 2966 and 2571.  1920 x 8064 over 3750 827 without, 850 in such patches.
+                place(t, ti, p.M < 2048 ? p.tiles_m : 1024 / TM);
                 // an expert's row range is cut at the rows the compact buffers hold
                 t.k_begin = min(max(__builtin_amdgcn_readfirstlane(p.offsets[e]), 0), p.K);
                 t.k_end = min(t.k_begin + min(max(__builtin_amdgcn_readfirstlane(p.counts[e]), 0), p.K), p.K);
@@ -122,11 +132,7 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
             const int lin = x * per + xi;
             t.valid = xi < per && lin < tiles_mn;
             if (t.valid) {
-                constexpr int GM = 8;
-                const int group = lin / (GM * p.tiles_n), first = group * GM;
-                const int gm = min(GM, p.tiles_m - first), in_group = lin - group * GM * p.tiles_n;
-                t.m0 = __builtin_amdgcn_readfirstlane((first + in_group % gm) * TM);
-                t.n0 = __builtin_amdgcn_readfirstlane((in_group / gm) * TN);
+                place(t, lin, 8);
                 t.k_end = p.K;
             }
         }

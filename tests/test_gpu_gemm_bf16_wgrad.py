@@ -59,9 +59,12 @@ def test_wgrad_large_c(cf, dev, M, N, ldc, f32, off):
     assert torch.isnan(C[:, N:]).all() and torch.isnan(buf[:off]).all() and torch.isnan(buf[off + M * ldc:]).all()
 
 
-# rows per expert from none to several tiles' worth of steps; enough tiles for every workgroup to walk several
+# rows per expert from none to several tiles' worth of steps; experts whose rows of tiles (6 and 11) end in a partial patch of four.
+# The last two have at least 176 tiles for an XCD's 64 workgroups, so that each walks several: of 256 x 128 and of 128 x 256 (fp32: streamed).
+SEVERAL = [40, 3, 64, 0, 65, 33, 1, 96, 31, 32, 70, 2, 129, 0, 17, 50]
 @pytest.mark.parametrize("M,N,counts", [(264, 136, [0, 1, 63, 64, 65, 0, 129, 300, 5]), (136, 264, [40, 0, 0, 7]),
-                                        (1408, 1024, [70, 0, 33, 1, 0, 64, 97, 128, 3, 200, 0, 32])])
+                                        (1408, 1024, [70, 0, 33, 1, 0, 64, 97, 128, 3, 200, 0, 32]),
+                                        (1416, 2056, SEVERAL), (1288, 2048, SEVERAL)])
 @pytest.mark.parametrize("f32", [True, False])
 def test_grouped_wgrad_edges(cf, dev, M, N, counts, f32):
     case(f"grouped bf16 wgrad {M}x{N} {counts} f32 {f32}")
