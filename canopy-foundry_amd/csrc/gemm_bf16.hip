@@ -1,5 +1,6 @@
 // bf16 GEMMs of the selected-expert MoE backward and of the bf16 expert bank, dense and grouped per expert: the input
-// gradients and the forward form.  (The weight gradients are gemm_bf16_duo.hip.)
+// gradients and the forward form; and the dense weight gradients whose operands are large.  (The others are gemm_bf16_duo.hip,
+// which also says where the line is.)
 //
 // The reference runs four cuBLAS calls per expert behind a host copy of the counts (src/trainer.cu:7727-7740,
 // wrappers :3069-3160), two of them input gradients  C[n,N] = A[n,K] . B[K,N]  (gemm_bf16, row-major, beta = 0).  Here one
@@ -40,22 +41,21 @@ namespace {
 constexpr int TM = 256, TN = 256, kThr = 256;
 constexpr int kMaxTK = 64;
 constexpr int kPitchKC = kMaxTK * 2;           // a K-contiguous tile: 128-byte rows, chunks swizzled
-constexpr int kPitchN = TN * 2 + 64;           // a [k][n] tile of the N side: 576-byte rows
+constexpr int kPitchKS = TN * 2 + 64;          // a [k][columns] tile: 576-byte rows
 // the pads put four consecutive k rows into four different quarters of the 256 bytes the banks span
-constexpr int kATile = TM * kPitchKC;              // 32,768 bytes
-constexpr int kBTile = kMaxTK * kPitchN;           // 36,864 bytes: covers both forms of the N-side tile (K-contiguous: 32,768)
-constexpr int kStage = kATile + kBTile;
-constexpr int kLds = 2 * kStage;               // 139,264 bytes: one workgroup per CU
+constexpr int kTileKC = TM * kPitchKC, kTileKS = kMaxTK * kPitchKS;        // 32,768 and 36,864 bytes
+// two stages of an M-side tile and the larger of the N side's forms: 139,264 or 147,456 bytes, one workgroup per CU
+constexpr int lds_bytes(bool a_ks) { return 2 * ((a_ks ? kTileKS : kTileKC) + kTileKS); }
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4bf* lds_v4bf_ptr;
 
-enum { OUT_STORE_BF16 = 0, OUT_STORE_F32 = 1 };
+enum { OUT_STORE_BF16 = 0, OUT_STORE_F32 = 1, OUT_ADD_BF16 = 2, OUT_ADD_F32 = 3 };
 
 struct BfArgs {
-    const uint16_t* A; int lda;     // M side: [M rows][K]
+    const uint16_t* A; int lda;     // M side: [M rows][K]; A_KS: [K rows][M]
     const uint16_t* B; int ldb;     // N side: [K rows][N]; NT (B_KC): [N rows][K]
     void* C; int ldc;               // [M][N], bf16 or fp32
     int M, N, K;
@@ -102,7 +102,8 @@ __device__ __forceinline__ int ks_lane_offset(int pitch, int lane) {
 // B_KC: the N-side operand is stored [N][K] (a weight matrix as the forward pass holds it); otherwise [K][N].
 // GATHER: the tile's rows of A are fetched through a row index, so a token permute
 // needs no pass of its own.
-template <int OUT, bool GROUPED, bool B_KC = false, bool GATHER = false>
+// A_KS: the M-side operand is stored [K][M] (the weight gradients, which add to C).
+template <int OUT, bool GROUPED, bool B_KC = false, bool GATHER = false, bool A_KS = false>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void k_gemm_bf16(const BfArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -120,6 +121,8 @@ void k_gemm_bf16(const BfArgs p) {
     // 8 row tiles x 4 column tiles, its workgroups taking every (grid / 8)-th tile of it.
     const int x = blockIdx.x % 8, xi_step = gridDim.x / 8;
     constexpr int TK = 64;
+    constexpr int kATile = A_KS ? kTileKS : kTileKC, kStage = lds_bytes(A_KS) / 2;
+    static_assert(!A_KS || !(GROUPED || B_KC || GATHER), "the weight gradients here are dense");
     constexpr int NA = 8, NB = TK / 8;       // 16-byte chunks per lane and K-tile
     constexpr uint32_t kOutside = 0x80000000u, kFar = 0x7ffffff0u;      // kOutside + kFar does not wrap; no operand is larger than kFar
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
@@ -207,6 +210,7 @@ void k_gemm_bf16(const BfArgs p) {
     };
     // [k][columns] operands: this lane's row within a group of eight k rows and its 16-byte column
     const uint32_t b_lane_ks = (tid >> 5) * static_cast<uint32_t>(p.ldb) * 2u + (tid & 31) * 16u;
+    [[maybe_unused]] const uint32_t a_lane_ks = (tid >> 5) * static_cast<uint32_t>(p.lda) * 2u + (tid & 31) * 16u;
     // [m][k] operand: this lane's row within a group of 32 rows and its 16-byte k chunk
     const uint32_t a_lane_kc = (tid >> 3) * static_cast<uint32_t>(p.lda) * 2u + (tid & 7) * 16u;
     const uint32_t b_lane_kc = (tid >> 3) * static_cast<uint32_t>(p.ldb) * 2u + (tid & 7) * 16u;
@@ -287,15 +291,20 @@ void k_gemm_bf16(const BfArgs p) {
     // differ in the lane offset only (one vector add each).
     __amdgpu_buffer_rsrc_t rs_a = a_all, rs_b = a_all;
     uint32_t off_a = kOutside, off_b = kOutside;
-    const uint32_t a_step = 32u * static_cast<uint32_t>(p.lda) * 2u;
+    const uint32_t a_step = (A_KS ? 8u : 32u) * static_cast<uint32_t>(p.lda) * 2u;
     const uint32_t b_step = (B_KC ? 32u : 8u) * static_cast<uint32_t>(p.ldb) * 2u;
     // chunk c (0 .. NA-1: M side, NA .. NA+NB-1: N side) of the cursor's K-tile into its staging register
     auto load_one = [&](auto cc, uint4 (&ra)[NA], uint4 (&rb)[NB]) {
         constexpr int c = decltype(cc)::value;
         const int k0 = lks * TK;
         if constexpr (c == 0 && !GATHER) {
-            rs_a = rows_rsrc(p.A, p.lda, L.m0, L.m_end, k0);
-            off_a = k0 + (tid & 7) * 8 < L.k_end ? a_lane_kc : kOutside;
+            if constexpr (A_KS) {
+                rs_a = rows_rsrc(p.A, p.lda, k0, L.k_end, L.m0);
+                off_a = L.m0 + (tid & 31) * 8 < p.M ? a_lane_ks : kOutside;
+            } else {
+                rs_a = rows_rsrc(p.A, p.lda, L.m0, L.m_end, k0);
+                off_a = k0 + (tid & 7) * 8 < L.k_end ? a_lane_kc : kOutside;
+            }
         }
         if constexpr (c == NA) {
             const uint16_t* B = p.B + L.b_off;
@@ -326,13 +335,17 @@ void k_gemm_bf16(const BfArgs p) {
         constexpr int c = decltype(cc)::value;
         uint8_t* as = smem + stage * kStage;
         if constexpr (c < NA) {
-            const int r = (tid >> 3) + 32 * c;
-            *reinterpret_cast<uint4*>(as + r * kPitchKC + (((tid & 7) ^ swz(r)) << 4)) = ra[c];
+            if constexpr (A_KS) {
+                *reinterpret_cast<uint4*>(as + ((tid >> 5) + 8 * c) * kPitchKS + (c & 1) * 32 + (tid & 31) * 16) = ra[c];
+            } else {
+                const int r = (tid >> 3) + 32 * c;
+                *reinterpret_cast<uint4*>(as + r * kPitchKC + (((tid & 7) ^ swz(r)) << 4)) = ra[c];
+            }
         } else if constexpr (B_KC) {
             const int r = (tid >> 3) + 32 * (c - NA);
             *reinterpret_cast<uint4*>(as + kATile + r * kPitchKC + (((tid & 7) ^ swz(r)) << 4)) = rb[c - NA];
         } else {
-            *reinterpret_cast<uint4*>(as + kATile + ((tid >> 5) + 8 * (c - NA)) * kPitchN + ((c - NA) & 1) * 32 + (tid & 31) * 16) = rb[c - NA];
+            *reinterpret_cast<uint4*>(as + kATile + ((tid >> 5) + 8 * (c - NA)) * kPitchKS + ((c - NA) & 1) * 32 + (tid & 31) * 16) = rb[c - NA];
         }
     };
 
@@ -349,7 +362,8 @@ void k_gemm_bf16(const BfArgs p) {
     clear_acc();
 
     const int r16 = lane & 15, kg = lane >> 4;
-    const int ks_n = ks_lane_offset(kPitchN, lane) + wn * 128 * 2;
+    const int ks_n = ks_lane_offset(kPitchKS, lane) + wn * 128 * 2;
+    [[maybe_unused]] const int ks_m = ks_lane_offset(kPitchKS, lane) + wm * 128 * 2;
     // K-contiguous tiles: this lane's row within a block and its chunk for either k-step (the swizzle depends on the
     // row modulo 16 only, so the block is an immediate offset)
     int kc[2];
@@ -363,15 +377,15 @@ void k_gemm_bf16(const BfArgs p) {
         constexpr int S = decltype(sc)::value, SET = decltype(setc)::value, R = decltype(rc_)::value;
         const uint8_t* as = smem + stage * kStage;
         constexpr bool NSIDE = SET < 2;
-        constexpr bool KC = NSIDE ? B_KC : true;
+        constexpr bool KC = NSIDE ? B_KC : !A_KS;
         constexpr int half = SET & 1, blk = half * 4 + R;
         v8bf v;
         if constexpr (KC) {
             const uint8_t* base = as + (NSIDE ? kATile + wn * 128 * kPitchKC : wm * 128 * kPitchKC);
             v = *reinterpret_cast<const v8bf*>(base + blk * 16 * kPitchKC + kc[S]);
         } else {
-            constexpr int PITCH = kPitchN;
-            const uint8_t* pl = as + kATile + ks_n + 32 * S * PITCH + 16 * blk * 2;
+            constexpr int PITCH = kPitchKS;
+            const uint8_t* pl = as + (NSIDE ? kATile + ks_n : ks_m) + 32 * S * PITCH + 16 * blk * 2;
             const v4bf lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf_ptr)(pl));
             const v4bf hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_v4bf_ptr)(pl + 4 * PITCH));
             v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -380,7 +394,8 @@ void k_gemm_bf16(const BfArgs p) {
     };
     constexpr int RN = 4, RM = 4;       // read_set calls per set
 
-    constexpr int CE = OUT == OUT_STORE_F32 ? 4 : 2;        // bytes per element of C
+    constexpr bool ADD = OUT == OUT_ADD_BF16 || OUT == OUT_ADD_F32;
+    constexpr int CE = OUT == OUT_STORE_F32 || OUT == OUT_ADD_F32 ? 4 : 2;        // bytes per element of C
     // the wavefront's block of the output tile `t`, rows beyond the tile's end cut off
     auto c_block_rsrc = [&](const Tile& t) {
         const int row_w = t.m0 + wm * 128;
@@ -388,6 +403,20 @@ void k_gemm_bf16(const BfArgs p) {
         return __builtin_amdgcn_make_buffer_rsrc(
             static_cast<uint8_t*>(p.C) + (static_cast<size_t>(row_w) * p.ldc + t.n0 + wn * 128) * CE, 0,
             static_cast<int>(static_cast<uint32_t>(rows) * static_cast<uint32_t>(p.ldc) * CE), 0x00020000);
+    };
+    // The forms that add to C read it in the epilogue, with idle matrix cores: a round trip to HBM per pass.  Under the
+    // tile's last pair of K-tiles every 128-byte line of the wavefront's block of C is therefore touched once (one dword per
+    // lane, distinct lines), so that the epilogue's reads find it in the L2 / the memory-side cache.  The touches
+    // are issued in every pair, from offsets beyond the descriptor in all but the last.
+    constexpr int NTOUCH = ADD ? 2 * CE : 1;                // 128 rows x CE lines / 64 lanes
+    [[maybe_unused]] int touched[NTOUCH] = {};
+    __amdgpu_buffer_rsrc_t rs_c = a_all;
+    [[maybe_unused]] bool touch_ok = false;
+    [[maybe_unused]] const uint32_t touch_lane = (lane / CE) * static_cast<uint32_t>(p.ldc) * CE + (lane % CE) * 128u;
+    [[maybe_unused]] const uint32_t touch_step = (64 / CE) * static_cast<uint32_t>(p.ldc) * CE;
+    [[maybe_unused]] auto touch_one = [&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        touched[t] = __builtin_amdgcn_raw_buffer_load_b32(rs_c, static_cast<int>(touch_ok ? touch_lane + t * touch_step : kOutside), 0, 0);
     };
 
     // One K-tile: two k-steps of four phases, 128 MFMAs per wavefront, with everything else woven between them (one
@@ -420,6 +449,7 @@ void k_gemm_bf16(const BfArgs p) {
                 if constexpr (q < 2 * RM && q % 2 == 0) read_set(S == 0 ? stage : stage ^ 1, std::integral_constant<int, 1 - S>{}, std::integral_constant<int, 2 + (1 - S)>{}, std::integral_constant<int, (q / 2) % RM>{});
             }
             if constexpr (m % 8 == 7) load_one(std::integral_constant<int, m / 8>{}, ra_new, rb_new);
+            if constexpr (ADD && stage == 0 && m % 8 == 1 && m / 8 < NTOUCH) touch_one(std::integral_constant<int, m / 8>{});
             // three LDS stores per sixteen MFMAs, after MFMAs that have neither an operand read nor a load behind them
             constexpr int park = 3 * (m / 16) + (q == 3 ? 0 : q == 10 ? 1 : 2);
             if constexpr ((q == 3 || q == 10 || q == 13) && park < 16) park_one(stage ^ 1, std::integral_constant<int, park % 16>{}, ra_next, rb_next);
@@ -442,24 +472,30 @@ void k_gemm_bf16(const BfArgs p) {
     static_for<0, RN>([&](auto r) { read_set(0, std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, r); });
     static_for<0, RM>([&](auto r) { read_set(0, std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{}, r); });
     while (true) {
+        if constexpr (ADD) rs_c = c_block_rsrc(cur);
         for (int ks = 0; ks < cur.nk2; ks += 2) {
+            if constexpr (ADD) touch_ok = ks + 2 >= cur.nk2 && cur.n0 + wn * 128 + (lane % CE) * (128 / CE) < p.N;
             ktile(std::integral_constant<int, 0>{}, ra0, rb0, ra1, rb1);
             ktile(std::integral_constant<int, 1>{}, ra1, rb1, ra0, rb0);
         }
         // the MFMAs above are opaque to the compiler's hazard handling: leave the wait states between the last of them
         // and the first read of an accumulator explicitly
         asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+        if constexpr (ADD) {
+#pragma unroll
+            for (int t = 0; t < NTOUCH; ++t) asm volatile("" : : "v"(touched[t]));     // the touches end here
+        }
         // ---- epilogue: accumulator register q of block (j, i) is output row m0 + wm*128 + 16 i + lane % 16,
         //      column n0 + wn*128 + 16 j + 4 (lane / 16) + q.  Written from there a store instruction would cover sixteen
         //      rows with 32 bytes each; instead the wavefront turns its 128 x 128 outputs round in LDS, 64 rows (bf16) or
-        //      32 rows (fp32) at a time, and stores whole 256-byte / 512-byte row pieces.  The staging area
+        //      32 rows (fp32) at a time, and stores (or adds to) whole 256-byte / 512-byte row pieces.  The staging area
         //      is the wavefront's quarter of LDS stage 1: every output tile ends on that stage, nobody reads it after
         //      the last K-tile's barrier, and nobody parks into it before the barrier below.
         // C is reached through a descriptor over the wavefront's block (rows beyond the tile's end lie beyond its size;
-        // a lane whose columns lie beyond N uses an offset beyond every size): stores are dropped there, so the epilogue
-        // has no branches.
+        // a lane whose columns lie beyond N uses an offset beyond every size): stores are dropped there and loads return zeros, so
+        // the epilogue has no branches and its loads can be issued ahead of the staging.
         uint8_t* stg = smem + kStage + wave * (kStage / 4);
-        const __amdgpu_buffer_rsrc_t rs_c = c_block_rsrc(cur);
+        if constexpr (!ADD) rs_c = c_block_rsrc(cur);
         const int col_w = cur.n0 + wn * 128;
         if constexpr (OUT == OUT_STORE_BF16) {
             // a lane's piece: eight columns (16 bytes of C) of row lane / 16 of every group of four rows
@@ -483,12 +519,56 @@ void k_gemm_bf16(const BfArgs p) {
                     __builtin_amdgcn_raw_buffer_store_b128(v, rs_c, static_cast<int>(c_lane + (16 * half + t) * c_rows4), 0, 0);
                 }
             }
+        } else if constexpr (OUT == OUT_ADD_BF16) {
+            const uint32_t c_lane = col_w + 8 * (lane & 15) < p.N ? (lane >> 4) * static_cast<uint32_t>(p.ldc) * 2u + (lane & 15) * 16u : kOutside;
+            const uint32_t c_rows4 = 4u * static_cast<uint32_t>(p.ldc) * 2u;
+            // fp32 sum of the old value and the product, one rounding (cublasGemmEx with a bf16 C, beta = 1)
+            constexpr int PF = 128 * 4 + 16;                    // staged row: 128 fp32 + pad (the sixteen rows of a quad column: 64 banks)
+            static_assert(32 * PF <= kStage / 4, "four passes of 32 rows");
+            // the next pass's rows of C are requested before this pass's are added to and stored
+            u32x4 c[8], c_ahead[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) c_ahead[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_c, static_cast<int>(c_lane + t * c_rows4), 0, 0);
+#pragma unroll
+            for (int pass = 0; pass < 4; ++pass) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) c[t] = c_ahead[t];
+                if (pass < 3) {
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) c_ahead[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_c, static_cast<int>(c_lane + (8 * (pass + 1) + t) * c_rows4), 0, 0);
+                }
+#pragma unroll
+                for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const v4f a = acc[j][2 * pass + ii];
+                        *reinterpret_cast<float4*>(stg + (16 * ii + r16) * PF + (16 * j + 4 * kg) * 4) =
+                            make_float4(acc_read(a[0]), acc_read(a[1]), acc_read(a[2]), acc_read(a[3]));
+                    }
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const uint8_t* src = stg + ((lane >> 4) + 4 * t) * PF + (lane & 15) * 32;
+                    const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 16);
+                    u32x4 v;
+                    v.x = pack_bf16x2_hw(lo.x + bf16_lo(c[t].x), lo.y + bf16_hi(c[t].x));
+                    v.y = pack_bf16x2_hw(lo.z + bf16_lo(c[t].y), lo.w + bf16_hi(c[t].y));
+                    v.z = pack_bf16x2_hw(hi.x + bf16_lo(c[t].z), hi.y + bf16_hi(c[t].z));
+                    v.w = pack_bf16x2_hw(hi.z + bf16_lo(c[t].w), hi.w + bf16_hi(c[t].w));
+                    __builtin_amdgcn_raw_buffer_store_b128(v, rs_c, static_cast<int>(c_lane + (8 * pass + t) * c_rows4), 0, 0);
+                }
+            }
         } else {
             // fp32 C.  A lane's piece: four columns (16 bytes) of row lane / 32 of every pair of rows
             constexpr int PF = 128 * 4 + 16;                    // staged row: 128 fp32 + pad (the sixteen rows of a quad column: 64 banks)
             static_assert(32 * PF <= kStage / 4, "four passes of 32 rows");
             const uint32_t c_lane = col_w + 4 * (lane & 31) < p.N ? (lane >> 5) * static_cast<uint32_t>(p.ldc) * 4u + (lane & 31) * 16u : kOutside;
             const uint32_t c_rows2 = 2u * static_cast<uint32_t>(p.ldc) * 4u;
+            // C is read in groups of eight row pairs, a group ahead of the adds and stores
+            [[maybe_unused]] u32x4 c[8], c_ahead[8];
+            if constexpr (ADD) {
+#pragma unroll
+                for (int t = 0; t < 8; ++t) c_ahead[t] = __builtin_amdgcn_raw_buffer_load_b128(rs_c, static_cast<int>(c_lane + t * c_rows2), 0, 0);
+            }
 #pragma unroll
             for (int pass = 0; pass < 4; ++pass) {
 #pragma unroll
@@ -501,8 +581,23 @@ void k_gemm_bf16(const BfArgs p) {
                     }
 #pragma unroll
                 for (int t = 0; t < 16; ++t) {
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(stg + ((lane >> 5) + 2 * t) * PF + (lane & 31) * 16);
-                    __builtin_amdgcn_raw_buffer_store_b128(v, rs_c, static_cast<int>(c_lane + (16 * pass + t) * c_rows2), 0, 0);
+                    if constexpr (ADD) {
+                        if (t % 8 == 0) {
+#pragma unroll
+                            for (int u = 0; u < 8; ++u) {
+                                c[u] = c_ahead[u];
+                                if (2 * pass + t / 8 < 7)
+                                    c_ahead[u] = __builtin_amdgcn_raw_buffer_load_b128(rs_c, static_cast<int>(c_lane + (16 * pass + t + 8 + u) * c_rows2), 0, 0);
+                            }
+                        }
+                    }
+                    const float4 v = *reinterpret_cast<const float4*>(stg + ((lane >> 5) + 2 * t) * PF + (lane & 31) * 16);
+                    u32x4 o = __builtin_bit_cast(u32x4, v);
+                    if constexpr (ADD) {
+                        const float4 was = __builtin_bit_cast(float4, c[t % 8]);
+                        o = __builtin_bit_cast(u32x4, make_float4(was.x + v.x, was.y + v.y, was.z + v.z, was.w + v.w));
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(o, rs_c, static_cast<int>(c_lane + (16 * pass + t) * c_rows2), 0, 0);
                 }
             }
         }
@@ -527,16 +622,16 @@ dim3 persistent_grid(long long tiles) {
     return dim3(static_cast<unsigned>(want < cus ? want : cus));
 }
 
-template <int OUT, bool GROUPED, bool B_KC = false, bool GATHER = false>
+template <int OUT, bool GROUPED, bool B_KC = false, bool GATHER = false, bool A_KS = false>
 int launch(const BfArgs& p, dim3 grid, hipStream_t st) {
     static std::once_flag once;
     static hipError_t attr = hipSuccess;      // kept: a failed set-up is reported by every call, not only the first
-    auto kern = k_gemm_bf16<OUT, GROUPED, B_KC, GATHER>;
+    auto kern = k_gemm_bf16<OUT, GROUPED, B_KC, GATHER, A_KS>;
     std::call_once(once, [&] {
-        attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+        attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(A_KS));
     });
     if (attr != hipSuccess) return static_cast<int>(attr);
-    kern<<<grid, kThr, kLds, st>>>(p);
+    kern<<<grid, kThr, lds_bytes(A_KS), st>>>(p);
     return launch_status();
 }
 
@@ -604,6 +699,16 @@ int grouped_gemm_bf16_nt(int total_rows, int N, int Kb, int terms, int num_exper
         return launch<OUT_STORE_F32, true, true, true>(p, grid, st);
     }
     return c_is_f32 ? launch<OUT_STORE_F32, true, true>(p, grid, st) : launch<OUT_STORE_BF16, true, true>(p, grid, st);
+}
+int gemm_bf16_tn_large(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb, void* C, int ldc, bool c_is_f32,
+                       hipStream_t st) {
+    BfArgs p{};
+    p.A = A; p.lda = lda; p.B = B; p.ldb = ldb; p.C = C; p.ldc = ldc;
+    p.M = M; p.N = N; p.K = K;
+    p.tiles_m = (M + TM - 1) / TM;
+    p.tiles_n = (N + TN - 1) / TN;
+    const dim3 grid = persistent_grid(static_cast<long long>(p.tiles_m) * p.tiles_n);
+    return c_is_f32 ? launch<OUT_ADD_F32, false, false, false, true>(p, grid, st) : launch<OUT_ADD_BF16, false, false, false, true>(p, grid, st);
 }
 }  // namespace cf
 

@@ -26,6 +26,7 @@
 #include "common.hpp"
 #include "internal.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -43,6 +44,7 @@ constexpr int kRingBytes = kStages * kStageBytes;
 constexpr int kStageOut = 2048;                            // per wavefront: what the epilogue turns round at a time
 constexpr int kLdsBytes = kRingBytes + 4 * kStageOut;      // 80 KiB: two workgroups per CU
 constexpr long long kStreamBytes = 96ll << 20;             // a larger C is streamed (see launch)
+constexpr long long kNearOperands = 300000000, kFarOperands = 600000000, kReadAgain = 1600000000;      // bytes (see large_operands)
 constexpr int kNonTemporal = 2;                            // cache policy of a buffer access
 constexpr int kWaitVm0 = 0x0f70, kWaitVm6 = 0x0f76;        // s_waitcnt vmcnt(n), the other counters left alone
 
@@ -409,6 +411,17 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
 }
 
+// two workgroups per CU, a multiple of 8 of them (launch position % 8 is the XCD)
+int resident_workgroups() {
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v < 8) return 512;
+        return 2 * (v - v % 8);
+    }();
+    return n;
+}
+long long tiles_of(int M, int N, int tm, int tn) { return static_cast<long long>((M + tm - 1) / tm) * ((N + tn - 1) / tn); }
+
 template <bool WIDE_M, bool F32, bool GROUPED, bool STREAM>
 int launch(TnArgs p, hipStream_t st) {
     static std::once_flag once;
@@ -418,12 +431,7 @@ int launch(TnArgs p, hipStream_t st) {
         attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     });
     if (attr != hipSuccess) return static_cast<int>(attr);
-    // two workgroups per CU, a multiple of 8 of them (launch position % 8 is the XCD), and no more than there are tiles
-    static const int most = [] {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v < 8) return 512;
-        return 2 * (v - v % 8);
-    }();
+    const int most = resident_workgroups();         // and no more than there are tiles
     constexpr int TM = WIDE_M ? kWide : kNarrow, TN = WIDE_M ? kNarrow : kWide;
     p.tiles_m = (p.M + TM - 1) / TM;
     p.tiles_n = (p.N + TN - 1) / TN;
@@ -447,10 +455,26 @@ int launch(const TnArgs& p, hipStream_t st) {
 }
 template <bool F32, bool GROUPED>
 int launch(const TnArgs& p, hipStream_t st) {
-    // the tile lies along C whichever way it covers it with fewer (64 x 2048 x 1408: 176 tiles fewer per expert's row of them)
-    const long long wide_m = static_cast<long long>((p.M + kWide - 1) / kWide) * ((p.N + kNarrow - 1) / kNarrow);
-    const long long wide_n = static_cast<long long>((p.M + kNarrow - 1) / kNarrow) * ((p.N + kWide - 1) / kWide);
-    return wide_m <= wide_n ? launch<true, F32, GROUPED>(p, st) : launch<false, F32, GROUPED>(p, st);
+    // the tile lies along C whichever way it covers it with fewer (2048 x 1408: 88 tiles against 96)
+    return tiles_of(p.M, p.N, kWide, kNarrow) <= tiles_of(p.M, p.N, kNarrow, kWide) ? launch<true, F32, GROUPED>(p, st) : launch<false, F32, GROUPED>(p, st);
+}
+
+// Which dense problems go to one workgroup of 256 x 256 per CU instead (gemm_bf16.hip, the same sums).  The 64 workgroups of an XCD drift apart in k,
+// beyond the 700 rows that its L2 holds of what they read; what they then read again comes from the 256 MiB memory-side cache, and from
+// memory where the operands are larger (8192 x 8192 over 32768 rows: 29 GB through the L2s instead of 8).  Their 32 larger tiles take a third less
+// per product and stay together.  Measured at 315 sizes, this kernel and that one: in several rounds of tiles the operands are read once a round
+// and the line is where that comes to 1.6 GB: 8192 x 8192 bf16 over 32768 4411 and 3589 us, over 16384 1966 and 1828, over 8192 814 and 914; 128256 x
+// 4096 fp32 over 2048 2830 and 2319, 50304 x 4096 over 2048 770 and 1000; 23168 x 49344 over 3234 9740 and 7600; 6072 x 18064 bf16 over 25114 7140 and
+// 4820.  Narrow ones (one side up to 2048) gain little until their operands are twice that large: 80192 x 1536 over 1917 403 and 501, 25600 x 2728
+// over 20295 3630 and 2622.  In a single round the partner's tile costs as much as the other half of a 256 x 256: 1136 x 9976 over 28204 810 and
+// 594, 11008 x 768 over 21389 392 and 442.  Where it decides wrongly: 2624 x 54016 over 4371 1020 and 1275, 50304 x 4096 over 8192 2600 and 3010,
+// and, kept here, 2760 x 5144 over 25895 868 and 585, 1848 x 13256 over 11575 662 and 518.
+bool large_operands(int M, int N, int K) {
+    if (K < 64) return false;
+    const long long most = resident_workgroups(), bytes = 2ll * K * (static_cast<long long>(M) + N);
+    const long long tiles = std::min(tiles_of(M, N, kWide, kNarrow), tiles_of(M, N, kNarrow, kWide)), rounds = (tiles + most - 1) / most;
+    if (rounds == 1) return bytes > kFarOperands && 2 * tiles > most && 2 * tiles_of(M, N, kWide, kWide) <= most;
+    return bytes * rounds > kReadAgain && (bytes > kFarOperands || (bytes > kNearOperands && std::min(M, N) > 2048));
 }
 
 // C[M,N] += A[K,M]^T . B[K,N]; grouped: per expert, K running over its rows of the compact buffers, C[E,M,N]
@@ -463,6 +487,7 @@ int gemm_tn(int M, int N, int K, int E, const int* counts, const int* offsets, c
     if (lda < M || ldb < N || ldc < N) return CF_ERR_INVALID_ARG;
     if (N % 8 != 0 || M % 8 != 0 || !bf16_operands_ok(A, lda, B, ldb, C, ldc, F32 ? 4 : 2)) return CF_ERR_UNSUPPORTED;
     if (static_cast<size_t>(K) * lda >= (1ull << 30) || static_cast<size_t>(K) * ldb >= (1ull << 30)) return CF_ERR_UNSUPPORTED;
+    if (!grouped && large_operands(M, N, K)) return gemm_bf16_tn_large(M, N, K, A, lda, B, ldb, C, ldc, F32, as_stream(stream));
     TnArgs p{};
     p.A = A; p.lda = lda; p.B = B; p.ldb = ldb; p.C = C; p.ldc = ldc;
     p.M = M; p.N = N; p.K = K;

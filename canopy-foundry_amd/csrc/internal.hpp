@@ -34,6 +34,10 @@ int grouped_gemm_nt_terms(int total_rows, int N, int Kb, int terms, int num_expe
 int grouped_gemm_bf16_nt(int total_rows, int N, int Kb, int terms, int num_experts, const uint16_t* A, int a_rows, int lda,
                          const int* d_a_row_index, const uint16_t* B, void* C, int ldc, bool c_is_f32, const int* d_tile_map,
                          cf_stream_t stream);
+// C[M,N] += A[K,M]^T . B[K,N] on one workgroup of 256 x 256 per CU (gemm_bf16.hip), for operands that gemm_bf16_duo.hip has checked and
+// K >= 64
+int gemm_bf16_tn_large(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb, void* C, int ldc, bool c_is_f32,
+                       hipStream_t st);
 // What both bf16 GEMM sources ask of their operands (their epilogues address a wavefront's 128 rows of C by 32-bit byte offsets from the block's first element)
 inline bool bf16_operands_ok(const void* A, int lda, const void* B, int ldb, const void* C, int ldc, int c_elem_bytes) {
     return aligned16(A) && aligned16(B) && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && ldc < (1 << 21) &&

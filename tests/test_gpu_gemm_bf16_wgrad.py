@@ -39,6 +39,27 @@ def test_wgrad_edges(cf, dev, M, N, K, f32):
     assert torch.isnan(got[:, N:]).all()           # the row padding of C is left alone
 
 
+# operands so large that one workgroup of 256 x 256 per CU takes them: beyond 1.6 GB in several rounds of tiles, one column short of and
+# beyond tiles, K one short of and beyond the pairs of 64; and in a single round of the smaller tiles
+@pytest.mark.parametrize("M,N,K,f32", [(8200, 4088, 22527, True), (4104, 8184, 22529, False), (1136, 9976, 28203, True), (9976, 1136, 28292, False)])
+def test_wgrad_large_operands(cf, dev, M, N, K, f32):
+    case(f"bf16 wgrad {M}x{N}x{K} f32 {f32}, large operands")
+    tiles = min(-(-M // 256) * -(-N // 128), -(-M // 128) * -(-N // 256))
+    assert 2 * (M + N) * K > (600e6 if 256 < tiles <= 512 else 1600e6 / -(-tiles // 512))
+    g = torch.Generator(device=dev).manual_seed(M)
+    A, B = (torch.randint(-4, 5, (K, n + 8), generator=g, device=dev).to(torch.bfloat16) for n in (M, N))
+    A[:, M:], B[:, N:] = float("nan"), float("nan")
+    dt = torch.float32 if f32 else torch.bfloat16
+    C = torch.full((M, N + 8), float("nan"), dtype=dt, device=dev)
+    C0 = torch.randint(-4, 5, (M, N), generator=g, device=dev).to(dt)
+    C[:, :N] = C0
+    call = cf.cf_gemm_bf16_tn_accum_f32 if f32 else cf.cf_gemm_bf16_tn_accum_bf16
+    call(M, N, K, A, M + 8, B, N + 8, C, N + 8, stream())
+    # sums of at most 16 x 28292 in magnitude: exact in fp32 on either side
+    want = (C0.float() + A[:, :M].float().T.contiguous() @ B[:, :N].float()).to(dt)
+    assert torch.equal(C[:, :N], want) and torch.isnan(C[:, N:]).all()
+
+
 # C larger than what is left to the caches: streamed where its rows begin at 128-byte lines, not where C itself begins off one
 @pytest.mark.parametrize("M,N,ldc,f32", [(5000, 5168, 5184, True), (10008, 5168, 5184, False)])
 @pytest.mark.parametrize("off", [0, 4])
