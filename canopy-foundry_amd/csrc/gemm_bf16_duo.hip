@@ -45,6 +45,7 @@ constexpr int kStageOut = 2048;                            // per wavefront: wha
 constexpr int kLdsBytes = kRingBytes + 4 * kStageOut;      // 80 KiB: two workgroups per CU
 constexpr long long kStreamBytes = 96ll << 20;             // a larger C is streamed (see launch)
 constexpr long long kNearOperands = 300000000, kFarOperands = 600000000, kReadAgain = 1600000000;      // bytes (see large_operands)
+constexpr int kTurn = 8;                                   // steps, an even number
 constexpr int kNonTemporal = 2;                            // cache policy of a buffer access
 constexpr int kWaitVm0 = 0x0f70, kWaitVm6 = 0x0f76;        // s_waitcnt vmcnt(n), the other counters left alone
 
@@ -84,8 +85,8 @@ __device__ __forceinline__ float acc_read(float a) {
 // (four consecutive ones of two neighbouring groups of eight) land in the eight different 32-byte units of 256 bytes.
 __device__ __forceinline__ int unit_swz(int row) { return ((row & 3) << 1) | ((row >> 3) & 1); }
 
-// STREAM: C is read and written past the caches
-template <bool WIDE_M, bool F32, bool GROUPED, bool STREAM>
+// STREAM: C is read and written past the caches.  TURNS: a CU's two workgroups go first by turns of kTurn steps, not of a tile.
+template <bool WIDE_M, bool F32, bool GROUPED, bool STREAM, bool TURNS>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_gemm_bf16_tn_duo(const TnArgs p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -285,10 +286,17 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
 
     // Left alone the matrix cores serve the older of a CU's two workgroups first, which then runs ahead by a quarter of the launch
     // (and out of step with what its XCD's L2 holds).  So the other one (its LDS starts above the first one's) goes first in
-    // every second of its tiles.
+    // every second of its tiles.  With one tile per workgroup and many steps that would leave the other one alone for the second
+    // half, when one wavefront per SIMD cannot fill the matrix cores: there they take turns inside the tile (TURNS; 1360 x 8944 fp32 over 17430 rows
+    // 509 -> 447 us, 2360 x 4984 bf16 over 11926 304 -> 287, 14384 x 840 over 3545 99 -> 91).
     unsigned lds_alloc;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_LDS_ALLOC, 0, 12)" : "=s"(lds_alloc));
     bool first_now = lds_alloc != 0;
+    auto go_first = [&]() {
+        if (first_now) __builtin_amdgcn_s_setprio(3);
+        else __builtin_amdgcn_s_setprio(0);
+        first_now = lds_alloc != 0 && !first_now;
+    };
 
     Tile cur = F;
     // the wavefront's block of C, rows from 16 im on: rows beyond the tile's end lie beyond the descriptor
@@ -311,15 +319,17 @@ void k_gemm_bf16_tn_duo(const TnArgs p) {
     static_for<0, 7>([&](auto ic) { read_w(rd_w, ic); });
 
     while (true) {
-        if (first_now) __builtin_amdgcn_s_setprio(3);
-        else __builtin_amdgcn_s_setprio(0);
-        first_now = lds_alloc != 0 && !first_now;
+        go_first();
         // the first pair's copies were waited for in the prologue or in the epilogue before
         step(B0{}, std::true_type{}, std::false_type{});
         step(B1{}, std::false_type{}, std::false_type{});
-        for (int ks = 2; ks < cur.nk; ks += 2) {
-            step(B0{}, std::false_type{}, std::true_type{});
-            step(B1{}, std::false_type{}, std::true_type{});
+        for (int ks = 2; ks < cur.nk;) {
+            const int stop = TURNS ? min(cur.nk, ks + kTurn) : cur.nk;
+            for (; ks < stop; ks += 2) {
+                step(B0{}, std::false_type{}, std::true_type{});
+                step(B1{}, std::false_type{}, std::true_type{});
+            }
+            if constexpr (TURNS) go_first();
         }
         // the MFMAs are opaque to the compiler's hazard handling
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -422,11 +432,11 @@ int resident_workgroups() {
 }
 long long tiles_of(int M, int N, int tm, int tn) { return static_cast<long long>((M + tm - 1) / tm) * ((N + tn - 1) / tn); }
 
-template <bool WIDE_M, bool F32, bool GROUPED, bool STREAM>
+template <bool WIDE_M, bool F32, bool GROUPED, bool STREAM, bool TURNS>
 int launch(TnArgs p, hipStream_t st) {
     static std::once_flag once;
     static hipError_t attr = hipSuccess;      // kept: a failed set-up is reported by every call, not only the first
-    auto kern = k_gemm_bf16_tn_duo<WIDE_M, F32, GROUPED, STREAM>;
+    auto kern = k_gemm_bf16_tn_duo<WIDE_M, F32, GROUPED, STREAM, TURNS>;
     std::call_once(once, [&] {
         attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
     });
@@ -451,7 +461,12 @@ int launch(const TnArgs& p, hipStream_t st) {
     // 848 rows 225 us streamed, 171 not; 30000 x 2056 fp32 over 256 213 and 107; rows at half lines 14336 x 4080 fp32 313 and 317).
     const long long bytes = static_cast<long long>(p.M) * p.ldc * (F32 ? 4 : 2) * (GROUPED ? p.num_experts : 1);
     const bool lines = (static_cast<long long>(p.ldc) * (F32 ? 4 : 2)) % 128 == 0 && (reinterpret_cast<uintptr_t>(p.C) & 127u) == 0;
-    return bytes > kStreamBytes && lines ? launch<WIDE_M, F32, GROUPED, true>(p, st) : launch<WIDE_M, F32, GROUPED, false>(p, st);
+    if (bytes > kStreamBytes && lines) return launch<WIDE_M, F32, GROUPED, true, false>(p, st);
+    if constexpr (!GROUPED) {
+        const long long tiles = WIDE_M ? tiles_of(p.M, p.N, kWide, kNarrow) : tiles_of(p.M, p.N, kNarrow, kWide);
+        if (tiles <= resident_workgroups() && 2 * tiles > resident_workgroups()) return launch<WIDE_M, F32, GROUPED, false, true>(p, st);
+    }
+    return launch<WIDE_M, F32, GROUPED, false, false>(p, st);
 }
 template <bool F32, bool GROUPED>
 int launch(const TnArgs& p, hipStream_t st) {

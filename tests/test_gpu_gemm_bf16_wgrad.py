@@ -20,9 +20,11 @@ def padded(x, ld):
 
 
 # tiles of 256 x 128 and of 128 x 256 (whichever are fewer), one column short of and beyond them; K around the steps of 32, the
-# pairs of steps and the shortest pipeline of four; the last size is as large as what is streamed, but its rows begin off the lines
+# pairs of steps and the shortest pipeline of four; the last size is as large as what is streamed, but its rows begin off the lines;
+# the two of 289 tiles have one tile per workgroup and two workgroups on some CUs: turns of eight steps, the last one short, and none
 @pytest.mark.parametrize("M,N,K", [(256, 128, 1), (128, 256, 31), (264, 120, 33), (120, 264, 64), (248, 136, 65), (8, 8, 127), (512, 384, 129),
-                                   (384, 512, 200), (2048, 2056, 96), (5128, 5192, 40)])
+                                   (384, 512, 200), (2048, 2056, 96), (5128, 5192, 40),
+                                   (2056, 4104, 709), (4104, 2056, 100)])
 @pytest.mark.parametrize("f32", [True, False])
 def test_wgrad_edges(cf, dev, M, N, K, f32):
     case(f"bf16 wgrad {M}x{N}x{K} f32 {f32}")
