@@ -2094,8 +2094,14 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
     }
     if (half && p.M > 128) {          // (with fewer rows half of the tile or more is padding)
-        const float d = half_estimate_us(p, epi);
-        if (d * (best.kernel == CF_GEMM_KERNEL_DUO ? 1.03f : 1.0f) < t) { t = d; best = {CF_GEMM_KERNEL_HALF, 0}; }
+        const bool over_duo = best.kernel == CF_GEMM_KERNEL_DUO;
+        const float d = half_estimate_us(p, epi, false);
+        if (d * (over_duo ? 1.03f : 1.0f) < t) {
+            // Rows of K that share lines cost both of them time.  The other kernels' estimates do not count that (they lose by more), so it is left out against
+            // those.  Half tiles and two per CU: 2665 x 15960 over 1584 104.8 us and 87.9, 1092 x 9432 over 3696 67.2 and 57.2, 869 x 5808 over 5072 40.7 and 47.0.
+            if (!over_duo || p.K % BK == 0 || half_estimate_us(p, epi, true) < t) best = {CF_GEMM_KERNEL_HALF, 0};
+            t = d;
+        }
     }
     if (small) {
         int shape = 0;

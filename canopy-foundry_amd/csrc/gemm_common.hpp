@@ -104,7 +104,7 @@ int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shap
 int grouped_gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int shape, hipStream_t st);
 // gemm_half.hip: whether it takes a problem, its time, the launch
 bool half_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
-float half_estimate_us(const GemmArgs& p, int epi);
+float half_estimate_us(const GemmArgs& p, int epi, bool shared);
 int gemm_nt_half(const GemmArgs& p, int fmt, int epi, int scale_mode, hipStream_t st);
 // gemm_duo.hip: whether it takes a problem, its time, the launch
 bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);

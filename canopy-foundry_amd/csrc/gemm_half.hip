@@ -405,7 +405,9 @@ bool half_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
 // the chip and the L2s, 0.57 where up to 144 CUs have a tile; per tile the store, which a long K hides part of; 6 (gate 4) for the launch
 // and the first fill.  Against the fastest of the other kernels there: 2048 x 4096 over K 14336 102.6 -> 90.8 us, over 50304 361 -> 317;
 // 700 x 2 x 14336 over 4096 88.7 -> 79.3; 4000 x 2048 over 32000 302 -> 189.
-float half_estimate_us(const GemmArgs& p, int epi) {
+// shared: with rows of K that share lines (K no multiple of 128).  A K-tile's copies then take 0.8 to 0.9 whatever the number of CUs, 0.95 in
+// problems of several rounds.
+float half_estimate_us(const GemmArgs& p, int epi, bool shared) {
     const int out_bn = 128;
     const long long tiles = epi == EPI_SILU_GATE ? static_cast<long long>((p.M + 127) / 128) * ((p.N + out_bn - 1) / out_bn)
                             : along_rows(p)      ? static_cast<long long>((p.M + 255) / 256) * ((p.N + 127) / 128)
@@ -414,8 +416,9 @@ float half_estimate_us(const GemmArgs& p, int epi) {
     const long long full = tiles / cus, rest = tiles % cus;
     const float nk = static_cast<float>(p.K <= 2 * BK ? 4 : (p.K + 2 * BK - 1) / (2 * BK) * 2);
     const float busy = static_cast<float>(rest) / static_cast<float>(cus), tile = 2.5f + 20.0f / nk;
-    const float slow = busy > 0.5625f ? 0.57f + 0.4f * (busy - 0.5625f) : 0.57f;
-    return (epi == EPI_SILU_GATE ? 4.0f : 6.0f) + static_cast<float>(full) * (nk * 0.74f + tile) + (rest ? nk * slow + tile : 0.0f);
+    const float crowd = busy > 0.5625f ? busy - 0.5625f : 0.0f;
+    const float whole = shared ? 0.95f : 0.74f, slow = !shared ? 0.57f + 0.4f * crowd : full ? 0.95f : 0.80f + 0.2f * crowd;
+    return (epi == EPI_SILU_GATE ? 4.0f : 6.0f) + static_cast<float>(full) * (nk * whole + tile) + (rest ? nk * slow + tile : 0.0f);
 }
 
 int gemm_nt_half(const GemmArgs& p, int fmt, int epi, int scale_mode, hipStream_t st) {

@@ -94,6 +94,10 @@ def test_silu_gate_kernel(cf, M, N, K, kernel):
     (8192, 4096, 14336, PLAIN, RING16),              # 346, 256 x 256 tiles 294
     (700, 14336, 4096, GATE, HALF),                  # 79.3, 256 x 256 tiles 88.7: 336 of those are one and a third rounds
     (8192, 14336, 4096, GATE, RING16),               # 733, 653
+    (2665, 15960, 1584, PLAIN, DUO),                 # 104.8, two per CU 87.9: rows of K that share lines
+    (1092, 9432, 3696, PLAIN, DUO),                  # 67.2, 57.2
+    (869, 5808, 5072, PLAIN, HALF),                  # 40.7, 47.0: a part of a round
+    (1348, 8352, 13296, GATE, HALF),                 # 297, small tiles 622
 ])
 def test_half_tiles(cf, M, N, K, epi, kernel):
     assert route(cf, M, N, K, mode=ROW_COL, epi=epi) == kernel
