@@ -10,8 +10,9 @@ namespace cf {
 constexpr uint32_t kGeluLo = 0x3680u, kGeluSpan = 22u * 128u;       // bits of 2^-18; magnitudes in the table
 constexpr int kGeluEntries = 2 * kGeluSpan;                         // entry 2 * magnitude + sign
 
-__device__ __forceinline__ void gelu_table_build(uint16_t* table) {
-    for (uint32_t i = threadIdx.x; i < kGeluEntries; i += blockDim.x)
+// lane `lane` of `lanes`
+__device__ __forceinline__ void gelu_table_build(uint16_t* table, uint32_t lane, uint32_t lanes) {
+    for (uint32_t i = lane; i < kGeluEntries; i += lanes)
         table[i] = f32_to_bf16(gelu_fwd(bf16_to_f32(static_cast<uint16_t>((i >> 1) + kGeluLo + ((i & 1u) << 15)))));
 }
 // Both halves of a pair.  worst keeps the largest index met, per half: kGeluEntries or more means that some value lay outside and

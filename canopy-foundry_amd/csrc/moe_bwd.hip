@@ -179,7 +179,7 @@ __global__ __launch_bounds__(kThreads) void k_gelu_scalar(const uint16_t* __rest
 constexpr int kLutThreads = 1024;
 __global__ __launch_bounds__(kLutThreads) void k_gelu_lut(const uint4* __restrict__ x, uint4* __restrict__ out, size_t nvec) {
     __shared__ uint16_t table[kGeluEntries];
-    gelu_table_build(table);
+    gelu_table_build(table, threadIdx.x, blockDim.x);
     __syncthreads();
     const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
     for (size_t i0 = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i0 < nvec; i0 += 4 * stride) {

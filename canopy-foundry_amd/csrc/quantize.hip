@@ -504,7 +504,7 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
                                                                      uint8_t* __restrict__ out, float* __restrict__ scale,
                                                                      float* __restrict__ descale) {
     __shared__ uint16_t table[kGeluEntries];
-    gelu_table_build(table);
+    gelu_table_build(table, threadIdx.x, blockDim.x);
     __syncthreads();
     const int lane = threadIdx.x & 63;
     const int waves = gridDim.x * (kLutThreads / 64);
@@ -548,16 +548,22 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
     }
 }
 
-// k_grouped_quant_delayed with GELU for all but small banks, on the same table: up to two workgroups per CU stay, build
-// the table once and then take the (expert, part) items w = blockIdx.x, blockIdx.x + gridDim.x, ...
-// (part p of `per` covers the expert's 16-element vectors p * 1024 + lane, stepping per * 1024).  An item ends as a
+// k_grouped_quant_delayed with GELU for all but small banks, on the same table: one workgroup per CU (its registers leave room for one) builds
+// the table and then takes items, parts of one expert's 16-element vectors.  The counts lie on the device, so every workgroup
+// works the same cut out for itself.  Where no expert has more than kLutHot times its even part, expert e's vectors
+// are dealt to `per` workgroups; otherwise, and for large banks (per = 0), the bank as a whole is cut into equal runs, and a workgroup's run
+// goes on from one expert to the next.  With `per` workgroups each a hot expert's went on alone: 64 experts, 98304 x 1408, one with half of the
+// rows 719 us (direct 318), now 80; rows as 1 / rank 319 (165), now 80; 24576 x 1408 360 (317), now 28.  Runs cost a balanced small bank
+// a second expert per workgroup (8 experts, 3818 x 1408: 13.0 us, dealt 10.9), so those are dealt.
+// An item ends as a
 // workgroup of the plain form does: maximum into the slot's running amax, one arrival; the item that arrives last of an
-// expert's `per` updates the slot.  The slot's state changes only in that last step, and only after every item of the
+// expert's updates the slot.  The slot's state changes only in that last step, and only after every item of the
 // expert has arrived, so what a workgroup reads of it at the start of the kernel (row range and scale pair of every
 // expert, into LDS, under the table build, and of an expert's history at the start of an item) is the state the call started
 // with.  Same bits as the plain form.
-// 24576 x 1408, 64 experts: direct 43.7 us, 22.9 (104 MB: 4.5 TB/s); x from memory 51.6 and 43.7.
+// 24576 x 1408, 64 equal experts: direct 47.2 us, 24.4 (104 MB: 4.3 TB/s).
 constexpr int kLutMaxExperts = 1024;
+constexpr float kLutHot = 2.0f;
 template <bool E5M2, bool RECOMPUTE>
 __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(const uint16_t* __restrict__ x, uint8_t* __restrict__ out,
                                                                                int K, const int* __restrict__ counts,
@@ -569,22 +575,84 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
     __shared__ float sh[2][kLutThreads / 64];
     __shared__ int sh_first[kLutMaxExperts], sh_rows[kLutMaxExperts];
     __shared__ float sh_scale[kLutMaxExperts], sh_descale[kLutMaxExperts];
-    for (int e = threadIdx.x; e < num_experts; e += kLutThreads) {
-        const int first = offsets[e];
-        sh_first[e] = first;
-        sh_rows[e] = first >= 0 && first < total_rows ? min(counts[e], total_rows - first) : 0;
-        const float* st = states + static_cast<size_t>(e) * stride;
-        sh_scale[e] = st[RECOMPUTE ? slotw::SCALE_SNAP : slotw::SCALE];
-        sh_descale[e] = st[RECOMPUTE ? slotw::DESCALE_SNAP : slotw::DESCALE];
+    __shared__ uint32_t sh_start[kLutMaxExperts];           // rows of the experts before
+    __shared__ uint32_t sh_sum[kLutThreads / 64];           // rows of 64 experts
+    __shared__ int sh_most[kLutThreads / 64];               // and of the largest of them
+    const int lane = threadIdx.x & 63;
+    const uint32_t kv = K / kVec;                           // K % 16 == 0; total_rows * kv < 2^31 (the launcher)
+    // A wavefront for every 64 experts adds their rows up; one alone leaves the table to the others, whose work hides its own.
+    const int wave = threadIdx.x >> 6, scans = (num_experts + 63) / 64;
+    auto add = [](uint32_t a, uint32_t b) { return min(a + b, 0x7fffffffu); };      // (experts may overlap: their rows can be more than there are)
+    if (wave < scans) {
+        const int e = threadIdx.x;
+        int rows = 0;
+        if (e < num_experts) {
+            const int first = offsets[e];
+            rows = first >= 0 && first < total_rows ? max(min(counts[e], total_rows - first), 0) : 0;
+            const float* st = states + static_cast<size_t>(e) * stride;
+            sh_first[e] = first;
+            sh_rows[e] = rows;
+            sh_scale[e] = st[RECOMPUTE ? slotw::SCALE_SNAP : slotw::SCALE];
+            sh_descale[e] = st[RECOMPUTE ? slotw::DESCALE_SNAP : slotw::DESCALE];
+        }
+        uint32_t incl = rows;
+        int most = rows;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(incl, off, 64);
+            if (lane >= off) incl = add(incl, o);
+            most = max(most, __shfl_xor(most, off, 64));
+        }
+        const uint32_t before = __shfl_up(incl, 1, 64);
+        if (e < num_experts) sh_start[e] = lane ? before : 0;
+        if (lane == 63) { sh_sum[wave] = incl; sh_most[wave] = most; }
     }
-    gelu_table_build(table);
+    if (scans > 1) gelu_table_build(table, threadIdx.x, kLutThreads);
+    else if (wave) gelu_table_build(table, threadIdx.x - 64, kLutThreads - 64);
     __syncthreads();
-    const int items = num_experts * per;
+    uint32_t rows_all = 0, rows_before = 0;                 // of all experts; of those before this lane's 64
+    int most = 0;
+    for (int i = 0; i < scans; ++i) {
+        if (i == wave) rows_before = rows_all;
+        rows_all = add(rows_all, sh_sum[i]);
+        most = max(most, sh_most[i]);
+    }
+    // (experts that overlap are cut each by itself)
+    const bool even = rows_all <= static_cast<uint32_t>(total_rows) &&
+                      (per == 0 || static_cast<float>(most) * static_cast<float>(gridDim.x) > kLutHot * static_cast<float>(per) * static_cast<float>(rows_all));
+    uint32_t at = 0, stop = 0, chunk = 1;                   // even: the vector of the bank that this workgroup is at, of those up to `stop`
+    int e = -1;                                             // even: the expert of vector `at`
+    if (even) {
+        if (scans > 1) {
+            if (static_cast<int>(threadIdx.x) < num_experts) sh_start[threadIdx.x] += rows_before;
+            __syncthreads();
+        }
+        chunk = max((rows_all * kv + gridDim.x - 1) / gridDim.x, 1u);
+        at = min(blockIdx.x * chunk, rows_all * kv);
+        stop = min(at + chunk, rows_all * kv);
+        for (int e0 = 0; e0 < num_experts; e0 += 64) e += __popcll(__ballot(e0 + lane < num_experts && sh_start[min(e0 + lane, num_experts - 1)] * kv <= at));
+    }
+    const int cut = max(per, 1);
     int parity = 0;
-    for (int w = blockIdx.x; w < items; w += gridDim.x) {
-        const int e = w / per, part = w - e * per;
-        const int rows = sh_rows[e];
-        if (rows <= 0) continue;                                     // uniform over the workgroup
+    for (int w = blockIdx.x; even ? at < stop : w < num_experts * cut; w += gridDim.x) {
+        uint32_t from, to, step;                            // of the expert's vectors; the lanes of the item take runs of kLutThreads, `step` apart
+        int parts;                                          // the expert's items
+        if (even) {
+            uint32_t begin = sh_start[e] * kv, end = begin + sh_rows[e] * kv;
+            while (end <= at) { ++e; begin = end; end += sh_rows[e] * kv; }
+            from = at - begin;
+            to = min(stop, end) - begin;
+            step = kLutThreads;
+            parts = static_cast<int>((end - 1) / chunk - begin / chunk) + 1;
+            at = begin + to;
+        } else {
+            e = w / cut;
+            to = sh_rows[e] * kv;
+            if (to == 0) continue;                          // uniform over the workgroup
+            from = (w - e * cut) * kLutThreads;
+            step = cut * kLutThreads;
+            parts = cut;
+        }
         const int first = sh_first[e];
         const float s = sh_scale[e], ds = sh_descale[e];
         // what the last arrival needs of the history, read under the streaming work
@@ -600,24 +668,23 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
                 if (i != cursor) pre_max = fmaxf(pre_max, st[slotw::HISTORY + i]);
         }
         const bool s_finite = fabsf(s) < __uint_as_float(0x7f800000u);
-        const size_t tid = static_cast<size_t>(part) * kLutThreads + threadIdx.x;
-        const size_t stride_t = static_cast<size_t>(per) * kLutThreads;
-        for (size_t r = tid; r < static_cast<size_t>(rows); r += stride_t) row_descale[first + r] = ds;
+        // rows whose first vector is the item's (even), or the item's share of them
+        const uint32_t r0 = even ? (from + kv - 1) / kv : from, r1 = even ? (to + kv - 1) / kv : static_cast<uint32_t>(sh_rows[e]);
+        for (uint32_t r = r0 + threadIdx.x; r < r1; r += step) row_descale[first + r] = ds;
         const uint16_t* xe = x + static_cast<size_t>(first) * K;
         uint8_t* oe = out + static_cast<size_t>(first) * K;
-        const size_t nvec = static_cast<size_t>(rows) * K / kVec;       // K % 16 == 0
         float local = 0.0f;
         int local_bits = 0;
         constexpr int kBatch = 4;                                    // loads in flight per lane
-        for (size_t i0 = tid; i0 < nvec; i0 += kBatch * stride_t) {
+        for (uint32_t i0 = from + threadIdx.x; i0 < to; i0 += kBatch * step) {
             Vec16 v[kBatch];
 #pragma unroll
             for (int b = 0; b < kBatch; ++b)
-                if (i0 + b * stride_t < nvec) v[b] = load16(xe + (i0 + b * stride_t) * kVec);
+                if (i0 + b * step < to) v[b] = load16(xe + static_cast<size_t>(i0 + b * step) * kVec);
 #pragma unroll
             for (int b = 0; b < kBatch; ++b) {
-                const size_t i = i0 + b * stride_t;
-                if (i < nvec) {
+                const size_t i = i0 + b * step;
+                if (i < to) {
                     v[b].lo = gelu_look8(table, v[b].lo);
                     v[b].hi = gelu_look8(table, v[b].hi);
                     store_stream16(oe + i * kVec, quant16_track<E5M2, !RECOMPUTE>(v[b], s, s_finite, local_bits, local));
@@ -633,7 +700,7 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
             if (threadIdx.x == 0) {
                 float* st = states + static_cast<size_t>(e) * stride;
                 unsigned* arrived = reinterpret_cast<unsigned*>(st) + slotw::ARRIVED;
-                if (arrive_with_max(st + slotw::RUNNING, arrived, m, static_cast<unsigned>(per))) {
+                if (arrive_with_max(st + slotw::RUNNING, arrived, m, static_cast<unsigned>(parts))) {
                     const float amax = atomic_load_agent(st + slotw::RUNNING);
                     st[slotw::SCALE_SNAP] = s;
                     st[slotw::DESCALE_SNAP] = ds;
@@ -929,7 +996,7 @@ int launch_quant(const uint16_t* x, void* out, const float* scale, float* amax, 
 // 2048 7.5 directly and 6.6.  Wider rows have few wavefronts at work in small tensors: 512 x 4096 5.5 and 9.5, 2048 x 4096 10.9 and
 // 10.0, 4096 x 4096 18.5 and 10.4.  The grouped form with its arrivals from twice the first line: 8 experts, 1500 x 1408 9.6 and 8.0,
 // 64 experts, 3072 x 1408 12.7 and 10.3.
-constexpr size_t kGeluTableFrom = 2u << 20, kGeluTableFromWide = 8u << 20, kGeluOneItem = 48u << 20, kGeluTableFromUneven = 32u << 20;
+constexpr size_t kGeluTableFrom = 2u << 20, kGeluTableFromWide = 8u << 20, kGeluRuns = 48u << 20, kGeluRunsUneven = 32u << 20;
 int resident_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
@@ -1063,22 +1130,21 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
                                           fp8_max, d_row_descale);
     };
     const int which = (is_e5m2 ? 4 : 0) | (apply_gelu ? 2 : 0) | (is_recompute ? 1 : 0);
-    // GELU: the table form (the direct form waits for erff).  Parts per expert: an item ends in an arrival of a few dependent atomics on
-    // the expert's slot, so at most one item per CU (64 experts, 6144 x 1408: 10.4 us, with two 15.7; 24576 x 1408 22.9 and 29.2) until
-    // the streaming outweighs that and wants both workgroups of a CU (180000 x 1408 from memory: 212 and 206).  Rounded down: a few CUs
+    // GELU: the table form (the direct form waits for erff), with one workgroup per CU.  Up to kGeluRuns elements experts without a hot one
+    // among them have the same number of workgroups (64 experts, 24576 x 1408: 24.4 us; 6144 x 1408 11.1), rounded down: a few CUs
     // with a second item hold up all others (100 experts, 4200 x 1408: 10.0 us, rounded up 14.2, direct 12.5).  Where that leaves more
-    // than a quarter of the CUs idle the direct form stays until two per CU pay (300 experts from memory, 12000 x 1408: 30.9 directly,
-    // 34.8 in table form; 24576 x 1408: 51.3, 49.7).
+    // than a quarter of the CUs idle the direct form stays until equal runs pay (300 experts from memory, 12000 x 1408: 30.9 directly).
+    // A larger bank is always cut into equal runs: 60 experts, 42263 x 2048 49 us, dealt 62; one expert of 54523 x 1408 47, dealt to 64 CUs 105.
     const size_t n = static_cast<size_t>(total_rows) * K;
     const int cus = resident_cus();
     int parts = cus / num_experts;
     parts = parts > 64 ? 64 : parts;
     const bool fills = parts * num_experts * 4 >= min(cus, 64 * num_experts) * 3;      // of the CUs that a part each can give work to
-    const bool two_per_cu = n >= (fills ? kGeluOneItem : kGeluTableFromUneven);
-    if (two_per_cu) parts = min((2 * cus + num_experts - 1) / num_experts, 64);
-    if (apply_gelu && num_experts <= kLutMaxExperts && (two_per_cu || (fills && n >= 2 * kGeluTableFrom))) {
+    const bool large = n >= (fills ? kGeluRuns : kGeluRunsUneven);
+    if (large) parts = 0;
+    if (apply_gelu && num_experts <= kLutMaxExperts && n / kVec < (1u << 31) && (large || (fills && n >= 2 * kGeluTableFrom))) {
         auto launch_lut = [&](auto kernel) {
-            kernel<<<min(2 * cus, parts * num_experts), kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
+            kernel<<<cus, kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
                                                     state_stride_words, history_len, fp8_max, d_row_descale);
         };
         switch (which & 5) {

@@ -155,66 +155,94 @@ def test_counts_beyond_the_bound(cf, dev):
         bank.close()
 
 
+SKEWED = [9000, 0, 7001, 300, 11000, 1, 8000, 4698]
+# expert counts, and by how much total_rows is larger; K; where the table form cuts them: a large bank into equal runs (an expert without rows, with one,
+# and 17 behind one another in a run); a small one with a hot expert (one with all rows); near-equal experts dealt to the same
+# number of workgroups each, several turns of the streaming loop; more than 64 and than 512 experts, whose rows several wavefronts add up
+BANKS = [(SKEWED, 0, 1408), (SKEWED, 10000, 1408), ([0, 300, 20000] + [3] * 17 + [0, 9000, 40, 0], 0, 1408), ([0, 0, 9000, 0], 0, 1024), ([5000], 77, 1408),
+         ([380 + 7 * (e % 9) for e in range(64)], 0, 1408), ([800, 900, 0, 1100, 700, 650, 1200, 990], 5, 1408), ([40 + e % 3 for e in range(100)], 0, 1408),
+         ([5 + 600 * (e % 97 == 5) for e in range(200)], 0, 4096), ([30 + e % 5 for e in range(600)], 0, 2048)]
+
+
+@pytest.mark.parametrize("counts,beyond,K", BANKS)
 @pytest.mark.parametrize("e5m2", [False, True])
-def test_large_banks_take_the_table_form_with_the_same_bits(cf, dev, e5m2):
-    """From 64 Mi elements (rows of the bound x K) the GELU form looks bf16(gelu(x)) up in a table held in LDS by
-    workgroups that stay resident; total_rows being an upper bound, the same routing runs through both forms."""
-    case(f"grouped delayed GELU quantize, table form against the direct form, e5m2={e5m2}")
-    E, K, hist = 8, 1408, 8
-    counts = np.array([9000, 0, 7001, 300, 11000, 1, 8000, 4698], np.int32)
+def test_table_form_is_gelu_then_quantize(cf, dev, counts, beyond, K, e5m2):
+    """The table form of the GELU step against gelu_forward, in pieces that it evaluates directly, followed by the step
+    without GELU, which has one form only: bytes, row descales and every state word over two calls, and the recompute pass."""
+    E, hist = len(counts), 8
+    case(f"grouped delayed GELU quantize in table form, {E} experts, {sum(counts)} + {beyond} rows of {K}, e5m2={e5m2}")
+    counts = np.array(counts, np.int32)
     offsets = np.concatenate([[0], np.cumsum(counts)[:-1]]).astype(np.int32)
-    total = int(counts.sum())                                              # 40000 rows: 56 Mi elements, the direct form
-    bound = 50000                                                          # 70 Mi elements: the table form
-    assert total * K < (64 << 20) <= bound * K
+    total, bound = int(counts.sum()), int(counts.sum()) + beyond
+    assert bound * K >= 4 << 20
     gen = torch.Generator(device=dev).manual_seed(11)
     x = (torch.randn(bound, K, device=dev, generator=gen) * 1.7).to(torch.bfloat16)
+    y = torch.empty_like(x)
+    for r in range(0, bound, 20000):
+        piece = y[r:r + 20000]
+        assert piece.numel() < 64 << 20                                    # evaluated directly
+        cf.cf_gelu_forward_bf16(x[r:r + 20000], piece, piece.numel(), stream())
     fp8_max = 57344.0 if e5m2 else 448.0
     stride = cf.raw_cf_act_slot_state_words(hist) + 3
     init = np.zeros((E, stride), np.float32)
-    init[:, W["scale"]] = fp8_max / 6.0
-    init[:, W["descale"]] = 6.0 / fp8_max
+    init[:, W["scale"]] = fp8_max / (6.0 + np.arange(E) % 5)
+    init[:, W["descale"]] = (6.0 + np.arange(E) % 5) / fp8_max
     init[:, W["history"]] = 6.0
     init.view(np.int32)[:, W["cursor"]] = 1
     init.view(np.int32)[:, W["count"]] = 1
     d_counts, d_offsets = dev_arr(counts, dev), dev_arr(offsets, dev)
-    results = []
-    for rows_bound in (total, bound):
-        state = torch.from_numpy(init.reshape(-1).copy()).to(dev)
-        per_call = []
-        for call in range(2):
-            out = torch.full((bound, K), 0xEE, dtype=torch.uint8, device=dev)
-            rd = torch.full((bound,), -1.0, dtype=torch.float32, device=dev)
-            cf.cf_moe_grouped_quantize_delayed(x, out, K, E, d_counts, d_offsets, rows_bound, state, stride, hist, int(e5m2), 1, 0, rd, stream())
-            out_r = torch.full((bound, K), 0xEE, dtype=torch.uint8, device=dev)
-            rd_r = torch.full((bound,), -1.0, dtype=torch.float32, device=dev)
-            cf.cf_moe_grouped_quantize_delayed(x, out_r, K, E, d_counts, d_offsets, rows_bound, state, stride, hist, int(e5m2), 1, 1, rd_r, stream())
-            torch.cuda.synchronize()
-            assert torch.equal(out_r, out) and torch.equal(rd_r, rd), "the recompute pass gives the forward call's bytes"
-            assert bool((out[total:] == 0xEE).all()) and bool((rd[total:] == -1.0).all())
-            per_call.append((out, rd, state.clone()))
-        results.append(per_call)
+    states = [torch.from_numpy(init.reshape(-1).copy()).to(dev) for _ in range(2)]
     for call in range(2):
-        (o_a, rd_a, st_a), (o_b, rd_b, st_b) = results[0][call], results[1][call]
-        assert torch.equal(o_a, o_b), f"call {call}: bytes differ between the two forms"
-        assert torch.equal(rd_a, rd_b)
-        assert torch.equal(st_a.view(torch.int32), st_b.view(torch.int32)), f"call {call}: slot states differ"
-    # and one expert against the oracle (the GPU's own GELU values as its input)
-    e = 3
-    o, n = int(offsets[e]), int(counts[e])
-    g = torch.empty((n, K), dtype=torch.bfloat16, device=dev)
-    cf.cf_gelu_forward_bf16(x[o:o + n].contiguous(), g, n * K, stream())
+        got = []
+        for src, gelu, state in ((x, 1, states[0]), (y, 0, states[1])):
+            for recompute in (0, 1):
+                out = torch.full((bound, K), 0xEE, dtype=torch.uint8, device=dev)
+                rd = torch.full((bound,), -1.0, dtype=torch.float32, device=dev)
+                cf.cf_moe_grouped_quantize_delayed(src, out, K, E, d_counts, d_offsets, bound, state, stride, hist, int(e5m2), gelu, recompute, rd,
+                                                   stream())
+                got.append((out, rd))
+        torch.cuda.synchronize()
+        for out, rd in got[:3]:
+            assert torch.equal(out, got[3][0]) and torch.equal(rd, got[3][1]), f"call {call}"
+        assert bool((got[0][0][total:] == 0xEE).all()) and bool((got[0][1][total:] == -1.0).all())
+        assert torch.equal(states[0].view(torch.int32), states[1].view(torch.int32)), f"call {call}: slot states differ"
+    st = states[0].cpu().numpy().reshape(E, stride)
+    assert np.array_equal(st[counts == 0], init[counts == 0]), "an expert without rows keeps its slot"
+    # and one expert's first call against the oracle (the GPU's own GELU values as its input)
+    e = int(np.flatnonzero(counts)[-1])
+    o, n = int(offsets[e]), min(int(counts[e]), 700)
+    state = torch.from_numpy(init.reshape(-1).copy()).to(dev)
+    out = torch.empty((bound, K), dtype=torch.uint8, device=dev)
+    cf.cf_moe_grouped_quantize_delayed(x, out, K, E, d_counts, d_offsets, bound, state, stride, hist, int(e5m2), 1, 0, got[0][1], stream())
     torch.cuda.synchronize()
     quant = orc.quantize_e5m2 if e5m2 else orc.quantize_e4m3
-    g_bits = bf16_bits(g).reshape(-1)
-    assert np.array_equal(host(results[1][0][0][o:o + n]).reshape(-1), quant(g_bits, np.float32(fp8_max / 6.0)))
-    st = results[1][0][2].cpu().numpy().reshape(E, stride)
-    amax = orc.amax_bf16(g_bits)
+    assert np.array_equal(host(out[o:o + n]).reshape(-1), quant(bf16_bits(y[o:o + n]).reshape(-1), init[e, W["scale"]]))
+    st = state.cpu().numpy().reshape(E, stride)
+    amax = orc.amax_bf16(bf16_bits(y[o:o + int(counts[e])]).reshape(-1))
     assert st[e, W["amax"]] == amax and st[e, W["history"] + 1] == max(amax, np.float32(1e-12))
     assert st[e, W["scale"]] == np.float32(fp8_max) / max(amax, np.float32(6.0))
-    assert np.array_equal(st[1], init[1]), "an expert without rows keeps its slot"
-    second = results[1][1][0]
-    want_scale = st[e, W["scale"]]
-    assert np.array_equal(host(second[o:o + n]).reshape(-1), quant(g_bits, np.float32(want_scale)))
+
+
+def test_table_form_with_experts_that_overlap(cf, dev):
+    """Experts that share rows have more of them than there are; with equal states they write the same."""
+    case("grouped delayed GELU quantize in table form, overlapping experts")
+    K, hist = 1408, 4
+    for E, bound in ((3, 3000), (40, 36000)):                              # dealt; a bank that is otherwise cut into runs
+        counts, offsets = np.full(E, bound, np.int32), np.zeros(E, np.int32)
+        x = torch.randn(bound, K, device=dev, generator=torch.Generator(device=dev).manual_seed(E)).to(torch.bfloat16)
+        y = torch.empty_like(x)
+        cf.cf_gelu_forward_bf16(x, y, bound * K, stream())
+        stride = cf.raw_cf_act_slot_state_words(hist)
+        init = torch.zeros((E, stride), dtype=torch.float32, device=dev)
+        init[:, W["scale"]], init[:, W["descale"]] = 50.0, 0.02
+        got = []
+        for src, gelu in ((x, 1), (y, 0)):
+            st, out, rd = init.clone(), torch.empty((bound, K), dtype=torch.uint8, device=dev), torch.empty(bound, device=dev)
+            cf.cf_moe_grouped_quantize_delayed(src, out, K, E, dev_arr(counts, dev), dev_arr(offsets, dev), bound, st, stride, hist, 0, gelu, 0, rd, stream())
+            got.append((out, rd, st))
+        torch.cuda.synchronize()
+        for a, b in zip(*got):
+            assert torch.equal(a.view(torch.int32) if a.dtype == torch.float32 else a, b.view(torch.int32) if b.dtype == torch.float32 else b)
 
 
 class LoopBank:
