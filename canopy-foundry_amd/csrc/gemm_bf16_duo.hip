@@ -470,8 +470,11 @@ int launch(const TnArgs& p, hipStream_t st) {
 }
 template <bool F32, bool GROUPED>
 int launch(const TnArgs& p, hipStream_t st) {
-    // the tile lies along C whichever way it covers it with fewer (2048 x 1408: 88 tiles against 96)
-    return tiles_of(p.M, p.N, kWide, kNarrow) <= tiles_of(p.M, p.N, kNarrow, kWide) ? launch<true, F32, GROUPED>(p, st) : launch<false, F32, GROUPED>(p, st);
+    // the tile lies along C whichever way it covers it with fewer (2048 x 1408: 88 tiles against 96); where both ways are alike and C is one wide tile
+    // across, it takes whole rows, since two tiles would read and write the lines they share twice (64 experts of 6040 x 136 fp32
+    // over 572 rows 143 us in two, 102 in one; 386560 x 136 over 9 136 and 93)
+    const long long wide_m = tiles_of(p.M, p.N, kWide, kNarrow), wide_n = tiles_of(p.M, p.N, kNarrow, kWide);
+    return wide_m < wide_n || (wide_m == wide_n && p.N > kWide) ? launch<true, F32, GROUPED>(p, st) : launch<false, F32, GROUPED>(p, st);
 }
 
 // Which dense problems go to one workgroup of 256 x 256 per CU instead (gemm_bf16.hip, the same sums).  The 64 workgroups of an XCD drift apart in k,

@@ -21,10 +21,11 @@ def padded(x, ld):
 
 # tiles of 256 x 128 and of 128 x 256 (whichever are fewer), one column short of and beyond them; K around the steps of 32, the
 # pairs of steps and the shortest pipeline of four; the last size is as large as what is streamed, but its rows begin off the lines;
-# the two of 289 tiles have one tile per workgroup and two workgroups on some CUs: turns of eight steps, the last one short, and none
+# the two of 289 tiles have one tile per workgroup and two workgroups on some CUs: turns of eight steps, the last one short, and none;
+# and 512 x 136 is as many tiles either way
 @pytest.mark.parametrize("M,N,K", [(256, 128, 1), (128, 256, 31), (264, 120, 33), (120, 264, 64), (248, 136, 65), (8, 8, 127), (512, 384, 129),
                                    (384, 512, 200), (2048, 2056, 96), (5128, 5192, 40),
-                                   (2056, 4104, 709), (4104, 2056, 100)])
+                                   (2056, 4104, 709), (4104, 2056, 100), (512, 136, 100)])
 @pytest.mark.parametrize("f32", [True, False])
 def test_wgrad_edges(cf, dev, M, N, K, f32):
     case(f"bf16 wgrad {M}x{N}x{K} f32 {f32}")
@@ -85,7 +86,7 @@ def test_wgrad_large_c(cf, dev, M, N, ldc, f32, off):
 # rows per expert from none to several tiles' worth of steps; experts whose rows of tiles (6 and 11) end in a partial patch of four.
 # The last two have at least 176 tiles for an XCD's 64 workgroups, so that each walks several: of 256 x 128 and of 128 x 256 (fp32: streamed).
 SEVERAL = [40, 3, 64, 0, 65, 33, 1, 96, 31, 32, 70, 2, 129, 0, 17, 50]
-@pytest.mark.parametrize("M,N,counts", [(264, 136, [0, 1, 63, 64, 65, 0, 129, 300, 5]), (136, 264, [40, 0, 0, 7]),
+@pytest.mark.parametrize("M,N,counts", [(264, 136, [0, 1, 63, 64, 65, 0, 129, 300, 5]), (136, 264, [40, 0, 0, 7]), (512, 136, [9, 0, 130, 3]),
                                         (1408, 1024, [70, 0, 33, 1, 0, 64, 97, 128, 3, 200, 0, 32]),
                                         (1416, 2056, SEVERAL), (1288, 2048, SEVERAL)])
 @pytest.mark.parametrize("f32", [True, False])
