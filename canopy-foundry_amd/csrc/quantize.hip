@@ -156,7 +156,7 @@ __global__ __launch_bounds__(THREADS) void k_amax_f32(const float* __restrict__ 
         for (size_t i = tid; i < nvec; i += LOADS * stride) {
             float4 v[LOADS];
 #pragma unroll
-            for (int b = 0; b < LOADS; ++b) v[b] = reinterpret_cast<const float4*>(x)[min(i + b * stride, nvec - 1)];
+            for (int b = 0; b < LOADS; ++b) v[b] = reinterpret_cast<const float4*>(x)[LOADS > 1 ? min(i + b * stride, nvec - 1) : i];
 #pragma unroll
             for (int b = 0; b < LOADS; ++b)
                 local = fmaxf(fmaxf(local, fabsf(v[b].x)), fmaxf(fmaxf(fabsf(v[b].y), fabsf(v[b].z)), fabsf(v[b].w)));
