@@ -1,4 +1,4 @@
-// bf16(gelu(x)) of bf16 values by table.  The result is a function of x's 16 bits; erff costs about 60 vector instructions, a look-up
+// bf16(gelu(x)) of bf16 values by table.  The result is a function of x's 16 bits; with erff it costs about 40 vector instructions, a look-up
 // five and an LDS read.  The table holds every x with 2^-18 <= |x| < 16, 5632 entries in 11 KiB, which a workgroup of 1024 builds with
 // five or six evaluations per lane (all 65536 bit patterns took 64 and 128 KiB); what lies outside (zeros, tiny, huge, non-finite
 // values) is evaluated directly.  The same bits either way: the table is built with gelu_fwd.

@@ -173,9 +173,8 @@ __global__ __launch_bounds__(kThreads) void k_gelu_scalar(const uint16_t* __rest
     }
 }
 
-// The forward for all but small tensors: workgroups that stay on their CU look every element up (gelu_table.hpp) instead of
-// evaluating erff, which is what the plain kernel waits for.  Same bits.  98304 x
-// 1408: 95.6 us (a table of all bf16 values: 107.7), x from memory 152 (158).
+// The forward for tensors of 64 Mi elements and more: workgroups that stay on their CU look every element up (gelu_table.hpp) instead of
+// evaluating erff.  Same bits.  98304 x 1408: 95.6 us (a table of all bf16 values: 107.7), x from memory 152 (158).
 constexpr int kLutThreads = 1024;
 __global__ __launch_bounds__(kLutThreads) void k_gelu_lut(const uint4* __restrict__ x, uint4* __restrict__ out, size_t nvec) {
     __shared__ uint16_t table[kGeluEntries];

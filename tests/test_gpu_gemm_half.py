@@ -12,26 +12,28 @@ HALF = 128
 
 
 # 256 x 128 and 128 x 256 tiles (whichever are fewer); a last K-tile of 16, 80 and 112 bytes, two and three K-tiles (the pipeline
-# has four); N that ends 8 columns into a tile; more tiles than workgroups (2816 x 3208: 22 x 13 of 128 x 256)
+# has four); N that ends 8 columns into a tile; more tiles than the card has CUs, so that workgroups go on from one to the next: 2816 x
+# 3208 is 11 x 26 of 256 x 128 (and as many of the other), 640 x 14344 5 x 57 of 128 x 256 (339 of the other)
 @pytest.mark.parametrize("M,N,K", [(256, 128, 144), (128, 256, 256), (300, 264, 208), (257, 392, 624), (1, 136, 2000), (2816, 3208, 384),
-                                   (130, 8, 512)])
-@pytest.mark.parametrize("kind", ["tensor", "e5m2_rows", "bias"])
+                                   (640, 14344, 384), (130, 8, 512)])
+@pytest.mark.parametrize("kind", ["tensor", "rows", "e5m2", "e5m2_rows", "bias", "bias_rows", "e5m2_bias_rows"])
 def test_half_forms(cf, dev, M, N, K, kind):
     case(f"half-tile gemm {M}x{N}x{K} {kind}")
     rng = np.random.default_rng(M + N + K)
-    A, sa = rand_fp8(rng, (M, K), e5m2=kind == "e5m2_rows")
+    e5m2 = kind.startswith("e5m2")
+    A, sa = rand_fp8(rng, (M, K), e5m2=e5m2)
     B, sb = rand_fp8(rng, (N, K), sigma=0.02)
-    mode = ROW_COL if kind == "e5m2_rows" else PER_TENSOR
+    mode = ROW_COL if kind.endswith("rows") else PER_TENSOR
     if mode == ROW_COL:
         sa, sb = (sa * rng.uniform(0.5, 2, M)).astype(np.float32), (sb * rng.uniform(0.5, 2, N)).astype(np.float32)
-    kw = dict(mode=mode, a_e5m2=kind == "e5m2_rows", flags=HALF, ldc=N + 8)
+    kw = dict(mode=mode, a_e5m2=e5m2, flags=HALF, ldc=N + 8)
     got = run_gemm(cf, dev, A, B, sa, sb, **kw)
     assert np.isnan(got[:, N:]).all()
     rows = np.unique(np.concatenate([np.arange(0, M, max(1, M // 60)), [M - 1]]))
     ref, absdot = orc.gemm_nt_ref(A[rows], B, np.atleast_1d(sa)[rows] if mode else np.atleast_1d(sa), np.atleast_1d(sb), scale_mode=mode,
-                                  a_e5m2=kind == "e5m2_rows")
+                                  a_e5m2=e5m2)
     orc.assert_gemm_close(got[rows][:, :N], ref, absdot, what=f"{M}x{N}x{K}")
-    if kind == "bias":                           # added to the bf16 result
+    if "bias" in kind:                           # added to the bf16 result
         bias = orc.bf16_from_f32(rng.standard_normal(N).astype(np.float32))
         biased = run_gemm(cf, dev, A, B, sa, sb, epi=EPI_BIAS, bias=bias, **kw)
         want = orc.bf16_to_f32(orc.bf16_from_f32((got[:, :N] + orc.bf16_to_f32(bias)).astype(np.float32)))

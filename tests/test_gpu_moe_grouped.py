@@ -508,7 +508,7 @@ def test_gelu_quantize_rows_argument_errors(cf, dev):
 
 @pytest.mark.parametrize("rows,K", [(49152, 1408), (16384, 4096)])
 def test_gelu_quantize_rows_table_form(cf, dev, rows, K):
-    """Enough rows for the form that looks GELU up in a per-workgroup table of all 65536 bf16 values: bytes and scales
+    """Enough rows for the form that looks GELU up in a table per workgroup: bytes and scales
     must equal gelu_forward followed by the per-row quantize (both pinned against the oracle elsewhere), NaN and
     infinity rows included."""
     case(f"gelu + per-row quantize, table form rows={rows} K={K}")
