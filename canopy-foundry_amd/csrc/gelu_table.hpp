@@ -1,7 +1,7 @@
 // bf16(gelu(x)) of bf16 values by table.  The result is a function of x's 16 bits; with erff it costs about 40 vector instructions, a look-up
 // five and an LDS read.  The table holds every x with 2^-18 <= |x| < 16, 5632 entries in 11 KiB, which a workgroup of 1024 builds with
-// five or six evaluations per lane (all 65536 bit patterns took 64 and 128 KiB); what lies outside (zeros, tiny, huge, non-finite
-// values) is evaluated directly.  The same bits either way: the table is built with gelu_fwd.
+// five or six evaluations per lane (all 65536 bit patterns took 64 and 128 KiB); what lies outside (zeros, tiny, huge
+// values) has a closed form, infinities and NaN are evaluated directly.  The same bits every way: the table is built with gelu_fwd.
 #pragma once
 #include "common.hpp"
 
@@ -28,11 +28,27 @@ __device__ __forceinline__ uint32_t gelu_look2(const uint16_t* table, uint32_t p
     return static_cast<uint32_t>(table[i & 0xffffu]) | (static_cast<uint32_t>(table[i >> 16]) << 16);
 }
 __device__ __forceinline__ bool gelu_outside(const u16x2& worst) { return max(worst.x, worst.y) >= kGeluEntries; }
-// Four pairs, evaluated directly where one lies outside
+// A pair of which a half may lie outside the table, `found` being what the table gave: below it erff(x / sqrt 2) is too small to reach the
+// bf16 result, x / 2; from 16 on erff is 1 or -1, and the result x or -0.  Infinities and NaN: `special`.
+__device__ __forceinline__ uint32_t gelu_edge2(uint32_t pair, uint32_t found, bool& special) {
+    const uint32_t half = pack_bf16x2_hw(0.5f * bf16_lo(pair), 0.5f * bf16_hi(pair));
+    auto one = [&](uint32_t x, uint32_t f, uint32_t h) {
+        const uint32_t m = x & 0x7fffu;
+        special |= m >= 0x7f80u;
+        return m < kGeluLo ? h : m < kGeluLo + kGeluSpan ? f : (x & 0x8000u) ? 0x8000u : x;
+    };
+    return one(pair & 0xffffu, found & 0xffffu, half & 0xffffu) | (one(pair >> 16, found >> 16, half >> 16) << 16);
+}
+// Four pairs.  A wavefront with one value outside takes the second half; evaluating its values with gelu_fwd there made data with a zero here
+// and there the slowest: 98304 x 1408 with per-row scales, half of the values zero, 221 us, now 125 (normal values 84, one in a thousand
+// 40.0 109 and 94).
 __device__ __forceinline__ uint4 gelu_look8(const uint16_t* table, const uint4& v) {
     u16x2 worst = {0, 0};
     const uint4 g = make_uint4(gelu_look2(table, v.x, worst), gelu_look2(table, v.y, worst), gelu_look2(table, v.z, worst), gelu_look2(table, v.w, worst));
     if (!gelu_outside(worst)) return g;
+    bool special = false;
+    const uint4 o = make_uint4(gelu_edge2(v.x, g.x, special), gelu_edge2(v.y, g.y, special), gelu_edge2(v.z, g.z, special), gelu_edge2(v.w, g.w, special));
+    if (!special) return o;
     return make_uint4(gelu2(v.x), gelu2(v.y), gelu2(v.z), gelu2(v.w));
 }
 

@@ -994,9 +994,9 @@ int launch_quant(const uint16_t* x, void* out, const float* scale, float* amax, 
 
 // From here on the table form of the row quantize is the faster one.  Rows of up to 2048 elements: 512 x 1408 7.5 us both ways, 1024 x
 // 2048 7.5 directly and 6.6.  Wider rows have few wavefronts at work in small tensors: 512 x 4096 5.5 and 9.5, 2048 x 4096 10.9 and
-// 10.0, 4096 x 4096 18.5 and 10.4.  The grouped form with its arrivals from twice the first line: 8 experts, 1500 x 1408 9.6 and 8.0,
+// 10.0 (with values outside the table 12 to 14), 4096 x 4096 18.5 and 10.4.  The grouped form with its arrivals from twice the first line: 8 experts, 1500 x 1408 9.6 and 8.0,
 // 64 experts, 3072 x 1408 12.7 and 10.3.
-constexpr size_t kGeluTableFrom = 2u << 20, kGeluTableFromWide = 8u << 20, kGeluRuns = 48u << 20, kGeluRunsUneven = 32u << 20;
+constexpr size_t kGeluTableFrom = 2u << 20, kGeluTableFromWide = 12u << 20, kGeluRuns = 48u << 20, kGeluRunsUneven = 32u << 20;
 int resident_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;

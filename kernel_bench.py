@@ -438,6 +438,25 @@ def main():
                    lambda: cf.cf_gemm_bf16_nn(Md, Nd, Kd, ad, Kd, bd, Nd, cd, Nd, st))
             del ad, bd, cd
 
+    # dense bf16 weight gradients: two workgroups per CU, and operands beyond the memory-side cache (one per CU)
+    for what, Mw, Nw, Kw in (("of the loss head", 50304, 4096, 2048), ("large operands", 8192, 8192, 32768)):
+        name = f"bf16 wgrad, dense, {what} (tn, fp32 C)"
+        if args.only not in name:
+            continue
+        aw = bf16(Kw, Mw); bw = bf16(Kw, Nw); cw = torch.zeros((Mw, Nw), dtype=torch.float32, device=dev)
+        mfma16(name, f"{Mw}x{Nw}x{Kw}", 2.0 * Mw * Nw * Kw, lambda: cf.cf_gemm_bf16_tn_accum_f32(Mw, Nw, Kw, aw, Mw, bw, Nw, cw, Nw, st))
+        del aw, bw, cw
+
+    # half-tile FP8 GEMM: the input gradient of the loss head
+    name = "gemm half tile, dX of the loss head"
+    if args.only in name:
+        Mh, Nh, Kh = 2048, 4096, 50304
+        ah = fp8(Mh, Kh); bh = fp8(Nh, Kh); ch = torch.empty((Mh, Nh), dtype=torch.bfloat16, device=dev)
+        sa = f32(Mh); sb = f32(Nh)
+        mfma(name, f"{Mh}x{Nh}x{Kh}", 2.0 * Mh * Nh * Kh,
+             lambda: cf.cf_fp8_gemm_nt_bf16_ex(Mh, Nh, Kh, ah, Kh, 0, sa, bh, Kh, sb, 1, 0, None, None, None, ch, Nh, 0, st))
+        del ah, bh, ch
+
     # the whole selected-expert backward of the GELU bank in one call: FP8 recompute, route gradient, four bf16 GEMMs,
     # gelu_backward, scatter-add (16 launches per expert in the reference's host loop)
     szb = ctypes.c_size_t(0)
