@@ -345,6 +345,9 @@ def main():
     gq = u8(total, Ie); gs = f32(total); gd = f32(total)
     hbm("gelu_quantize_rows_e4m3 (gelu_forward + per-token quantize)", f"{total}x{Ie}", 3.0 * total * Ie,
         lambda: cf.cf_gelu_quantize_rows_e4m3(act, total, Ie, gq, gs, gd, st))
+    gact = bf16(total, Ie)              # the row above: values of a gate/up product under these scales, nearly all beyond the GELU table
+    hbm("gelu_quantize_rows_e4m3, values of N(0, 1)", f"{total}x{Ie}", 3.0 * total * Ie,
+        lambda: cf.cf_gelu_quantize_rows_e4m3(gact, total, Ie, gq, gs, gd, st))
     mfma("grouped GELU expert bank, whole pipeline (re-quantizing)", f"T={T} E={E} k={k}", 4.0 * total * Ie * H,
          lambda: cf.cf_moe_grouped_gelu_forward_fp8(hq, one, 0, rw, counts, offs, idx, wg, one, wd, one, mixed, T, H, Ie, E, total,
                                                     ws3, sz3.value, st))
@@ -357,6 +360,9 @@ def main():
     rowd = f32(total)
     hbm("grouped per-expert delayed-scale quantize with GELU (1 launch, 64 slots)", f"{total}x{Ie}", 3.0 * total * Ie,
         lambda: cf.cf_moe_grouped_quantize_delayed(act, gq, Ie, E, counts, offs, total, bank, words, 8, 0, 1, 0, rowd, st))
+    hbm("grouped per-expert delayed-scale quantize with GELU, values of N(0, 1)", f"{total}x{Ie}", 3.0 * total * Ie,
+        lambda: cf.cf_moe_grouped_quantize_delayed(gact, gq, Ie, E, counts, offs, total, bank, words, 8, 0, 1, 0, rowd, st))
+    del gact
     mfma("grouped GELU expert bank with per-expert activation slots", f"T={T} E={E} k={k}", 4.0 * total * Ie * H,
          lambda: cf.cf_moe_grouped_gelu_forward_fp8_slots(hq, one, 0, rw, counts, offs, idx, wg, one, wd, one, mixed, T, H, Ie, E, total,
                                                           bank, words, 8, 0, 0, ws3, sz3.value, st))
