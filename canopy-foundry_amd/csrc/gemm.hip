@@ -8,7 +8,8 @@
 //                         grouped per expert).  Needs K % 128 == 0, K >= 256 and a full-width, aligned C.
 //   k_gemm_nt             the same tile with register-staged, double-buffered LDS: any K % 16 == 0, any N.
 //   k_gemm_nt_block_ring  1 x 128 / 128 x 128 block scales on the persistent structure (eight wavefronts, partial
-//                         products folded into running sums every K-tile); k_gemm_nt_block is its staged fallback.
+//                         products folded into running sums every K-tile); k_gemm_nt_block is its staged fallback.  Where
+//                         256 x 256 tiles fill the rounds as well, gemm_block.hip's kernel is the faster one.
 //   k_gemm_nt_naive       one lane per output element: any shape and alignment, and the on-device cross-check.
 //
 // Common to the tiled kernels: workgroup tile 256 x 256 x 128 (128 x 256 x 128 with block scales), wavefronts own
@@ -2075,7 +2076,9 @@ float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.
+// shape: of the small-tile kernel; kWideBlocks marks the 256 x 256-tile one of the persistent block-scaled kernels.
 struct Route { int kernel, shape; };
+constexpr int kWideBlocks = 1;
 Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_naive) {
     if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
         (epi == EPI_SILU_GATE && !aligned16(p.B2)))
@@ -2089,6 +2092,10 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
     if (p.half && half) return {CF_GEMM_KERNEL_HALF, 0};
     if (p.small || p.duo || p.half || p.ring || p.force_staged) return best;
     float t = persistent_estimate_us(p, epi, scale_mode);
+    if (scale_mode == SCALE_BLOCK && block_wide_ok(p)) {
+        const float d = block_wide_estimate_us(p);
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_RING, kWideBlocks}; }
+    }
     if (duo) {
         const float d = duo_estimate_us(p, epi);
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
@@ -2139,6 +2146,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kBlkLds);
         });
         if (attr_err != hipSuccess) return static_cast<int>(attr_err);
+        if (route.kernel == CF_GEMM_KERNEL_RING && route.shape == kWideBlocks) return gemm_nt_block_wide(p, st);
         p.tiles_m = (p.M + BSM - 1) / BSM;
         p.tiles_n = (p.N + BN - 1) / BN;
         if (route.kernel == CF_GEMM_KERNEL_RING) {
@@ -2232,7 +2240,7 @@ int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int sca
     p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
     p.half = (flags & CF_GEMM_FLAG_HALF) != 0;
     const Route r = gemm_route(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE);
-    *kernel = r.kernel + r.shape;
+    *kernel = r.kernel == CF_GEMM_KERNEL_SMALL ? r.kernel + r.shape : r.kernel;
     return CF_OK;
 }
 

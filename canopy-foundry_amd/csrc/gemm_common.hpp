@@ -110,5 +110,9 @@ int gemm_nt_half(const GemmArgs& p, int fmt, int epi, int scale_mode, hipStream_
 bool duo_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
 float duo_estimate_us(const GemmArgs& p, int epi);
 int gemm_nt_duo(GemmArgs p, int fmt, int epi, int scale_mode, hipStream_t st);
+// gemm_block.hip (block scales on 256 x 256 tiles): whether it takes a problem, its time, the launch
+bool block_wide_ok(const GemmArgs& p);
+float block_wide_estimate_us(const GemmArgs& p);
+int gemm_nt_block_wide(GemmArgs p, hipStream_t st);
 
 }  // namespace cf
