@@ -1,9 +1,11 @@
-"""Builds libcf_fp8.so (hand-written HIP for gfx950) in-tree with hipcc."""
+"""Builds libcf_fp8.so (hand-written HIP for gfx950) in-tree with hipcc, and _cf_call.so (Python's way into it) with the host compiler."""
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -11,6 +13,8 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 INCLUDE = PKG.parent / "include"
 LIB = Path(os.environ.get("CF_LIB_OUT", PKG / "libcf_fp8.so"))
+
+CALL = PKG / "_cf_call.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -35,6 +39,23 @@ def _compile(src: Path, obj: Path, extra: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
+def build_call(objdir: Path) -> Path:
+    """Compiles csrc/call.cpp against this interpreter, with the names the header declares."""
+    spec = importlib.util.spec_from_file_location("cf_native", PKG / "native.py")
+    native = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(native)
+    names = [n for n, (ret, _) in native.parse_header().items() if ret == "int"]
+    (objdir / "call_names.inc").write_text("".join(f"CF_CALL({n})\n" for n in names))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-missing-field-initializers",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"), "-o", str(CALL)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"call.cpp:\n{proc.stderr}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr)
+    return CALL
+
+
 def build(force: bool = True, extra: list[str] | None = None, jobs: int = 8) -> Path:
     """Compiles every .hip under csrc/ and links libcf_fp8.so next to this file."""
     extra = list(extra or [])
@@ -55,6 +76,7 @@ def build(force: bool = True, extra: list[str] | None = None, jobs: int = 8) -> 
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
+    build_call(objdir)
     return LIB
 
 

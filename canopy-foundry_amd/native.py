@@ -1,13 +1,17 @@
-"""ctypes binding generated from include/cf_fp8.h.
+"""Python binding generated from include/cf_fp8.h.
 
 Every `int cf_*(...)` declared in the header becomes an attribute of `Lib` whose
 call raises `CfError` on a non-zero return (the reference's functions throw where
 the C ABI returns a code).  Pointer arguments accept an int address, None, or any
-object with `data_ptr()` (a torch tensor).
+object with `data_ptr()` (a torch tensor).  The calls go through _cf_call.so
+(csrc/call.cpp), which hands arguments of any other type to ctypes; `raw_cf_*` are
+the plain ctypes functions.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import re
 from pathlib import Path
 
@@ -65,6 +69,17 @@ def _conv(v):
     return v
 
 
+def _call_module():
+    path = PKG / "_cf_call.so"
+    if not path.exists():
+        raise RuntimeError(f"{path} is missing: build the library first (python -c 'import __graft_entry__ as g; g.build()')")
+    loader = importlib.machinery.ExtensionFileLoader("_cf_call", str(path))
+    spec = importlib.util.spec_from_file_location("_cf_call", path, loader=loader)
+    module = importlib.util.module_from_spec(spec)
+    loader.exec_module(module)
+    return module
+
+
 class Lib:
     def __init__(self, path: Path | None = None):
         path = Path(path) if path else lib_path()
@@ -78,16 +93,23 @@ class Lib:
         import torch  # noqa: F401
         self._dll = ctypes.CDLL(str(path))
         self.decls = parse_header()
+        make = _call_module().make
         for name, (ret, args) in self.decls.items():
             fn = getattr(self._dll, name)      # raises AttributeError if a declared symbol is not exported
             fn.argtypes = [_ctype(t) for t, _ in args]
             if ret == "int":
                 fn.restype = ctypes.c_int
-                setattr(self, name, self._checked(name, fn))
+                setattr(self, name, make(name, ctypes.cast(fn, ctypes.c_void_p).value, self._checked(name, fn), self._failed(name)))
             else:
                 fn.restype = ctypes.c_char_p if "char" in ret else None
                 setattr(self, name, fn)
             setattr(self, "raw_" + name, fn)
+
+    @staticmethod
+    def _failed(name):
+        def fail(rc):
+            raise CfError(name, rc)
+        return fail
 
     @staticmethod
     def _checked(name, fn):
