@@ -2025,15 +2025,31 @@ __global__ __launch_bounds__(64) void k_build_tile_map(const int* __restrict__ c
     build_tile_map_wave(counts, offsets, num_experts, max_row_tiles, total_rows, tile_map, threadIdx.x);
 }
 
+__device__ __forceinline__ void spread_descales(const DescaleSpread& s, size_t first, size_t step) {
+    const size_t n0 = s.n[0], n1 = n0 + s.n[1], n2 = n1 + s.n[2];
+    if (first >= n2) return;
+    const float f0 = n0 ? *s.src[0] : 0.0f, f1 = s.n[1] ? *s.src[1] : 0.0f, f2 = s.n[2] ? *s.src[2] : 0.0f;
+    for (size_t i = first; i < n2; i += step) {
+        if (i < n0) s.dst[0][i] = f0;
+        else if (i < n1) s.dst[1][i - n0] = f1;
+        else s.dst[2][i - n1] = f2;
+    }
+}
+
 // Everything an expert bank derives from (counts, row lists) in one launch.  Workgroup e < num_experts: the offset
 // of expert e (the sum of the counts before it; stored when the caller wants the array), its row list copied into the compact index at that offset and,
-// when slot_index is given, the inverse entries slot_index[row, e] = position.  The last workgroup: the tile table.
+// when slot_index is given, the inverse entries slot_index[row, e] = position.  Workgroup num_experts: the tile table.  Those after it: the
+// spread descales.
 // Entries at or beyond total_rows (the size of the compact buffers) are left out.
 __global__ __launch_bounds__(256) void k_bank_setup(const int* __restrict__ counts, const int* __restrict__ row_indices, int rows,
                                                     int num_experts, int max_row_tiles, int total_rows, int* __restrict__ offsets,
                                                     int* __restrict__ compact, int* __restrict__ slot_index,
-                                                    int* __restrict__ tile_map) {
+                                                    int* __restrict__ tile_map, const DescaleSpread spread) {
     const int e = blockIdx.x, tid = threadIdx.x;
+    if (e > num_experts) {
+        spread_descales(spread, static_cast<size_t>(e - num_experts - 1) * 256 + tid, static_cast<size_t>(gridDim.x - num_experts - 1) * 256);
+        return;
+    }
     if (e == num_experts) {
         if (tid < 64) build_tile_map_wave(counts, nullptr, num_experts, max_row_tiles, total_rows, tile_map, tid);
         return;
@@ -2054,6 +2070,68 @@ __global__ __launch_bounds__(256) void k_bank_setup(const int* __restrict__ coun
         compact[base + s] = row;
         if (slot_index) slot_index[static_cast<size_t>(row) * num_experts + e] = base + s;
     }
+}
+
+// What the backward of an expert bank derives from (counts, offsets, row lists), and the zeros it starts from, in one launch: between
+// large kernels a launch of next to no work takes 4.8 us (five of them did: 24 us of a GELU bank's step at 24576 rows).
+// Workgroups 0 ... (num_experts + 1) * parts - 1, the compact row index.  (e, part): expert e's rows from its offset on, and zeros from their end
+// up to the next expert's first row where no other expert's rows lie; e = num_experts: zeros before the first row of all.  The entries
+// must all be there: the elementwise stages run over total_rows rows and gather by them.  Any offsets will do, in any order.
+// Next workgroup: the tile table and the clamped counts.  The rest: descales and zeros.
+struct BackwardSetup {
+    const int *counts, *offsets, *row_indices;
+    int rows, num_experts, parts, max_row_tiles, total_rows;
+    int *clamped, *compact, *tile_map;
+    DescaleSpread spread;
+    float* zero;
+    size_t zeros;
+};
+__device__ __forceinline__ int kept_rows(const int* counts, const int* offsets, int e, int total_rows) {
+    const int first = offsets[e];
+    return first >= 0 && first < total_rows ? max(0, min(counts[e], total_rows - first)) : 0;
+}
+__global__ __launch_bounds__(256) void k_bank_backward_setup(const BackwardSetup a) {
+    const int tid = threadIdx.x, index_blocks = (a.num_experts + 1) * a.parts;
+    if (static_cast<int>(blockIdx.x) < index_blocks) {
+        const int e = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
+        int end = 0;
+        if (e < a.num_experts) {
+            const int first = a.offsets[e], n = kept_rows(a.counts, a.offsets, e, a.total_rows);
+            const int* list = a.row_indices + static_cast<size_t>(e) * a.rows;
+            for (int s = part * 256 + tid; s < n; s += a.parts * 256) a.compact[first + s] = list[s];
+            if (n == 0) return;              // what lies behind it is behind some other expert's rows, or before all
+            end = first + n;
+        }
+        // [from, to): no expert's rows begin up to `to`, and those that began by `end` are over by `from`
+        int from = end, to = a.total_rows;
+        for (int i = tid; i < a.num_experts; i += 256) {
+            const int n = kept_rows(a.counts, a.offsets, i, a.total_rows), first = a.offsets[i];
+            if (n == 0) continue;
+            if (e == a.num_experts || first > end) to = min(to, first);
+            else from = max(from, first + n);
+        }
+        __shared__ int sh[2][4];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            from = max(from, __shfl_xor(from, off, 64));
+            to = min(to, __shfl_xor(to, off, 64));
+        }
+        if ((tid & 63) == 0) { sh[0][tid >> 6] = from; sh[1][tid >> 6] = to; }
+        __syncthreads();
+        from = max(max(sh[0][0], sh[0][1]), max(sh[0][2], sh[0][3]));
+        to = min(min(sh[1][0], sh[1][1]), min(sh[1][2], sh[1][3]));
+        for (int p = from + part * 256 + tid; p < to; p += a.parts * 256) a.compact[p] = 0;
+        return;
+    }
+    if (static_cast<int>(blockIdx.x) == index_blocks) {
+        if (tid < 64) build_tile_map_wave(a.counts, a.offsets, a.num_experts, a.max_row_tiles, a.total_rows, a.tile_map, tid);
+        else
+            for (int i = tid - 64; i < a.num_experts; i += 192) a.clamped[i] = kept_rows(a.counts, a.offsets, i, a.total_rows);
+        return;
+    }
+    const size_t first = static_cast<size_t>(blockIdx.x - index_blocks - 1) * 256 + tid, step = static_cast<size_t>(gridDim.x - index_blocks - 1) * 256;
+    for (size_t i = first; i < a.zeros; i += step) a.zero[i] = 0.0f;
+    spread_descales(a.spread, first, step);
 }
 
 // What the kernels of this file take for a dense problem, in microseconds: tiles in rounds over the CUs, so much per K-tile and
@@ -2353,9 +2431,27 @@ void cf::build_tile_map(const int* d_counts, const int* d_offsets, int num_exper
 }
 
 void cf::bank_setup(const int* d_counts, const int* d_row_indices, int rows, int num_experts, int total_rows, int* d_offsets,
-                    int* d_compact_index, int* d_slot_index, int* tile_map, hipStream_t stream) {
-    k_bank_setup<<<num_experts + 1, 256, 0, stream>>>(d_counts, d_row_indices, rows, num_experts, total_rows / BM + num_experts,
-                                                      total_rows, d_offsets, d_compact_index, d_slot_index, tile_map);
+                    int* d_compact_index, int* d_slot_index, int* tile_map, const DescaleSpread& spread, hipStream_t stream) {
+    const size_t spread_blocks = (spread.n[0] + spread.n[1] + spread.n[2] + 1023) / 1024;
+    k_bank_setup<<<num_experts + 1 + static_cast<unsigned>(spread_blocks < 1024 ? spread_blocks : 1024), 256, 0, stream>>>(
+        d_counts, d_row_indices, rows, num_experts, total_rows / BM + num_experts, total_rows, d_offsets, d_compact_index, d_slot_index,
+        tile_map, spread);
+}
+
+void cf::bank_backward_setup(const int* d_counts, const int* d_offsets, const int* d_row_indices, int rows, int num_experts, int total_rows,
+                             int* d_clamped, int* d_compact_index, int* tile_map, const DescaleSpread& spread, float* d_zero, size_t zeros,
+                             hipStream_t stream) {
+    BackwardSetup a{};
+    a.counts = d_counts; a.offsets = d_offsets; a.row_indices = d_row_indices;
+    a.rows = rows; a.num_experts = num_experts; a.max_row_tiles = total_rows / BM + num_experts; a.total_rows = total_rows;
+    // 1024 rows of an even expert to a workgroup, and enough of them for one that has most of the rows
+    a.parts = total_rows / 4096 / (num_experts < 4 ? 1 : num_experts / 4) + 1;
+    a.parts = a.parts < 64 ? a.parts : 64;
+    a.clamped = d_clamped; a.compact = d_compact_index; a.tile_map = tile_map;
+    a.spread = spread; a.zero = d_zero; a.zeros = zeros;
+    const size_t items = zeros + spread.n[0] + spread.n[1] + spread.n[2];
+    const size_t blocks = (items + 1023) / 1024;
+    k_bank_backward_setup<<<(num_experts + 1) * a.parts + 1 + static_cast<unsigned>(blocks < 1024 ? (blocks ? blocks : 1) : 1024), 256, 0, stream>>>(a);
 }
 
 // build_map = false: d_workspace already holds the tile table of these counts and offsets (an earlier call of

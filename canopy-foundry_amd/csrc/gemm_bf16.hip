@@ -637,7 +637,7 @@ int launch(const BfArgs& p, dim3 grid, hipStream_t st) {
 
 // C[M,N] = A[M,K] . B[K,N]; grouped: per expert over its rows of the compact buffers
 int gemm_nn(int M, int N, int K, int E, const int* counts, const int* offsets, const uint16_t* A, int lda, const uint16_t* B,
-            int ldb, uint16_t* C, int ldc, void* ws, size_t ws_bytes, bool grouped, cf_stream_t stream) {
+            int ldb, uint16_t* C, int ldc, void* ws, size_t ws_bytes, bool grouped, bool build_map, cf_stream_t stream) {
     if (M < 0 || N < 0 || K < 0 || E < 0) return CF_ERR_INVALID_ARG;
     if (M == 0 || N == 0 || (grouped && E == 0)) return CF_OK;
     if (!A || !B || !C || (grouped && (!counts || !offsets || !ws))) return CF_ERR_INVALID_ARG;
@@ -656,7 +656,7 @@ int gemm_nn(int M, int N, int K, int E, const int* counts, const int* offsets, c
         cf_fp8_grouped_gemm_workspace_bytes(M, E, &need);
         if (ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 3u)) return CF_ERR_INVALID_ARG;
         tiles_m = M / TM + E;
-        build_tile_map(counts, offsets, E, tiles_m, M, static_cast<int*>(ws), st);
+        if (build_map) build_tile_map(counts, offsets, E, tiles_m, M, static_cast<int*>(ws), st);
         p.tile_map = static_cast<const int*>(ws);
         p.b_expert_stride = static_cast<long long>(K) * ldb;
         p.tiles_m = tiles_m;
@@ -700,6 +700,10 @@ int grouped_gemm_bf16_nt(int total_rows, int N, int Kb, int terms, int num_exper
     }
     return c_is_f32 ? launch<OUT_STORE_F32, true, true>(p, grid, st) : launch<OUT_STORE_BF16, true, true>(p, grid, st);
 }
+int grouped_gemm_bf16_nn_mapped(int total_rows, int N, int K, int num_experts, const int* d_counts, const int* d_offsets, const uint16_t* A,
+                                int lda, const uint16_t* B, uint16_t* C, int ldc, void* d_workspace, size_t workspace_bytes, cf_stream_t stream) {
+    return gemm_nn(total_rows, N, K, num_experts, d_counts, d_offsets, A, lda, B, N, C, ldc, d_workspace, workspace_bytes, true, false, stream);
+}
 int gemm_bf16_tn_large(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb, void* C, int ldc, bool c_is_f32,
                        hipStream_t st) {
     BfArgs p{};
@@ -718,12 +722,12 @@ extern "C" {
 
 int cf_gemm_bf16_nn(int M, int N, int K, const uint16_t* A, int lda, const uint16_t* B, int ldb, uint16_t* C, int ldc,
                     cf_stream_t stream) {
-    return gemm_nn(M, N, K, 0, nullptr, nullptr, A, lda, B, ldb, C, ldc, nullptr, 0, false, stream);
+    return gemm_nn(M, N, K, 0, nullptr, nullptr, A, lda, B, ldb, C, ldc, nullptr, 0, false, false, stream);
 }
 int cf_moe_grouped_gemm_bf16_nn(int total_rows, int N, int K, int num_experts, const int* d_counts, const int* d_offsets,
                                 const uint16_t* A, int lda, const uint16_t* B, uint16_t* C, int ldc, void* d_workspace,
                                 size_t workspace_bytes, cf_stream_t stream) {
-    return gemm_nn(total_rows, N, K, num_experts, d_counts, d_offsets, A, lda, B, N, C, ldc, d_workspace, workspace_bytes, true,
+    return gemm_nn(total_rows, N, K, num_experts, d_counts, d_offsets, A, lda, B, N, C, ldc, d_workspace, workspace_bytes, true, true,
                    stream);
 }
 

@@ -56,8 +56,26 @@ int unpermute_f32(uint16_t* d_mixed, const float* d_y, const float* d_route_weig
 // One launch for what an expert bank derives from (counts, row lists [num_experts, rows]): the offsets, the compact
 // row index, the (row, expert) -> compact row table (d_offsets and d_slot_index may be null) and the tile table of a grouped GEMM
 // over total_rows rows.
+// spread: per-tensor descales to be written out as the vectors a grouped GEMM reads (n = 0: none).
+struct DescaleSpread { const float* src[3]; float* dst[3]; size_t n[3]; };
 void bank_setup(const int* d_counts, const int* d_row_indices, int rows, int num_experts, int total_rows, int* d_offsets,
-                int* d_compact_index, int* d_slot_index, int* tile_map, hipStream_t stream);
+                int* d_compact_index, int* d_slot_index, int* tile_map, const DescaleSpread& spread, hipStream_t stream);
+// The same for the backward, where the offsets are the caller's: the counts cut to what the compact buffers hold (clamped), the compact
+// row index (0 where no expert's rows lie), the tile table, the spread descales, and zeros in d_zero.
+void bank_backward_setup(const int* d_counts, const int* d_offsets, const int* d_row_indices, int rows, int num_experts, int total_rows,
+                         int* d_clamped, int* d_compact_index, int* tile_map, const DescaleSpread& spread, float* d_zero, size_t zeros,
+                         hipStream_t stream);
+// cf_moe_grouped_gemm_bf16_nn over a tile table that is already in d_workspace (gemm_bf16.hip)
+int grouped_gemm_bf16_nn_mapped(int total_rows, int N, int K, int num_experts, const int* d_counts, const int* d_offsets, const uint16_t* A,
+                                int lda, const uint16_t* B, uint16_t* C, int ldc, void* d_workspace, size_t workspace_bytes, cf_stream_t stream);
+// cf_moe_grouped_route_grad_bf16 without the zeros (moe_bwd.hip)
+int grouped_route_grad_selected(const uint16_t* d_grad_mixed, uint16_t* d_expert_out, float* d_grad_route_weights, const float* d_route_weights,
+                                const int* d_counts, const int* d_offsets, const int* d_row_indices, int rows, int num_experts, int H,
+                                cf_stream_t stream);
+// bf16(gelu(x)) into d_post and, quantized by each expert's snapshot scale (cf_moe_grouped_quantize_delayed with is_recompute), into d_out
+int grouped_gelu_quantize_recompute(const uint16_t* d_x, uint16_t* d_post, void* d_out, int K, int num_experts, const int* d_counts,
+                                    const int* d_offsets, int total_rows, float* d_slot_states, int state_stride_words, int history_len,
+                                    int is_e5m2, float* d_row_descale, cf_stream_t stream);
 
 // The one-kernel forms of the GELU expert bank (moe.hip): what cf_moe_grouped_expert_forward_fp8 / _bf16 run when no
 // workspace is at hand.  Arguments checked by the callers.

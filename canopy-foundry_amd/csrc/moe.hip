@@ -1534,7 +1534,7 @@ int cf_moe_grouped_swiglu_forward_fp8(const void* d_hidden_e4m3, const float* d_
     int* slot = indexed ? reinterpret_cast<int*>(base + w.slot) : nullptr;
     // with the tile table of both projections in the same launch
     bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, nullptr, index, slot,
-               reinterpret_cast<int*>(base + w.tile_map), as_stream(stream));
+               reinterpret_cast<int*>(base + w.tile_map), DescaleSpread{}, as_stream(stream));
     int rc = launch_status();
     if (rc) return rc;
     // gate/up: rows gathered through the compact index (the token permute is fused into the operand fetch)
@@ -1570,18 +1570,6 @@ GeluWs gelu_layout(int rows, int total_rows, int num_experts, int H, int Ie) {
     w.out_descale = off; off = up(off + sizeof(float) * static_cast<size_t>(num_experts) * H);
     w.total = off;
     return w;
-}
-
-__global__ __launch_bounds__(kThreads) void k_spread_descales(const float* __restrict__ a, float* __restrict__ av, size_t na,
-                                                              const float* __restrict__ b, float* __restrict__ bv, size_t nb,
-                                                              const float* __restrict__ c, float* __restrict__ cv, size_t nc) {
-    const float fa = *a, fb = *b, fc = *c;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < na + nb + nc;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        if (i < na) av[i] = fa;
-        else if (i < na + nb) bv[i - na] = fb;
-        else cv[i - na - nb] = fc;
-    }
 }
 }  // namespace
 
@@ -1624,16 +1612,12 @@ int gelu_bank_forward(const void* d_hidden, const float* d_fcin_descale, int fci
     hipStream_t st = as_stream(stream);
     const bool indexed = sizeof(int) * static_cast<size_t>(rows) * num_experts <= w.s.slot_bytes;
     int* slot = indexed ? reinterpret_cast<int*>(base + w.s.slot) : nullptr;
+    const DescaleSpread spread{{d_fcin_descale, d_fc_in_descale, d_fc_out_descale},
+                               {hidden_descale, in_descale, out_descale},
+                               {static_cast<size_t>(rows), static_cast<size_t>(num_experts) * Ie, static_cast<size_t>(num_experts) * H}};
     bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, nullptr, index, slot,
-               reinterpret_cast<int*>(base + w.s.tile_map), st);
+               reinterpret_cast<int*>(base + w.s.tile_map), spread, st);
     int rc = launch_status();
-    if (rc) return rc;
-    {
-        const size_t na = static_cast<size_t>(rows), nb = static_cast<size_t>(num_experts) * Ie, nc = static_cast<size_t>(num_experts) * H;
-        k_spread_descales<<<grid_for(na + nb + nc), kThreads, 0, st>>>(d_fcin_descale, hidden_descale, na, d_fc_in_descale, in_descale, nb,
-                                                                      d_fc_out_descale, out_descale, nc);
-    }
-    rc = launch_status();
     if (rc) return rc;
     // fc_in: token rows gathered through the compact index in the operand fetch
     rc = grouped_gemm_nt_bf16(total_selected_rows, Ie, H, num_experts, d_counts, d_offsets, d_hidden, rows, H, index, hidden_descale,

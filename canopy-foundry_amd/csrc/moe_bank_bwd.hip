@@ -31,37 +31,7 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__global__ __launch_bounds__(kThreads) void k_zero_f32(float* __restrict__ p, size_t n) {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        p[i] = 0.0f;
-}
-__global__ __launch_bounds__(kThreads) void k_zero_i32(int* __restrict__ p, size_t n) {
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        p[i] = 0;
-}
-__global__ __launch_bounds__(kThreads) void k_spread3(const float* __restrict__ a, float* __restrict__ av, size_t na,
-                                                      const float* __restrict__ b, float* __restrict__ bv, size_t nb,
-                                                      const float* __restrict__ c, float* __restrict__ cv, size_t nc) {
-    const float fa = *a, fb = *b, fc = *c;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < na + nb + nc;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        if (i < na) av[i] = fa;
-        else if (i < na + nb) bv[i - na] = fb;
-        else cv[i - na - nb] = fc;
-    }
-}
-
 struct Layout { size_t off[CF_MOE_BWD_WS_COUNT]; size_t counts; size_t total; };
-
-// counts[e] cut to what the compact buffers hold: total_rows is the caller's bound on the selected rows (the
-// reference's callers pass rows * top_k), and every later stage walks (these counts, the caller's offsets)
-__global__ __launch_bounds__(kThreads) void k_clamp_counts(const int* __restrict__ counts, const int* __restrict__ offsets, int E,
-                                                           int total_rows, int* __restrict__ out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= E) return;
-    const int first = offsets[e];
-    out[e] = first >= 0 && first < total_rows ? max(0, min(counts[e], total_rows - first)) : 0;
-}
 
 Layout layout(int rows, int total_rows, int E, int H, int Ie) {
     auto up = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
@@ -154,47 +124,35 @@ int gelu_bank_backward(const uint16_t* d_grad_mixed, const void* d_hidden_fp8, c
     cf_fp8_grouped_gemm_workspace_bytes(total_selected_rows, num_experts, &map_bytes);
     hipStream_t st = as_stream(stream);
     const int total = total_selected_rows;
-    auto grid = [](size_t items) { return static_cast<unsigned>(min((items + kThreads - 1) / kThreads, static_cast<size_t>(2048))); };
 
-    // the route-weight gradient starts from zero (cudaMemsetAsync at src/trainer.cu:7670-7672): cleared by a kernel, so
-    // that the call can be recorded into a graph
-    k_zero_f32<<<grid(static_cast<size_t>(rows) * num_experts), kThreads, 0, st>>>(d_grad_route_weights, static_cast<size_t>(rows) * num_experts);
+    // Everything the stages below take from the routing, and the route-weight gradient's zeros (cudaMemsetAsync at
+    // src/trainer.cu:7670-7672), in one kernel that a graph can record.  total_selected_rows bounds the selected rows from above (the
+    // reference's callers pass rows * top_k, src/trainer.cu:6863): no stage may go past it, whatever the counts say.
+    int* clamped = reinterpret_cast<int*>(base + l.counts);
+    const DescaleSpread spread{{d_fcin_descale, d_fc_in_descale, d_fc_out_descale},
+                               {hidden_descale, in_descale, out_descale},
+                               {static_cast<size_t>(rows), static_cast<size_t>(num_experts) * Ie, static_cast<size_t>(num_experts) * H}};
+    bank_backward_setup(d_counts, d_offsets, d_row_indices, rows, num_experts, total, clamped, index, static_cast<int*>(tile_map),
+                        spread, d_grad_route_weights, static_cast<size_t>(rows) * num_experts, st);
     int rc = launch_status();
     if (rc) return rc;
     if (total == 0) return CF_OK;
-    {
-        const size_t na = static_cast<size_t>(rows), nb = static_cast<size_t>(num_experts) * Ie, nc = static_cast<size_t>(num_experts) * H;
-        k_spread3<<<grid(na + nb + nc), kThreads, 0, st>>>(d_fcin_descale, hidden_descale, na, d_fc_in_descale, in_descale, nb,
-                                                           d_fc_out_descale, out_descale, nc);
-    }
-    if ((rc = launch_status())) return rc;
-    // total_selected_rows bounds the selected rows from above (the reference's callers pass rows * top_k,
-    // src/trainer.cu:6863): no stage may go past it, whatever the counts say
-    {
-        int* clamped = reinterpret_cast<int*>(base + l.counts);
-        k_clamp_counts<<<(num_experts + kThreads - 1) / kThreads, kThreads, 0, st>>>(d_counts, d_offsets, num_experts, total, clamped);
-        if ((rc = launch_status())) return rc;
-        d_counts = clamped;
-    }
-    // entries of the index past the experts' lists (a total above the sum of the counts) point at row 0: the
-    // elementwise stages run over all `total` rows and must not gather from a stale index
-    k_zero_i32<<<grid(static_cast<size_t>(total)), kThreads, 0, st>>>(index, static_cast<size_t>(total));
-    if ((rc = launch_status())) return rc;
-    if ((rc = cf_moe_compact_row_index(d_counts, d_offsets, d_row_indices, rows, num_experts, index, stream))) return rc;
+    d_counts = clamped;
 
     // ---- recompute of the forward from the FP8 hidden states ----
     if ((rc = grouped_gemm_nt_bf16(total, Ie, H, num_experts, d_counts, d_offsets, d_hidden_fp8, rows, H, index, hidden_descale,
                                    d_fc_in_w8, in_descale, CF_SCALE_ROW_COL, CF_EPI_NONE, nullptr, nullptr, pre, Ie, tile_map, map_bytes,
-                                   true, fcin_is_e5m2 ? 1 : 0, stream)))
+                                   false, fcin_is_e5m2 ? 1 : 0, stream)))
         return rc;
-    if ((rc = cf_gelu_forward_bf16(pre, post, static_cast<size_t>(total) * Ie, stream))) return rc;
-    // one scale per token row, or the recompute call of fp8_quant_act on the expert's slot (is_recompute = true: the
+    // GELU, and one scale per token row or the recompute call of fp8_quant_act on the expert's slot (is_recompute = true: the
     // scale the forward's call snapshotted, no side effects; src/trainer.cu:7707-7712)
-    if (slots.states)
-        rc = cf_moe_grouped_quantize_delayed(post, postq, Ie, num_experts, d_counts, d_offsets, total, slots.states, slots.stride,
-                                             slots.history_len, slots.is_e5m2, 0, 1, post_descale, stream);
-    else
-        rc = cf_fp8_quantize_rows(post, total, Ie, 0, postq, post_scale, post_descale, stream);
+    if (slots.states) {
+        rc = grouped_gelu_quantize_recompute(pre, post, postq, Ie, num_experts, d_counts, d_offsets, total, slots.states, slots.stride,
+                                             slots.history_len, slots.is_e5m2, post_descale, stream);
+    } else {
+        rc = cf_gelu_forward_bf16(pre, post, static_cast<size_t>(total) * Ie, stream);
+        if (!rc) rc = cf_fp8_quantize_rows(post, total, Ie, 0, postq, post_scale, post_descale, stream);
+    }
     if (rc) return rc;
     if ((rc = grouped_gemm_nt_bf16(total, H, Ie, num_experts, d_counts, d_offsets, postq, total, Ie, nullptr, post_descale,
                                    d_fc_out_w8, out_descale, CF_SCALE_ROW_COL, CF_EPI_NONE, nullptr, nullptr, d_out, H, tile_map, map_bytes,
@@ -202,14 +160,14 @@ int gelu_bank_backward(const uint16_t* d_grad_mixed, const void* d_hidden_fp8, c
         return rc;
 
     // ---- route-weight gradient; the expert outputs become their gradients in place ----
-    if ((rc = cf_moe_grouped_route_grad_bf16(d_grad_mixed, d_out, d_grad_route_weights, d_route_weights, d_counts, d_offsets,
-                                             d_row_indices, rows, num_experts, H, stream)))
+    if ((rc = grouped_route_grad_selected(d_grad_mixed, d_out, d_grad_route_weights, d_route_weights, d_counts, d_offsets, d_row_indices,
+                                          rows, num_experts, H, stream)))
         return rc;
 
     // ---- fc_out: weight gradient and input gradient ----
     if ((rc = cf_moe_grouped_gemm_bf16_tn_accum_bf16(H, Ie, total, num_experts, d_counts, d_offsets, d_out, H, post, Ie, d_grad_fc_out, stream)))
         return rc;
-    if ((rc = cf_moe_grouped_gemm_bf16_nn(total, Ie, H, num_experts, d_counts, d_offsets, d_out, H, d_fc_out_w, d_post, Ie, tile_map, map_bytes,
+    if ((rc = grouped_gemm_bf16_nn_mapped(total, Ie, H, num_experts, d_counts, d_offsets, d_out, H, d_fc_out_w, d_post, Ie, tile_map, map_bytes,
                                           stream)))
         return rc;
     if ((rc = cf_gelu_backward_bf16(pre, d_post, d_pre, static_cast<size_t>(total) * Ie, stream))) return rc;
@@ -218,7 +176,7 @@ int gelu_bank_backward(const uint16_t* d_grad_mixed, const void* d_hidden_fp8, c
     if ((rc = cf_moe_gather_rows_bf16(d_hidden_bf16, x, index, total, H, stream))) return rc;
     if ((rc = cf_moe_grouped_gemm_bf16_tn_accum_bf16(Ie, H, total, num_experts, d_counts, d_offsets, d_pre, Ie, x, H, d_grad_fc_in, stream)))
         return rc;
-    if ((rc = cf_moe_grouped_gemm_bf16_nn(total, H, Ie, num_experts, d_counts, d_offsets, d_pre, Ie, d_fc_in_w, d_x, H, tile_map, map_bytes,
+    if ((rc = grouped_gemm_bf16_nn_mapped(total, H, Ie, num_experts, d_counts, d_offsets, d_pre, Ie, d_fc_in_w, d_x, H, tile_map, map_bytes,
                                           stream)))
         return rc;
     return cf_moe_unpermute_add_bf16(d_grad_hidden, d_x, d_route_weights, d_counts, d_offsets, d_row_indices, rows, num_experts, H,

@@ -204,7 +204,7 @@ int cf_moe_grouped_expert_forward_fp8_ws(const void* d_hidden, const float* d_fc
     hipStream_t st = as_stream(stream);
 
     // the reference takes the row lists without their offsets; the tile table and the compact index need them
-    bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, offsets, index, slot, tile_map, st);
+    bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, offsets, index, slot, tile_map, DescaleSpread{}, st);
     int rc = launch_status();
     if (rc) return rc;
     rc = grouped_gemm_nt_store_f32(total_selected_rows, Ie, H, num_experts, d_hidden, rows, H, index, d_fcin_descale, d_fc_in_w,
@@ -272,7 +272,7 @@ int cf_moe_grouped_expert_forward_bf16_ws(const uint16_t* d_hidden, const float*
     float* y = reinterpret_cast<float*>(base + w.off[CF_MOE_FWD_WS_Y]);
     hipStream_t st = as_stream(stream);
 
-    bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, offsets, index, slot, tile_map, st);
+    bank_setup(d_counts, d_row_indices, rows, num_experts, total_selected_rows, offsets, index, slot, tile_map, DescaleSpread{}, st);
     int rc = launch_status();
     if (rc) return rc;
     // the token permute rides in fc_in's operand fetch

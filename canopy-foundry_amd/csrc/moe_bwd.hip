@@ -15,6 +15,7 @@
 // Any other H takes a workgroup of T threads per row and the tree through LDS.
 #include "common.hpp"
 #include "gelu_table.hpp"
+#include "internal.hpp"
 
 namespace cf {
 namespace {
@@ -295,15 +296,23 @@ int cf_moe_grouped_route_grad_bf16(const uint16_t* d_grad_mixed, uint16_t* d_exp
     if (H == 0 || !d_grad_mixed || !d_expert_out || !d_grad_route_weights || !d_route_weights || !d_counts || !d_offsets ||
         !d_row_indices)
         return CF_ERR_INVALID_ARG;
-    hipStream_t st = as_stream(stream);
     // unselected (row, expert) pairs carry no gradient (src/trainer.cu:7667-7670 clears the buffer the same way)
     const size_t cells = static_cast<size_t>(rows) * num_experts;
-    k_fill_zero_f32<<<static_cast<unsigned>(min(ceil_div(cells, kThreads), 4096u)), kThreads, 0, st>>>(d_grad_route_weights, cells);
+    k_fill_zero_f32<<<static_cast<unsigned>(min(ceil_div(cells, kThreads), 4096u)), kThreads, 0, as_stream(stream)>>>(d_grad_route_weights, cells);
+    const int rc = launch_status();
+    if (rc) return rc;
+    return grouped_route_grad_selected(d_grad_mixed, d_expert_out, d_grad_route_weights, d_route_weights, d_counts, d_offsets, d_row_indices,
+                                       rows, num_experts, H, stream);
+}
+
+}  // extern "C"
+
+int cf::grouped_route_grad_selected(const uint16_t* d_grad_mixed, uint16_t* d_expert_out, float* d_grad_route_weights,
+                                    const float* d_route_weights, const int* d_counts, const int* d_offsets, const int* d_row_indices, int rows,
+                                    int num_experts, int H, cf_stream_t stream) {
     RouteGradArgs p{};
     p.a_full = d_grad_mixed; p.b = d_expert_out; p.dst = d_expert_out; p.out = d_grad_route_weights; p.rw = d_route_weights;
     p.counts = d_counts; p.offsets = d_offsets; p.row_indices = d_row_indices;
     p.rows = rows; p.E = num_experts; p.H = H; p.out_stride = num_experts;
-    return launch_route_grad<true, true>(p, rows, st);
+    return launch_route_grad<true, true>(p, rows, as_stream(stream));
 }
-
-}  // extern "C"

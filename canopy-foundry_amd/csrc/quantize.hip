@@ -564,9 +564,11 @@ __global__ __launch_bounds__(kLutThreads) void k_gelu_quant_rows_lut(const uint1
 // 24576 x 1408, 64 equal experts: direct 47.2 us, 24.4 (104 MB: 4.3 TB/s).
 constexpr int kLutMaxExperts = 1024;
 constexpr float kLutHot = 2.0f;
-template <bool E5M2, bool RECOMPUTE>
+// POST: bf16(gelu(x)) is written too (the backward's recompute needs both: one pass over x instead of a GELU and a quantize pass; 24576 x
+// 1408, 32 + 22 us before).
+template <bool E5M2, bool RECOMPUTE, bool POST = false>
 __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(const uint16_t* __restrict__ x, uint8_t* __restrict__ out,
-                                                                               int K, const int* __restrict__ counts,
+                                                                               uint16_t* __restrict__ post, int K, const int* __restrict__ counts,
                                                                                const int* __restrict__ offsets, int total_rows,
                                                                                int num_experts, int per, float* __restrict__ states,
                                                                                int stride, int history_len, float fp8_max,
@@ -687,6 +689,11 @@ __global__ __launch_bounds__(kLutThreads) void k_grouped_gelu_quant_delayed_lut(
                 if (i < to) {
                     v[b].lo = gelu_look8(table, v[b].lo);
                     v[b].hi = gelu_look8(table, v[b].hi);
+                    if constexpr (POST) {
+                        uint16_t* pe = post + static_cast<size_t>(first) * K + i * kVec;
+                        store_stream16(pe, v[b].lo);
+                        store_stream16(pe + 8, v[b].hi);
+                    }
                     store_stream16(oe + i * kVec, quant16_track<E5M2, !RECOMPUTE>(v[b], s, s_finite, local_bits, local));
                 }
             }
@@ -1109,10 +1116,12 @@ int cf_fp8_quantize_f32_e5m2(const float* d_x, void* d_out, const float* d_scale
     return launch_status();
 }
 
-int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int num_experts, const int* d_counts,
-                                    const int* d_offsets, int total_rows, float* d_slot_states, int state_stride_words,
-                                    int history_len, int is_e5m2, int apply_gelu, int is_recompute, float* d_row_descale,
-                                    cf_stream_t stream) {
+}  // extern "C"
+namespace {
+// d_post: also bf16(gelu(x)) (GELU and recompute only); by a pass of its own where the table form is not taken.
+int grouped_quantize_delayed(const uint16_t* d_x, void* d_out, uint16_t* d_post, int K, int num_experts, const int* d_counts,
+                             const int* d_offsets, int total_rows, float* d_slot_states, int state_stride_words, int history_len, int is_e5m2,
+                             int apply_gelu, int is_recompute, float* d_row_descale, cf_stream_t stream) {
     if (K < 0 || num_experts < 0 || total_rows < 0 || history_len < 0) return CF_ERR_INVALID_ARG;
     if (K == 0 || num_experts == 0 || total_rows == 0) return CF_OK;
     if (!d_x || !d_out || !d_counts || !d_offsets || !d_slot_states || !d_row_descale) return CF_ERR_INVALID_ARG;
@@ -1144,9 +1153,14 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
     if (large) parts = 0;
     if (apply_gelu && num_experts <= kLutMaxExperts && n / kVec < (1u << 31) && (large || (fills && n >= 2 * kGeluTableFrom))) {
         auto launch_lut = [&](auto kernel) {
-            kernel<<<cus, kLutThreads, 0, st>>>(d_x, o, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
+            kernel<<<cus, kLutThreads, 0, st>>>(d_x, o, d_post, K, d_counts, d_offsets, total_rows, num_experts, parts, d_slot_states,
                                                     state_stride_words, history_len, fp8_max, d_row_descale);
         };
+        if (d_post) {
+            if (is_e5m2) launch_lut(k_grouped_gelu_quant_delayed_lut<true, true, true>);
+            else launch_lut(k_grouped_gelu_quant_delayed_lut<false, true, true>);
+            return launch_status();
+        }
         switch (which & 5) {
             case 0: launch_lut(k_grouped_gelu_quant_delayed_lut<false, false>); break;
             case 1: launch_lut(k_grouped_gelu_quant_delayed_lut<false, true>); break;
@@ -1154,6 +1168,11 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
             default: launch_lut(k_grouped_gelu_quant_delayed_lut<true, true>); break;
         }
         return launch_status();
+    }
+    if (d_post) {
+        const int rc = cf_gelu_forward_bf16(d_x, d_post, n, stream);
+        return rc ? rc : grouped_quantize_delayed(d_post, d_out, nullptr, K, num_experts, d_counts, d_offsets, total_rows, d_slot_states,
+                                                  state_stride_words, history_len, is_e5m2, 0, is_recompute, d_row_descale, stream);
     }
     switch (which) {
         case 0: launch(k_grouped_quant_delayed<false, false, false>); break;
@@ -1166,6 +1185,16 @@ int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int
         default: launch(k_grouped_quant_delayed<true, true, true>); break;
     }
     return launch_status();
+}
+
+}  // namespace
+extern "C" {
+int cf_moe_grouped_quantize_delayed(const uint16_t* d_x, void* d_out, int K, int num_experts, const int* d_counts,
+                                    const int* d_offsets, int total_rows, float* d_slot_states, int state_stride_words,
+                                    int history_len, int is_e5m2, int apply_gelu, int is_recompute, float* d_row_descale,
+                                    cf_stream_t stream) {
+    return grouped_quantize_delayed(d_x, d_out, nullptr, K, num_experts, d_counts, d_offsets, total_rows, d_slot_states, state_stride_words,
+                                    history_len, is_e5m2, apply_gelu, is_recompute, d_row_descale, stream);
 }
 
 int cf_fp8_quantize_delayed_step(const uint16_t* d_x, void* d_out, size_t n, int is_e5m2, float* d_amax, float* d_scale,
@@ -1297,3 +1326,10 @@ int cf_fp8_unpack_e4m3_raw_bf16(const uint8_t* d_in, const float* d_descale, uin
 }
 
 }  // extern "C"
+
+int cf::grouped_gelu_quantize_recompute(const uint16_t* d_x, uint16_t* d_post, void* d_out, int K, int num_experts, const int* d_counts,
+                                        const int* d_offsets, int total_rows, float* d_slot_states, int state_stride_words, int history_len,
+                                        int is_e5m2, float* d_row_descale, cf_stream_t stream) {
+    return grouped_quantize_delayed(d_x, d_out, d_post, K, num_experts, d_counts, d_offsets, total_rows, d_slot_states, state_stride_words,
+                                    history_len, is_e5m2, 1, 1, d_row_descale, stream);
+}
