@@ -18,6 +18,7 @@ namespace {
 constexpr int kCeThreads = 256;
 constexpr int kCeWide = 1024;                          // lanes per row for rows beyond 32768 logits
 constexpr int kCeMaxChunks = 16;                       // 8-element chunks per lane: rows up to 32768 logits
+constexpr int kCeFewChunks = 7;                        // ... of a wide workgroup that leaves room for a second one: up to 57344
 constexpr float kLog2e = 1.44269504088896340736f, kLn2 = 0.69314718055994530942f;
 
 struct CeArgs {
@@ -60,8 +61,12 @@ __device__ __forceinline__ void opaque_words(const uint4& v, uint32_t (&w)[4]) {
 // Row in registers: V % 8 == 0, V <= 128 T, 16-byte aligned rows (8-byte for the fp8 gradient).  T lanes per row: 256
 // for rows up to 32768 logits, 1024 (a CU's sixteen wavefronts, 128 registers each) for rows up to 131072, so that a
 // 128k vocabulary is still read from memory once.
-template <bool QUANT, int T>
-__global__ __launch_bounds__(T) void k_ce_rows(const CeArgs p) {
+// CHUNKS: 8-element chunks per lane.  With sixteen a wide workgroup fills its CU's registers and its phases (load, maximum, sum, gradient)
+// run one after the other with nothing to overlap them; with seven, 64 registers in all, a second one's loads and stores run under
+// them: 2048 x 50304, 142 -> 110 us (4.7 TB/s).
+template <bool QUANT, int T, int CHUNKS>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(CHUNKS == kCeFewChunks ? 8 : 4)))
+void k_ce_rows(const CeArgs p) {
     __shared__ float sh[T / 64];
     const int tid = threadIdx.x, V = p.V, nchunks = V / 8;
     const size_t row = blockIdx.x;
@@ -76,10 +81,10 @@ __global__ __launch_bounds__(T) void k_ce_rows(const CeArgs p) {
         return;
     }
     const uint16_t* lrow = p.logits + row * V;
-    uint4 v[kCeMaxChunks];
+    uint4 v[CHUNKS];
     float m = -3.402823466e38f;
 #pragma unroll
-    for (int j = 0; j < kCeMaxChunks; ++j) {
+    for (int j = 0; j < CHUNKS; ++j) {
         const int c = tid + j * T;
         if (c < nchunks) {
             v[j] = reinterpret_cast<const uint4*>(lrow)[c];
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(T) void k_ce_rows(const CeArgs p) {
     const float bias2 = -row_max * kLog2e;
     float s = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kCeMaxChunks; ++j) {
+    for (int j = 0; j < CHUNKS; ++j) {
         if (tid + j * T < nchunks) {
             uint32_t w[4];
             opaque_words(v[j], w);
@@ -113,7 +118,7 @@ __global__ __launch_bounds__(T) void k_ce_rows(const CeArgs p) {
     float llp = 0.0f;
     uint32_t absacc = 0;
 #pragma unroll
-    for (int j = 0; j < kCeMaxChunks; ++j) {
+    for (int j = 0; j < CHUNKS; ++j) {
         const int c = tid + j * T;
         if (c < nchunks) {
             uint32_t w[4];
@@ -298,8 +303,9 @@ template <bool QUANT>
 int launch_ce(const CeArgs& p, int rows, hipStream_t st) {
     const bool vec = p.V % 8 == 0 && aligned16(p.logits) && aligned16(p.grad) &&
                      (!QUANT || (reinterpret_cast<uintptr_t>(p.grad8) & 7u) == 0);
-    if (vec && p.V <= kCeMaxChunks * kCeThreads * 8)      k_ce_rows<QUANT, kCeThreads><<<rows, kCeThreads, 0, st>>>(p);
-    else if (vec && p.V <= kCeMaxChunks * kCeWide * 8)    k_ce_rows<QUANT, kCeWide><<<rows, kCeWide, 0, st>>>(p);
+    if (vec && p.V <= kCeMaxChunks * kCeThreads * 8)      k_ce_rows<QUANT, kCeThreads, kCeMaxChunks><<<rows, kCeThreads, 0, st>>>(p);
+    else if (vec && p.V <= kCeFewChunks * kCeWide * 8)    k_ce_rows<QUANT, kCeWide, kCeFewChunks><<<rows, kCeWide, 0, st>>>(p);
+    else if (vec && p.V <= kCeMaxChunks * kCeWide * 8)    k_ce_rows<QUANT, kCeWide, kCeMaxChunks><<<rows, kCeWide, 0, st>>>(p);
     else if (vec)                                         k_ce_rows_stream<QUANT><<<rows, kCeThreads, 0, st>>>(p);
     else                                             k_ce_rows_generic<QUANT><<<rows, kCeThreads, 0, st>>>(p);
     return launch_status();

@@ -120,3 +120,9 @@ def test_cross_entropy_argument_errors(cf):
     assert cf.raw_cf_cross_entropy_fwd_bwd_chunk(None, None, None, None, 0, 8, None, None) == 0
     assert cf.raw_cf_cross_entropy_fwd_bwd_chunk(None, None, None, None, -1, 8, None, None) == -1
     assert cf.raw_cf_cross_entropy_count_valid(None, 0, None, None) == -1
+
+
+# the edges of the form that leaves room for two wide workgroups on a CU, and rows enough that there are two
+@pytest.mark.parametrize("rows,V", [(3, 32776), (2, 57344), (2, 57352), (600, 33000)])
+def test_cross_entropy_seven_chunks_a_lane(cf, dev, rows, V):
+    test_cross_entropy_chunk_fused_with_e5m2_quantize(cf, dev, rows, V)
