@@ -43,6 +43,9 @@ inline bool bf16_operands_ok(const void* A, int lda, const void* B, int ldb, con
     return aligned16(A) && aligned16(B) && lda % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && ldc < (1 << 21) &&
            (reinterpret_cast<uintptr_t>(C) & (4u * c_elem_bytes - 1u)) == 0;
 }
+// cf_fp8_scale_from_amax (E4M3) and cf_fp8_quant_and_transpose_e4m3 in one launch, K and N above 0 (transpose.hip)
+int quant_and_transpose_from_amax(const uint16_t* d_in, void* d_straight, void* d_transposed, const float* d_amax, float* d_scale,
+                                  float* d_descale, int K, int N, cf_stream_t stream);
 // The tile table of a grouped GEMM (k_build_tile_map in gemm.hip): tile_map[0] = number of row tiles of 256 rows,
 // then per row tile (expert, its first row, its end row, its first row tile, its row-tile count), experts back to back.
 // An expert's row range is cut at total_rows, the number of rows the compact buffers hold.

@@ -8,6 +8,7 @@
 // into LDS and the tile leaves as 128-byte row segments.  Other shapes take a
 // 64 x 64 scalar tile.
 #include "common.hpp"
+#include "internal.hpp"
 
 namespace cf {
 namespace {
@@ -51,6 +52,19 @@ __device__ __forceinline__ uint2 load_row8(const void* src, size_t elem_index, f
     }
 }
 
+// A scale that is still to be made from an amax (k_scale_from_amax's two divisions): every workgroup makes it for itself, the first
+// one writes it out.  A launch of its own for that took 4.8 us between two passes over a weight.
+struct FromAmax { const float* amax; float *scale, *descale; };
+__device__ __forceinline__ float tile_scale(const float* scale, const FromAmax& from) {
+    if (!from.amax) return *scale;
+    const float a = fmaxf(*from.amax, 1e-12f), s = CF_E4M3_MAX / a;
+    if (threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+        *from.scale = s;
+        *from.descale = a / CF_E4M3_MAX;
+    }
+    return s;
+}
+
 // in[R,C] (bf16 when QUANT, bytes otherwise) -> outT[C,R] bytes, and straight[R,C] when DUAL.
 // Bound by memory: 2 bytes in and 2 out per element of the dual form.  RAGGED: the last tile of a row or column of tiles is
 // cut off; a lane's 8 x 8 block lies inside the matrix or outside it, and so does a 16-byte piece of the output.  The two
@@ -59,14 +73,14 @@ template <bool QUANT, bool DUAL, bool RAGGED>
 __global__ __launch_bounds__(kThreads) void k_transpose_tiled(const void* __restrict__ in,
                                                               uint8_t* __restrict__ straight,
                                                               uint8_t* __restrict__ outT,
-                                                              const float* __restrict__ scale, int R, int C) {
+                                                              const float* __restrict__ scale, int R, int C, const FromAmax from) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[kTile * kPitch];   // [c][r]
     const int r0 = blockIdx.y * kTile, c0 = blockIdx.x * kTile;
     // lane = 16 * (row block within the wavefront) + column block; row blocks 0 and 2 of a wavefront (lanes 0-15 and
     // 32-47) are the neighbours 2h and 2h + 1, as are row blocks 1 and 3
     const int tx = threadIdx.x & 15, tyl = (threadIdx.x >> 4) & 3, wave = threadIdx.x >> 6;
     const int ty = 2 * (2 * wave + (tyl & 1)) + (tyl >> 1);
-    const float s = QUANT ? *scale : 1.0f;
+    const float s = QUANT ? tile_scale(scale, from) : 1.0f;
 
     uint2 rowb[8] = {};
     if (!RAGGED || (r0 + ty * 8 < R && c0 + tx * 8 < C)) {
@@ -108,10 +122,10 @@ template <bool QUANT, bool DUAL>
 __global__ __launch_bounds__(kThreads) void k_transpose_generic(const void* __restrict__ in,
                                                                 uint8_t* __restrict__ straight,
                                                                 uint8_t* __restrict__ outT,
-                                                                const float* __restrict__ scale, int R, int C) {
+                                                                const float* __restrict__ scale, int R, int C, const FromAmax from) {
     __shared__ uint8_t tile[64][65];
     const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
-    const float s = QUANT ? *scale : 1.0f;
+    const float s = QUANT ? tile_scale(scale, from) : 1.0f;
     for (int i = threadIdx.x; i < 64 * 64; i += kThreads) {
         const int r = r0 + (i >> 6), c = c0 + (i & 63);
         uint8_t b = 0;
@@ -131,10 +145,10 @@ __global__ __launch_bounds__(kThreads) void k_transpose_generic(const void* __re
 }
 
 template <bool QUANT, bool DUAL>
-int launch_transpose(const void* in, void* straight, void* outT, const float* scale, int R, int C, cf_stream_t st) {
+int launch_transpose(const void* in, void* straight, void* outT, const float* scale, int R, int C, cf_stream_t st, const FromAmax& from = {}) {
     if (R < 0 || C < 0) return CF_ERR_INVALID_ARG;
     if (R == 0 || C == 0) return CF_OK;
-    if (!in || !outT || (QUANT && !scale) || (DUAL && !straight)) return CF_ERR_INVALID_ARG;
+    if (!in || !outT || (QUANT && !scale && !from.amax) || (DUAL && !straight)) return CF_ERR_INVALID_ARG;
     auto* o = static_cast<uint8_t*>(outT);
     auto* d = static_cast<uint8_t*>(straight);
     // 16-byte pieces of an output row need R % 16, 8-byte (bytes in) or 16-byte (bf16 in) pieces of an input row C % 8
@@ -142,12 +156,12 @@ int launch_transpose(const void* in, void* straight, void* outT, const float* sc
     if (fast) {
         dim3 grid((C + kTile - 1) / kTile, (R + kTile - 1) / kTile);
         if (R % kTile == 0 && C % kTile == 0)
-            k_transpose_tiled<QUANT, DUAL, false><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C);
+            k_transpose_tiled<QUANT, DUAL, false><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C, from);
         else
-            k_transpose_tiled<QUANT, DUAL, true><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C);
+            k_transpose_tiled<QUANT, DUAL, true><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C, from);
     } else {
         dim3 grid((C + 63) / 64, (R + 63) / 64);
-        k_transpose_generic<QUANT, DUAL><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C);
+        k_transpose_generic<QUANT, DUAL><<<grid, kThreads, 0, as_stream(st)>>>(in, d, o, scale, R, C, from);
     }
     return launch_status();
 }
@@ -174,3 +188,8 @@ int cf_transpose_u8(const void* d_in, void* d_out, int rows, int cols, cf_stream
 }
 
 }  // extern "C"
+
+int cf::quant_and_transpose_from_amax(const uint16_t* d_in, void* d_straight, void* d_transposed, const float* d_amax, float* d_scale,
+                                      float* d_descale, int K, int N, cf_stream_t stream) {
+    return launch_transpose<true, true>(d_in, d_straight, d_transposed, nullptr, K, N, stream, FromAmax{d_amax, d_scale, d_descale});
+}
