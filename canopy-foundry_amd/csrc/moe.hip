@@ -921,6 +921,8 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma(const ui
 // load so addressed touches a line per lane (25 bytes a nanosecond and CU).  So weights are fetched as runs of 64 or 128
 // bytes of a row by neighbouring lanes and turned in 4 KiB of LDS per wavefront; the sums go to `mixed` as whole rows.
 // 2048 tokens, 6 of 64 experts, 2048 x 1408: 620 -> 375 us (the swaps alone 160 us of the former); 64 tokens 280 -> 187.
+// What then bounds it is neither memory (with every fetch from one line 329 us) nor the matrix cores (busy 28 % of the time) but the
+// chains of LDS writes, reads and MFMAs of two wavefronts per SIMD; fc_in takes 55 us of a workgroup's 170, fc_out 105.
 constexpr int kWideRows = 32;
 constexpr int kWideBlocks = 16;
 constexpr int kWideInDepth = 4;     // weight fetches in flight per wavefront in fc_in
@@ -961,16 +963,25 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
     if (first >= n_active) return;
     const int n_rows = min(kWideRows, n_active - first);
     const int* my_rows = row_indices + static_cast<size_t>(e) * rows + first;
+    // the expert's weights through descriptors: a fetch's address is one lane offset and one scalar (H Ie < 2^31, checked by the launcher)
     const uint8_t* w_in = fc_in_w + static_cast<size_t>(e) * H * Ie;
     const uint8_t* w_out = fc_out_w + static_cast<size_t>(e) * Ie * H;
+    const int w_bytes = H * Ie;                 // below 2^31, checked by the launcher
+    // weights come through descriptors: a fetch's address is one lane offset and one scalar
+    auto fetch = [&](const uint8_t* w, uint32_t lane_at, int at) {
+        return __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(w), 0, w_bytes, 0x00020000), static_cast<int>(lane_at), at, 0));
+    };
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t = lane & 15, g = lane >> 4;
 
-    const int vec_per_row = H / 16;
-    for (int i = threadIdx.x; i < kWideRows * vec_per_row; i += kMfmaThreads) {
-        const int r = i / vec_per_row, c = i % vec_per_row;
+    // the rows are continued with zeros to whole rings of steps: what fc_in multiplies there (its last step again) adds nothing
+    const int vec_per_row = H / 16, vec_padded = (H + 511) / 512 * 32;
+    for (int i = threadIdx.x; i < kWideRows * vec_padded; i += kMfmaThreads) {
+        const int r = i / vec_padded, c = i % vec_padded;
         const int src = my_rows[min(r, n_rows - 1)];
-        *reinterpret_cast<uint4*>(sh_hidden + r * hs + wide_hidden_at(c * 16)) =
-            *reinterpret_cast<const uint4*>(hidden + static_cast<size_t>(src) * H + c * 16);
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (c < vec_per_row) v = *reinterpret_cast<const uint4*>(hidden + static_cast<size_t>(src) * H + c * 16);
+        *reinterpret_cast<uint4*>(sh_hidden + r * hs + wide_hidden_at(c * 16)) = v;
     }
     __syncthreads();
 
@@ -990,28 +1001,39 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
         acc[b][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
 
+    // One stream of fetches runs through the whole kernel: the last steps of a phase already request the first ones of the next, into the
+    // same eight registers (a chunk has two phases of some 10 us each, and began each of them with a round trip to memory).
+    // fc_in: a step is 16 weight rows x 128 bytes, fetched 8 lanes to a row and turned in LDS: registers 2 j and 2 j + 1.  in_pad: steps of a
+    // block, rounded up to the ring's length.
+    const int in_pad = (in_steps + kWideInDepth - 1) / kWideInDepth * kWideInDepth;
+    const uint32_t in_lane = static_cast<uint32_t>(lane >> 3) * static_cast<uint32_t>(H) + (lane & 7) * 16;
+    const uint32_t out_lane = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(Ie) + (lane & 3) * 16;
+    v4u wr[2 * kWideInDepth];
+    auto in_at = [&](int base, int width, int n0, int st) { return (base + min(n0, width - 16)) * H + min(st, in_steps - 1) * 128; };
+    // fc_out: 64 bytes of each of a block's 16 weight rows, fetched 4 lanes to a row: step j, block i of the group: register 4 j + i.
+    // Block blk of this wavefront; past the last one: that one again, whose sums are not used.
+    auto out_at = [&](int c, int width, int blk, int st) { return c + (min(blk, nblk - 1) * kWaves + wave) * 16 * Ie + min(st, width / 64 - 1) * 64; };
+    // Register pair x (fc_in's step x, or two blocks of fc_out's step x / 2) from fc_out or from fc_in.  Clamped and selected, never skipped or
+    // branched around: the compiler counts what is in flight, and behind a branch it waits for more than it needs.
+    auto fetch_pair = [&](int x, bool out, int at_in, int at_out0, int at_out1) {
+        const uint8_t* w = out ? w_out : w_in;
+        const uint32_t at_lane = out ? out_lane : in_lane;
+        wr[2 * x] = fetch(w, at_lane, out ? at_out0 : at_in);
+        wr[2 * x + 1] = fetch(w, at_lane, out ? at_out1 : at_in + 8 * H);
+        __builtin_amdgcn_sched_barrier(0);      // in the order they are waited for
+    };
+#pragma unroll
+    for (int j = 0; j < kWideInDepth; ++j) fetch_pair(j, false, in_at(0, min(chunk, Ie), wave * 16, j), 0, 0);
     for (int c0 = 0; c0 < Ie; c0 += chunk) {
         const int cw = min(chunk, Ie - c0);         // a multiple of 64
         // ---- fc_in + GELU for columns c0 .. c0 + cw - 1 ----
-        // A step is 16 weight rows x 128 bytes, fetched 8 lanes to a row and turned in LDS.  One stream of fetches over the
-        // wavefront's column blocks, kWideInDepth steps ahead: the first ones of the next block are requested under the last
-        // ones of this.  in_pad: steps of a block, rounded up to the ring's length.
-        const int in_pad = (in_steps + kWideInDepth - 1) / kWideInDepth * kWideInDepth;
-        // addresses are a scalar base plus one 32-bit lane offset, here and in fc_out: the registers go to the fetches
-        const uint32_t in_lane = static_cast<uint32_t>(lane >> 3) * static_cast<uint32_t>(H) + (lane & 7) * 16;
-        v4u w0[kWideInDepth], w1[kWideInDepth];
-        auto fetch_in = [&](int j, int n0, int st) {          // clamped, not skipped: loads under a condition cannot be counted
-            const uint8_t* wr = w_in + static_cast<size_t>(c0 + min(n0, cw - 16)) * H + min(st, in_steps - 1) * 128;
-            w0[j] = *reinterpret_cast<const v4u*>(wr + in_lane);
-            w1[j] = *reinterpret_cast<const v4u*>(wr + static_cast<size_t>(8) * H + in_lane);
-        };
         // row r's 16-byte piece c sits at slot c ^ (r / 2): rows 0-7 of one k-group and 8-15 of the next fill 256 bytes each
         uint8_t* in_put = turn + (lane >> 3) * 128;
         const int in_put0 = ((lane & 7) ^ (lane >> 4)) << 4, in_put1 = ((lane & 7) ^ (4 + (lane >> 4))) << 4;
         const uint8_t* in_get = turn + t * 128;
         const int in_get0 = ((2 * g) ^ (t >> 1)) << 4, in_get1 = ((2 * g + 1) ^ (t >> 1)) << 4;
-#pragma unroll
-        for (int j = 0; j < kWideInDepth; ++j) fetch_in(j, wave * 16, j);
+        // No step is skipped, so that the compiler can count the fetches in flight and wait for the two it turns: with a branch around the
+        // padded ones it waited for all of them at the head of the loop.
         for (int n0 = wave * 16; n0 < cw; n0 += kWaves * 16) {
             v4f a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = {0.0f, 0.0f, 0.0f, 0.0f};
             const uint8_t* hr0 = sh_hidden + t * hs + wide_hidden_at(32 * g);
@@ -1023,26 +1045,29 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
                     turned();
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        *reinterpret_cast<v4u*>(in_put + q * 2048 + in_put0) = w0[j + q];
-                        *reinterpret_cast<v4u*>(in_put + q * 2048 + 1024 + in_put1) = w1[j + q];
-                        fetch_in(j + q, last ? n0 + kWaves * 16 : n0, last ? j + q : s0 + j + q + kWideInDepth);
+                        *reinterpret_cast<v4u*>(in_put + q * 2048 + in_put0) = wr[2 * (j + q)];
+                        *reinterpret_cast<v4u*>(in_put + q * 2048 + 1024 + in_put1) = wr[2 * (j + q) + 1];
+                        const int x = j + q;
+                        fetch_pair(x, last && n0 + kWaves * 16 >= cw, in_at(c0, cw, last ? n0 + kWaves * 16 : n0, last ? x : s0 + x + kWideInDepth),
+                                   out_at(c0, cw, x % 2 * 2, x / 2), out_at(c0, cw, x % 2 * 2 + 1, x / 2));
                     }
                     turned();
+                    v8i w[2], x[2], y[2];
+                    auto pair = [](const uint4& lo, const uint4& hi) {
+                        return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+                    };
 #pragma unroll
                     for (int q = 0; q < 2; ++q) {
-                        const int st = s0 + j + q;
-                        if (st < in_steps) {
-                            const uint4 u0 = *reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get0);
-                            const uint4 u1 = *reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get1);
-                            const v8i a = {(int)u0.x, (int)u0.y, (int)u0.z, (int)u0.w, (int)u1.x, (int)u1.y, (int)u1.z, (int)u1.w};
-                            const int at = wide_hidden_at(st * 128);
-                            const uint4 x0 = *reinterpret_cast<const uint4*>(hr0 + at), x1 = *reinterpret_cast<const uint4*>(hr0 + at + 16);
-                            const uint4 y0 = *reinterpret_cast<const uint4*>(hr1 + at), y1 = *reinterpret_cast<const uint4*>(hr1 + at + 16);
-                            const v8i b0 = {(int)x0.x, (int)x0.y, (int)x0.z, (int)x0.w, (int)x1.x, (int)x1.y, (int)x1.z, (int)x1.w};
-                            const v8i b1 = {(int)y0.x, (int)y0.y, (int)y0.z, (int)y0.w, (int)y1.x, (int)y1.y, (int)y1.z, (int)y1.w};
-                            a0 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b0, a0, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
-                            a1 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b1, a1, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
-                        }
+                        const int at = wide_hidden_at((s0 + j + q) * 128);
+                        w[q] = pair(*reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get0), *reinterpret_cast<const uint4*>(in_get + q * 2048 + in_get1));
+                        x[q] = pair(*reinterpret_cast<const uint4*>(hr0 + at), *reinterpret_cast<const uint4*>(hr0 + at + 16));
+                        y[q] = pair(*reinterpret_cast<const uint4*>(hr1 + at), *reinterpret_cast<const uint4*>(hr1 + at + 16));
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        a0 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[q], x[q], a0, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
+                        a1 = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(w[q], y[q], a1, 0, E5M2 ? 1 : 0, 0, 0, 0, 0);
                     }
                 }
             }
@@ -1062,19 +1087,14 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
             }
         }
         // ---- this chunk's share of fc_out ----
-        // Four blocks at a time (an activation read feeds eight MFMAs).  A step is 64 k: 64 bytes of each of a block's 16 weight
-        // rows, fetched 4 lanes to a row and turned in LDS; one stream of fetches over the groups of blocks, two steps ahead.
+        // Four blocks at a time (an activation read feeds eight MFMAs), 64 k to a step, turned in LDS.
         const int steps = cw / 64, out_pad = (steps + 1) & ~1;
-        const uint32_t out_lane = static_cast<uint32_t>(lane >> 2) * static_cast<uint32_t>(Ie) + (lane & 3) * 16;
-        // the weights of this wavefront's block blk (past the last one: that one again; those sums are not used)
-        auto block = [&](int blk) { return w_out + c0 + static_cast<size_t>((min(blk, nblk - 1) * kWaves + wave) * 16) * Ie; };
-        v4u w[2][kWideGroup];
-        auto fetch_out = [&](int j, int blk, int st) {
+        if (wave * 16 >= cw) {                      // a wavefront that had no block of fc_in has not asked for these yet
 #pragma unroll
-            for (int i = 0; i < kWideGroup; ++i) w[j][i] = *reinterpret_cast<const v4u*>(block(blk + i) + min(st, steps - 1) * 64 + out_lane);
-        };
-        fetch_out(0, 0, 0);
-        fetch_out(1, 0, 1);
+            for (int x = 0; x < kWideInDepth; ++x)
+                fetch_pair(x, true, 0, out_at(c0, cw, x % 2 * 2, x / 2), out_at(c0, cw, x % 2 * 2 + 1, x / 2));
+        }
+        const int c1 = min(c0 + chunk, Ie - 64), cw1 = min(chunk, Ie - c1);        // the next chunk (past the last one: something that is there)
         __syncthreads();                            // the activations are complete
         // row r's piece c sits at slot c ^ (r / 4), for the same reason as above
         uint8_t* out_put = turn + (lane >> 2) * 64 + (((lane & 3) ^ (lane >> 4)) << 4);
@@ -1092,8 +1112,12 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
                     for (int j = 0; j < 2; ++j) {
                         turned();
 #pragma unroll
-                        for (int i = 0; i < kWideGroup; ++i) *reinterpret_cast<v4u*>(out_put + i * 1024) = w[j][i];
-                        fetch_out(j, last ? bg + kWideGroup : bg, last ? j : s0 + j + 2);
+                        for (int i = 0; i < kWideGroup; ++i) *reinterpret_cast<v4u*>(out_put + i * 1024) = wr[kWideGroup * j + i];
+#pragma unroll
+                        for (int x = 2 * j; x < 2 * j + 2; ++x) {
+                            const int blk = (last ? bg + kWideGroup : bg) + x % 2 * 2, st = last ? j : s0 + j + 2;
+                            fetch_pair(x, !(last && bg + kWideGroup >= nblk), in_at(c1, cw1, wave * 16, x), out_at(c0, cw, blk, st), out_at(c0, cw, blk + 1, st));
+                        }
                         turned();
                         if (s0 + j < steps) {
                             uint4 x[kWideGroup];
@@ -1695,7 +1719,8 @@ int cf::expert_forward_fp8_one_kernel(const void* d_hidden, const float* d_fcin_
                          (reinterpret_cast<uintptr_t>(d_mixed) & 7u) == 0;
     // 32 rows per workgroup where the output blocks fit a wavefront's registers; Ie is walked in the fewest equal chunks whose
     // activations fit the LDS beside the hidden rows
-    if (mfma_ok && H <= 128 * kWideBlocks) {
+    // (its weight offsets are 32-bit)
+    if (mfma_ok && H <= 128 * kWideBlocks && static_cast<long long>(H) * Ie < (1ll << 31)) {
         const int room = 160 * 1024 - kWideRows * wide_hidden_stride(H) - (kMfmaThreads / 64) * kWideTurn;
         const int most = (room / (4 * kWideRows) - 8) / 256 * 256, passes = (Ie + most - 1) / most;     // >= 256 at H = 2048
         const int chunk = ((Ie + passes - 1) / passes + 63) / 64 * 64;
