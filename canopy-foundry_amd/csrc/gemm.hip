@@ -2162,9 +2162,10 @@ float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.
-// shape: of the small-tile kernel; kWideBlocks marks the 256 x 256-tile one of the persistent block-scaled kernels.
+// shape: of the small-tile kernel; kWideBlocks marks the 256 x 256-tile one of the persistent block-scaled kernels, kWideAccum the one of the
+// kernels that accumulate over any K.
 struct Route { int kernel, shape; };
-constexpr int kWideBlocks = 1;
+constexpr int kWideBlocks = 1, kWideAccum = 1;
 Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_naive) {
     if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
         (epi == EPI_SILU_GATE && !aligned16(p.B2)))
@@ -2185,6 +2186,10 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
     if (duo) {
         const float d = duo_estimate_us(p, epi);
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
+    }
+    if (accum_wide_ok(p, fmt, epi, scale_mode)) {
+        const float d = accum_wide_estimate_us(p);
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, kWideAccum}; }
     }
     if (half && p.M > 128) {          // (with fewer rows half of the tile or more is padding)
         const bool over_duo = best.kernel == CF_GEMM_KERNEL_DUO;
@@ -2222,6 +2227,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         return launch_status();
     }
     if (route.kernel == CF_GEMM_KERNEL_SMALL) return gemm_nt_direct(p, fmt, epi, scale_mode, route.shape, st);
+    if (route.kernel == CF_GEMM_KERNEL_DUO && route.shape == kWideAccum) return gemm_nt_accum_wide(p, st);
     if (route.kernel == CF_GEMM_KERNEL_DUO) return gemm_nt_duo(p, fmt, epi, scale_mode, st);
     if (route.kernel == CF_GEMM_KERNEL_HALF) return gemm_nt_half(p, fmt, epi, scale_mode, st);
     if (scale_mode == SCALE_BLOCK) {

@@ -8,7 +8,8 @@
 //   - too few 256 x 256 tiles to fill the chip (4096 columns, 1000 rows, K 4096: 38 -> 19 us; 2048 rows, K 14336: 123 -> 98);
 //   - the accumulating forms over a short K: while one workgroup of a CU adds its tile to what C holds, the other multiplies.
 //     With one workgroup per CU all of them multiply and all of them wait for memory in turn.  14336 x 4096 fp32 (470 MB read
-//     and written, 85 us): K 1024 126 -> 108 us, K 2048 164 -> 147, K 2000 262 (register-staged kernel) -> 188, K 4096 240 -> 250.
+//     and written, 85 us): K 1024 126 -> 108 us, K 2048 164 -> 147, K 2000 262 (register-staged kernel) -> 188 (164 in gemm_accum.hip, which has
+//     the longer K that are no multiple of 128), K 4096 240 -> 250.
 // Operand rows and bytes of K beyond the operands are read as zeros (buffer copies with the operand's size in their
 // descriptor), so K only has to be a multiple of 16.
 #include "gemm_common.hpp"

@@ -306,7 +306,8 @@ int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const 
 #define CF_GEMM_KERNEL_STAGED 1    /* 256 x 256 (block scales: 128 x 256) tiles through registers and LDS */
 #define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: 128 x 256 or 256 x 256 tiles, kernels of their own) */
 #define CF_GEMM_KERNEL_RING16 3    /* the same on 16 x 16 x 128 MFMAs */
-#define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU */
+#define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU (+= into fp32 over a K that is no multiple of 128: those or 256 x 256 tiles,
+                                      a kernel of its own) */
 #define CF_GEMM_KERNEL_HALF   5    /* persistent, 256 x 128 or 128 x 256 tiles, one workgroup per CU */
 #define CF_GEMM_KERNEL_SMALL  16   /* + tile shape (see CF_GEMM_FLAG_SMALL): K split over a workgroup's wavefronts */
 
