@@ -277,7 +277,7 @@ bool accum_wide_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
 
 // Microseconds: per round of tiles 1.42 a K-tile and, for C, 21; 26 where a few whole rounds leave no workgroup to start later, 34 where there is
 // one round and all go to C at once, 39 where the rows of C do not begin at lines.  Beside the two workgroups per CU (them, this), a line
-// on each side: 14336 x 4096, K 1040 123 and 120 with C at hand (a step's is not), K 1488 152 and 144; 14336 x 4100, K 1488 209 and 222, K 2000 241 and 237; 5632 x 2048 (one round,
+// on each side: 14336 x 4096, K 1040 123 and 120 alone, K 1488 152 and 144; 14336 x 4100, K 1488 209 and 222, K 2000 241 and 237; 5632 x 2048 (one round,
 // part filled), K 4016 70.7 and 66.4 alone but no difference within a step, K 8176 121 and 110; 5120 x 4096 (a quarter of the second round
 // filled), K 8176 198 and 210.
 float accum_wide_estimate_us(const GemmArgs& p) {
