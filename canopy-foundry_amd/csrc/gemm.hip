@@ -2162,10 +2162,10 @@ float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.
-// shape: of the small-tile kernel; kWideBlocks marks the 256 x 256-tile one of the persistent block-scaled kernels, kWideAccum the one of the
-// kernels that accumulate over any K.
+// shape: of the small-tile kernel; kWideBlocks and kSlimBlocks mark the 256 x 256- and the 128 x 128-tile one of the persistent block-scaled
+// kernels, kWideAccum the 256 x 256-tile one of those that accumulate over any K.
 struct Route { int kernel, shape; };
-constexpr int kWideBlocks = 1, kWideAccum = 1;
+constexpr int kWideBlocks = 1, kSlimBlocks = 2, kWideAccum = 1;
 Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_naive) {
     if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
         (epi == EPI_SILU_GATE && !aligned16(p.B2)))
@@ -2182,6 +2182,10 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
     if (scale_mode == SCALE_BLOCK && block_wide_ok(p)) {
         const float d = block_wide_estimate_us(p);
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_RING, kWideBlocks}; }
+    }
+    if (scale_mode == SCALE_BLOCK && block_slim_ok(p)) {
+        const float d = block_slim_estimate_us(p);
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_RING, kSlimBlocks}; }
     }
     if (duo) {
         const float d = duo_estimate_us(p, epi);
@@ -2239,6 +2243,7 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         });
         if (attr_err != hipSuccess) return static_cast<int>(attr_err);
         if (route.kernel == CF_GEMM_KERNEL_RING && route.shape == kWideBlocks) return gemm_nt_block_wide(p, st);
+        if (route.kernel == CF_GEMM_KERNEL_RING && route.shape == kSlimBlocks) return gemm_nt_block_slim(p, st);
         p.tiles_m = (p.M + BSM - 1) / BSM;
         p.tiles_n = (p.N + BN - 1) / BN;
         if (route.kernel == CF_GEMM_KERNEL_RING) {

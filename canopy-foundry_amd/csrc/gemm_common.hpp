@@ -114,6 +114,9 @@ int gemm_nt_duo(GemmArgs p, int fmt, int epi, int scale_mode, hipStream_t st);
 bool block_wide_ok(const GemmArgs& p);
 float block_wide_estimate_us(const GemmArgs& p);
 int gemm_nt_block_wide(GemmArgs p, hipStream_t st);
+bool block_slim_ok(const GemmArgs& p);
+float block_slim_estimate_us(const GemmArgs& p);
+int gemm_nt_block_slim(GemmArgs p, hipStream_t st);
 // gemm_accum.hip
 bool accum_wide_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
 float accum_wide_estimate_us(const GemmArgs& p);

@@ -304,7 +304,7 @@ int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const 
                               int ldc_dw, cf_stream_t stream);
 #define CF_GEMM_KERNEL_NAIVE  0    /* one lane per output: K no multiple of 16, or asked for */
 #define CF_GEMM_KERNEL_STAGED 1    /* 256 x 256 (block scales: 128 x 256) tiles through registers and LDS */
-#define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: 128 x 256 or 256 x 256 tiles, kernels of their own) */
+#define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: 128 x 128, 128 x 256 or 256 x 256 tiles, kernels of their own) */
 #define CF_GEMM_KERNEL_RING16 3    /* the same on 16 x 16 x 128 MFMAs */
 #define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU (+= into fp32 over a K that is no multiple of 128: those or 256 x 256 tiles,
                                       a kernel of its own) */

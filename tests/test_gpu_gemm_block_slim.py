@@ -1,0 +1,40 @@
+"""The block-scaled GEMM on 128 x 128 tiles: the fewest K-tiles it takes and counts after them that leave each of its four stages last, rows that end
+inside a tile, a wavefront's part and a 16-row block, one tile per workgroup and several, an odd number of column blocks, rows of C beyond N."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle_lib as orc
+from gpu_util import bf16_bits, case, dev_arr, stream
+
+pytestmark = pytest.mark.gpu
+BLOCK, RING = 2, 2
+
+
+# one round of these tiles that is less than one of 128 x 256, or columns that those do not take
+@pytest.mark.parametrize("M,N,K,pad", [
+    (257, 7168, 512, 0), (300, 7168, 640, 8), (1000, 4096, 768, 0), (1900, 2048, 1024, 0), (513, 4096, 1152, 0),
+    (1153, 2176, 1536, 8),          # 17 column blocks
+    (600, 8576, 2048, 0),           # 335 tiles: some workgroups take two, others one
+    (2049, 4224, 2048, 0),          # 561 tiles, two or three a workgroup; one row in the last row tile
+])
+def test_block_scales_on_small_tiles(cf, dev, M, N, K, pad):
+    case(f"block-scaled gemm, 128 x 128 tiles {M}x{N}x{K} ldc N + {pad}")
+    kernel = ctypes.c_int(-1)
+    cf.cf_fp8_gemm_route(M, N, K, 0, 0, BLOCK, 0, N + pad, 0, ctypes.byref(kernel))
+    assert kernel.value == RING
+    rng = np.random.default_rng(M + N + K)
+    A = orc.quantize_e4m3(orc.bf16_from_f32(rng.standard_normal((M, K)).astype(np.float32)), np.float32(100.0))
+    B = orc.quantize_e4m3(orc.bf16_from_f32(rng.standard_normal((N, K)).astype(np.float32)), np.float32(100.0))
+    sa = (2.0 ** rng.uniform(-8, 2, (M, K // 128))).astype(np.float32)
+    sb = (2.0 ** rng.uniform(-8, 2, (N // 128, K // 128))).astype(np.float32)
+    C = torch.full((M, N + pad), -7.0, dtype=torch.bfloat16, device=dev)
+    cf.cf_fp8_gemm_nt_bf16_ex(M, N, K, dev_arr(A, dev), K, 0, dev_arr(sa, dev), dev_arr(B, dev), K, dev_arr(sb, dev), BLOCK, 0, None, None,
+                              None, C, N + pad, 0, stream())
+    got = orc.bf16_to_f32(bf16_bits(C))
+    assert (got[:, N:] == -7.0).all()
+    rows = np.unique(np.concatenate([np.arange(min(M, 48)), np.arange(max(M - 48, 0), M), rng.integers(0, M, 32)]))
+    ref, absdot = orc.gemm_nt_ref(A[rows], B, sa[rows], sb, scale_mode=BLOCK)
+    orc.assert_gemm_close(got[rows, :N], ref, absdot, what=f"slim block {M}x{N}x{K}")
