@@ -2517,7 +2517,7 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
     p.b_expert_stride = static_cast<long long>(N) * K;
     p.sb_expert_stride = scale_mode == SCALE_ROWCOL ? N : 0;
     const int out_bn = epilogue == EPI_SILU_GATE ? BN / 2 : BN;
-    p.tiles_m = max_row_tiles;
+    p.tiles_m = p.map_entries = max_row_tiles;
     p.tiles_n = (N + out_bn - 1) / out_bn;
     // Few rows per expert: the small-tile kernel, which walks an expert's rows 16 mb at a time, where its estimate is lower.
     // It is sized for half as many rows again as the bound's average, so that most experts take one pass over their weights;
@@ -2531,6 +2531,20 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
         const int row_tiles = total_rows < num_experts ? total_rows : num_experts;
         if (direct < ring_estimate_us(row_tiles * BM, N, K, BM, out_bn, 0.95f, 6.0f)) {
             const int rc = grouped_gemm_nt_direct(p, a_is_e5m2, epilogue, shape, st);
+            if (rc != CF_ERR_UNSUPPORTED) return rc;
+        }
+    }
+    // More rows, up to a ring tile's, where few experts leave the ring kernel few tiles: its largest pass of 64 rows, with workgroups enough that
+    // all passes of an entry run side by side, wherever the rows lie.  The routed layer around 8 experts of 1024 x 2048, two a token: 200 tokens
+    // (50 rows each) 72 -> 45 us, 256 72 -> 50, 600 74 -> 63, 1000 77 -> 71.  64 experts of 2048 x 1408 fill the chip with ring tiles and keep them
+    // (600 tokens 193, with passes 221).
+    else if (total_rows <= static_cast<long long>(BM) * num_experts) {
+        int shape = 0;
+        const float direct = grouped_direct_many_estimate_us(total_rows, N, K, num_experts, epilogue == EPI_SILU_GATE, &shape);
+        if (direct < ring_estimate_us(num_experts * BM, N, K, BM, out_bn, 0.95f, 6.0f)) {
+            GemmArgs q = p;
+            q.tiles_m *= std::min(4, (total_rows + 64 * num_experts - 1) / (64 * num_experts) + 1);
+            const int rc = grouped_gemm_nt_direct(q, a_is_e5m2, epilogue, shape, st);
             if (rc != CF_ERR_UNSUPPORTED) return rc;
         }
     }

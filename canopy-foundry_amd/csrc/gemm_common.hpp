@@ -34,6 +34,7 @@ struct GemmArgs {
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
     // grouped (per-expert) form, ring and small-tile kernels; all null / 0 for a dense GEMM
     const int* tile_map;         // [0] = number of row tiles, then kMapWords words per row tile: expert, its first row, end row, first tile, tiles
+    int map_entries;             // small-tile kernel: row tiles the table has room for (tiles_m may be several times that: workgroups that share an entry)
     const int* a_row_index;      // compact row r reads A row (and its descale) a_row_index[r]; null = r
     int a_rows;                  // rows of the A buffer (= M without a row index)
     long long b_expert_stride;   // bytes between the weight matrices of consecutive experts
@@ -100,6 +101,7 @@ bool direct_ok(const GemmArgs& p, int fmt, int epi, int scale_mode);
 bool direct_takes(const GemmArgs& p, int epi, int scale_mode, int shape);
 float direct_estimate_us(const GemmArgs& p, int epi, int scale_mode, int* shape);
 float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape);
+float grouped_direct_many_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape);
 int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st);
 int grouped_gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int shape, hipStream_t st);
 // gemm_half.hip: whether it takes a problem, its time, the launch

@@ -50,9 +50,9 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
         // A table entry is up to 256 rows of an expert, walked TM at a time.  Where the rows lie on few experts there are fewer entries
         // than workgroups to a column of tiles: those beyond the last entry take every second, third, ... pass of the entries
         // before.  (64 experts of 2 x 1408 x 2048, 1280 rows all on one: 53 us with its entries walked by a workgroup each.)
-        const int* e = p.tile_map + 1 + kMapWords * tm;            // the usual one, read beside the number of entries
+        const int* e = p.tile_map + 1 + kMapWords * min(tm, p.map_entries - 1);            // the usual one, read beside the number of entries
         int number = e[0], first = e[1], last = e[2], first_tile = e[3];
-        const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], p.tiles_m));
+        const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], min(p.map_entries, p.tiles_m)));
         if (entries <= 0) return;
         int entry = tm, part = 0, parts = tm + entries < p.tiles_m ? 2 : 1;
         if (tm >= entries || 2 * entries < p.tiles_m) {
@@ -456,6 +456,16 @@ float grouped_direct_estimate_us(int total_rows, int N, int K, int num_experts, 
         *shape = kWideShape + i;
     }
     return best;
+}
+
+// The same in passes of 64 rows that run side by side: half a pass an expert more than the rows fill.
+float grouped_direct_many_estimate_us(int total_rows, int N, int K, int num_experts, bool gate, int* shape) {
+    *shape = gate ? 2 : 3;
+    const Shape& sh = gate ? kGate[2] : kPlain[3];
+    const int tn = 16 * sh.nt / (gate ? 2 : 1);
+    const float passes = static_cast<float>(total_rows) / 64.0f + 0.5f * static_cast<float>(num_experts);
+    const float rounds = passes * static_cast<float>((N + tn - 1) / tn) / static_cast<float>(num_cus());
+    return (rounds < 1.0f ? 1.0f : rounds) * (sh.fixed + static_cast<float>(K) * 16.0f * static_cast<float>(sh.mb + sh.nt) / 93e3f);
 }
 
 int gemm_nt_direct(const GemmArgs& p, int fmt, int epi, int scale_mode, int shape, hipStream_t st) {
