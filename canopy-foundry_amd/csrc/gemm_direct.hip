@@ -52,7 +52,7 @@ void k_gemm_nt_direct(const GemmArgs p, const int rowcol, const int bias, const 
         // before.  (64 experts of 2 x 1408 x 2048, 1280 rows all on one: 53 us with its entries walked by a workgroup each.)
         const int* e = p.tile_map + 1 + kMapWords * min(tm, p.map_entries - 1);            // the usual one, read beside the number of entries
         int number = e[0], first = e[1], last = e[2], first_tile = e[3];
-        const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], min(p.map_entries, p.tiles_m)));
+        const int entries = __builtin_amdgcn_readfirstlane(min(p.tile_map[0], p.map_entries));
         if (entries <= 0) return;
         int entry = tm, part = 0, parts = tm + entries < p.tiles_m ? 2 : 1;
         if (tm >= entries || 2 * entries < p.tiles_m) {
