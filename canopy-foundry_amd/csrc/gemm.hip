@@ -2162,10 +2162,9 @@ float persistent_estimate_us(const GemmArgs& p, int epi, int scale_mode) {
 }
 
 // Which kernel a dense problem runs on: the one asked for by a flag where it applies, otherwise the one with the lowest estimate.
-// shape: of the small-tile kernel; kWideBlocks and kSlimBlocks mark the 256 x 256- and the 128 x 128-tile one of the persistent block-scaled
-// kernels, kWideAccum the 256 x 256-tile one of those that accumulate over any K.
+// shape: of the small-tile kernel.
 struct Route { int kernel, shape; };
-constexpr int kWideBlocks = 1, kSlimBlocks = 2, kWideAccum = 1;
+int tile_edge(int flags) { return flags & CF_GEMM_FLAG_WIDE ? 256 : flags & CF_GEMM_FLAG_SLIM ? 128 : 0; }
 Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_naive) {
     if (force_naive || p.K <= 0 || p.K % 16 != 0 || p.lda % 16 != 0 || p.ldb % 16 != 0 || !aligned16(p.A) || !aligned16(p.B) ||
         (epi == EPI_SILU_GATE && !aligned16(p.B2)))
@@ -2177,23 +2176,28 @@ Route gemm_route(const GemmArgs& p, int fmt, int epi, int scale_mode, int force_
     if (p.small && small && direct_takes(p, epi, scale_mode, p.small - 1)) return {CF_GEMM_KERNEL_SMALL, p.small - 1};
     if (p.duo && duo) return {CF_GEMM_KERNEL_DUO, 0};
     if (p.half && half) return {CF_GEMM_KERNEL_HALF, 0};
-    if (p.small || p.duo || p.half || p.ring || p.force_staged) return best;
+    const bool block_wide = scale_mode == SCALE_BLOCK && block_wide_ok(p), block_slim = scale_mode == SCALE_BLOCK && block_slim_ok(p);
+    const bool accum_wide = accum_wide_ok(p, fmt, epi, scale_mode);
+    if (p.edge == 256 && block_wide) return {CF_GEMM_KERNEL_BLOCK_WIDE, 0};
+    if (p.edge == 256 && accum_wide) return {CF_GEMM_KERNEL_ACCUM_WIDE, 0};
+    if (p.edge == 128 && block_slim) return {CF_GEMM_KERNEL_BLOCK_SLIM, 0};
+    if (p.small || p.duo || p.half || p.edge || p.ring || p.force_staged) return best;
     float t = persistent_estimate_us(p, epi, scale_mode);
-    if (scale_mode == SCALE_BLOCK && block_wide_ok(p)) {
+    if (block_wide) {
         const float d = block_wide_estimate_us(p);
-        if (d < t) { t = d; best = {CF_GEMM_KERNEL_RING, kWideBlocks}; }
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_BLOCK_WIDE, 0}; }
     }
-    if (scale_mode == SCALE_BLOCK && block_slim_ok(p)) {
+    if (block_slim) {
         const float d = block_slim_estimate_us(p);
-        if (d < t) { t = d; best = {CF_GEMM_KERNEL_RING, kSlimBlocks}; }
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_BLOCK_SLIM, 0}; }
     }
     if (duo) {
         const float d = duo_estimate_us(p, epi);
         if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, 0}; }
     }
-    if (accum_wide_ok(p, fmt, epi, scale_mode)) {
+    if (accum_wide) {
         const float d = accum_wide_estimate_us(p);
-        if (d < t) { t = d; best = {CF_GEMM_KERNEL_DUO, kWideAccum}; }
+        if (d < t) { t = d; best = {CF_GEMM_KERNEL_ACCUM_WIDE, 0}; }
     }
     if (half && p.M > 128) {          // (with fewer rows half of the tile or more is padding)
         const bool over_duo = best.kernel == CF_GEMM_KERNEL_DUO;
@@ -2231,7 +2235,9 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
         return launch_status();
     }
     if (route.kernel == CF_GEMM_KERNEL_SMALL) return gemm_nt_direct(p, fmt, epi, scale_mode, route.shape, st);
-    if (route.kernel == CF_GEMM_KERNEL_DUO && route.shape == kWideAccum) return gemm_nt_accum_wide(p, st);
+    if (route.kernel == CF_GEMM_KERNEL_ACCUM_WIDE) return gemm_nt_accum_wide(p, st);
+    if (route.kernel == CF_GEMM_KERNEL_BLOCK_WIDE) return gemm_nt_block_wide(p, st);
+    if (route.kernel == CF_GEMM_KERNEL_BLOCK_SLIM) return gemm_nt_block_slim(p, st);
     if (route.kernel == CF_GEMM_KERNEL_DUO) return gemm_nt_duo(p, fmt, epi, scale_mode, st);
     if (route.kernel == CF_GEMM_KERNEL_HALF) return gemm_nt_half(p, fmt, epi, scale_mode, st);
     if (scale_mode == SCALE_BLOCK) {
@@ -2242,8 +2248,6 @@ int gemm_nt(GemmArgs p, int fmt, int epi, int scale_mode, int force_naive, cf_st
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kBlkLds);
         });
         if (attr_err != hipSuccess) return static_cast<int>(attr_err);
-        if (route.kernel == CF_GEMM_KERNEL_RING && route.shape == kWideBlocks) return gemm_nt_block_wide(p, st);
-        if (route.kernel == CF_GEMM_KERNEL_RING && route.shape == kSlimBlocks) return gemm_nt_block_slim(p, st);
         p.tiles_m = (p.M + BSM - 1) / BSM;
         p.tiles_n = (p.N + BN - 1) / BN;
         if (route.kernel == CF_GEMM_KERNEL_RING) {
@@ -2317,6 +2321,7 @@ int cf_fp8_gemm_nt_bf16_ex(int M, int N, int K, const void* A, int lda, int a_is
     p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
     p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
     p.half = (flags & CF_GEMM_FLAG_HALF) != 0;
+    p.edge = tile_edge(flags);
     return gemm_nt(p, a_is_e5m2 ? 1 : 0, epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE, stream);
 }
 
@@ -2336,8 +2341,9 @@ int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int sca
     p.ring = (flags & (CF_GEMM_FLAG_RING | CF_GEMM_FLAG_MFMA32)) != 0;
     p.small = (flags & CF_GEMM_FLAG_SMALL) ? 1 + ((flags >> 8) & 15) : 0;
     p.half = (flags & CF_GEMM_FLAG_HALF) != 0;
+    p.edge = tile_edge(flags);
     const Route r = gemm_route(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), epilogue, scale_mode, flags & CF_GEMM_FLAG_NAIVE);
-    *kernel = r.kernel == CF_GEMM_KERNEL_SMALL ? r.kernel + r.shape : r.kernel;
+    *kernel = r.kernel + r.shape;
     return CF_OK;
 }
 
@@ -2643,6 +2649,7 @@ int accum_ex(int M, int N, int K, const void* A, int lda, int a_is_e5m2, const f
     p.force_staged = (flags & CF_GEMM_FLAG_STAGED) != 0;
     p.duo = (flags & CF_GEMM_FLAG_DUO) ? ((flags & CF_GEMM_FLAG_DUO_IN_STEP) ? 2 : 1) : 0;
     p.ring = (flags & CF_GEMM_FLAG_RING) != 0;
+    p.edge = tile_edge(flags);
     return gemm_nt(p, (a_is_e5m2 ? 1 : 0) | (b_is_e5m2 ? 2 : 0), Cf ? EPI_ACCUM_F32 : EPI_ACCUM_BF16, SCALE_TENSOR,
                    flags & CF_GEMM_FLAG_NAIVE, stream);
 }

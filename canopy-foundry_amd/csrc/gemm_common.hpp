@@ -32,6 +32,7 @@ struct GemmArgs {
     int half;                    // take the half-tile kernel where it applies
     int ring;                    // keep the persistent kernels where a smaller-tile kernel's estimate is lower
     int mfma32;                  // keep k_gemm_nt_ring (the 32 x 32 x 64 MFMA shape) where k_gemm_nt_ring16 would apply
+    int edge;                    // 256, 128: take the kernel of that tile edge of gemm_block.hip or gemm_accum.hip where it applies
     // grouped (per-expert) form, ring and small-tile kernels; all null / 0 for a dense GEMM
     const int* tile_map;         // [0] = number of row tiles, then kMapWords words per row tile: expert, its first row, end row, first tile, tiles
     int map_entries;             // small-tile kernel: row tiles the table has room for (tiles_m may be several times that: workgroups that share an entry)

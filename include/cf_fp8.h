@@ -271,6 +271,10 @@ int cf_cross_entropy_fwd_bwd_chunk_quant_e5m2(const uint16_t* d_logits, const in
 
 #define CF_GEMM_FLAG_HALF 128  /* take the kernel of 256 x 128 or 128 x 256 tiles (SiLU gate: 128 x 128 outputs) where it applies:
                                   plain, bias and SiLU-gate epilogues, otherwise as CF_GEMM_FLAG_DUO (gate: N a multiple of 8) */
+#define CF_GEMM_FLAG_WIDE 4096 /* take the kernel of 256 x 256 tiles of its own where it applies: block scales, K of 3 to 256 times 128, N a
+                                  multiple of 256; E4M3 x E5M2 accumulating into fp32 over a K above 256 that is a multiple of 16 and not
+                                  of 128, N and ldc multiples of 4 */
+#define CF_GEMM_FLAG_SLIM 8192 /* take the kernel of 128 x 128 tiles and block scales where it applies: K of 4 to 256 times 128, N a multiple of 128 */
 
 /* lt_gemm_fp8_nt, static at src/trainer.cu:4498-4534 (plan lookup :4402-4496).
  * C[M,N] bf16 (row stride ldc) = (A[M,K] fp8, row stride lda, E4M3 or E5M2) .
@@ -304,11 +308,13 @@ int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const 
                               int ldc_dw, cf_stream_t stream);
 #define CF_GEMM_KERNEL_NAIVE  0    /* one lane per output: K no multiple of 16, or asked for */
 #define CF_GEMM_KERNEL_STAGED 1    /* 256 x 256 (block scales: 128 x 256) tiles through registers and LDS */
-#define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs (block scales: 128 x 128, 128 x 256 or 256 x 256 tiles, kernels of their own) */
+#define CF_GEMM_KERNEL_RING   2    /* persistent, 256 x 256 (128 x 256) tiles, 32 x 32 x 64 MFMAs */
 #define CF_GEMM_KERNEL_RING16 3    /* the same on 16 x 16 x 128 MFMAs */
-#define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU (+= into fp32 over a K that is no multiple of 128: those or 256 x 256 tiles,
-                                      a kernel of its own) */
+#define CF_GEMM_KERNEL_DUO    4    /* persistent, 128 x 128 tiles, two workgroups per CU */
 #define CF_GEMM_KERNEL_HALF   5    /* persistent, 256 x 128 or 128 x 256 tiles, one workgroup per CU */
+#define CF_GEMM_KERNEL_BLOCK_WIDE 6  /* block scales: persistent, 256 x 256 tiles, 16 x 16 x 128 MFMAs */
+#define CF_GEMM_KERNEL_BLOCK_SLIM 7  /* block scales: persistent, 128 x 128 tiles, 16 x 16 x 128 MFMAs */
+#define CF_GEMM_KERNEL_ACCUM_WIDE 8  /* += into fp32 over a K that is no multiple of 128: persistent, 256 x 256 tiles */
 #define CF_GEMM_KERNEL_SMALL  16   /* + tile shape (see CF_GEMM_FLAG_SMALL): K split over a workgroup's wavefronts */
 
 /* Which kernel (CF_GEMM_KERNEL_*) the dense GEMM entry points run a problem on (16-byte aligned operands, descales and
@@ -318,7 +324,7 @@ int cf_fp8_gemm_tn_accum_bf16(int M, int N, int K, const void* d_Xt_e4m3, const 
 int cf_fp8_gemm_route(int M, int N, int K, int a_is_e5m2, int b_is_e5m2, int scale_mode, int epilogue, int ldc,
                       int flags, int* kernel);
 /* The accumulate GEMMs of src/trainer.cu:4596-4627 and :4670-4691 with free operand formats and row strides, and a
- * kernel of the caller's choice: CF_GEMM_FLAG_NAIVE, _STAGED, _DUO (E4M3 x E5M2, N and ldc multiples of 4), _RING; used
+ * kernel of the caller's choice: CF_GEMM_FLAG_NAIVE, _STAGED, _DUO (E4M3 x E5M2, N and ldc multiples of 4), _RING, _WIDE (fp32); used
  * by the tests and for fp32 inspection of the accumulators. */
 int cf_fp8_gemm_nt_accum_f32_ex(int M, int N, int K, const void* d_A, int lda, int a_is_e5m2,
                                 const float* d_a_descale, const void* d_B, int ldb, int b_is_e5m2,

@@ -4,10 +4,10 @@ import ctypes
 
 import pytest
 
-NAIVE, STAGED, RING, RING16, DUO, HALF, SMALL = 0, 1, 2, 3, 4, 5, 16
+NAIVE, STAGED, RING, RING16, DUO, HALF, BLOCK_WIDE, BLOCK_SLIM, ACCUM_WIDE, SMALL = 0, 1, 2, 3, 4, 5, 6, 7, 8, 16
 TENSOR, ROW_COL, BLOCK = 0, 1, 2
 PLAIN, BIAS, GATE, ACCUM_F32, ACCUM_BF16 = range(5)
-F_NAIVE, F_STAGED, F_DUO, F_MFMA32, F_RING, F_SMALL, F_HALF = 1, 2, 4, 16, 32, 64, 128
+F_NAIVE, F_STAGED, F_DUO, F_MFMA32, F_RING, F_SMALL, F_HALF, F_WIDE, F_SLIM = 1, 2, 4, 16, 32, 64, 128, 4096, 8192
 
 
 def route(cf, M, N, K, mode=TENSOR, epi=PLAIN, flags=0, pad=0, a_e5m2=0):
@@ -25,7 +25,13 @@ def test_flags_name_kernels(cf):
     assert route(cf, 512, 512, 512, flags=F_DUO) == DUO == route(cf, 512, 512, 512, flags=F_DUO, epi=ACCUM_BF16)
     for shape in range(6):
         assert route(cf, 512, 512, 512, flags=F_SMALL | shape << 8) == SMALL + shape
+    assert route(cf, 512, 512, 512, flags=F_WIDE, mode=BLOCK) == BLOCK_WIDE and route(cf, 512, 640, 512, flags=F_SLIM, mode=BLOCK) == BLOCK_SLIM
+    assert route(cf, 512, 512, 528, flags=F_WIDE, epi=ACCUM_F32) == ACCUM_WIDE
+    assert route(cf, 14336, 4096, 2000, flags=F_DUO, epi=ACCUM_F32) == DUO and route(cf, 4096, 7168, 7168, flags=F_RING, mode=BLOCK) == RING
     # what a kernel does not take falls to the persistent or the staged one
+    assert route(cf, 512, 512, 256, flags=F_WIDE, mode=BLOCK) == STAGED == route(cf, 512, 640, 512, flags=F_WIDE, mode=BLOCK)
+    assert route(cf, 512, 512, 384, flags=F_SLIM, mode=BLOCK) == RING == route(cf, 512, 512, 512, flags=F_WIDE, epi=ACCUM_F32)
+    assert route(cf, 512, 512, 512, flags=F_WIDE) == RING16 == route(cf, 512, 512, 512, flags=F_SLIM)
     assert route(cf, 512, 516, 512, flags=F_DUO) == STAGED
     assert route(cf, 512, 512, 512, flags=F_SMALL | 4 << 8, epi=GATE) == RING16
     assert route(cf, 512, 512, 512, flags=F_SMALL, epi=ACCUM_F32) == RING
@@ -49,23 +55,29 @@ def test_estimates_ask_what_the_launch_asks(cf):
     (4096, 14336, 512, 4, ACCUM_F32, RING),          # 191, 222: rows of C that do not begin at a line
     (4100, 5636, 256, 0, ACCUM_F32, DUO),            # 116 (register-staged), 94
     (1024, 4096, 1024, 0, ACCUM_F32, DUO),           # 24.1, 13.5: 64 tiles
-    (14336, 4096, 2000, 0, ACCUM_F32, DUO),          # 262, 188: K no multiple of 128
+    (14336, 4096, 2000, 0, ACCUM_F32, ACCUM_WIDE),   # 262, 188 and, on 256 x 256 tiles, 164: K no multiple of 128
+    (14336, 4096, 512 + 16, 0, ACCUM_F32, DUO),      # few K-tiles
+    (14336, 4100, 1488, 0, ACCUM_F32, DUO),          # 209, 256 x 256 tiles 222: rows of C off the lines
+    (5120, 4096, 8176, 0, ACCUM_F32, DUO),           # 198, 210: a quarter of the second round filled
     (14336, 4096, 8192, 0, ACCUM_F32, RING),         # 389, 431
 ])
 def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
     assert route(cf, M, N, K, epi=epi, pad=pad) == kernel
 
 
-# times of the tile shapes 32x32, 64x32, 64x64 and of the persistent kernel (128 x 256 tiles)
+# times of the tile shapes 32x32, 64x32, 64x64 and of the persistent kernels (128 x 256 tiles, and the one named)
 @pytest.mark.parametrize("M,N,K,kernel", [
-    (3000, 512, 4096, (RING, SMALL + 3)),            # 33.9, 42.4, 28.7, 29.9
-    (3000, 512, 2048, (RING, SMALL + 3)),            # 19.1, 23.6, 18.0, 16.9
+    (3000, 512, 4096, (BLOCK_SLIM,)),                # 34.3, 42.7, 29.1, 36.9, 27.0
+    (3000, 512, 2048, (BLOCK_SLIM,)),                # 18.5, 22.7, 17.5, 16.3, 11.9
     (6000, 1000, 7168, (STAGED,)),                   # 197, 227, 137, 103 (register-staged)
     (4096, 1000, 2000, (STAGED,)),                   # 56.6, 70.0, 44.1, 35.6 (register-staged)
     (100, 1000, 4096, (SMALL + 1,)),                 # 16x16 8.3; 6.7, 8.9, 11.5, 55.5 (register-staged)
     (1024, 128, 7168, (SMALL + 1,)),                 # 16x16 12.5; 10.7, 15.5, 16.6, 97.4
     (1000, 512, 4096, (SMALL + 1, SMALL + 2)),       # 11.7, 12.1, 13.7, 28.6
-    (4096, 7168, 7168, (RING,)),
+    (4096, 7168, 7168, (BLOCK_WIDE,)),               # 210, 186
+    (2560, 7168, 7168, (RING,)),                     # 154, 256 x 256 tiles 169: 1.1 rounds of those
+    (512, 7168, 7168, (BLOCK_SLIM,)),                # with the quantize 59.7, 43.3
+    (700, 7168, 7168, (RING,)),                      # with the quantize 61.1, 128 x 128 tiles 70.7
 ])
 def test_block_scaled_kernel(cf, M, N, K, kernel):
     assert route(cf, M, N, K, mode=BLOCK) in kernel

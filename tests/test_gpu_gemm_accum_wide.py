@@ -11,10 +11,12 @@ import oracle_lib as orc
 from gpu_util import case, dev_arr, stream
 
 pytestmark = pytest.mark.gpu
-TENSOR, ACCUM_F32, DUO = 0, 3, 4
+TENSOR, ACCUM_F32, DUO, ACCUM_WIDE = 0, 3, 4, 8
+F_DUO, F_WIDE = 4, 4096
 
 
-# sizes at which two workgroups of 128 x 128 tiles per CU are estimated to take longer
+# sizes at which two workgroups of 128 x 128 tiles per CU are estimated to take longer; both are asked for here, so that the test does
+# not hang on the estimates
 @pytest.mark.parametrize("M,N,K,pad", [
     (3841, 4092, 2704, 4),          # 256 tiles; one row in the last row tile, 252 columns in the last column tile
     (4096, 4000, 2992, 0),          # the last column tile 160 columns
@@ -27,15 +29,17 @@ TENSOR, ACCUM_F32, DUO = 0, 3, 4
 def test_ragged_k_on_wide_tiles(cf, dev, M, N, K, pad):
     case(f"wgrad accumulate, wide tiles {M}x{N}x{K} ldc N + {pad}")
     kernel = ctypes.c_int(-1)
-    cf.cf_fp8_gemm_route(M, N, K, 0, 1, TENSOR, ACCUM_F32, N + pad, 0, ctypes.byref(kernel))
-    assert kernel.value == DUO
+    for flag, which in ((F_WIDE, ACCUM_WIDE), (F_DUO, DUO)):
+        cf.cf_fp8_gemm_route(M, N, K, 0, 1, TENSOR, ACCUM_F32, N + pad, flag, ctypes.byref(kernel))
+        assert kernel.value == which
     rng = np.random.default_rng(M + N + K)
     A = orc.quantize_e4m3(orc.bf16_from_f32(rng.standard_normal((M, K), dtype=np.float32)), np.float32(100.0))
     B = orc.quantize_e5m2(orc.bf16_from_f32(rng.standard_normal((N, K), dtype=np.float32)), np.float32(1000.0))
     sa, sb = np.float32([0.01]), np.float32([3e-5])
     C = torch.randn(M, N + pad, device=dev, generator=torch.Generator(device=dev).manual_seed(K)) * 0.01
     held = C.clone()
-    cf.cf_fp8_gemm_tn_accum_f32(M, N, K, dev_arr(A, dev), dev_arr(sa, dev), dev_arr(B, dev), dev_arr(sb, dev), C, N + pad, stream())
+    cf.cf_fp8_gemm_nt_accum_f32_ex(M, N, K, dev_arr(A, dev), K, 0, dev_arr(sa, dev), dev_arr(B, dev), K, 1, dev_arr(sb, dev), C, N + pad, F_WIDE,
+                                   stream())
     assert torch.equal(C[:, N:], held[:, N:])
     rows = np.unique(np.concatenate([np.arange(32), np.arange(M - 32, M), rng.integers(0, M, 32)]))
     at = torch.from_numpy(rows).to(dev)
@@ -45,7 +49,7 @@ def test_ragged_k_on_wide_tiles(cf, dev, M, N, K, pad):
     assert np.all(np.abs(got - want) <= orc.ACC_MFMA * absdot + 2.0 ** -22 * (np.abs(want) + np.abs(before)))
     # every other element: against the 128 x 128 tiles, whose sums differ in their order alone
     other = held.clone()
-    cf.cf_fp8_gemm_nt_accum_f32_ex(M, N, K, dev_arr(A, dev), K, 0, dev_arr(sa, dev), dev_arr(B, dev), K, 1, dev_arr(sb, dev), other, N + pad, 4,
+    cf.cf_fp8_gemm_nt_accum_f32_ex(M, N, K, dev_arr(A, dev), K, 0, dev_arr(sa, dev), dev_arr(B, dev), K, 1, dev_arr(sb, dev), other, N + pad, F_DUO,
                                    stream())
     bound = 2 * orc.ACC_MFMA * float(absdot.max()) * 2 + 2.0 ** -20 * float(C.abs().max())      # (absdot of other rows: at most twice the largest seen)
     assert float((C - other).abs().max()) <= bound
