@@ -1,4 +1,4 @@
-"""Builds libcf_fp8.so (hand-written HIP for gfx950) in-tree with hipcc, and _cf_call.so (Python's way into it) with the host compiler."""
+"""Builds libcf_fp8.so (hand-written HIP for gfx950) in-tree with hipcc, and beside it Python's compiled calls into it with the host compiler."""
 from __future__ import annotations
 
 import importlib.util
@@ -13,8 +13,6 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 INCLUDE = PKG.parent / "include"
 LIB = Path(os.environ.get("CF_LIB_OUT", PKG / "libcf_fp8.so"))
-
-CALL = PKG / "_cf_call.so"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -44,16 +42,17 @@ def build_call(objdir: Path) -> Path:
     spec = importlib.util.spec_from_file_location("cf_native", PKG / "native.py")
     native = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(native)
+    out = native.call_path(LIB)
     names = [n for n, (ret, _) in native.parse_header().items() if ret == "int"]
     (objdir / "call_names.inc").write_text("".join(f"CF_CALL({n})\n" for n in names))
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-missing-field-initializers",
-           f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"), "-o", str(CALL)]
+           f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"), "-o", str(out)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"call.cpp:\n{proc.stderr}")
     if proc.stderr.strip():
         sys.stderr.write(proc.stderr)
-    return CALL
+    return out
 
 
 def build(force: bool = True, extra: list[str] | None = None, jobs: int = 8) -> Path:

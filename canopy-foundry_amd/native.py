@@ -3,9 +3,9 @@
 Every `int cf_*(...)` declared in the header becomes an attribute of `Lib` whose
 call raises `CfError` on a non-zero return (the reference's functions throw where
 the C ABI returns a code).  Pointer arguments accept an int address, None, or any
-object with `data_ptr()` (a torch tensor).  The calls go through _cf_call.so
-(csrc/call.cpp), which hands arguments of any other type to ctypes; `raw_cf_*` are
-the plain ctypes functions.
+object with `data_ptr()` (a torch tensor).  The calls go through a compiled module
+beside the library (csrc/call.cpp), which hands arguments of any other type to
+ctypes; `raw_cf_*` are the plain ctypes functions.
 """
 from __future__ import annotations
 
@@ -13,6 +13,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import re
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -29,6 +30,10 @@ class CfError(RuntimeError):
 def lib_path() -> Path:
     return PKG / "libcf_fp8.so"
 
+
+def call_path(lib: Path) -> Path:
+    """The compiled calls of a library: beside it, for one interpreter's ABI."""
+    return lib.with_name(lib.name.removesuffix(".so") + "_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 _CTYPES = {
@@ -69,8 +74,8 @@ def _conv(v):
     return v
 
 
-def _call_module():
-    path = PKG / "_cf_call.so"
+def _call_module(lib: Path):
+    path = call_path(lib)
     if not path.exists():
         raise RuntimeError(f"{path} is missing: build the library first (python -c 'import __graft_entry__ as g; g.build()')")
     loader = importlib.machinery.ExtensionFileLoader("_cf_call", str(path))
@@ -93,7 +98,7 @@ class Lib:
         import torch  # noqa: F401
         self._dll = ctypes.CDLL(str(path))
         self.decls = parse_header()
-        make = _call_module().make
+        make = _call_module(path).make
         for name, (ret, args) in self.decls.items():
             fn = getattr(self._dll, name)      # raises AttributeError if a declared symbol is not exported
             fn.argtypes = [_ctype(t) for t, _ in args]

@@ -1,7 +1,16 @@
 """The compiled call path takes, refuses and raises what the ctypes path it stands in for does."""
 import ctypes
+import importlib.util
+import os
+import subprocess
+import sys
+import sysconfig
+from pathlib import Path
 
 import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+PKG = ROOT / "canopy-foundry_amd"
 
 
 class Holder:
@@ -36,3 +45,21 @@ def test_floats_sizes_and_outputs(cf):
         with pytest.raises(type(cf)._failed.__globals__["CfError"]):
             cf.cf_fp8_scale_from_amax(None, value, None, None, None)
     assert cf.cf_fp8_quantize_e4m3.__name__ == "cf_fp8_quantize_e4m3"
+
+
+def build_calls(out, **env):
+    """build_call() for a library elsewhere, in a process of its own: the path it returns."""
+    code = ("import importlib.util, pathlib; s = importlib.util.spec_from_file_location('b', %r); b = importlib.util.module_from_spec(s); "
+            "s.loader.exec_module(b); print(b.build_call(pathlib.Path(%r)))" % (str(PKG / "build.py"), str(out)))
+    done = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env={**os.environ, "CF_LIB_OUT": str(out / "libvariant.so"), **env})
+    assert done.returncode == 0, done.stderr
+    return done.stdout.strip(), done.stderr
+
+
+def test_a_variant_has_compiled_calls_of_its_own(tmp_path):
+    before = {p.name: p.stat().st_mtime_ns for p in PKG.glob("*.so")}
+    made, _ = build_calls(tmp_path)
+    assert Path(made).parent == tmp_path and Path(made).exists()
+    assert {p.name: p.stat().st_mtime_ns for p in PKG.glob("*.so")} == before
+    # another interpreter looks for another file
+    assert made.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
