@@ -14,6 +14,7 @@ import importlib.machinery
 import importlib.util
 import re
 import sysconfig
+import warnings
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -75,9 +76,11 @@ def _conv(v):
 
 
 def _call_module(lib: Path):
+    """The compiled calls of a library, or None: every call then goes through ctypes, as any of them can."""
     path = call_path(lib)
     if not path.exists():
-        raise RuntimeError(f"{path} is missing: build the library first (python -c 'import __graft_entry__ as g; g.build()')")
+        warnings.warn(f"{path} is missing: calls go through ctypes, which takes several microseconds more each", RuntimeWarning, stacklevel=3)
+        return None
     loader = importlib.machinery.ExtensionFileLoader("_cf_call", str(path))
     spec = importlib.util.spec_from_file_location("_cf_call", path, loader=loader)
     module = importlib.util.module_from_spec(spec)
@@ -98,13 +101,16 @@ class Lib:
         import torch  # noqa: F401
         self._dll = ctypes.CDLL(str(path))
         self.decls = parse_header()
-        make = _call_module(path).make
+        calls = _call_module(path)
         for name, (ret, args) in self.decls.items():
             fn = getattr(self._dll, name)      # raises AttributeError if a declared symbol is not exported
             fn.argtypes = [_ctype(t) for t, _ in args]
             if ret == "int":
                 fn.restype = ctypes.c_int
-                setattr(self, name, make(name, ctypes.cast(fn, ctypes.c_void_p).value, self._checked(name, fn), self._failed(name)))
+                call = self._checked(name, fn)
+                if calls:
+                    call = calls.make(name, ctypes.cast(fn, ctypes.c_void_p).value, call, self._failed(name))
+                setattr(self, name, call)
             else:
                 fn.restype = ctypes.c_char_p if "char" in ret else None
                 setattr(self, name, fn)

@@ -63,3 +63,29 @@ def test_a_variant_has_compiled_calls_of_its_own(tmp_path):
     assert {p.name: p.stat().st_mtime_ns for p in PKG.glob("*.so")} == before
     # another interpreter looks for another file
     assert made.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def copied_package(tmp_path, header=lambda text: text, calls=True):
+    """The package's binding over a copy of the header, the library linked: the module of native.py."""
+    pkg, include = tmp_path / "pkg", tmp_path / "include"
+    pkg.mkdir()
+    include.mkdir()
+    (include / "cf_fp8.h").write_text(header((ROOT / "include" / "cf_fp8.h").read_text()))
+    (pkg / "native.py").write_text((PKG / "native.py").read_text())
+    for lib in PKG.glob("*.so"):
+        if calls or lib.name == "libcf_fp8.so":
+            (pkg / lib.name).symlink_to(lib)
+    spec = importlib.util.spec_from_file_location("cf_native_copy", pkg / "native.py")
+    native = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(native)
+    return native
+
+
+def test_loads_without_the_compiled_calls(tmp_path):
+    native = copied_package(tmp_path, calls=False)
+    with pytest.warns(RuntimeWarning):
+        lib = native.Lib()
+    assert lib.cf_swiglu_forward(None, None, None, 0, None) is None
+    with pytest.raises(native.CfError):
+        lib.cf_swiglu_forward(None, None, None, 4, None)
+    assert lib.cf_swiglu_forward.__name__ == "cf_swiglu_forward"
