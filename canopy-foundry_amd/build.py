@@ -45,7 +45,7 @@ def build_call(objdir: Path) -> Path:
     out = native.call_path(LIB)
     names = [n for n, (ret, _) in native.parse_header().items() if ret == "int"]
     (objdir / "call_names.inc").write_text("".join(f"CF_CALL({n})\n" for n in names))
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-missing-field-initializers",
+    cmd = [os.environ.get("CXX", "g++"), f'-DCF_HEADER_HASH="{native.header_hash()}"', "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-missing-field-initializers",
            f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"), "-o", str(out)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -170,5 +170,8 @@ PyMODINIT_FUNC PyInit__cf_call() {
     CallableType.tp_clear = clear;
     CallableType.tp_dealloc = dealloc;
     if (PyType_Ready(&CallableType) < 0) return nullptr;
-    return PyModule_Create(&kModule);
+    PyObject* module = PyModule_Create(&kModule);
+    // the text these prototypes came from: the binding goes by what it reads, and uses none of them if that is another
+    if (module && PyModule_AddStringConstant(module, "header", CF_HEADER_HASH) < 0) Py_CLEAR(module);
+    return module;
 }

@@ -10,6 +10,7 @@ ctypes; `raw_cf_*` are the plain ctypes functions.
 from __future__ import annotations
 
 import ctypes
+import hashlib
 import importlib.machinery
 import importlib.util
 import re
@@ -60,6 +61,10 @@ def parse_header(path: Path = HEADER) -> dict[str, tuple[str, list[tuple[str, st
     return out
 
 
+def header_hash() -> str:
+    return hashlib.sha256(HEADER.read_bytes()).hexdigest()
+
+
 def _ctype(tstr: str):
     if "*" in tstr:
         return ctypes.c_void_p
@@ -85,6 +90,9 @@ def _call_module(lib: Path):
     spec = importlib.util.spec_from_file_location("_cf_call", path, loader=loader)
     module = importlib.util.module_from_spec(spec)
     loader.exec_module(module)
+    if getattr(module, "header", None) != header_hash():
+        warnings.warn(f"{path} was built for another {HEADER.name}: calls go through ctypes", RuntimeWarning, stacklevel=3)
+        return None
     return module
 
 

@@ -89,3 +89,14 @@ def test_loads_without_the_compiled_calls(tmp_path):
     with pytest.raises(native.CfError):
         lib.cf_swiglu_forward(None, None, None, 4, None)
     assert lib.cf_swiglu_forward.__name__ == "cf_swiglu_forward"
+
+
+def test_goes_by_the_header_that_is_read(tmp_path):
+    """A prototype that changed since the compiled calls were built, and a function that was not there then."""
+    native = copied_package(tmp_path, lambda text: text.replace("int cf_fp8_scale_from_amax(const float* d_amax, float fp8_max,",
+                                                                "int cf_fp8_scale_from_amax(const float* d_amax, int fp8_max,"))
+    assert native.parse_header()["cf_fp8_scale_from_amax"][1][1] == ("int", "fp8_max")
+    with pytest.warns(RuntimeWarning):
+        lib = native.Lib()
+    with pytest.raises(ctypes.ArgumentError):
+        lib.cf_fp8_scale_from_amax(None, 448.0, None, None, None)
