@@ -37,21 +37,29 @@ def _compile(src: Path, obj: Path, extra: list[str]) -> None:
         sys.stderr.write(err + "\n")
 
 
-def build_call(objdir: Path) -> Path:
-    """Compiles csrc/call.cpp against this interpreter, with the names the header declares."""
+def build_call(objdir: Path) -> Path | None:
+    """Compiles csrc/call.cpp against this interpreter, with the names the header declares.  Where that cannot be done (no host compiler, no
+    Python.h) there is none, not even an earlier one, and the binding uses ctypes: None, with the reason on stderr."""
     spec = importlib.util.spec_from_file_location("cf_native", PKG / "native.py")
     native = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(native)
     out = native.call_path(LIB)
+    out.unlink(missing_ok=True)
     names = [n for n, (ret, _) in native.parse_header().items() if ret == "int"]
     (objdir / "call_names.inc").write_text("".join(f"CF_CALL({n})\n" for n in names))
-    cmd = [os.environ.get("CXX", "g++"), f'-DCF_HEADER_HASH="{native.header_hash()}"', "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-Wno-missing-field-initializers",
-           f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"), "-o", str(out)]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"call.cpp:\n{proc.stderr}")
-    if proc.stderr.strip():
-        sys.stderr.write(proc.stderr)
+    cmd = [os.environ.get("CXX", "g++"), f'-DCF_HEADER_HASH="{native.header_hash()}"', "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+           "-Wno-missing-field-initializers", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{objdir}", str(CSRC / "call.cpp"),
+           "-o", str(out)]
+    try:
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        failed, said = proc.returncode != 0, proc.stderr
+    except OSError as e:
+        failed, said = True, str(e)
+    if failed:
+        sys.stderr.write(f"call.cpp did not compile, calls will go through ctypes:\n{said}\n")
+        return None
+    if said.strip():
+        sys.stderr.write(said)
     return out
 
 

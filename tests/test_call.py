@@ -100,3 +100,12 @@ def test_goes_by_the_header_that_is_read(tmp_path):
         lib = native.Lib()
     with pytest.raises(ctypes.ArgumentError):
         lib.cf_fp8_scale_from_amax(None, 448.0, None, None, None)
+
+
+def test_a_build_without_a_host_compiler_has_none(tmp_path):
+    earlier, _ = build_calls(tmp_path)
+    made, said = build_calls(tmp_path, CXX=str(tmp_path / "no-such-compiler"))
+    assert made == "None" and "no-such-compiler" in said and not Path(earlier).exists()
+    (tmp_path / "fails").write_text("#!/bin/sh\necho Python.h: not found >&2\nexit 1\n")
+    (tmp_path / "fails").chmod(0o755)
+    assert build_calls(tmp_path, CXX=str(tmp_path / "fails"))[0] == "None"
