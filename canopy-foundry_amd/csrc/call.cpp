@@ -31,7 +31,7 @@ struct Callable {
     PyObject* name;
 };
 
-// false: not plainly of the parameter's type (no exception left behind)
+// false: not plainly of the parameter's type, or data_ptr() raised (what it raised is then set)
 template <class T>
 bool convert(PyObject* o, T& out) {
     if constexpr (std::is_pointer_v<T>) {
@@ -45,7 +45,7 @@ bool convert(PyObject* o, T& out) {
         }
         PyObject* r = PyObject_VectorcallMethod(g_data_ptr, &o, 1 | PY_VECTORCALL_ARGUMENTS_OFFSET, nullptr);
         if (!r) {
-            PyErr_Clear();
+            if (PyErr_ExceptionMatches(PyExc_AttributeError)) PyErr_Clear();       // no such method: not a tensor
             return false;
         }
         const bool ok = PyLong_CheckExact(r);
@@ -79,7 +79,7 @@ struct Thunk<int (*)(A...)> {
         std::tuple<A...> v;
         if (names || PyVectorcall_NARGS(nargsf) != static_cast<Py_ssize_t>(sizeof...(A)) ||
             !convert_all(args, v, std::index_sequence_for<A...>{}))
-            return PyObject_Vectorcall(c->fallback, args, nargsf, names);
+            return PyErr_Occurred() ? nullptr : PyObject_Vectorcall(c->fallback, args, nargsf, names);
         int rc;
         auto fn = reinterpret_cast<int (*)(A...)>(c->fn);
         Py_BEGIN_ALLOW_THREADS

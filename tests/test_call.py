@@ -109,3 +109,21 @@ def test_a_build_without_a_host_compiler_has_none(tmp_path):
     (tmp_path / "fails").write_text("#!/bin/sh\necho Python.h: not found >&2\nexit 1\n")
     (tmp_path / "fails").chmod(0o755)
     assert build_calls(tmp_path, CXX=str(tmp_path / "fails"))[0] == "None"
+
+
+@pytest.mark.parametrize("error", [KeyboardInterrupt, RuntimeError, MemoryError])
+def test_what_data_ptr_raises_is_raised(cf, error):
+    class Once:
+        """Raises the first time it is asked (an interrupt that arrives there), and would answer the second."""
+        asked = 0
+
+        def data_ptr(self):
+            self.asked += 1
+            if self.asked == 1:
+                raise error
+            return 0
+
+    once = Once()
+    with pytest.raises(error):
+        cf.cf_swiglu_forward(None, once, None, 0, None)
+    assert once.asked == 1
