@@ -526,14 +526,16 @@ bool block_wide_ok(const GemmArgs& p) {
            aligned16(p.C);
 }
 
-// Microseconds: 1.12 a K-tile and 6 a tile beside the 0.65 and 6 of k_gemm_nt_block_ring's 128 x 256 tiles.  4096 columns or more in whole rounds:
-// 186 against 210 (4096 x 7168 x 7168), 61 against 68 (4096^3), 93 against 104 (2048 x 7168 x 7168).  Where the large tiles leave a round
-// nearly empty or half of the CUs without one the small ones stay: 169 against 154 (2560 x 7168 x 7168, 1.1 rounds and 2.2), 78 against 60
-// (4096 x 2048 x 7168, half a round and one).  Of 80 sizes from 211 to 15044 rows none came out slower than before by more than two runs differ.
+// Microseconds: 1.12 a K-tile and 10 a tile beside the 0.65 and 6 of k_gemm_nt_block_ring's 128 x 256 tiles.  Whole rounds: 186 against 210 (4096 x 7168
+// x 7168), 61 against 68 (4096^3), 93 against 104 (2048 x 7168 x 7168).  Where the large tiles leave a round nearly empty or half of the CUs
+// without one the small ones stay: 169 against 154 (2560 x 7168 x 7168, 1.1 rounds and 2.2), 78 against 60 (4096 x 2048 x 7168, half a round and one).
+// With few K-tiles the fixed part decides.  At 6 these went to the large ones: 3000 x 7168 x 2048 54.5 against 48.2, 2892 x 11008 x 640 34.9 and 27.7,
+// 3644 x 5888 x 1536 44.1 and 38.4; 3500 x 7168 x 2048 still does, 54.2 against 63.0.  Of 1400 sizes (K 384 to 9000) 44 of 900 were slower than before these
+// kernels by more than 3 %, the worst 1.19 times; now 3 of 500 are, all with K 512 to 768.
 float block_wide_estimate_us(const GemmArgs& p) {
     const long long tiles = static_cast<long long>((p.M + BM - 1) / BM) * (p.N / BN);
     const int cus = num_cus();
-    return static_cast<float>((tiles + cus - 1) / cus) * (static_cast<float>(p.K / BK) * 1.12f + 6.0f);
+    return static_cast<float>((tiles + cus - 1) / cus) * (static_cast<float>(p.K / BK) * 1.12f + 10.0f);
 }
 
 int gemm_nt_block_wide(GemmArgs p, hipStream_t st) {

@@ -76,6 +76,9 @@ def test_accumulating_kernel(cf, M, N, K, pad, epi, kernel):
     (1000, 512, 4096, (SMALL + 1, SMALL + 2)),       # 11.7, 12.1, 13.7, 28.6
     (4096, 7168, 7168, (BLOCK_WIDE,)),               # 210, 186
     (2560, 7168, 7168, (RING,)),                     # 154, 256 x 256 tiles 169: 1.1 rounds of those
+    (3000, 7168, 2048, (RING,)),                     # 48.2, 256 x 256 tiles 54.5: few K-tiles
+    (3500, 7168, 2048, (BLOCK_WIDE,)),               # 63.0, 54.2
+    (2892, 11008, 640, (RING,)),                     # 27.7, 34.9
     (512, 7168, 7168, (BLOCK_SLIM,)),                # with the quantize 59.7, 43.3
     (700, 7168, 7168, (RING,)),                      # with the quantize 61.1, 128 x 128 tiles 70.7
 ])
