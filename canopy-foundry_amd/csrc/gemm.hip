@@ -2545,9 +2545,10 @@ int cf::grouped_gemm_nt_bf16(int total_rows, int N, int K, int num_experts, cons
     // (50 rows each) 72 -> 45 us, 256 72 -> 50, 600 74 -> 63, 1000 77 -> 71.  64 experts of 2048 x 1408 fill the chip with ring tiles and keep them
     // (600 tokens 193, with passes 221).
     else if (total_rows <= static_cast<long long>(BM) * num_experts) {
+        const bool gate = epilogue == EPI_SILU_GATE;
         int shape = 0;
-        const float direct = grouped_direct_many_estimate_us(total_rows, N, K, num_experts, epilogue == EPI_SILU_GATE, &shape);
-        if (direct < ring_estimate_us(num_experts * BM, N, K, BM, out_bn, 0.95f, 6.0f)) {
+        const float direct = grouped_direct_many_estimate_us(total_rows, N, K, num_experts, gate, &shape);
+        if (direct < ring_estimate_us(num_experts * BM, N, K, BM, out_bn, gate ? 0.88f : 0.89f, gate ? 8.3f : 6.1f)) {
             GemmArgs q = p;
             q.tiles_m *= std::min(4, (total_rows + 64 * num_experts - 1) / (64 * num_experts) + 1);
             const int rc = grouped_gemm_nt_direct(q, a_is_e5m2, epilogue, shape, st);

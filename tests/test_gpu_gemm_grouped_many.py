@@ -53,3 +53,43 @@ def test_grouped_passes(cf, dev, counts, gate):
             assert np.sqrt(((mine - exact) ** 2).sum() / (exact ** 2).sum()) <= 4e-3, e
         else:
             orc.assert_gemm_close(mine, ref, absdot, what=f"expert {e}")
+
+
+RING, PASSES = 32, 64 | 3 << 8          # flags of the dense form: the persistent kernel, the small tiles of 64 x 64
+
+
+# times with passes and on the ring kernel
+@pytest.mark.parametrize("E,N,K,per,kernel", [
+    (24, 640, 5376, 186, RING),          # 77.6, 50.5: three passes an expert, and the first XCDs have most of them
+    (32, 256, 4864, 239, RING),          # 59.3, 45.6
+    (8, 1024, 2048, 64, PASSES),         # 10.1, 25.3
+    (8, 1024, 2048, 250, PASSES),        # 19.9, 25.5
+])
+def test_which_kernel_takes_the_experts(cf, dev, E, N, K, per, kernel):
+    """The two sum K in different orders, which shows where values of every exponent meet: an expert's rows have the bits of the dense product
+    on the kernel that the grouped one took, and not all of the other one's."""
+    case(f"grouped gemm, kernel of {E} experts {N}x{K} rows {per}")
+    g = torch.Generator(device=dev).manual_seed(E + N)
+
+    def fp8(*shape):
+        t = torch.randint(0, 256, shape, dtype=torch.uint8, device=dev, generator=g)
+        return torch.where((t & 0x7f) == 0x7f, 0x3c, t)
+
+    total = E * per
+    A, B = fp8(total, K), fp8(E, N, K)
+    sa, sb = torch.rand(total, device=dev, generator=g) + 0.5, torch.rand(E, N, device=dev, generator=g) + 0.5
+    counts = torch.full((E,), per, dtype=torch.int32, device=dev)
+    offsets = torch.arange(E, dtype=torch.int32, device=dev) * per
+    sz = ctypes.c_size_t(0)
+    assert cf.raw_cf_fp8_grouped_gemm_workspace_bytes(total, E, ctypes.byref(sz)) == 0
+    ws = torch.empty(sz.value, dtype=torch.uint8, device=dev)
+    C = torch.empty((total, N), dtype=torch.bfloat16, device=dev)
+    cf.cf_fp8_grouped_gemm_nt_bf16_ex(total, N, K, E, counts, offsets, A, total, K, None, sa, B, sb, ROW_COL, EPI_NONE, None, None, C, N, ws,
+                                      sz.value, stream())
+    for flag in (RING, PASSES):
+        D = torch.empty_like(C)
+        for e in range(E):
+            rows = slice(e * per, (e + 1) * per)
+            cf.cf_fp8_gemm_nt_bf16_ex(per, N, K, A[rows], K, 0, sa[rows].clone(), B[e], K, sb[e], ROW_COL, EPI_NONE, None, None, None, D[rows], N,
+                                      flag, stream())
+        assert torch.equal(C.view(torch.int16), D.view(torch.int16)) == (flag == kernel)
