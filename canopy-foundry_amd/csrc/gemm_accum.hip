@@ -275,15 +275,15 @@ bool accum_wide_ok(const GemmArgs& p, int fmt, int epi, int scale_mode) {
            p.ldc < (1 << 23) && static_cast<size_t>(p.M) * p.lda < (1ull << 31) && static_cast<size_t>(p.N) * p.ldb < (1ull << 31);
 }
 
-// Microseconds: per round of tiles 1.42 a K-tile and, for C, 21; 26 where a few whole rounds leave no workgroup to start later, 34 where there is
-// one round and all go to C at once, 39 where the rows of C do not begin at lines.  Beside the two workgroups per CU (them, this), a line
-// on each side: 14336 x 4096, K 1040 123 and 120 alone, K 1488 152 and 144; 14336 x 4100, K 1488 209 and 222, K 2000 241 and 237; 5632 x 2048 (one round,
-// part filled), K 4016 70.7 and 66.4 alone but no difference within a step, K 8176 121 and 110; 5120 x 4096 (a quarter of the second round
-// filled), K 8176 198 and 210.
+// Microseconds: per round of tiles 1.42 a K-tile and, for C, 21; 26 where a few rounds, the last of them more than four fifths full, leave hardly a workgroup to
+// start later, 34 where there is one round and all go to C at once, 39 where the rows of C do not begin at lines.  Beside the two workgroups per CU (them,
+// this), a line on each side: 14336 x 4096, K 1040 123 and 120 alone, K 1488 152 and 144; 14336 x 4100, K 1488 209 and 222, K 2000 241 and 237; 10620 x 3072, K
+// 800 64.4 and 70.7 (504 tiles); 5632 x 2048 (one round, part filled), K 4016 70.7 and 66.4 alone but no difference within a step, K 8176 121 and 110; 5120 x 4096
+// (a quarter of the second round filled), K 8176 198 and 210.  Of 453 random sizes that come here 14 are slower by more than 3 %, the worst 1.06 times (K 800 to 1350).
 float accum_wide_estimate_us(const GemmArgs& p) {
     const int most = num_cus();
     const long long tiles = static_cast<long long>((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN), rounds = (tiles + most - 1) / most;
-    const float c = c_lines_shared(p, 4) ? 39.0f : rounds == 1 ? 34.0f : tiles % most == 0 && rounds < kManyTiles ? 26.0f : 21.0f;
+    const float c = c_lines_shared(p, 4) ? 39.0f : rounds == 1 ? 34.0f : 5 * (rounds * most - tiles) < most && rounds < kManyTiles ? 26.0f : 21.0f;
     return static_cast<float>(rounds) * (static_cast<float>((p.K + BK - 1) / BK) * 1.42f + c);
 }
 

@@ -58,6 +58,9 @@ def test_estimates_ask_what_the_launch_asks(cf):
     (14336, 4096, 2000, 0, ACCUM_F32, ACCUM_WIDE),   # 262, 188 and, on 256 x 256 tiles, 164: K no multiple of 128
     (14336, 4096, 512 + 16, 0, ACCUM_F32, DUO),      # few K-tiles
     (14336, 4100, 1488, 0, ACCUM_F32, DUO),          # 209, 256 x 256 tiles 222: rows of C off the lines
+    (10620, 3072, 800, 0, ACCUM_F32, DUO),           # 64.4, 70.7: two rounds, nearly full
+    (10023, 4864, 928, 0, ACCUM_F32, DUO),           # 98.6, 104.8: three
+    (14336, 4096, 1488, 0, ACCUM_F32, ACCUM_WIDE),   # 152, 144: three and a half
     (5120, 4096, 8176, 0, ACCUM_F32, DUO),           # 198, 210: a quarter of the second round filled
     (14336, 4096, 8192, 0, ACCUM_F32, RING),         # 389, 431
 ])
