@@ -1,7 +1,8 @@
 // Python calls into libcf_fp8.so without ctypes: one callable per declared function, its arguments converted by templates over
 // the header's own prototypes.  A pass over a small layer is bound by its host calls; through ctypes and a Python loop over the
-// arguments a GEMM's nineteen took 4.7 us beside a launch of about two, here 0.8 (an FP8 linear layer, four calls and five launches: 23.9 -> 21.5 us
-// at 512 x 1024 x 1024, where the GPU takes over, 23.1 -> 17.8 at a smaller one).
+// arguments a GEMM's nineteen took 4.7 us beside a launch of about two, here 0.8.  An FP8 linear layer, four calls and five launches: 512 x 1024 x 1024,
+// where the GPU takes over, 23.2 to 25.7 -> 18.8 to 21.2 us in five pairs of runs (two runs of one side differ by 3 to 24 %); smaller passes that the
+// host bounds 24.4 -> 20.1 and 13.2 -> 11.4 (within 2 %).
 //
 // A pointer is None, an int or an object with data_ptr() (a torch tensor).  Whatever is not plainly one of the types a parameter
 // takes, and any other number of arguments, goes to the ctypes callable that each of these carries, which converts it or raises.

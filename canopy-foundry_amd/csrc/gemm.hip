@@ -795,9 +795,10 @@ void k_gemm_nt_ring(const GemmArgs p) {
     if (my_tiles <= 0) return;        // grouped launches size the grid by an upper bound of the tile count
     const int ktiles = p.K / BK;      // >= 2, checked by the launcher
     // The accumulating forms: all workgroups take the same time to a tile, and would read and write C all at once with the matrix cores idle
-    // and leave memory idle in between.  Where some have a tile fewer than others, those start half a tile late (0.7 us a K-tile; they are
-    // done before the others still), so that the two groups' turns at C fall apart.  The backward of a 14336 x 4096 projection (896 tiles:
-    // 128 workgroups with four, 128 with three): 4096 tokens 544 -> 522 us, 6144 731 -> 716, 8192 909 -> 898.
+    // and leave memory idle in between.  Where some have a tile fewer than others, those start late, by 0.7 us a K-tile (two fifths of a tile at K
+    // 4096, two thirds at the longest K; they are done before the others still), so that the two groups' turns at C fall apart.  The backward of
+    // a 14336 x 4096 projection (896 tiles: 128 workgroups with four, 128 with three), without and with it in turn: 3072 tokens 457 -> 438 us, 4096 564 ->
+    // 544, 6144 758 -> 743, 8192 940 -> 930 (the last by less than cards differ); the product alone, K 4096 245 -> 228, 8192 396 -> 390.
     if constexpr (EPI == EPI_ACCUM_F32 || EPI == EPI_ACCUM_BF16) {
         if (my_tiles * static_cast<int>(gridDim.x) < total_tiles)
             for (int i = 0; i < ktiles; ++i) __builtin_amdgcn_s_sleep(23);
@@ -2144,7 +2145,8 @@ __global__ __launch_bounds__(256) void k_bank_backward_setup(const BackwardSetup
 
 // What the kernels of this file take for a dense problem, in microseconds: tiles in rounds over the CUs, so much per K-tile and
 // so much per tile.  Measured with a tile on every CU: 256 x 256 tiles 0.95 a K-tile (the
-// register-staged kernel 2.3), 128 x 256 block-scaled tiles 0.65 (1.5).  (At the power limit all of them slow down together.)
+// register-staged kernel 2.3), 128 x 256 block-scaled tiles 0.65 (1.5).  (At the power limit all of them slow down together: many rounds of grouped
+// tiles take 1.31 a K-tile and 8.9 a tile, 16384 tokens, 6 of 64 experts, 2048 x 1408: gate/up 537 us in 18 rounds of 16 K-tiles, down 303 in 13 of 11.)
 float ring_estimate_us(int M, int N, int K, int bm, int out_bn, float per_ktile, float per_tile) {
     const long long tiles = static_cast<long long>((M + bm - 1) / bm) * ((N + out_bn - 1) / out_bn);
     const int cus = num_cus();

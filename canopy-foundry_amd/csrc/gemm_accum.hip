@@ -57,10 +57,12 @@ void k_gemm_nt_accum_wide(const GemmArgs p) {
         lin0 = blockIdx.x;
     }
     if (my_tiles <= 0) return;
-    // Turns at memory: the workgroups start in eight groups within about the time that C takes (24 K-tiles; one takes 1 us), which costs the last group
-    // that much once, so over many tiles each, or a few of few K-tiles.  Over few otherwise, those with a tile fewer start a tile's MFMAs late and
-    // still end before the others.  In step, the second and the first: 14336 x 4096 (four tiles or three) K 2000 179, 164, 159 us, within a step 376, 367,
-    // 354; K 4016 there 645, 595, 600.  28672 x 8192 (14 tiles), K 2000: 634, 571 in eight groups.  8192 x 8192 (four whole rounds), K 2000: 197, 171.
+    // Turns at memory: the workgroups start in eight groups within about the time that C takes (24 us; `late` counts in us, a K-tile takes 1.42), which
+    // costs the last group that much once, so over many tiles each, or a few of few K-tiles.  Over few otherwise, those with a tile fewer start late by
+    // 1 us a K-tile and still end before the others.  In step, the second and the first: 14336 x 4096 (four tiles or three) K 2000 179, 164, 159 us, within
+    // a step 376, 367, 354; K 4016 there 645, 595, 600.  28672 x 8192 (14 tiles), K 2000: 634, 571 in eight groups.  8192 x 8192 (four whole rounds), K 2000:
+    // 197, 171.  The line at 20 K-tiles, within a step, second and first: 14336 x 4096 K 2000 382 and 367, 2512 452 and 441, 2768 470 and 463, 3024 489 and 485,
+    // 3536 567 and 572; 12288 x 4096 K 2512 362 and 355, 3536 461 and 462; 11008 x 5120 (3.4 rounds) K 2000 388 and 392, 2512 and 3024 the same.
     int late = 0;
     if (total_tiles >= kManyTiles * static_cast<int>(gridDim.x)) late = min(ktiles, 24) * static_cast<int>(blockIdx.x / 8 % 8) / 8;
     else if (ktiles <= 20 && total_tiles >= 3 * static_cast<int>(gridDim.x)) late = ktiles * 3 * static_cast<int>(blockIdx.x / 8 % 8) / 16;

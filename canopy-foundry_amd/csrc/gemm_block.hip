@@ -7,8 +7,8 @@
 // v_mfma_f32_16x16x128 one MFMA is a whole scale group of a 16 x 16 block, its four registers are folded three MFMAs later, and
 // the tile is 64 x 128 (sums 128 registers, activations 32, weights 2 x 16, partial products 16 of the 256 that two wavefronts per SIMD have).
 // A workgroup's 256 x 256 tile takes two thirds of the L2-to-LDS bytes per FLOP of the 128 x 256 tile of k_gemm_nt_block_ring, three
-// quarters of its LDS reads and half of its barriers.  4096 x 7168 x 7168, random operands: 210 -> 186 us (2.26 PFLOP/s), 242 -> 203 on
-// a slower card; 1.75 rounds of tiles, so 87.5 % at best.
+// quarters of its LDS reads and half of its barriers.  4096 x 7168 x 7168, quantized normal operands: 210 -> 186 us (2.26 PFLOP/s) on one pair of
+// operands over and over, 243 -> 199 on eight pairs in turn, so from memory (202 in a profile of the quantize and it); 1.75 rounds of tiles, so 87.5 % at best.
 //
 // LDS: two stages of 64 KiB.  A K-tile is 32 MFMAs per wavefront in four groups of eight (two weight blocks x four activation blocks).
 // The weights of the next group are read under the current one; before the last group every wavefront has the rest of the K-tile in

@@ -58,12 +58,12 @@ __device__ __forceinline__ void opaque_words(const uint4& v, uint32_t (&w)[4]) {
     asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
 }
 
-// Row in registers: V % 8 == 0, V <= 128 T, 16-byte aligned rows (8-byte for the fp8 gradient).  T lanes per row: 256
+// Row in registers: V % 8 == 0, V <= 8 CHUNKS T, 16-byte aligned rows (8-byte for the fp8 gradient).  T lanes per row: 256
 // for rows up to 32768 logits, 1024 (a CU's sixteen wavefronts, 128 registers each) for rows up to 131072, so that a
 // 128k vocabulary is still read from memory once.
 // CHUNKS: 8-element chunks per lane.  With sixteen a wide workgroup fills its CU's registers and its phases (load, maximum, sum, gradient)
-// run one after the other with nothing to overlap them; with seven, 64 registers in all, a second one's loads and stores run under
-// them: 2048 x 50304, 142 -> 110 us (4.7 TB/s).
+// run one after the other with nothing to overlap them; with seven it gets by on 64 and one spilled (8 bytes of scratch a lane), and a second one's loads
+// and stores run under them: 2048 x 50304, 142 -> 110 us (4.7 TB/s); 1 to 256 rows, a workgroup per CU at most, as before.
 template <bool QUANT, int T, int CHUNKS>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(CHUNKS == kCeFewChunks ? 8 : 4)))
 void k_ce_rows(const CeArgs p) {

@@ -920,8 +920,8 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma(const ui
 // What bounds it is how fast a CU gets the weights into the MFMAs' layout: there, 16 neighbouring lanes hold 16 rows, and a
 // load so addressed touches a line per lane (25 bytes a nanosecond and CU).  So weights are fetched as runs of 64 or 128
 // bytes of a row by neighbouring lanes and turned in 4 KiB of LDS per wavefront; the sums go to `mixed` as whole rows.
-// 2048 tokens, 6 of 64 experts, 2048 x 1408: 620 -> 375 us (the swaps alone 160 us of the former); 64 tokens 280 -> 187.
-// What then bounds it is neither memory (with every fetch from one line 329 us) nor the matrix cores (busy 28 % of the time) but the
+// 2048 tokens, 6 of 64 experts, 2048 x 1408: 620 -> 375 us (the swaps alone 160 us of the former); 64 tokens 280 -> 187; with the fetches of all phases
+// in one stream 353 and 178 (H = 128, one step of a ring of four, pays 3 % for the zeros: 24.0 -> 24.7 us).  What then bounds it is neither memory (with every fetch from one line 329 us) nor the matrix cores (busy 28 % of the time) but the
 // chains of LDS writes, reads and MFMAs of two wavefronts per SIMD; fc_in takes 55 us of a workgroup's 170, fc_out 105.
 constexpr int kWideRows = 32;
 constexpr int kWideBlocks = 16;
@@ -963,7 +963,6 @@ __global__ __launch_bounds__(kMfmaThreads) void k_grouped_gelu_fp8_mfma32(const 
     if (first >= n_active) return;
     const int n_rows = min(kWideRows, n_active - first);
     const int* my_rows = row_indices + static_cast<size_t>(e) * rows + first;
-    // the expert's weights through descriptors: a fetch's address is one lane offset and one scalar (H Ie < 2^31, checked by the launcher)
     const uint8_t* w_in = fc_in_w + static_cast<size_t>(e) * H * Ie;
     const uint8_t* w_out = fc_out_w + static_cast<size_t>(e) * Ie * H;
     const int w_bytes = H * Ie;                 // below 2^31, checked by the launcher
