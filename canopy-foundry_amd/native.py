@@ -117,7 +117,7 @@ class Lib:
                 fn.restype = ctypes.c_int
                 call = self._checked(name, fn)
                 if calls:
-                    call = calls.make(name, ctypes.cast(fn, ctypes.c_void_p).value, call, self._failed(name))
+                    call = calls.make(name, ctypes.cast(fn, ctypes.c_void_p).value, call, self._failed(name)) or call
                 setattr(self, name, call)
             else:
                 fn.restype = ctypes.c_char_p if "char" in ret else None

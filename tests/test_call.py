@@ -127,3 +127,16 @@ def test_what_data_ptr_raises_is_raised(cf, error):
     with pytest.raises(error):
         cf.cf_swiglu_forward(None, once, None, 0, None)
     assert once.asked == 1
+
+
+def test_a_function_the_compiled_calls_do_not_know(tmp_path, monkeypatch):
+    native = copied_package(tmp_path)
+
+    class Calls:
+        @staticmethod
+        def make(name, address, fallback, failed):
+            return None
+
+    monkeypatch.setattr(native, "_call_module", lambda lib: Calls)
+    with pytest.raises(native.CfError):
+        native.Lib().cf_swiglu_forward(None, None, None, 4, None)
